@@ -7,13 +7,14 @@
 // interior system A_II (mass, interior convection, outflow faces, in-cell
 // scattering and any self-coupling link), identity on inflow-boundary DOFs.
 //
-// Build: one workgroup per cell assembles the block from its structure
-// (per-node angular scattering blocks, the diagonal, the x/y derivative
-// lines) in LDS (or in a global scratch block when it does not fit), inverts
-// it by Gauss-Jordan with partial pivoting (column-parallel elimination, one
-// pivot search per wavefront-shuffle reduction), and stores the inverse
-// column-major so the apply is a coalesced batched GEMV.
+// Build: one workgroup per block assembles it from its structure (per-node
+// angular scattering blocks, the diagonal, the x/y derivative lines), inverts
+// it by Gauss-Jordan with partial pivoting (blocked, in registers with matrix
+// instructions, for blocks of up to 128 DOFs; in LDS or a global scratch block
+// otherwise), and stores the inverse column-major so the apply is a coalesced
+// batched GEMV.
 #include <algorithm>
+#include <type_traits>
 
 #include "rtx_internal.h"
 
@@ -244,18 +245,7 @@ __global__ __launch_bounds__(BJ_THREADS) void k_bj_build(DevMesh m, int restrict
         for (int row = tid; row < n; row += BJ_THREADS) o[size_t(col) * n + row] = A[size_t(row) * n + col];
 }
 
-// ---- register-resident build for blocks of up to 16 RR DOFs.
-//
-// The block is distributed cyclically over a 16 x TJ thread grid (thread
-// (ti, tj) holds rows ti + 16 u, u < RR, and columns tj + TJ v, v < CC; 16 RR
-// = TJ CC), each entry evaluated directly from the operator's structure
-// (same terms, same summation order as bj_assemble).  Inversion is
-// Gauss-Jordan with partial pivoting done as a sequence of sweeps on the
-// pivot entries (p_k, k) without moving rows: only the pivot column and the
-// pivot row pass through LDS, so a workgroup needs about 3 KB of LDS
-// instead of n^2 doubles and several cells run per CU.  After all sweeps
-// the register matrix M holds the inverse with permuted indices:
-// inv[q_i][p_j] = M[i][j], q = p^-1.
+// ---- register-resident build for blocks of up to 128 DOFs.
 struct BJCell {
     int nx, ny, nth, n, nyt, ao, na, quad, bd;
     double dx, dy, dth;
@@ -319,32 +309,195 @@ __device__ inline double bj_entry(const DevMesh &m, const BJCell &x, const BJSel
 }
 
 // One workgroup per block, the block's index from the size-class list bl
-// (blocks of at most 16 RR DOFs).  T: the elimination's arithmetic and the
-// inverse's storage (FP64, or FP32 for the reduced-precision copies alone;
-// the entries are assembled in FP64 either way).
-template <int RR, int CC, int TJ, typename T = double>
-__global__ __launch_bounds__(16 * TJ)
-__attribute__((amdgpu_waves_per_eu(TJ == 24 ? 5 : (TJ == 32 && sizeof(T) == 4 ? 6 : 1))))
-void k_bj_build_reg(DevMesh m, int restrict_,
-                                                         const int64_t *inv_off,
-                                                         const int32_t *__restrict__ blk,
-                                                         const int32_t *__restrict__ bl,
-                                                         T *__restrict__ out,
-                                                         int *__restrict__ status) {
-    constexpr int NR = 16 * RR;
-    static_assert(NR == TJ * CC, "square register tiles");
-    static_assert(NR <= 128, "pivot rows fit the key's 7 low bits");
-    __shared__ double cth[NMq], sth[NMq];
-    __shared__ T colk[2][NR];
-    __shared__ T prow[NR];
-    // pivot key of each step (double-buffered): the bits of |value| with the
-    // low 7 mantissa bits replaced by 127 - row, so the largest key is the
-    // largest value (to 45 mantissa bits), the lowest row among ties
-    __shared__ unsigned long long red_key[2];
-    __shared__ int perm[NR], qinv[NR];
-    __shared__ int used[NR];
+// (blocks of 16 (NT - 1) + 1 .. 16 NT DOFs).  T: the elimination's arithmetic
+// and the inverse's storage (FP64, or FP32 for the reduced-precision copies
+// alone; the entries are assembled in FP64 either way).
+//
+// Blocked Gauss-Jordan on M = (block)^T, in registers.  Wave w holds columns
+// 16 w .. 16 w + 15 of M in the accumulator layout of the 16 x 16 matrix
+// instruction.  The columns are eliminated in panels of 16, panel k by wave k
+// alone: it turns its tile to one row (two for NT > 4) per lane through LDS,
+// sweeps its 16 columns with partial pivoting (wavefront maximum by DPP, the
+// pivot row broadcast by readlane, no block barrier), and leaves the swept
+// panel W in LDS.  After the sweeps every other column c is
+//     M[:, c] <- M[:, c] with the panel's pivot rows zeroed + W M_P[:, c],
+// M_P the 16 pivot rows before the panel: four matrix instructions per 16 x
+// 16 tile.  Rows are never moved: with p_k the pivot row of column k and q =
+// p^-1, inv(M)[q_i][p_j] is what M[i][j] ends as, so inv(block)[p_j][q_i],
+// and a tile's 16 lanes store runs of one column of the inverse.
+//
+// Bound by the panels (half of the FP64 time: pivot search, broadcast and
+// division in series) and the matrix instructions.  A rank-1 form with two
+// block barriers per column and five instructions per element and column
+// took 14.6 ms for 16,384 blocks of 125 in FP64 (this: 3.5, the FP64 rate's
+// floor 0.9) and 31.3 ms for the 91,352 blocks of an hp mesh of 8.3 M DOF in
+// FP32 (this: 7.6).  One barrier per panel is left; the next panel's wave
+// starts as soon as its own tile is updated (W is double-buffered), at raised
+// priority because the panels are the serial chain.  Registers: two blocks of
+// eight waves per CU in FP64 (128 VGPRs); in FP32 four (64 VGPRs with a few
+// spills: 16,384 blocks of 125 in 1.83 ms, against 2.0 at 80 VGPRs and 2.5
+// without a limit).
+template <int NT, typename T>
+struct BJReg {
+    static constexpr int NR = 16 * NT;
+    static constexpr int WS = 18;                 // row stride of W: lane rows and operand
+                                                  // reads both spread over the banks
+    static constexpr int SS = NR + 2;             // row stride of the assembly strip
+    static constexpr int H = NT > 4 ? 2 : 1;      // rows per lane of a panel
+    static_assert(32 * SS <= 2 * NR * WS, "a 32-row strip fits the panel buffers");
+};
+
+__device__ inline uint32_t bj_key(double v) {
+    return static_cast<uint32_t>(__double2hiint(v)) & 0x7fffff80u;
+}
+__device__ inline uint32_t bj_key(float v) { return __float_as_uint(v) & 0x7fffff80u; }
+// keys of infinities and NaN start here
+template <typename T>
+__device__ constexpr uint32_t bj_key_inf() { return sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u; }
+
+__device__ inline double bj_lane(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+__device__ inline float bj_lane(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// Largest value over the wavefront, in every lane's scalar view.
+__device__ inline uint32_t bj_wave_max(uint32_t v) {
+    auto step = [&](uint32_t o) { v = o > v ? o : v; };
+    step(uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x111, 0xf, 0xf, false)));   // row_shr:1
+    step(uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x112, 0xf, 0xf, false)));   // row_shr:2
+    step(uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x114, 0xf, 0xf, false)));   // row_shr:4
+    step(uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x118, 0xf, 0xf, false)));   // row_shr:8
+    step(uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x142, 0xf, 0xf, false)));   // row_bcast:15
+    step(uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x143, 0xf, 0xf, false)));   // row_bcast:31
+    return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+}
+
+template <typename T> struct BJMma;
+template <> struct BJMma<double> {
+    typedef double v4 __attribute__((ext_vector_type(4)));
+    __device__ static v4 step(double a, double b, v4 c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    // row of accumulator v in lane group lg, and its inverse: row r is entry
+    // (r >> 4) 4 + v of lane group lg
+    __device__ static int row(int lg, int v) { return lg + 4 * v; }
+    __device__ static int slot(int r) { return (r & 3) * 32 + (r >> 2); }
+};
+template <> struct BJMma<float> {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    __device__ static v4 step(float a, float b, v4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ static int row(int lg, int v) { return 4 * lg + v; }
+    __device__ static int slot(int r) { return ((r >> 2) & 3) * 32 + (r >> 4) * 4 + (r & 3); }
+};
+
+// A wave's own LDS writes made visible to its other lanes.
+__device__ inline void bj_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sweep the 16 columns of a panel held one row (H rows, 64 apart) per lane.
+// q: byte table of the step that each row was pivot of (BJMma::slot order);
+// perm: pivot row of each step.  False on a zero or non-finite pivot (the
+// same for every lane; what the panel holds then is void).
+template <int H, typename T>
+__device__ __forceinline__ bool bj_panel(T (&P0)[16], T (&P1)[16], int k0, int lane, bool used0,
+                                         bool used1, uint8_t *q, int32_t *perm) {
+    bool bad = false;
+    // In-place Gauss-Jordan with the pivot rows' division left to the end: a
+    // step adds -c_r / p times the pivot row to every other row (the pivot
+    // row's factor is 0) and puts -c_r / p (1 in the pivot row) in its
+    // column; the panel's pivot rows are divided by their pivots at the end.
+    // Nothing but the FMAs touches a whole row, and the pivot row's values
+    // are scalar operands of them.
+    T s0 = T(1), s1 = T(1);
+    int step0 = -1, step1 = -1;          // steps that this lane's rows were pivots of
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        // key: the high bits of |value| (13 mantissa bits in FP64, 16 in
+        // FP32) over 127 - row: a pivot within 2^-13 of the largest, the
+        // lowest row among ties
+        uint32_t key = used0 ? 0u : bj_key(P0[k]) | uint32_t(127 - lane);
+        if constexpr (H == 2) {
+            const uint32_t v = used1 ? 0u : bj_key(P1[k]) | uint32_t(63 - lane);
+            key = v > key ? v : key;
+        }
+        key = bj_wave_max(key);
+        bad |= key < 0x80u || key >= bj_key_inf<T>();
+        const int pr = 127 - int(key & 127u), pl = pr & 63;
+        const bool low = H == 1 || pr < 64;
+        T row[16];
+        if (low) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) row[c] = bj_lane(P0[c], pl);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) row[c] = bj_lane(P1[c], pl);
+        }
+        const T inv = T(1) / row[k];
+        const bool is0 = low && lane == pl, is1 = !low && lane == pl;
+        const T f0 = P0[k] * inv, f1 = P1[k] * inv;
+        const T g0 = is0 ? T(0) : -f0, g1 = is1 ? T(0) : -f1;
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+            if (c != k) {
+                P0[c] = fma(g0, row[c], P0[c]);
+                if constexpr (H == 2) P1[c] = fma(g1, row[c], P1[c]);
+            }
+        P0[k] = is0 ? T(1) : g0;
+        s0 = is0 ? inv : s0;
+        used0 = used0 || is0;
+        if constexpr (H == 2) {
+            P1[k] = is1 ? T(1) : g1;
+            s1 = is1 ? inv : s1;
+            used1 = used1 || is1;
+        }
+        step0 = is0 ? k0 + k : step0;
+        if constexpr (H == 2) step1 = is1 ? k0 + k : step1;
+    }
+    if (step0 >= 0) {
+        q[BJMma<T>::slot(lane)] = uint8_t(step0);
+        perm[step0] = lane;
+    }
+    if (H == 2 && step1 >= 0) {
+        q[BJMma<T>::slot(lane + 64)] = uint8_t(step1);
+        perm[step1] = lane + 64;
+    }
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+        P0[c] *= s0;
+        if constexpr (H == 2) P1[c] *= s1;
+    }
+    return !bad;
+}
+
+template <int NT, typename T>
+__global__ __launch_bounds__(64 * NT)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? (NT > 4 ? 4 : 5) : 8)))
+void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
+                    const int32_t *__restrict__ blk, const int32_t *__restrict__ bl,
+                    T *__restrict__ out, int *__restrict__ status) {
+    typedef BJReg<NT, T> R;
+    typedef BJMma<T> Mma;
+    typedef typename Mma::v4 v4;
+    constexpr int NR = R::NR, WS = R::WS, SS = R::SS, H = R::H;
+    __shared__ __attribute__((aligned(16))) T buf[2 * NR * WS];   // strip, then W of two panels
+    __shared__ T piv[NT][17 * 16];                // each wave's pivot rows of its own columns
+    __shared__ double cth[NMq], sth[NMq], wx[NMq], wy[NMq], wt[NMq];
+    __shared__ double Dx[NMq * NMq], Dy[NMq * NMq], kap[NMq * NMq], sig[NMq * NMq];
+    __shared__ __attribute__((aligned(16))) uint8_t q[4 * 32];
+    __shared__ int32_t perm[NR];
+    __shared__ int failed;
     __shared__ BJSelf sl;
-    const int b = bl[blockIdx.x], tid = threadIdx.x, ti = tid / TJ, tj = tid % TJ;
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = bl[blockIdx.x];
     const int k = blk[3 * b], a0 = blk[3 * b + 1], g = blk[3 * b + 2];
     BJCell x;
     const int c = m.cell_col[k];
@@ -357,18 +510,32 @@ void k_bj_build_reg(DevMesh m, int restrict_,
     x.dy = m.col_geom[4 * c + 3] - m.col_geom[4 * c + 1];
     const double th0 = m.cell_geom[2 * k];
     x.dth = m.cell_geom[2 * k + 1] - th0;
-    x.wx = m.lgl_w + x.nx * NMq;
-    x.wy = m.lgl_w + x.ny * NMq;
-    x.wt = m.lg_w + x.nth * NMq;
-    x.Dx = m.lgl_D + size_t(x.nx) * NMq * NMq;
-    x.Dy = m.lgl_D + size_t(x.ny) * NMq * NMq;
+    x.wx = wx;
+    x.wy = wy;
+    x.wt = wt;
+    x.Dx = Dx;
+    x.Dy = Dy;
     x.ao = m.cell_ang_off[k];
     x.na = m.col_nang[c];
     x.G = m.G + m.col_G_off[c];
-    x.kap = m.kappa + m.col_sp_off[c];
-    x.sig = m.sigma + m.col_sp_off[c];
+    x.kap = kap;
+    x.sig = sig;
     x.quad = m.cell_quad[k];
     x.bd = restrict_ ? m.cell_bdry[k] : 0;
+    const int nsp = x.nx * x.ny, sp0 = m.col_sp_off[c];
+    for (int t = tid; t < NMq * NMq; t += 64 * NT) {
+        Dx[t] = m.lgl_D[size_t(x.nx) * NMq * NMq + t];
+        Dy[t] = m.lgl_D[size_t(x.ny) * NMq * NMq + t];
+        if (t < nsp) {
+            kap[t] = m.kappa[sp0 + t];
+            sig[t] = m.sigma[sp0 + t];
+        }
+        if (t < NMq) {
+            wx[t] = m.lgl_w[x.nx * NMq + t];
+            wy[t] = m.lgl_w[x.ny * NMq + t];
+            wt[t] = m.lg_w[x.nth * NMq + t];
+        }
+    }
     if (tid == 0) {
         int ns = 0;
         for (int l = m.link_start[k]; l < m.link_start[k + 1] && ns < 4; ++l)
@@ -379,6 +546,7 @@ void k_bj_build_reg(DevMesh m, int restrict_,
                 ++ns;
             }
         sl.n = ns;
+        failed = 0;
     }
     if (tid < x.nth) {
         double s, cc;
@@ -386,114 +554,138 @@ void k_bj_build_reg(DevMesh m, int restrict_,
         cth[tid] = cc;
         sth[tid] = s;
     }
-    if (tid < NR) used[tid] = 0;
-    if (tid < 2) red_key[tid] = 0ull;
+    for (int t = tid; t < 4 * 32; t += 64 * NT) q[t] = 0xff;
     // the block: angles a0 .. a0 + g - 1 of the cell at every spatial node;
     // block index t <-> cell DOF (t / g) nth + a0 + t % g
-    const int n = (x.n / x.nth) * g;
-    __syncthreads();
-    T A[RR][CC];
+    const int n = nsp * g;
+    // Assembly by strips of 32 rows of M (columns of the block): of a row's n
+    // entries at most g + nx + ny - 2 are not zero (the node's angles, the
+    // two derivative lines), so those alone are evaluated, one per thread.
+    v4 acc[NT];
+    const int per = g + x.nx + x.ny - 2;
 #pragma unroll
-    for (int u = 0; u < RR; ++u)
-#pragma unroll
-        for (int v = 0; v < CC; ++v) {
-            const int row = ti + 16 * u, col = tj + TJ * v;
-            A[u][v] = (row < n && col < n)
-                          ? T(bj_entry(m, x, sl, cth, sth, (row / g) * x.nth + a0 + row % g,
-                                       (col / g) * x.nth + a0 + col % g))
-                          : T(0);
-        }
-    // Every step is written without per-element branches (selects around
-    // one FMA per element), so the wave runs straight-line code.
-    for (int kk = 0; kk < n; ++kk) {
-        const int buf = kk & 1, vk = kk / TJ;
-        if (tj == kk % TJ) {           // the 16 owners of column kk
-            double best = -1.0;
-            int bi = n;
-#pragma unroll
-            for (int u = 0; u < RR; ++u) {
-                T val = A[u][0];
-#pragma unroll
-                for (int v = 1; v < CC; ++v) val = (v == vk) ? A[u][v] : val;
-                const int row = ti + 16 * u;
-                const bool ok = row < n;
-                if (ok) colk[buf][row] = val;
-                const double av = fabs(double(val));
-                const bool better = ok && !used[ok ? row : 0] && (av > best || (av == best && row < bi));
-                best = better ? av : best;
-                bi = better ? row : bi;
+    for (int s = 0; s < (NT + 1) / 2; ++s) {
+        for (int t = tid; t < 32 * SS; t += 64 * NT) buf[t] = T(0);
+        __syncthreads();
+        // unit diagonal past the block: those columns pivot on their own rows
+        if (tid < 32 && 32 * s + tid >= n && 32 * s + tid < NR) buf[tid * SS + 32 * s + tid] = T(1);
+        const int rows = min(32, n - 32 * s), each = sl.n ? n : per;
+        for (int e = tid; e < rows * each; e += 64 * NT) {
+            const int rr = e / each, f = e - rr * each, u = 32 * s + rr;
+            const int node = u / g, r = u - node * g, i = node / x.ny, j = node - i * x.ny;
+            int t;
+            if (sl.n)                                // self links couple whole faces
+                t = f;
+            else if (f < g)
+                t = node * g + f;
+            else if (f < g + x.nx - 1) {
+                const int p = f - g, pi = p + (p >= i);
+                t = (pi * x.ny + j) * g + r;
+            } else {
+                const int p = f - g - (x.nx - 1), pj = p + (p >= j);
+                t = (i * x.ny + pj) * g + r;
             }
-            // no candidate (or a zero column): key 0, which fails below
-            const unsigned long long key =
-                (bi < n && best > 0.0)
-                    ? ((static_cast<unsigned long long>(__double_as_longlong(best)) & ~0x7Full) |
-                       static_cast<unsigned long long>(127 - bi))
-                    : 0ull;
-            atomicMax(&red_key[buf], key);
+            const int tn = t / g;
+            buf[rr * SS + t] = T(bj_entry(m, x, sl, cth, sth, tn * x.nth + a0 + (t - tn * g),
+                                          node * x.nth + a0 + r));
         }
         __syncthreads();
-        const unsigned long long key = red_key[buf];
-        const double best = __longlong_as_double(static_cast<long long>(key & ~0x7Full));
-        const int pr = 127 - int(key & 0x7Full);
-        // the other buffer is next read after this step's second barrier
-        if (tid == 0) red_key[buf ^ 1] = 0ull;
-        if (!(best > 0.0) || pr >= n) {
-            if (tid == 0) atomicMax(status, k + 1);
-            return;                    // uniform across the workgroup
-        }
-        if (ti == (pr & 15)) {
-            const int up = pr >> 4;
 #pragma unroll
-            for (int v = 0; v < CC; ++v) {
-                T pval = A[0][v];
+        for (int h = 0; h < 2; ++h)
+            if (2 * s + h < NT) {
 #pragma unroll
-                for (int u = 1; u < RR; ++u) pval = (u == up) ? A[u][v] : pval;
-                const int col = tj + TJ * v;
-                if (col < n) prow[col] = pval;
+                for (int v = 0; v < 4; ++v)
+                    acc[2 * s + h][v] = buf[(16 * h + Mma::row(lg, v)) * SS + 16 * wave + l16];
             }
-        }
-        if (tid == 0) {
-            used[pr] = 1;
-            perm[kk] = pr;
-        }
         __syncthreads();
-        // in-place Gauss-Jordan: pivot row -> row / p with 1 / p in column
-        // kk; other rows -> row - c_r (pivot row / p) with -c_r / p in column
-        // kk.  With the pivot row's kk entry taken as 1 and the other rows'
-        // kk entries as 0 this is one FMA per element.
-        const T invp = T(1) / colk[buf][pr];
-        T pv[CC];
-#pragma unroll
-        for (int v = 0; v < CC; ++v) {
-            const int col = tj + TJ * v;
-            const T pr_v = (col == kk) ? T(1) : ((col < n) ? prow[col] : T(0));
-            pv[v] = pr_v * invp;
-        }
-#pragma unroll
-        for (int u = 0; u < RR; ++u) {
-            const int row = ti + 16 * u;
-            const bool isp = row == pr;
-            const T ck = (row < n) ? colk[buf][row] : T(0);
-#pragma unroll
-            for (int v = 0; v < CC; ++v) {
-                const int col = tj + TJ * v;
-                const T base = (col == kk) ? T(0) : A[u][v];
-                const T upd = fma(-ck, pv[v], base);
-                A[u][v] = isp ? pv[v] : upd;
-            }
-        }
     }
-    __syncthreads();
-    if (tid < n) qinv[perm[tid]] = tid;
-    __syncthreads();
-    T *o = out + inv_off[b];
+    // Panel p of another wave: update this wave's tile.
+    auto update = [&](int p) {
+        const T *W = buf + (p & 1) * NR * WS;
+        __syncthreads();
+        // This wave's entries of the panel's pivot rows -> piv, zero in M.
+        // q may get entries of the next panel meanwhile: those steps are
+        // 16 (p + 1) or more, no match either way.
 #pragma unroll
-    for (int u = 0; u < RR; ++u)
+        for (int rt = 0; rt < NT; ++rt) {
+            const uint32_t qs = *reinterpret_cast<const uint32_t *>(q + lg * 32 + rt * 4);
+            // a byte of t is zero where a row of this lane is a pivot of
+            // panel p; most row tiles have none
+            const uint32_t t = ((qs >> 4) & 0x0f0f0f0fu) ^ (uint32_t(p) * 0x01010101u);
+            if (__any(((t - 0x01010101u) & ~t & 0x80808080u) != 0)) {
+                v4 keep;
 #pragma unroll
-        for (int v = 0; v < CC; ++v) {
-            const int row = ti + 16 * u, col = tj + TJ * v;
-            if (row < n && col < n) o[size_t(perm[col]) * n + qinv[row]] = A[u][v];
+                for (int v = 0; v < 4; ++v) {
+                    // rows that are no pivots go to the spare row 16
+                    const uint32_t s = min(((qs >> (8 * v)) & 255u) - 16u * p, 16u);
+                    piv[wave][s * 16 + l16] = acc[rt][v];
+                    keep[v] = s < 16u ? T(0) : T(1);
+                }
+                acc[rt] *= keep;
+            }
         }
+        bj_wave_sync();
+#pragma unroll 1
+        for (int s = 0; s < 4; ++s) {
+            const T bv = piv[wave][(4 * s + lg) * 16 + l16];
+#pragma unroll
+            for (int rt = 0; rt < NT; ++rt)
+                acc[rt] = Mma::step(W[(16 * rt + l16) * WS + 4 * s + lg], bv, acc[rt]);
+        }
+        bj_wave_sync();                              // piv is written again by the next panel
+    };
+    // Straight-line phases rather than one loop with a branch on the panel's
+    // owner: the branch made the compiler keep two copies of the tile.
+#pragma unroll 1
+    for (int p = 0; p < wave; ++p) update(p);
+    {
+        T *W = buf + (wave & 1) * NR * WS;
+        __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) W[(16 * rt + Mma::row(lg, v)) * WS + l16] = acc[rt][v];
+        bj_wave_sync();
+        // rows that earlier panels took are no candidates
+        const int r0 = NT > 3 ? lane : min(lane, NR - 1), r1 = H == 2 ? min(lane + 64, NR - 1) : 0;
+        T P0[16], P1[16];
+#pragma unroll
+        for (int cc = 0; cc < 16; ++cc) {
+            P0[cc] = W[r0 * WS + cc];
+            P1[cc] = H == 2 ? W[r1 * WS + cc] : T(0);
+        }
+        const bool ok = bj_panel<H, T>(P0, P1, 16 * wave, lane,
+                                       lane >= NR || q[Mma::slot(r0)] != 0xff,
+                                       lane + 64 >= NR || q[Mma::slot(r1)] != 0xff, q, perm);
+        if (!ok && lane == 0) {
+            failed = 1;
+            atomicMax(status, k + 1);
+        }
+#pragma unroll
+        for (int cc = 0; cc < 16; ++cc) {
+            if (NT > 3 || lane < NR) W[r0 * WS + cc] = P0[cc];
+            if (H == 2 && lane + 64 < NR) W[r1 * WS + cc] = P1[cc];
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __syncthreads();
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[rt][v] = W[(16 * rt + Mma::row(lg, v)) * WS + l16];
+    }
+#pragma unroll 1
+    for (int p = wave + 1; p < NT; ++p) update(p);
+    __syncthreads();
+    const int j = 16 * wave + l16;
+    if (failed || j >= n) return;
+    T *o = out + inv_off[b] + perm[j];
+#pragma unroll
+    for (int rt = 0; rt < NT; ++rt) {
+        const uint32_t qs = *reinterpret_cast<const uint32_t *>(q + lg * 32 + rt * 4);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (16 * rt + Mma::row(lg, v) < n) o[size_t((qs >> (8 * v)) & 255u) * n] = acc[rt][v];
+    }
 }
 
 __global__ void k_to_f32_bj(const double *__restrict__ s, float *__restrict__ d, int64_t n) {
@@ -968,7 +1160,7 @@ extern "C" int rtx_bjacobi_size(rtx_plan *p, int64_t *n_entries) {
     std::vector<int32_t> dof0(p->m.ncell);
     RTX_HIP(hipMemcpy(dof0.data(), p->m.cell_dof_off, dof0.size() * 4, hipMemcpyDeviceToHost));
     const int split = (p->bj_method != 0) ? 1 : 0;
-    std::vector<int32_t> blk, apd, cls[4];
+    std::vector<int32_t> blk, apd, cls[BJ_NCLS];
     std::vector<int64_t> off(1, 0), off16(1, 0), off8(1, 0), soff(1, 0);
     int32_t maxb = 0;
     for (int k = 0; k < p->m.ncell; ++k) {
@@ -984,8 +1176,7 @@ extern "C" int rtx_bjacobi_size(rtx_plan *p, int64_t *n_entries) {
             apd.push_back(dof0[k] + a0);
             apd.push_back(nth);
             apd.push_back(gg);
-            const int q = n <= 32 ? 0 : n <= 64 ? 1 : n <= 96 ? 2 : 3;
-            cls[q].push_back(int32_t(blk.size() / 3 - 1));
+            cls[std::min<int64_t>((n - 1) / 16, BJ_NCLS - 1)].push_back(int32_t(blk.size() / 3 - 1));
             off.push_back(off.back() + n * n);
             off16.push_back(off16.back() + n * ((n + 7) / 8 * 8));
             off8.push_back(off8.back() + n * ((n + 15) / 16 * 16));
@@ -1022,11 +1213,11 @@ extern "C" int rtx_bjacobi_size(rtx_plan *p, int64_t *n_entries) {
         RTX_HIP(hipMemcpy(p->bj_apd, apd.data(), apd.size() * sizeof(int32_t),
                           hipMemcpyHostToDevice));
         std::vector<int32_t> all;
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < BJ_NCLS; ++q) {
             p->bj_cls_start[q] = int32_t(all.size());
             all.insert(all.end(), cls[q].begin(), cls[q].end());
         }
-        p->bj_cls_start[4] = int32_t(all.size());
+        p->bj_cls_start[BJ_NCLS] = int32_t(all.size());
         RTX_HIP(hipMalloc(&p->bj_cls, std::max<size_t>(all.size(), 1) * sizeof(int32_t)));
         if (!all.empty())
             RTX_HIP(hipMemcpy(p->bj_cls, all.data(), all.size() * sizeof(int32_t),
@@ -1147,24 +1338,26 @@ extern "C" int rtx_bjacobi_factor(rtx_plan *p, int restrict_interior, double *d_
         return RTX_ERR_ARG;
     }
     if (reg) {
-        // each size class on the smallest register grid that holds it:
-        // fewer padded elements per elimination step, more blocks per CU
+        // each size class (steps of 16 DOFs, one wave per 16) on the kernel that holds it
         const int32_t *cs = p->bj_cls, *c0 = p->bj_cls_start;
         auto cnt = [&](int q) { return c0[q + 1] - c0[q]; };
         auto run = [&](auto *out) {
             using T = typename std::remove_pointer<decltype(out)>::type;
-            if (cnt(0))
-                k_bj_build_reg<2, 2, 16, T><<<cnt(0), 256, 0, st>>>(
-                    p->m, restrict_interior, p->bj_off, p->bj_blk, cs + c0[0], out, d_status);
-            if (cnt(1))
-                k_bj_build_reg<4, 4, 16, T><<<cnt(1), 256, 0, st>>>(
-                    p->m, restrict_interior, p->bj_off, p->bj_blk, cs + c0[1], out, d_status);
-            if (cnt(2))
-                k_bj_build_reg<6, 4, 24, T><<<cnt(2), 384, 0, st>>>(
-                    p->m, restrict_interior, p->bj_off, p->bj_blk, cs + c0[2], out, d_status);
-            if (cnt(3))
-                k_bj_build_reg<8, 4, 32, T><<<cnt(3), 512, 0, st>>>(
-                    p->m, restrict_interior, p->bj_off, p->bj_blk, cs + c0[3], out, d_status);
+            auto build = [&](auto nt) {
+                constexpr int NT = decltype(nt)::value;
+                if (cnt(NT - 1))
+                    k_bj_build_reg<NT, T><<<cnt(NT - 1), 64 * NT, 0, st>>>(
+                        p->m, restrict_interior, p->bj_off, p->bj_blk, cs + c0[NT - 1], out, d_status);
+            };
+            // the largest blocks first: the small classes fill the tail
+            build(std::integral_constant<int, 8>());
+            build(std::integral_constant<int, 7>());
+            build(std::integral_constant<int, 6>());
+            build(std::integral_constant<int, 5>());
+            build(std::integral_constant<int, 4>());
+            build(std::integral_constant<int, 3>());
+            build(std::integral_constant<int, 2>());
+            build(std::integral_constant<int, 1>());
         };
         if (f32_only)
             run(d_inv_f32);

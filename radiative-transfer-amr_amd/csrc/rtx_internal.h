@@ -112,6 +112,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d);
 int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
                  int accumulate);
 
+constexpr int BJ_NCLS = 8;          // size classes of the block-Jacobi build
 constexpr int RTX_NBINS = 6;
 // Tiled scattering work items: 16 spatial nodes x SC_RG output angles
 constexpr int SC_RG = 128;
@@ -210,10 +211,10 @@ struct rtx_plan {
     // per block, for the applies: (n, first DOF, cell angle count, angle
     // count g), one 16-byte load instead of a chain through the mesh tables
     int32_t *bj_apd = nullptr;
-    // the register build's size classes (blocks of <= 32, 64, 96, 128
-    // DOFs): block indices, concatenated, with the class starts
+    // the register build's size classes (blocks of <= 16, 32, .. 128 DOFs):
+    // block indices, concatenated, with the class starts
     int32_t *bj_cls = nullptr;
-    int32_t bj_cls_start[5] = {0, 0, 0, 0, 0};
+    int32_t bj_cls_start[rtx::BJ_NCLS + 1] = {};
     int32_t bj_nblk = 0, bj_max_block = 0;
     int bj_split = -1;           // split setting the block table was built with
     // coarse grid of the learned correction: per column a list of

@@ -592,6 +592,37 @@ def _device_inverses(pc, blocks, invs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [(2, 2, 2), (2, 2, 4), (3, 3, 2), (4, 4, 2), (3, 3, 4), (3, 4, 4),
+                               (7, 7, 1), (4, 4, 4), (5, 5, 3), (5, 4, 4), (3, 9, 3), (4, 6, 4),
+                               (5, 5, 4), (4, 7, 4), (5, 5, 5), (8, 4, 4), (6, 6, 6)])
+@pytest.mark.parametrize("self_links", [False, True])
+def test_block_jacobi_build_sizes(cuda, n, self_links):
+    """The register build at the edges of its size classes (16, 32, .. 128
+    DOFs, and cells split into groups), with inflow-masked cells on open
+    boundaries, and with cells coupled to themselves (one column, periodic):
+    every inverse in FP64 and from the FP32 elimination to 8 n u cond(B)."""
+    from rtx.operator import TransportOperator
+    from rtx.krylov import BlockJacobi
+    mesh = problems.uniform_mesh([1.0, 1.3], list(n), 2, 0 if self_links else 1,
+                                 pbcs=(self_links, self_links))
+    wl = problems.two_scatterers()
+    A, f, b, mask = _oracle_system(mesh, wl)
+    op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
+    blocks = osys.bj_block_dofs(mesh, 128)
+    invs = osys.block_jacobi_inverses(A, mesh, mask, split=128)
+    pc = BlockJacobi(op)
+    inv64 = pc.inv.cpu().numpy()
+    off = 0
+    for idx, inv in zip(blocks, invs):
+        m = len(idx)
+        err = np.linalg.norm(inv64[off:off + m * m].reshape(m, m).T - inv) / np.linalg.norm(inv)
+        assert err <= 8 * m * 2.0 ** -53 * np.linalg.cond(inv), (m, err)
+        off += m * m
+    assert off == inv64.size
+    _device_inverses(BlockJacobi(op, keep_f64=False, keep_f32=True), blocks, invs)
+
+
+@pytest.mark.gpu
 def test_block_jacobi_fp8_apply(cuda):
     """FP8 block-Jacobi (e4m3 codes, one FP32 scale max|column| / 448 per
     column) against the oracle's inverses quantised the same way in numpy
