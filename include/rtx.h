@@ -248,6 +248,14 @@ int rtx_bjacobi_size_fp4(rtx_plan *plan, int64_t *n_bytes);
    saturating) with the scale max |column| / 6 per column, into the FP4
    pool.  No counterpart in the reference. */
 int rtx_bjacobi_pack_fp4(rtx_plan *plan, const float *d_inv32, uint8_t *d_inv4, void *stream);
+/* rtx_bjacobi_factor (FP32 elimination) and rtx_bjacobi_pack_fp8 / _fp4 in one
+   pass, without the FP32 pool: the same bytes into the pool of
+   rtx_bjacobi_size_fp8 (precision RTX_PREC_FP8) or _fp4 (RTX_PREC_FP4), 16-byte
+   aligned.  Register build only (blocks of up to 128 DOFs, else RTX_ERR_ARG).
+   Synchronises the stream; RTX_ERR_NUMERIC on a singular block.  No
+   counterpart in the reference. */
+int rtx_bjacobi_factor_coded(rtx_plan *plan, int restrict_interior, int precision,
+                             uint8_t *d_codes, void *stream);
 /* z = blockdiag(inv) r, precision RTX_PREC_F64 (double inverses, vectors),
    RTX_PREC_F32 (float inverses, vectors), RTX_PREC_MIXED (the packed BF16
    pool of rtx_bjacobi_pack_bf16, float vectors, FP32 accumulation),

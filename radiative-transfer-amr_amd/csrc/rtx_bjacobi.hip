@@ -245,11 +245,27 @@ __global__ __launch_bounds__(BJ_THREADS) void k_bj_build(DevMesh m, int restrict
         for (int row = tid; row < n; row += BJ_THREADS) o[size_t(col) * n + row] = A[size_t(row) * n + col];
 }
 
+// FP8 e4m3 (bias 7, largest finite 448, no infinities): nearest code, ties to
+// even, by the hardware conversion; |v| above 448 saturates; -0 gets code 0.
+__device__ inline uint8_t bj_to_e4m3(float v) {
+    v = fminf(fmaxf(v, -448.f), 448.f) + 0.f;
+    return uint8_t(__builtin_amdgcn_cvt_pk_fp8_f32(v, v, 0, false));
+}
+
+// FP4 e2m1 (OCP: bias 1, one mantissa bit, largest 6, no infinities or
+// NaN; magnitudes 0, 0.5, 1, 1.5, 2, 3, 4, 6 for codes 0..7): nearest code,
+// ties to the even code, by the hardware conversion; |v| above 6 saturates;
+// -0 gets code 0.
+__device__ inline uint32_t bj_to_e2m1(float v) {
+    v = fminf(fmaxf(v, -6.f), 6.f) + 0.f;
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v, v, 1.f, 0) & 15u;
+}
+
 // ---- register-resident build for blocks of up to 128 DOFs.
 struct BJCell {
-    int nx, ny, nth, n, nyt, ao, na, quad, bd;
+    int nx, ny, nth, quad, bd;
     double dx, dy, dth;
-    const double *wx, *wy, *wt, *Dx, *Dy, *G, *kap, *sig;
+    const double *wx, *wy, *wt, *Dx, *Dy, *kap, *sig;
 };
 
 struct BJSelf {                  // links of a cell to itself (periodic faces), in LDS
@@ -258,19 +274,20 @@ struct BJSelf {                  // links of a cell to itself (periodic faces), 
     int es[4], et[4];
 };
 
+// The block's entry at row (p, q, r), column (i, j, a): spatial nodes and
+// angles of the cell; Gb = the cell's scattering block G[a][r] from angle a0
+// on, g x g.
 __device__ inline double bj_entry(const DevMesh &m, const BJCell &x, const BJSelf &sl,
-                                  const double *cth, const double *sth, int t, int u) {
-    const int p = t / x.nyt, q = (t / x.nth) % x.ny, r = t % x.nth;
-    const int i = u / x.nyt, j = (u / x.nth) % x.ny, a = u % x.nth;
+                                  const double *cth, const double *sth, const double *Gb, int a0,
+                                  int g, int p, int q, int r, int i, int j, int a) {
     if (x.bd) {
         const bool rb = bj_on_bdry(x.bd, p, q, x.nx, x.ny);
         const bool cb = bj_on_bdry(x.bd, i, j, x.nx, x.ny);
-        if (rb || cb) return (t == u) ? 1.0 : 0.0;
+        if (rb || cb) return (p == i && q == j && r == a) ? 1.0 : 0.0;
     }
     double v = 0.0;
     if (p == i && q == j) {
-        v = -x.dx * x.dy * x.wx[p] * x.wy[q] * x.sig[p * x.ny + q] *
-            x.G[size_t(x.ao + a) * x.na + x.ao + r];
+        v = -x.dx * x.dy * x.wx[p] * x.wy[q] * x.sig[p * x.ny + q] * Gb[(a - a0) * g + r - a0];
         if (r == a) {
             double d = (x.dx * x.dy * x.dth * 0.125) * x.wx[p] * x.wy[q] * x.wt[r] * x.kap[p * x.ny + q];
             if (x.quad >= 0)
@@ -327,16 +344,16 @@ __device__ inline double bj_entry(const DevMesh &m, const BJCell &x, const BJSel
 // and a tile's 16 lanes store runs of one column of the inverse.
 //
 // Bound by the panels (half of the FP64 time: pivot search, broadcast and
-// division in series) and the matrix instructions.  A rank-1 form with two
+// reciprocal in series) and the matrix instructions.  A rank-1 form with two
 // block barriers per column and five instructions per element and column
-// took 14.6 ms for 16,384 blocks of 125 in FP64 (this: 3.5, the FP64 rate's
+// took 14.6 ms for 16,384 blocks of 125 in FP64 (this: 3.2, the FP64 rate's
 // floor 0.9) and 31.3 ms for the 91,352 blocks of an hp mesh of 8.3 M DOF in
-// FP32 (this: 7.6).  One barrier per panel is left; the next panel's wave
+// FP32 (this: 6.9).  One barrier per panel is left; the next panel's wave
 // starts as soon as its own tile is updated (W is double-buffered), at raised
 // priority because the panels are the serial chain.  Registers: two blocks of
 // eight waves per CU in FP64 (128 VGPRs); in FP32 four (64 VGPRs with a few
 // spills: 16,384 blocks of 125 in 1.83 ms, against 2.0 at 80 VGPRs and 2.5
-// without a limit).
+// without a limit, before the assembly's index tables took it to 1.68).
 template <int NT, typename T>
 struct BJReg {
     static constexpr int NR = 16 * NT;
@@ -402,6 +419,18 @@ __device__ inline void bj_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// 1 / p to an ulp (hardware reciprocal and Newton steps): a pivot's relative
+// perturbation of that size is one rounding of the elimination.
+__device__ inline double bj_recip(double p) {
+    double r = __builtin_amdgcn_rcp(p);
+    r = fma(fma(-p, r, 1.0), r, r);
+    return fma(fma(-p, r, 1.0), r, r);
+}
+__device__ inline float bj_recip(float p) {
+    const float r = __builtin_amdgcn_rcpf(p);
+    return fmaf(fmaf(-p, r, 1.f), r, r);
+}
+
 // Sweep the 16 columns of a panel held one row (H rows, 64 apart) per lane.
 // q: byte table of the step that each row was pivot of (BJMma::slot order);
 // perm: pivot row of each step.  False on a zero or non-finite pivot (the
@@ -440,7 +469,7 @@ __device__ __forceinline__ bool bj_panel(T (&P0)[16], T (&P1)[16], int k0, int l
 #pragma unroll
             for (int c = 0; c < 16; ++c) row[c] = bj_lane(P1[c], pl);
         }
-        const T inv = T(1) / row[k];
+        const T inv = bj_recip(row[k]);
         const bool is0 = low && lane == pl, is1 = !low && lane == pl;
         const T f0 = P0[k] * inv, f1 = P1[k] * inv;
         const T g0 = is0 ? T(0) : -f0, g1 = is1 ? T(0) : -f1;
@@ -477,12 +506,19 @@ __device__ __forceinline__ bool bj_panel(T (&P0)[16], T (&P1)[16], int k0, int l
     return !bad;
 }
 
-template <int NT, typename T>
+//
+// BITS 8 or 4 (T = float): the inverse is not stored; each of its columns is
+// scaled and rounded to FP8 / FP4 codes in registers, in the layout and with
+// the bytes of k_bj_pack_fp8 / _fp4, through an image in the dead panel
+// buffers. The FP32 pool that the separate pass reads (3.2 GB on the hp mesh
+// above) is neither allocated nor written: 7.5 ms instead of 7.2 + 2.7.
+template <int NT, typename T, int BITS = 0>
 __global__ __launch_bounds__(64 * NT)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? (NT > 4 ? 4 : 5) : 8)))
 void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
                     const int32_t *__restrict__ blk, const int32_t *__restrict__ bl,
-                    T *__restrict__ out, int *__restrict__ status) {
+                    typename std::conditional<BITS == 0, T, uint8_t>::type *__restrict__ out,
+                    const int64_t *soff, float *__restrict__ scales, int *__restrict__ status) {
     typedef BJReg<NT, T> R;
     typedef BJMma<T> Mma;
     typedef typename Mma::v4 v4;
@@ -490,7 +526,8 @@ void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
     __shared__ __attribute__((aligned(16))) T buf[2 * NR * WS];   // strip, then W of two panels
     __shared__ T piv[NT][17 * 16];                // each wave's pivot rows of its own columns
     __shared__ double cth[NMq], sth[NMq], wx[NMq], wy[NMq], wt[NMq];
-    __shared__ double Dx[NMq * NMq], Dy[NMq * NMq], kap[NMq * NMq], sig[NMq * NMq];
+    __shared__ double Dx[NMq * NMq], Dy[NMq * NMq], kap[NMq * NMq], sig[NMq * NMq], Gb[NMq * NMq];
+    __shared__ int32_t at[NR];                    // node i | j << 8 | angle << 16 of a block index
     __shared__ __attribute__((aligned(16))) uint8_t q[4 * 32];
     __shared__ int32_t perm[NR];
     __shared__ int failed;
@@ -504,8 +541,6 @@ void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
     x.nx = m.col_nx[c];
     x.ny = m.col_ny[c];
     x.nth = m.cell_nth[k];
-    x.n = x.nx * x.ny * x.nth;
-    x.nyt = x.ny * x.nth;
     x.dx = m.col_geom[4 * c + 2] - m.col_geom[4 * c + 0];
     x.dy = m.col_geom[4 * c + 3] - m.col_geom[4 * c + 1];
     const double th0 = m.cell_geom[2 * k];
@@ -515,15 +550,17 @@ void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
     x.wt = wt;
     x.Dx = Dx;
     x.Dy = Dy;
-    x.ao = m.cell_ang_off[k];
-    x.na = m.col_nang[c];
-    x.G = m.G + m.col_G_off[c];
     x.kap = kap;
     x.sig = sig;
     x.quad = m.cell_quad[k];
     x.bd = restrict_ ? m.cell_bdry[k] : 0;
-    const int nsp = x.nx * x.ny, sp0 = m.col_sp_off[c];
+    const int nsp = x.nx * x.ny, sp0 = m.col_sp_off[c], na = m.col_nang[c];
+    const double *G = m.G + m.col_G_off[c] + size_t(m.cell_ang_off[k] + a0) * (na + 1);
+    // the block: angles a0 .. a0 + g - 1 of the cell at every spatial node;
+    // block index t <-> cell DOF (t / g) nth + a0 + t % g
+    const int n = nsp * g;
     for (int t = tid; t < NMq * NMq; t += 64 * NT) {
+        if (t < g * g) Gb[t] = G[size_t(t / g) * na + t % g];
         Dx[t] = m.lgl_D[size_t(x.nx) * NMq * NMq + t];
         Dy[t] = m.lgl_D[size_t(x.ny) * NMq * NMq + t];
         if (t < nsp) {
@@ -555,40 +592,46 @@ void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
         sth[tid] = s;
     }
     for (int t = tid; t < 4 * 32; t += 64 * NT) q[t] = 0xff;
-    // the block: angles a0 .. a0 + g - 1 of the cell at every spatial node;
-    // block index t <-> cell DOF (t / g) nth + a0 + t % g
-    const int n = nsp * g;
+    for (int t = tid; t < n; t += 64 * NT) {
+        const int node = t / g, i = node / x.ny;
+        at[t] = i | (node - i * x.ny) << 8 | (t - node * g) << 16;
+    }
+    for (int t = tid; t < 32 * SS; t += 64 * NT) buf[t] = T(0);
     // Assembly by strips of 32 rows of M (columns of the block): of a row's n
     // entries at most g + nx + ny - 2 are not zero (the node's angles, the
-    // two derivative lines), so those alone are evaluated, one per thread.
+    // two derivative lines), so those alone are evaluated, one per thread,
+    // and cleared again after the strip is read.
     v4 acc[NT];
-    const int per = g + x.nx + x.ny - 2;
+    __syncthreads();
+    const int each = sl.n ? n : g + x.nx + x.ny - 2;   // self links couple whole faces
+    const float r_each = 1.f / float(each);            // e < 32 128: exact quotients
+    const auto entries = [&](int s, auto put) {
+        const int rows = min(32, n - 32 * s);
+        for (int e = tid; e < rows * each; e += 64 * NT) {
+            const int rr = int((float(e) + 0.5f) * r_each), f = e - rr * each;
+            const int c0 = at[32 * s + rr], i = c0 & 255, j = (c0 >> 8) & 255, r = c0 >> 16;
+            int p = i, pq = j, a = r;
+            if (sl.n) {
+                const int c1 = at[f];
+                p = c1 & 255;
+                pq = (c1 >> 8) & 255;
+                a = c1 >> 16;
+            } else if (f < g)
+                a = f;
+            else if (f < g + x.nx - 1)
+                p = f - g + (f - g >= i);
+            else
+                pq = f - g - x.nx + 1 + (f - g - x.nx + 1 >= j);
+            put(rr * SS + (p * x.ny + pq) * g + a, p, pq, a, i, j, r);
+        }
+    };
 #pragma unroll
     for (int s = 0; s < (NT + 1) / 2; ++s) {
-        for (int t = tid; t < 32 * SS; t += 64 * NT) buf[t] = T(0);
-        __syncthreads();
+        entries(s, [&](int o, int p, int pq, int a, int i, int j, int r) {
+            buf[o] = T(bj_entry(m, x, sl, cth, sth, Gb, a0, g, p, pq, a0 + a, i, j, a0 + r));
+        });
         // unit diagonal past the block: those columns pivot on their own rows
         if (tid < 32 && 32 * s + tid >= n && 32 * s + tid < NR) buf[tid * SS + 32 * s + tid] = T(1);
-        const int rows = min(32, n - 32 * s), each = sl.n ? n : per;
-        for (int e = tid; e < rows * each; e += 64 * NT) {
-            const int rr = e / each, f = e - rr * each, u = 32 * s + rr;
-            const int node = u / g, r = u - node * g, i = node / x.ny, j = node - i * x.ny;
-            int t;
-            if (sl.n)                                // self links couple whole faces
-                t = f;
-            else if (f < g)
-                t = node * g + f;
-            else if (f < g + x.nx - 1) {
-                const int p = f - g, pi = p + (p >= i);
-                t = (pi * x.ny + j) * g + r;
-            } else {
-                const int p = f - g - (x.nx - 1), pj = p + (p >= j);
-                t = (i * x.ny + pj) * g + r;
-            }
-            const int tn = t / g;
-            buf[rr * SS + t] = T(bj_entry(m, x, sl, cth, sth, tn * x.nth + a0 + (t - tn * g),
-                                          node * x.nth + a0 + r));
-        }
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -598,6 +641,10 @@ void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
                     acc[2 * s + h][v] = buf[(16 * h + Mma::row(lg, v)) * SS + 16 * wave + l16];
             }
         __syncthreads();
+        if (2 * s + 2 < NT) {
+            entries(s, [&](int o, int, int, int, int, int, int) { buf[o] = T(0); });
+            __syncthreads();
+        }
     }
     // Panel p of another wave: update this wave's tile.
     auto update = [&](int p) {
@@ -676,15 +723,81 @@ void k_bj_build_reg(DevMesh m, int restrict_, const int64_t *inv_off,
 #pragma unroll 1
     for (int p = wave + 1; p < NT; ++p) update(p);
     __syncthreads();
+    if (failed) return;
     const int j = 16 * wave + l16;
-    if (failed || j >= n) return;
-    T *o = out + inv_off[b] + perm[j];
+    if constexpr (BITS == 0) {
+        if (j >= n) return;
+        T *o = out + inv_off[b] + perm[j];
 #pragma unroll
-    for (int rt = 0; rt < NT; ++rt) {
-        const uint32_t qs = *reinterpret_cast<const uint32_t *>(q + lg * 32 + rt * 4);
+        for (int rt = 0; rt < NT; ++rt) {
+            const uint32_t qs = *reinterpret_cast<const uint32_t *>(q + lg * 32 + rt * 4);
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (16 * rt + Mma::row(lg, v) < n) o[size_t((qs >> (8 * v)) & 255u) * n] = acc[rt][v];
+            for (int v = 0; v < 4; ++v)
+                if (16 * rt + Mma::row(lg, v) < n) o[size_t((qs >> (8 * v)) & 255u) * n] = acc[rt][v];
+        }
+    } else {
+        // largest magnitude of each row i of M (column q_i of the inverse):
+        // over a wave's 16 columns, then over the waves; columns past the
+        // block are zero there
+        static_assert(NT * 17 * 16 >= NT * NR, "row maxima of every wave fit piv");
+        static_assert(NR * NR <= int(sizeof(buf)), "the code image fits the panel buffers");
+        static_assert(NR * 4 <= int(sizeof(Dx)), "the scales fit Dx");
+        float *const mx = reinterpret_cast<float *>(piv);
+        float *const inv_s = reinterpret_cast<float *>(Dx);
+        uint8_t *const img = reinterpret_cast<uint8_t *>(buf);
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float a = fabsf(acc[rt][v]);
+#pragma unroll
+                for (int o = 8; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o, 16));
+                if (l16 == 0) mx[wave * NR + 16 * rt + Mma::row(lg, v)] = a;
+            }
+        __syncthreads();
+        for (int i = tid; i < NR; i += 64 * NT) {
+            float a = 0.f;
+#pragma unroll
+            for (int w = 0; w < NT; ++w) a = fmaxf(a, mx[w * NR + i]);
+            const float sc = a > 0.f ? a / (BITS == 8 ? 448.f : 6.f) : 1.f;
+            inv_s[i] = 1.f / sc;
+            if (i < n) scales[soff[b] + q[Mma::slot(i)]] = sc;
+        }
+        __syncthreads();
+        // one code per byte at [column q_i][row p_j] of the inverse; rows
+        // past the block are zero in M, so they get code 0
+        const int pj = perm[j];
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt) {
+            const uint32_t qs = *reinterpret_cast<const uint32_t *>(q + lg * 32 + rt * 4);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = 16 * rt + Mma::row(lg, v);
+                const float f = acc[rt][v] * inv_s[i];
+                const uint32_t cd = BITS == 8 ? uint32_t(bj_to_e4m3(f)) : bj_to_e2m1(f);
+                img[((qs >> (8 * v)) & 255u) * NR + pj] = uint8_t(cd);
+            }
+        }
+        __syncthreads();
+        const uint4 *I = reinterpret_cast<const uint4 *>(img);
+        if constexpr (BITS == 8) {
+            uint4 *D = reinterpret_cast<uint4 *>(out + inv_off[b]);
+            for (int e = tid; e < n * NT; e += 64 * NT) D[e] = I[e];
+        } else {
+            // bytes 2 t and 2 t + 1 -> the nibbles of byte t
+            auto two = [](uint32_t lo, uint32_t hi) {
+                auto half = [](uint32_t w) {
+                    w |= w >> 4;
+                    return (w & 0xffu) | ((w >> 8) & 0xff00u);
+                };
+                return half(lo) | (half(hi) << 16);
+            };
+            uint2 *D = reinterpret_cast<uint2 *>(out + inv_off[b] / 2);
+            for (int e = tid; e < n * NT; e += 64 * NT) {
+                const uint4 w = I[e];
+                D[e] = make_uint2(two(w.x, w.y), two(w.z, w.w));
+            }
+        }
     }
 }
 
@@ -821,30 +934,6 @@ __global__ __launch_bounds__(NT) void k_bj_apply_bf16(DevMesh m, const int64_t *
     }
 }
 
-// FP8 e4m3 (bias 7, largest finite 448, no infinities): nearest code,
-// ties to even; |v| above 448 saturates.
-__device__ inline uint8_t bj_to_e4m3(float v) {
-    const uint8_t sgn = v < 0.f ? 0x80 : 0;
-    const float a = fabsf(v);
-    if (!(a > 0.f)) return sgn;
-    if (a >= 448.f) return sgn | 0x7E;
-    int e;
-    (void)frexpf(a, &e);                       // a = f 2^e, f in [0.5, 1)
-    int E = e - 1;                             // a = (1 + m / 8) 2^E for normals
-    if (E < -6) {                              // subnormals: m 2^-9
-        const int mq = int(rintf(a * 512.f));
-        return sgn | uint8_t(mq >= 8 ? 8 : mq);
-    }
-    int mq = int(rintf((ldexpf(a, -E) - 1.f) * 8.f));
-    if (mq == 8) {
-        mq = 0;
-        ++E;
-    }
-    const int eb = E + 7;
-    if (eb > 15 || (eb == 15 && mq > 6)) return sgn | 0x7E;
-    return sgn | uint8_t((eb << 3) | mq);
-}
-
 // Column scales of one block for the coded copies: scale_j = max_i |B_ij| /
 // div (1 for an all-zero column) into sc[j] and its reciprocal into inv_s[j].
 // One wavefront per column: coalesced loads of the column and a shuffle
@@ -887,26 +976,6 @@ __global__ __launch_bounds__(BJ_THREADS) void k_bj_pack_fp8(DevMesh m, const int
         const int j = e / ldp, i = e % ldp;
         D[e] = i < n ? bj_to_e4m3(S[size_t(j) * n + i] * inv_s[j]) : uint8_t(0);
     }
-}
-
-// FP4 e2m1 (OCP: bias 1, one mantissa bit, largest 6, no infinities or
-// NaN; magnitudes 0, 0.5, 1, 1.5, 2, 3, 4, 6 for codes 0..7): nearest code,
-// ties to the even code; |v| above 6 saturates.
-__device__ inline uint32_t bj_to_e2m1(float v) {
-    const uint32_t sgn = v < 0.f ? 8u : 0u;
-    const float a = fabsf(v);
-    // midpoints between consecutive magnitudes; at a midpoint the even code
-    // (0, 2, 4, 6) wins
-    uint32_t c;
-    if (a <= 0.25f) c = 0;
-    else if (a < 0.75f) c = 1;
-    else if (a <= 1.25f) c = 2;
-    else if (a < 1.75f) c = 3;
-    else if (a <= 2.5f) c = 4;
-    else if (a < 3.5f) c = 5;
-    else if (a <= 5.f) c = 6;
-    else c = 7;
-    return sgn | c;
 }
 
 // FP4 copy of block b: the FP8 copy's layout at half the bytes (column j's
@@ -1152,6 +1221,11 @@ using namespace rtx;
 
 extern "C" int rtx_bjacobi_size(rtx_plan *p, int64_t *n_entries) {
     RTX_CHECK(p && n_entries, "rtx_bjacobi_size: null argument");
+    const int split = (p->bj_method != 0) ? 1 : 0;
+    if (p->bj_off && p->bj_split == split) {      // the plan's mesh never changes
+        *n_entries = p->bj_entries;
+        return RTX_OK;
+    }
     std::vector<int32_t> nx(p->m.ncol), ny(p->m.ncol), cc(p->m.ncell), nt(p->m.ncell);
     RTX_HIP(hipMemcpy(nx.data(), p->m.col_nx, nx.size() * 4, hipMemcpyDeviceToHost));
     RTX_HIP(hipMemcpy(ny.data(), p->m.col_ny, ny.size() * 4, hipMemcpyDeviceToHost));
@@ -1159,7 +1233,6 @@ extern "C" int rtx_bjacobi_size(rtx_plan *p, int64_t *n_entries) {
     RTX_HIP(hipMemcpy(nt.data(), p->m.cell_nth, nt.size() * 4, hipMemcpyDeviceToHost));
     std::vector<int32_t> dof0(p->m.ncell);
     RTX_HIP(hipMemcpy(dof0.data(), p->m.cell_dof_off, dof0.size() * 4, hipMemcpyDeviceToHost));
-    const int split = (p->bj_method != 0) ? 1 : 0;
     std::vector<int32_t> blk, apd, cls[BJ_NCLS];
     std::vector<int64_t> off(1, 0), off16(1, 0), off8(1, 0), soff(1, 0);
     int32_t maxb = 0;
@@ -1184,47 +1257,46 @@ extern "C" int rtx_bjacobi_size(rtx_plan *p, int64_t *n_entries) {
             maxb = std::max<int32_t>(maxb, int32_t(n));
         }
     }
-    if (p->bj_split != split || !p->bj_off) {
-        if (p->bj_off) RTX_HIP(hipFree(p->bj_off));
-        if (p->bj_off16) RTX_HIP(hipFree(p->bj_off16));
-        if (p->bj_off8) RTX_HIP(hipFree(p->bj_off8));
-        if (p->bj_soff) RTX_HIP(hipFree(p->bj_soff));
-        if (p->bj_blk) RTX_HIP(hipFree(p->bj_blk));
-        if (p->bj_apd) RTX_HIP(hipFree(p->bj_apd));
-        if (p->bj_cls) RTX_HIP(hipFree(p->bj_cls));
-        p->bj_off = p->bj_off16 = p->bj_off8 = p->bj_soff = nullptr;
-        p->bj_blk = p->bj_apd = p->bj_cls = nullptr;
-        RTX_HIP(hipMalloc(&p->bj_off, off.size() * sizeof(int64_t)));
-        RTX_HIP(hipMemcpy(p->bj_off, off.data(), off.size() * sizeof(int64_t),
-                          hipMemcpyHostToDevice));
-        RTX_HIP(hipMalloc(&p->bj_off16, off16.size() * sizeof(int64_t)));
-        RTX_HIP(hipMemcpy(p->bj_off16, off16.data(), off16.size() * sizeof(int64_t),
-                          hipMemcpyHostToDevice));
-        RTX_HIP(hipMalloc(&p->bj_off8, off8.size() * sizeof(int64_t)));
-        RTX_HIP(hipMemcpy(p->bj_off8, off8.data(), off8.size() * sizeof(int64_t),
-                          hipMemcpyHostToDevice));
-        RTX_HIP(hipMalloc(&p->bj_soff, soff.size() * sizeof(int64_t)));
-        RTX_HIP(hipMemcpy(p->bj_soff, soff.data(), soff.size() * sizeof(int64_t),
-                          hipMemcpyHostToDevice));
-        RTX_HIP(hipMalloc(&p->bj_blk, blk.size() * sizeof(int32_t)));
-        RTX_HIP(hipMemcpy(p->bj_blk, blk.data(), blk.size() * sizeof(int32_t),
-                          hipMemcpyHostToDevice));
-        RTX_HIP(hipMalloc(&p->bj_apd, apd.size() * sizeof(int32_t)));
-        RTX_HIP(hipMemcpy(p->bj_apd, apd.data(), apd.size() * sizeof(int32_t),
-                          hipMemcpyHostToDevice));
-        std::vector<int32_t> all;
-        for (int q = 0; q < BJ_NCLS; ++q) {
-            p->bj_cls_start[q] = int32_t(all.size());
-            all.insert(all.end(), cls[q].begin(), cls[q].end());
-        }
-        p->bj_cls_start[BJ_NCLS] = int32_t(all.size());
-        RTX_HIP(hipMalloc(&p->bj_cls, std::max<size_t>(all.size(), 1) * sizeof(int32_t)));
-        if (!all.empty())
-            RTX_HIP(hipMemcpy(p->bj_cls, all.data(), all.size() * sizeof(int32_t),
-                              hipMemcpyHostToDevice));
-        p->bj_split = split;
-        p->bj_ready = false;
+    p->bj_split = -1;
+    if (p->bj_off) RTX_HIP(hipFree(p->bj_off));
+    if (p->bj_off16) RTX_HIP(hipFree(p->bj_off16));
+    if (p->bj_off8) RTX_HIP(hipFree(p->bj_off8));
+    if (p->bj_soff) RTX_HIP(hipFree(p->bj_soff));
+    if (p->bj_blk) RTX_HIP(hipFree(p->bj_blk));
+    if (p->bj_apd) RTX_HIP(hipFree(p->bj_apd));
+    if (p->bj_cls) RTX_HIP(hipFree(p->bj_cls));
+    p->bj_off = p->bj_off16 = p->bj_off8 = p->bj_soff = nullptr;
+    p->bj_blk = p->bj_apd = p->bj_cls = nullptr;
+    RTX_HIP(hipMalloc(&p->bj_off, off.size() * sizeof(int64_t)));
+    RTX_HIP(hipMemcpy(p->bj_off, off.data(), off.size() * sizeof(int64_t),
+                      hipMemcpyHostToDevice));
+    RTX_HIP(hipMalloc(&p->bj_off16, off16.size() * sizeof(int64_t)));
+    RTX_HIP(hipMemcpy(p->bj_off16, off16.data(), off16.size() * sizeof(int64_t),
+                      hipMemcpyHostToDevice));
+    RTX_HIP(hipMalloc(&p->bj_off8, off8.size() * sizeof(int64_t)));
+    RTX_HIP(hipMemcpy(p->bj_off8, off8.data(), off8.size() * sizeof(int64_t),
+                      hipMemcpyHostToDevice));
+    RTX_HIP(hipMalloc(&p->bj_soff, soff.size() * sizeof(int64_t)));
+    RTX_HIP(hipMemcpy(p->bj_soff, soff.data(), soff.size() * sizeof(int64_t),
+                      hipMemcpyHostToDevice));
+    RTX_HIP(hipMalloc(&p->bj_blk, blk.size() * sizeof(int32_t)));
+    RTX_HIP(hipMemcpy(p->bj_blk, blk.data(), blk.size() * sizeof(int32_t),
+                      hipMemcpyHostToDevice));
+    RTX_HIP(hipMalloc(&p->bj_apd, apd.size() * sizeof(int32_t)));
+    RTX_HIP(hipMemcpy(p->bj_apd, apd.data(), apd.size() * sizeof(int32_t),
+                      hipMemcpyHostToDevice));
+    std::vector<int32_t> all;
+    for (int q = 0; q < BJ_NCLS; ++q) {
+        p->bj_cls_start[q] = int32_t(all.size());
+        all.insert(all.end(), cls[q].begin(), cls[q].end());
     }
+    p->bj_cls_start[BJ_NCLS] = int32_t(all.size());
+    RTX_HIP(hipMalloc(&p->bj_cls, std::max<size_t>(all.size(), 1) * sizeof(int32_t)));
+    if (!all.empty())
+        RTX_HIP(hipMemcpy(p->bj_cls, all.data(), all.size() * sizeof(int32_t),
+                          hipMemcpyHostToDevice));
+    p->bj_split = split;
+    p->bj_ready = false;
     p->bj_nblk = int32_t(blk.size() / 3);
     p->bj_max_block = maxb;
     p->bj_entries = off.back();
@@ -1304,6 +1376,45 @@ extern "C" int rtx_bjacobi_pack_bf16(rtx_plan *p, const float *d_inv32, uint16_t
     return RTX_OK;
 }
 
+// The register build, each size class (steps of 16 DOFs, one wave per 16) on
+// the kernel that holds it, the largest blocks first: the small classes fill
+// the tail.
+template <typename T, int BITS, typename O>
+static void launch_bj_build(const rtx_plan *p, int restrict_interior, const int64_t *off, O *out,
+                            float *scales, int *d_status, hipStream_t st) {
+    const int32_t *cs = p->bj_cls, *c0 = p->bj_cls_start;
+    auto build = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        const int cnt = c0[NT] - c0[NT - 1];
+        if (cnt)
+            k_bj_build_reg<NT, T, BITS><<<cnt, 64 * NT, 0, st>>>(
+                p->m, restrict_interior, off, p->bj_blk, cs + c0[NT - 1], out, p->bj_soff, scales,
+                d_status);
+    };
+    build(std::integral_constant<int, 8>());
+    build(std::integral_constant<int, 7>());
+    build(std::integral_constant<int, 6>());
+    build(std::integral_constant<int, 5>());
+    build(std::integral_constant<int, 4>());
+    build(std::integral_constant<int, 3>());
+    build(std::integral_constant<int, 2>());
+    build(std::integral_constant<int, 1>());
+}
+
+// Wait for a build and read its status: the 1-based cell of a singular block.
+static int bj_build_status(rtx_plan *p, int *d_status, hipStream_t st, const char *who) {
+    int h_status = 0;
+    RTX_HIP(hipMemcpyAsync(&h_status, d_status, sizeof(int), hipMemcpyDeviceToHost, st));
+    RTX_HIP(hipStreamSynchronize(st));
+    RTX_HIP(hipFreeAsync(d_status, st));
+    if (h_status) {
+        set_error("%s: singular diagonal block in cell %d", who, h_status - 1);
+        return RTX_ERR_NUMERIC;
+    }
+    p->bj_ready = true;
+    return RTX_OK;
+}
+
 extern "C" int rtx_bjacobi_factor(rtx_plan *p, int restrict_interior, double *d_inv,
                                   float *d_inv_f32, double *d_scratch, void *stream) {
     RTX_CHECK(p && (d_inv || d_inv_f32), "rtx_bjacobi_factor: null argument");
@@ -1337,32 +1448,10 @@ extern "C" int rtx_bjacobi_factor(rtx_plan *p, int restrict_interior, double *d_
                   (long long)nmax);
         return RTX_ERR_ARG;
     }
-    if (reg) {
-        // each size class (steps of 16 DOFs, one wave per 16) on the kernel that holds it
-        const int32_t *cs = p->bj_cls, *c0 = p->bj_cls_start;
-        auto cnt = [&](int q) { return c0[q + 1] - c0[q]; };
-        auto run = [&](auto *out) {
-            using T = typename std::remove_pointer<decltype(out)>::type;
-            auto build = [&](auto nt) {
-                constexpr int NT = decltype(nt)::value;
-                if (cnt(NT - 1))
-                    k_bj_build_reg<NT, T><<<cnt(NT - 1), 64 * NT, 0, st>>>(
-                        p->m, restrict_interior, p->bj_off, p->bj_blk, cs + c0[NT - 1], out, d_status);
-            };
-            // the largest blocks first: the small classes fill the tail
-            build(std::integral_constant<int, 8>());
-            build(std::integral_constant<int, 7>());
-            build(std::integral_constant<int, 6>());
-            build(std::integral_constant<int, 5>());
-            build(std::integral_constant<int, 4>());
-            build(std::integral_constant<int, 3>());
-            build(std::integral_constant<int, 2>());
-            build(std::integral_constant<int, 1>());
-        };
-        if (f32_only)
-            run(d_inv_f32);
-        else
-            run(d_inv);
+    if (reg && f32_only)
+        launch_bj_build<float, 0>(p, restrict_interior, p->bj_off, d_inv_f32, nullptr, d_status, st);
+    else if (reg) {
+        launch_bj_build<double, 0>(p, restrict_interior, p->bj_off, d_inv, nullptr, d_status, st);
     } else if (p->bj_method == 1) {
         (void)hipFreeAsync(d_status, st);
         set_error("rtx_bjacobi_factor: the register build handles blocks of up to 128 DOFs, "
@@ -1387,16 +1476,37 @@ extern "C" int rtx_bjacobi_factor(rtx_plan *p, int restrict_interior, double *d_
     RTX_HIP(hipGetLastError());
     if (d_inv_f32 && !f32_only)
         k_to_f32_bj<<<2048, 256, 0, st>>>(d_inv, d_inv_f32, p->bj_entries);
-    int h_status = 0;
-    RTX_HIP(hipMemcpyAsync(&h_status, d_status, sizeof(int), hipMemcpyDeviceToHost, st));
-    RTX_HIP(hipStreamSynchronize(st));
-    RTX_HIP(hipFreeAsync(d_status, st));
-    if (h_status) {
-        set_error("rtx_bjacobi_factor: singular diagonal block in cell %d", h_status - 1);
-        return RTX_ERR_NUMERIC;
+    return bj_build_status(p, d_status, st, "rtx_bjacobi_factor");
+}
+
+extern "C" int rtx_bjacobi_factor_coded(rtx_plan *p, int restrict_interior, int precision,
+                                        uint8_t *d_codes, void *stream) {
+    RTX_CHECK(p && d_codes, "rtx_bjacobi_factor_coded: null argument");
+    RTX_CHECK(precision == RTX_PREC_FP8 || precision == RTX_PREC_FP4,
+              "rtx_bjacobi_factor_coded: precision must be RTX_PREC_FP8 or RTX_PREC_FP4, not %d",
+              precision);
+    if (!p->has_coeffs) {
+        set_error("rtx_bjacobi_factor_coded: coefficients not set");
+        return RTX_ERR_STATE;
     }
-    p->bj_ready = true;
-    return RTX_OK;
+    int64_t n;
+    if (const int rc = rtx_bjacobi_size(p, &n)) return rc;
+    RTX_CHECK(p->bj_method != 0 && p->bj_max_block <= BJ_SPLIT,
+              "rtx_bjacobi_factor_coded: the FP32-only factorisation needs the register build "
+              "(blocks of up to 128 DOFs, method -1 or 1); blocks of %d DOFs",
+              int(p->bj_max_block));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    int *d_status = nullptr;
+    RTX_HIP(hipMallocAsync((void **)&d_status, sizeof(int), st));
+    RTX_HIP(hipMemsetAsync(d_status, 0, sizeof(int), st));
+    if (precision == RTX_PREC_FP8)
+        launch_bj_build<float, 8>(p, restrict_interior, p->bj_off8, d_codes,
+                                  reinterpret_cast<float *>(d_codes + p->bj_codes8), d_status, st);
+    else
+        launch_bj_build<float, 4>(p, restrict_interior, p->bj_off8, d_codes,
+                                  reinterpret_cast<float *>(d_codes + p->bj_codes4), d_status, st);
+    RTX_HIP(hipGetLastError());
+    return bj_build_status(p, d_status, st, "rtx_bjacobi_factor_coded");
 }
 
 extern "C" int rtx_bjacobi_set_method(rtx_plan *p, int method) {

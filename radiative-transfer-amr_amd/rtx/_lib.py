@@ -66,6 +66,7 @@ SIGNATURES = [
     ("rtx_bjacobi_size", C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]),
     ("rtx_bjacobi_factor", C.c_int, [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p,
                                      C.c_void_p]),
+    ("rtx_bjacobi_factor_coded", C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p]),
     ("rtx_bjacobi_set_method", C.c_int, [C.c_void_p, C.c_int]),
     ("rtx_bjacobi_size_bf16", C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]),
     ("rtx_bjacobi_size_fp8", C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]),

@@ -67,6 +67,11 @@ class BlockJacobi:
         check(self.lib.rtx_bjacobi_size(op.plan, C.byref(n)), "rtx_bjacobi_size")
         self.entries = int(n.value)
         dev = op.device
+        self.inv = self.inv32 = self.inv16 = self.inv8 = self.inv4 = None
+        self.entries16 = self.bytes8 = self.bytes4 = 0
+        if (keep_fp8 != keep_fp4 and not (keep_f64 or keep_f32 or keep_bf16)
+                and self._factor_coded(restrict, PREC_FP8 if keep_fp8 else PREC_FP4)):
+            return
         # BF16 / FP8 / FP4 are rounded from FP32
         need32 = keep_f32 or keep_bf16 or keep_fp8 or keep_fp4
         self.inv32 = torch.empty(self.entries, dtype=torch.float32, device=dev) if need32 else None
@@ -75,7 +80,6 @@ class BlockJacobi:
         if need32 and not keep_f64:
             # no FP64 copy wanted: eliminate in FP32 straight into inv32
             # (register build, blocks of up to 128 DOFs; else the FP64 path)
-            self.inv = None
             rc = self.lib.rtx_bjacobi_factor(op.plan, 1 if restrict else 0, None,
                                              _vp(self.inv32), None, st)
             if rc != 0 and not (rc == -1 and b"FP32-only" in self.lib.rtx_last_error()):
@@ -91,8 +95,6 @@ class BlockJacobi:
                                              _vp(scratch), st)
             del scratch
         check(rc, "rtx_bjacobi_factor")
-        self.inv16 = None
-        self.entries16 = 0
         if keep_bf16:
             n16 = C.c_int64()
             check(self.lib.rtx_bjacobi_size_bf16(op.plan, C.byref(n16)), "rtx_bjacobi_size_bf16")
@@ -101,8 +103,6 @@ class BlockJacobi:
             self.inv16 = torch.empty(self.entries16, dtype=torch.int16, device=dev)
             check(self.lib.rtx_bjacobi_pack_bf16(op.plan, _vp(self.inv32), _vp(self.inv16), st),
                   "rtx_bjacobi_pack_bf16")
-        self.inv8 = None
-        self.bytes8 = 0
         if keep_fp8:
             n8 = C.c_int64()
             check(self.lib.rtx_bjacobi_size_fp8(op.plan, C.byref(n8)), "rtx_bjacobi_size_fp8")
@@ -111,8 +111,6 @@ class BlockJacobi:
             self.inv8 = torch.empty(self.bytes8, dtype=torch.uint8, device=dev)
             check(self.lib.rtx_bjacobi_pack_fp8(op.plan, _vp(self.inv32), _vp(self.inv8), st),
                   "rtx_bjacobi_pack_fp8")
-        self.inv4 = None
-        self.bytes4 = 0
         if keep_fp4:
             n4 = C.c_int64()
             check(self.lib.rtx_bjacobi_size_fp4(op.plan, C.byref(n4)), "rtx_bjacobi_size_fp4")
@@ -128,6 +126,24 @@ class BlockJacobi:
                 self.inv32 = None
         if not keep_f64:
             self.inv = None
+
+    def _factor_coded(self, restrict, precision):
+        """One reduced-precision copy alone: eliminated in FP32 and rounded
+        to its codes in one pass, with no FP32 pool.  False when a block has
+        more than 128 DOFs."""
+        size, name = {PREC_FP8: (self.lib.rtx_bjacobi_size_fp8, "8"),
+                      PREC_FP4: (self.lib.rtx_bjacobi_size_fp4, "4")}[precision]
+        nb = C.c_int64()
+        check(size(self.op.plan, C.byref(nb)), "rtx_bjacobi_size_fp" + name)
+        pool = torch.empty(int(nb.value), dtype=torch.uint8, device=self.op.device)
+        rc = self.lib.rtx_bjacobi_factor_coded(self.op.plan, 1 if restrict else 0, precision,
+                                               _vp(pool), stream_handle())
+        if rc == -1 and b"FP32-only" in self.lib.rtx_last_error():
+            return False
+        check(rc, "rtx_bjacobi_factor_coded")
+        setattr(self, "inv" + name, pool)
+        setattr(self, "bytes" + name, int(nb.value))
+        return True
 
     def bytes_per_apply(self, precision=PREC_F64):
         if precision == PREC_MIXED:

@@ -619,7 +619,17 @@ def test_block_jacobi_build_sizes(cuda, n, self_links):
         assert err <= 8 * m * 2.0 ** -53 * np.linalg.cond(inv), (m, err)
         off += m * m
     assert off == inv64.size
-    _device_inverses(BlockJacobi(op, keep_f64=False, keep_f32=True), blocks, invs)
+    # the FP8 / FP4 pools of the one-pass build: the bytes of the separate
+    # quantisation of the FP32 inverses
+    two = BlockJacobi(op, keep_f64=False, keep_f32=True, keep_fp8=True, keep_fp4=True)
+    _device_inverses(two, blocks, invs)
+    for one, ref in ((BlockJacobi(op, keep_f64=False, keep_fp8=True).inv8, two.inv8),
+                     (BlockJacobi(op, keep_f64=False, keep_fp4=True).inv4, two.inv4)):
+        # without the gap between the codes and the 16-byte aligned scales
+        ncodes = sum(len(i) * ((len(i) + 15) // 16 * 16) for i in blocks) // (1 if ref is two.inv8 else 2)
+        gap = (-ncodes) % 16
+        assert bool((one[:ncodes] == ref[:ncodes]).all())
+        assert bool((one[ncodes + gap:] == ref[ncodes + gap:]).all())
 
 
 @pytest.mark.gpu
