@@ -662,9 +662,7 @@ extern "C" int rtx_plan_info(const rtx_plan *p, int64_t *out, int n) {
     v[20] = p->n_gen_cols;
     v[21] = p->n_gen_cells;
     v[22] = p->hp_default ? 1 : 0;
-    int hp_cols = 0;
-    for (int k = 0; k < HP_NCLS; ++k) hp_cols += p->hp_cls[k].n;
-    v[23] = hp_cols;
+    v[23] = p->hp_ncols;
     v[24] = (p->uni_ok && p->uni_H == 0 && p->m.ncol <= 4 * p->n_cu) ? 1 : 0;
     for (int i = 0; i < NV && i < n && out; ++i) out[i] = v[i];
     return NV;

@@ -1,41 +1,45 @@
-// Matrix-free DG transport operator for uneven-order hp meshes: one fused
-// pass per spatial column.
+// Matrix-free DG transport operator for uneven-order hp meshes: two kernels.
 //
 // A column's DOFs are contiguous in the reference's global order (columns by
-// key, cells by key, then beta = nth ny i + nth j + a inside a cell).  One
-// workgroup of 512 threads owns one column of N x N spatial nodes:
+// key, cells by key, then beta = nth ny i + nth j + a inside a cell).
 //
-//   phase 0  the column's cell, angle, node and link tables -> LDS
-//   phase 1  x of the column -> LDS, angle-major (row = column angle A, one
-//            entry per spatial node; inflow-boundary DOFs zeroed; mixed
-//            precision also keeps a node-major BF16 copy for the matrix-core
-//            operands), and, for every upwind link, the neighbour's trace
-//            contracted with E^theta over the neighbour's angles:
-//            inn[m1, r] = sum_a E^th[a, r] tr[m1, a]
-//            (boundary_convection_matrix.py:348-524, the angular half), then
-//            with E^s over the neighbour's face nodes, summed over the links
-//            of each cell face: one value per (cell, face, face node, angle)
-//   phase 2  each wavefront takes (tile of 16 output angles R, group of
-//            node tiles) items: it accumulates the scattering contraction
-//            sum_A x[s, A] G^T[A, R] on the matrix cores
-//            (scattering_matrix.py:142-237), then, in the accumulator layout,
-//            adds for each of its (s, R) the mass (mass_matrix.py:140-173),
-//            interior convection (interior_convection_matrix.py:161-243), the
-//            outflow faces (boundary_convection_matrix.py:284-346) and the
-//            inflow-face sums of the node's faces, and stores y.
+//   k_hp_flux  the upwind face coupling (boundary_convection_matrix.py:
+//              348-524).  One wavefront per cell, no LDS: for every link the
+//              neighbour's trace is contracted with E^theta over the
+//              neighbour's angles, then with E^s over its face nodes, both on
+//              the matrix cores with operands read from memory; the links of
+//              a face add up in the accumulators.  The sums of the cell's
+//              inflow faces are stored at their DOFs of y.
+//   k_hpcol    everything else, one workgroup of 512 threads per column of
+//              N x N nodes: x of the column -> LDS (angle-major); each
+//              wavefront owns 16 output angles R and every node: it
+//              accumulates the scattering sum_A x[s, A] G^T[A, R] on the
+//              matrix cores (scattering_matrix.py:142-237), then adds mass
+//              (mass_matrix.py:140-173), interior convection
+//              (interior_convection_matrix.py:161-243), the outflow faces
+//              (boundary_convection_matrix.py:284-346) and the sums that
+//              k_hp_flux left in y, and stores y.
 //
-// Phases 1 and 2 are compiled per node count N (3..10), so the line reads of
-// the derivative terms and the E^s rows have compile-time offsets.  Every
-// output has one owner and a fixed order of additions, so results are
+// The two share no workspace: y itself carries the face sums from one to the
+// other, so concurrent applies on several streams stay independent.
+//
+// The nodes are the rows of the scattering product in an order of our own: a
+// lane's accumulators are whole lines of nodes (x-lines q = lane group,
+// lane group + 4, ..), so the derivative along x reads a line once for all of
+// its outputs, with the derivative matrix in scalar registers, and the
+// derivative along y reads each row of nodes once per line.  That is about 6
+// LDS reads per output; evaluated output by output it was about 30, and the
+// LDS pipe was what bounded the column.
+//
+// Every output has one owner and a fixed order of additions, so results are
 // bit-reproducible; x is read from HBM once (plus the neighbours' face
-// traces), G once and y written once.  Columns are grouped by the LDS they
-// need into two launches, so columns of up to about 70 KB run two
-// workgroups per CU.  Arithmetic: FP64 (v_mfma_f64_16x16x4f64), FP32
+// traces), G once, y written once (plus the face sums).  Columns are grouped
+// by LDS need into two classes (one launch each) sized so that the first runs
+// two workgroups per CU.  Arithmetic: FP64 (v_mfma_f64_16x16x4f64), FP32
 // (v_mfma_f32_16x16x4f32) or mixed (FP32 transport terms, BF16 scattering
 // operands on v_mfma_f32_16x16x16bf16_1k with FP32 accumulation).
 #include <algorithm>
 #include <type_traits>
-#include <utility>
 
 #include "rtx_internal.h"
 
@@ -44,14 +48,9 @@ namespace rtx {
 constexpr int HP_THREADS = 512;
 constexpr int HP_WAVES = HP_THREADS / 64;
 constexpr int HP_NM = RTX_NMAX;
-constexpr int HP_MT = (RTX_NMAX * RTX_NMAX + 15) / 16;   // node tiles of 16
 constexpr int HP_XCD = 8;
-constexpr int HP_TG = 2;          // node tiles per scattering pass (accumulators in registers)
 constexpr int HP_NMIN = 3;        // node counts compiled for the column kernel
-constexpr int HP_FV = 8;          // inflow-face sums per thread (a column holds <= HP_FV * HP_THREADS)
-constexpr int HP_LINK_LOG = 8;    // 2^8 >= HP_MAX_LINKS
-constexpr int HP_CELL_LOG = 6;    // 2^6 >= HP_MAX_CELLS
-static_assert((1 << HP_LINK_LOG) >= HP_MAX_LINKS && (1 << HP_CELL_LOG) >= HP_MAX_CELLS, "search range");
+constexpr int HP_WD = HP_NM + HP_NM * HP_NM;   // one n's entry of the line tables
 
 typedef double hp_d4 __attribute__((ext_vector_type(4)));
 typedef float hp_f4 __attribute__((ext_vector_type(4)));
@@ -72,19 +71,175 @@ __device__ inline uint16_t hp_bf16(float f) {
     return uint16_t(u >> 16);
 }
 
-// Largest i in [0, hi) with starts[i] <= t (starts ascending, starts[0] <= t,
-// hi <= 2^LOG).  A fixed number of steps, so the searches of an unrolled
-// loop's iterations are independent and their LDS reads overlap.
-template <int LOG>
-__device__ inline int hp_find(const int *starts, int hi, int t) {
-    int lo = 0;
-#pragma unroll
-    for (int s = 1 << (LOG - 1); s > 0; s >>= 1) {
-        const int mid = lo + s;
-        if (mid < hi && starts[mid] <= t) lo = mid;
+// 16 x 16 x 4 products.  A operand: row lane % 16, k = lane / 16; B operand:
+// k = lane / 16, column lane % 16; D: column lane % 16, row(lane / 16, v).
+// A D is the next product's B operand as it stands, with k = row(lane / 16, s)
+// in step s.
+template <typename A> struct HpMma;
+template <> struct HpMma<double> {
+    typedef hp_d4 v4;
+    __device__ static v4 step(double a, double b, v4 c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    return lo;
+    __host__ __device__ static int row(int lg, int v) { return lg + 4 * v; }
+    // lane group and register that hold D row r
+    __host__ __device__ static int group(int r) { return r & 3; }
+    __host__ __device__ static int reg(int r) { return r >> 2; }
+};
+template <> struct HpMma<float> {
+    typedef hp_f4 v4;
+    __device__ static v4 step(float a, float b, v4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __host__ __device__ static int row(int lg, int v) { return 4 * lg + v; }
+    __host__ __device__ static int group(int r) { return r >> 2; }
+    __host__ __device__ static int reg(int r) { return r & 3; }
+};
+
+// XCD-aware index: block b runs on XCD b % 8, and XCD j takes the j-th
+// contiguous run of the (key-ordered) work, so neighbouring columns are mostly
+// read through the same L2.  -1 past the end.
+__device__ inline int hp_xcd(int n) {
+    const int per = (n + HP_XCD - 1) / HP_XCD;
+    const int i = (blockIdx.x % HP_XCD) * per + blockIdx.x / HP_XCD;
+    return (int(blockIdx.x / HP_XCD) < per && i < n) ? i : -1;
 }
+
+// ---- the upwind face coupling
+
+constexpr int HF_WAVES = 4;       // cells per workgroup
+
+// v where keep, else 0.  Bits rather than a select: the compiler turns a
+// select of a loaded value into a branch around the load, and a link's loads
+// then wait for each other.
+__device__ inline float hp_keep(float v, bool keep) {
+    return __uint_as_float(__float_as_uint(v) & (keep ? ~0u : 0u));
+}
+__device__ inline double hp_keep(double v, bool keep) {
+    const int k = keep ? ~0 : 0;
+    return __hiloint2double(__double2hiint(v) & k, __double2loint(v) & k);
+}
+
+// One link's operands in matrix-core layout: the neighbour's trace, E^theta
+// and E^s.  Indices past the sizes read the last entry; the trace is zero
+// there (one mask serves both products: the rows past the face's nodes that
+// the first leaves are zero too), and rows and columns past this cell's sizes
+// reach no stored value.  Offsets are 32-bit from uniform bases.
+template <typename A>
+struct HpLink {
+    A tv[3], ev[3], sv[4];
+    int F, n1, nt1;
+};
+
+template <typename T, typename A>
+__device__ __forceinline__ HpLink<A> hp_load_link(const DevMesh &m, const int4 rec, uint32_t N,
+                                                  uint32_t nt, int restrict_, uint32_t l16,
+                                                  uint32_t lg, const T *x) {
+    const uint32_t w = rec.y, n1 = (w >> 2) & 15, nt1 = (w >> 6) & 15, stride = (w >> 10) & 255;
+    HpLink<A> o;
+    o.F = w & 3;
+    o.n1 = n1;
+    o.nt1 = nt1;
+    const uint32_t row = min(l16, n1 - 1);
+    // masked inflow nodes of the neighbour count as zero
+    bool live = l16 < n1;
+    if (restrict_) live = live && !((w >> (18 + row)) & 1);
+    const T *tr = x + rec.x;
+    const double *Et = m.Eth_pool + rec.w, *Es = m.Es_pool + rec.z;
+    const uint32_t r = min(l16, nt - 1), m0 = min(l16, N - 1);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+        const uint32_t a = 4 * s + lg, ac = min(a, nt1 - 1);
+        o.tv[s] = hp_keep(A(tr[row * stride + ac]), live && a < nt1);
+        o.ev[s] = A(Et[ac * nt + r]);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        o.sv[s] = A(Es[min(uint32_t(HpMma<A>::row(lg, s)), n1 - 1) * N + m0]);
+    return o;
+}
+
+// Bound by instructions and latency (cell record -> link record -> operands,
+// then short matrix chains): records of one load each instead of a walk
+// through the mesh tables, no LDS, no branches around loads, and registers
+// for 8 wavefronts per SIMD to cover the chains.  An hp mesh's 34,279 cells
+// (86,793 links) in FP64: 42 us; loading the next link's operands while the
+// current one is multiplied costs two wavefronts per SIMD and measures the
+// same.  In FP32 the links of 1,024 columns of 7 x 7 nodes take 9.4 us.
+template <typename T, typename A>
+__global__ __launch_bounds__(64 * HF_WAVES)
+__attribute__((amdgpu_waves_per_eu(8)))
+void k_hp_flux(DevMesh m, const HpCell *__restrict__ cells, const int4 *__restrict__ links,
+               int ncells, int restrict_, int accumulate, const T *__restrict__ x,
+               T *__restrict__ y) {
+    typedef HpMma<A> Mma;
+    typedef typename Mma::v4 v4;
+    const int blk = hp_xcd((ncells + HF_WAVES - 1) / HF_WAVES);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
+    const int ci = blk * HF_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (blk < 0 || ci >= ncells) return;
+    // the cell's scalars are uniform over the wavefront
+    const HpCell cl = cells[ci];
+    const int nl = cl.w & 255, N = (cl.w >> 8) & 15, nt = (cl.w >> 12) & 15;
+    const int bd = restrict_ ? (cl.w >> 16) & 15 : 0, lf = (cl.w >> 20) & 15;
+    if (nl == 0) return;
+    const v4 zero = v4{0, 0, 0, 0};
+    v4 cur = zero;
+    // A face shares its first node (m0 = 0) with one neighbouring face and its
+    // last with another; the later of the two in face order stores the sum.
+    // c0, c1: the values that an earlier face leaves at face F's first and
+    // last node, [F] (faces 1, 2, 3)
+    A c0[4] = {A(0), A(0), A(0), A(0)}, c1[4] = {A(0), A(0), A(0), A(0)};
+    for (int i = 0; i < nl; ++i) {           // ascending faces
+        const HpLink<A> lk = hp_load_link<T, A>(m, links[cl.l0 + i], N, nt, restrict_, l16, lg, x);
+        // inn[m1, r] = sum_a tr[m1, a] E^theta[a, r], then
+        // sum_m1 E^s[m1, m0] inn[m1, r] onto the face's sums
+        v4 inn = zero;
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+            if (4 * s < lk.nt1) inn = Mma::step(lk.tv[s], lk.ev[s], inn);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (Mma::row(0, s) < lk.n1) cur = Mma::step(lk.sv[s], inn[s], cur);
+        if (i + 1 == nl || (links[cl.l0 + i + 1].y & 3) != lk.F) {
+            const int F = lk.F;
+            cur *= (F & 1) ? A(cl.fy) : A(cl.fx);
+            // the faces at the first and last node: for an x-face the y-faces
+            // 3 and 1, for a y-face the x-faces 2 and 0
+            const int f0 = (F & 1) ? 2 : 3, f1 = (F & 1) ? 0 : 1;
+            const int rgN = Mma::reg(N - 1);
+            const A first = __shfl(cur[0], l16);
+            const A last = __shfl(rgN == 0 ? cur[0] : rgN == 1 ? cur[1] : rgN == 2 ? cur[2] : cur[3],
+                                  Mma::group(N - 1) * 16 + l16);
+            // left for a later face f: at its last node if this is face 0 (an
+            // x-face's p = N - 1) or face 1, at its first if face 2
+            if (F == 0) { c1[1] = last; c1[3] = first; }
+            if (F == 1) c1[2] = first;
+            if (F == 2) c0[3] = first;
+            const A add0 = F == 3 ? c0[3] : A(0);
+            const A add1 = F == 1 ? c1[1] : F == 2 ? c1[2] : F == 3 ? c1[3] : A(0);
+            const bool skip0 = ((bd >> f0) & 1) || (((lf >> f0) & 1) && f0 > F);
+            const bool skip1 = ((bd >> f1) & 1) || (((lf >> f1) & 1) && f1 > F);
+            const int fixed = F < 2 ? N - 1 : 0;
+            const int ms = (F & 1) ? N * nt : nt;
+            T *yf = y + cl.off + ((F & 1) ? fixed * nt : fixed * N * nt) + l16;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if (Mma::row(0, v) >= N) continue;           // uniform
+                const int m0 = Mma::row(lg, v);
+                const bool at0 = m0 == 0, at1 = m0 == N - 1;
+                const A val = cur[v] + (at0 ? add0 : A(0)) + (at1 ? add1 : A(0));
+                if (m0 < N && l16 < nt && !(at0 && skip0) && !(at1 && skip1)) {
+                    T *yp = yf + m0 * ms;
+                    *yp = accumulate ? T(A(*yp) + val) : T(val);
+                }
+            }
+            cur = zero;
+        }
+    }
+}
+
+// ---- the column kernel
 
 // Row stride (elements) of a node-major copy: at least na rounded up to the
 // K step, and congruent to c modulo M, so that the 16 rows x K lanes of one
@@ -96,18 +251,16 @@ __host__ __device__ inline int hp_stride(int na, int kstep, int c, int M) {
 }
 
 struct HpLayout {           // dynamic LDS of one column, in bytes from the base
-    int xs, xb, inn, es, cth, sth, wr, acell, total;
+    int xs, xb, ct, sn, wr, dth, pk, fl, total;
     int S, NA, XSB;         // angle-major row (node) stride, padded angle rows, BF16 stride
 };
 
 // Angle-major copy: NA rows (the column's angles, padded to the K step with
-// zero rows) of S = nsp rounded up to odd entries; the same region first
-// holds the ntr neighbour-trace values of the column's links.  The inn
-// region holds nin = max(ninn, nffc) entries: the E^theta-contracted traces,
-// then the inflow-face sums written over them; the es region the column's
-// nes distinct E^s values.  A: LDS element type.
+// zero rows) of S = nsp rounded up to odd entries, so that lanes on
+// consecutive angles or nodes read distinct banks; mixed adds the node-major
+// BF16 copy.  Then four values and two words per angle.  A: LDS element type.
 template <typename A, int PREC>
-__host__ __device__ inline HpLayout hp_layout(int nsp, int na, int nin, int ntr, int nes) {
+__host__ __device__ inline HpLayout hp_layout(int nsp, int na) {
     HpLayout L;
     const int ea = int(sizeof(A));
     const int kstep = (PREC == RTX_PREC_MIXED) ? 16 : 4;
@@ -116,211 +269,139 @@ __host__ __device__ inline HpLayout hp_layout(int nsp, int na, int nin, int ntr,
     L.XSB = (PREC == RTX_PREC_MIXED) ? hp_stride(na, 16, 8, 16) : 0;
     int o = 0;
     L.xs = o;
-    o += (L.NA * L.S > ntr ? L.NA * L.S : ntr) * ea;
+    o += L.NA * L.S * ea;
     o = (o + 15) & ~15;
     L.xb = o;
     o += nsp * L.XSB * 2;
     o = (o + 15) & ~15;
-    L.inn = o;
-    o += nin * ea;
-    L.es = o;
-    o += nes * ea;
-    L.cth = o;
+    L.ct = o;
     o += na * ea;
-    L.sth = o;
+    L.sn = o;
     o += na * ea;
     L.wr = o;
     o += na * ea;
-    L.acell = o;
+    L.dth = o;
+    o += na * ea;
+    L.pk = o;
+    o += na * 4;
+    L.fl = o;
     o += na * 4;
     L.total = (o + 15) & ~15;
     return L;
 }
 
-// LDS tables of one column (phase 0).
 template <typename A>
 struct HpShared {
-    int c_nth[HP_MAX_CELLS], c_bd[HP_MAX_CELLS], c_lf[HP_MAX_CELLS];
-    int c_quad[HP_MAX_CELLS], c_ao[HP_MAX_CELLS + 1], c_l0[HP_MAX_CELLS + 1];
-    int c_fo[HP_MAX_CELLS + 1];     // offsets of the cells' inflow-face sums
-    A c_dth[HP_MAX_CELLS];
-    int l_w[HP_MAX_LINKS], l_inn[HP_MAX_LINKS + 1], l_es[HP_MAX_LINKS];
-    // per link: packed source shape word (link_meta[4 l + 1]), source cell's
-    // first DOF, E^theta offset, column-local trace offset
-    int l_m1[HP_MAX_LINKS], l_src[HP_MAX_LINKS], l_et[HP_MAX_LINKS], l_tr[HP_MAX_LINKS + 1];
-    A w2k[HP_NM * HP_NM], sgw[HP_NM * HP_NM];
-    A wxs[HP_NM], wys[HP_NM], WDx[HP_NM * HP_NM], WDy[HP_NM * HP_NM];
+    __attribute__((aligned(16))) A nf[2 * HP_NM * HP_NM];   // mass and scattering factor of each node
+    A wd[HP_WD];                                // weights, then w_i l'_p(xi_i) (N x N)
 };
 
-// Phases 1 and 2 of one column of N x N nodes.
+// Operand row i of node tile t of the scattering product: register e = 4 t + v
+// of lane group g holds node p = e % N of line q = g + 4 (l0 + e / N).  Rows
+// past the lines read a valid node; their outputs are not stored.
+template <typename A, int N>
+__device__ inline int hp_node(int t, int i, int l0) {
+    const int e = 4 * t + HpMma<A>::reg(i), q = HpMma<A>::group(i) + 4 * (l0 + e / N);
+    return (e % N) * N + (q < N ? q : N - 1);
+}
+
+// What bounds a column: latency in its phases and the LDS pipe in the lines.
+// FP64, N = 6, 88 angles, two workgroups per CU, cycles: tables and first G
+// rows 7,900, x to LDS 4,200, a wavefront's 16 angles 9,700 (matrix) + 6,600
+// (lines), those of the second round 15,100.  Times of the two kernels
+// together, against one kernel with the contraction's operands in LDS and 30
+// LDS reads per output: hp mesh of 34,279 cells FP64 283 -> 226 us, 9,150
+// cells mixed 87 -> 45 us, 1,024 columns of 7 x 7 nodes FP32 52 -> 35 us.
 template <typename T, typename A, int PREC, int N>
-__device__ __forceinline__ void hp_column(const DevMesh &m, uint32_t ops, int accumulate,
-                                          HpShared<A> &sh, unsigned char *lds, int c, int k0,
-                                          int ncells, int na, int cdof, int L0, int nl,
-                                          int ninn, int nffc, int ntr, int es0, int nes,
-                                          const double *__restrict__ h_es, double dx,
-                                          double dy, const T *__restrict__ x,
+__device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, uint32_t ops,
+                                          int accumulate, HpShared<A> &sh, unsigned char *lds,
+                                          const int32_t *hd, const T *__restrict__ x,
                                           T *__restrict__ y) {
     constexpr int NSP = N * N;
-    constexpr int MT = (NSP + 15) / 16;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // x-lines: NL per lane group, LI of them in one item (16 output angles x
+    // 4 LI lines).  FP64 takes one: with all of them its accumulators leave
+    // too few of the 128 registers of 4 wavefronts per SIMD for the lines
+    // (252 spilled, against 24), and two or three times the items spread
+    // better over the wavefronts; G is then read from L2 once per item.
+    constexpr int NL = (N + 3) / 4;
+    constexpr int LI = sizeof(A) == 8 ? 1 : NL, NI = NL / LI;
+    constexpr int MT = (N * LI + 3) / 4;         // node tiles
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, lg = lane >> 4;
     const bool restrict_ = (ops & RTX_OP_RESTRICT) != 0;
     const bool bconv = (ops & RTX_OP_BCONV) != 0;
+    const int na = hd[3], cdof = hd[4], ga0 = hd[7], sp0 = hd[13], c = hd[14];
     const int ncd = NSP * na;
-    const HpLayout Lo = hp_layout<A, PREC>(NSP, na, ninn > nffc ? ninn : nffc, ntr, nes);
+    const double dx = m.col_geom[4 * c + 2] - m.col_geom[4 * c + 0];
+    const double dy = m.col_geom[4 * c + 3] - m.col_geom[4 * c + 1];
+    const HpLayout Lo = hp_layout<A, PREC>(NSP, na);
     const int S = Lo.S, XSB = Lo.XSB;
     A *xs = reinterpret_cast<A *>(lds + Lo.xs);
     uint16_t *xb = reinterpret_cast<uint16_t *>(lds + Lo.xb);
-    A *inn = reinterpret_cast<A *>(lds + Lo.inn);
-    A *es = reinterpret_cast<A *>(lds + Lo.es);
-    const A *cth = reinterpret_cast<const A *>(lds + Lo.cth);
-    const A *sth = reinterpret_cast<const A *>(lds + Lo.sth);
-    const A *wr = reinterpret_cast<const A *>(lds + Lo.wr);
-    const int *acell = reinterpret_cast<const int *>(lds + Lo.acell);
+    A *ct = reinterpret_cast<A *>(lds + Lo.ct);
+    A *sn = reinterpret_cast<A *>(lds + Lo.sn);
+    A *wr = reinterpret_cast<A *>(lds + Lo.wr);
+    A *dt = reinterpret_cast<A *>(lds + Lo.dth);
+    int *pk = reinterpret_cast<int *>(lds + Lo.pk);
+    int *fl = reinterpret_cast<int *>(lds + Lo.fl);
 
-    // ---- phase 1.  The first batch of x is loaded into registers; while it
-    // is in flight the neighbour traces of the column's links are gathered
-    // into the x region (batched loads), then contracted with E^theta into
-    // inn; then x is written over them, angle-major and masked.  DOF t of
-    // the column lies in the cell of angle t / NSP (cell kk's DOFs start at
-    // NSP * c_ao[kk]).
-    constexpr int XU = 4;                 // x and trace values per thread and pass
+    // ---- the first G rows of this wavefront's first 16 output angles, in
+    // flight through the staging phases.  PD load groups of four K steps (one
+    // of 16 in mixed precision); lanes past the last angle, and rows past it,
+    // read valid addresses: those angle rows of the copy are zero, and those
+    // lanes' outputs are not stored.
+    constexpr int PD = PREC == RTX_PREC_F32 && N <= 7 ? 4 : 2;
+    typedef typename std::conditional<PREC == RTX_PREC_MIXED, uint16_t, A>::type GT;
+    const GT *Gc = PREC == RTX_PREC_MIXED ? (const GT *)(m.G_bf16 + m.col_G_off[c])
+                   : PREC == RTX_PREC_F64 ? (const GT *)(m.G + m.col_G_off[c])
+                                          : (const GT *)(m.G_f + m.col_G_off[c]);
+    struct Group { GT g[4]; };
+    const auto gload = [&](int Rc, int kb) {
+        Group o;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int Ak = kb + (PREC == RTX_PREC_MIXED ? 4 * lg + u : 4 * u + lg);
+            o.g[u] = Gc[size_t(Ak < na ? Ak : na - 1) * na + Rc];
+        }
+        return o;
+    };
+    Group gq[PD];
+    const bool scat = (ops & RTX_OP_SCAT) != 0;
+    if (scat) {
+        const int R = wave / NI * 16 + l16;
+#pragma unroll
+        for (int d = 0; d < PD; ++d) gq[d] = gload(R < na ? R : na - 1, 16 * d);
+    }
+    // ---- x of the column and its tables.  The first batch of x is loaded
+    // while the angles' tables go to LDS.
+    // x values per thread and pass: a column of 96 angles in one
+    constexpr int XU = (NSP * 96 + HP_THREADS - 1) / HP_THREADS < 16 ? (NSP * 96 + HP_THREADS - 1) / HP_THREADS : 16;
     A vv[XU];
 #pragma unroll
     for (int u = 0; u < XU; ++u) {
         const int t = tid + u * HP_THREADS;
         vv[u] = (t < ncd) ? A(x[cdof + t]) : A(0);
     }
-    if (bconv) {
-        // the column's distinct E^s blocks -> LDS (read after two barriers)
-        for (int e = tid; e < nes; e += HP_THREADS) es[e] = A(h_es[es0 + e]);
-        A *tr = xs;
-        for (int e0 = tid; e0 < ntr; e0 += XU * HP_THREADS) {
-            int addr[XU];
-#pragma unroll
-            for (int u = 0; u < XU; ++u) {
-                const int e = e0 + u * HP_THREADS;
-                addr[u] = -1;
-                if (e < ntr) {
-                    const int li = hp_find<HP_LINK_LOG>(sh.l_tr, nl, e);
-                    const int w1 = sh.l_m1[li];
-                    const int F = w1 & 3, nx1 = (w1 >> 2) & 15, ny1 = (w1 >> 6) & 15;
-                    const int nt1 = (w1 >> 10) & 15, bd1 = restrict_ ? ((w1 >> 14) & 15) : 0;
-                    const int le = e - sh.l_tr[li];
-                    const int m1 = hp_div(le, 1.0f / float(nt1)), a = le - m1 * nt1;
-                    int i1, j1;
-                    if (F == 0) { i1 = 0; j1 = m1; }
-                    else if (F == 2) { i1 = nx1 - 1; j1 = m1; }
-                    else if (F == 1) { i1 = m1; j1 = 0; }
-                    else { i1 = m1; j1 = ny1 - 1; }
-                    if (!(bd1 && hp_on_bdry(bd1, i1, j1, nx1, ny1)))
-                        addr[u] = sh.l_src[li] + (i1 * ny1 + j1) * nt1 + a;
-                }
-            }
-            A tv[XU];
-#pragma unroll
-            for (int u = 0; u < XU; ++u) tv[u] = (addr[u] >= 0) ? A(x[addr[u]]) : A(0);
-#pragma unroll
-            for (int u = 0; u < XU; ++u) {
-                const int e = e0 + u * HP_THREADS;
-                if (e < ntr) tr[e] = tv[u];
-            }
-        }
-        __syncthreads();
-        // two entries per thread and step, so that their searches and E^theta
-        // loads are in flight together
-        for (int e0 = tid; e0 < ninn; e0 += 2 * HP_THREADS) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int e = e0 + u * HP_THREADS;
-                if (e < ninn) {
-                    const int li = hp_find<HP_LINK_LOG>(sh.l_inn, nl, e);
-                    const int w1 = sh.l_m1[li];
-                    const int nt1 = (w1 >> 10) & 15, kk = w1 >> 18;
-                    const int nt = sh.c_nth[kk];
-                    const int le = e - sh.l_inn[li], m1 = hp_div(le, 1.0f / float(nt));
-                    const int r = le - m1 * nt;
-                    const double *Et = m.Eth_pool + sh.l_et[li] + r;
-                    const A *trl = tr + sh.l_tr[li] + m1 * nt1;
-                    // the E^theta column's (at most RTX_NMAX) loads in flight
-                    // together: unconditional (rows past nt1 reload row
-                    // nt1 - 1), so that no conversion or wait sits between
-                    // them
-                    double ev[HP_NM];
-#pragma unroll
-                    for (int a = 0; a < HP_NM; ++a) ev[a] = Et[(a < nt1 ? a : nt1 - 1) * nt];
-                    // the trace reads likewise unconditional; terms past nt1
-                    // are zero times a finite trace value
-                    A acc = A(0);
-#pragma unroll
-                    for (int a = 0; a < HP_NM; ++a) {
-                        const A tv = trl[a < nt1 ? a : nt1 - 1];
-                        acc += (a < nt1 ? A(ev[a]) : A(0)) * tv;
-                    }
-                    inn[e] = acc;
-                }
-            }
-        }
-        __syncthreads();
-        // inflow-face sums.  Entry (kk, h, m0, r): cell kk, the h-th of its
-        // faces that carry links (ascending face number F), own face node
-        // m0, angle r of the cell:
-        //   sum over kk's links on F, in link order, of
-        //   (face factor) * sum_m1 E^s[m0, m1] inn[link, m1, r]
-        // (the spatial half of boundary_convection_matrix.py:348-524).  They
-        // are held in registers over a barrier, then written over inn, which
-        // no one reads after them.
-        A fv[HP_FV];
-#pragma unroll
-        for (int u = 0; u < HP_FV; ++u) {
-            const int e = tid + u * HP_THREADS;
-            fv[u] = A(0);
-            if (e < nffc) {
-                const int kk = hp_find<HP_CELL_LOG>(sh.c_fo, ncells, e);
-                const int nt = sh.c_nth[kk], lf = sh.c_lf[kk];
-                const int le = e - sh.c_fo[kk];
-                const int row = hp_div(le, 1.0f / float(nt)), r = le - row * nt;
-                const int hs = hp_div(row, 1.0f / float(N)), m0 = row - hs * N;
-                int F = 0;
-                for (int cnt = hs; F < 4; ++F)
-                    if ((lf >> F) & 1) {
-                        if (cnt == 0) break;
-                        --cnt;
-                    }
-                const A fxy = A(((F & 1) ? dx : dy) * 0.25) * sh.c_dth[kk];
-                A sum = A(0);
-                for (int li = sh.c_l0[kk]; li < sh.c_l0[kk + 1]; ++li) {
-                    const int w1 = sh.l_w[li];
-                    if ((w1 & 3) != F) continue;
-                    const int n1 = w1 >> 2;
-                    const A *Es = es + sh.l_es[li] + m0;
-                    const A *in_ = inn + sh.l_inn[li] + r;
-                    // the E^s row's and the traces' (at most RTX_NMAX each)
-                    // reads in flight together: unconditional, rows past n1
-                    // reread row n1 - 1 and add zero times a finite value
-                    A ev[HP_NM], iv[HP_NM];
-#pragma unroll
-                    for (int m1 = 0; m1 < HP_NM; ++m1) {
-                        const int mm = m1 < n1 ? m1 : n1 - 1;
-                        ev[m1] = Es[mm * N];
-                        iv[m1] = in_[mm * nt];
-                    }
-                    A f = A(0);
-#pragma unroll
-                    for (int m1 = 0; m1 < HP_NM; ++m1) f += (m1 < n1 ? ev[m1] : A(0)) * iv[m1];
-                    sum += fxy * f;
-                }
-                fv[u] = sum;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < HP_FV; ++u) {
-            const int e = tid + u * HP_THREADS;
-            if (e < nffc) inn[e] = fv[u];
-        }
+    for (int a = tid; a < na; a += HP_THREADS) {
+        ct[a] = A(m.ang_trig[3 * (ga0 + a)]);
+        sn[a] = A(m.ang_trig[3 * (ga0 + a) + 1]);
+        wr[a] = A(m.ang_trig[3 * (ga0 + a) + 2]);
+        dt[a] = A(h.ang_dth[ga0 + a]);
+        pk[a] = m.ang_pack[ga0 + a];
+        fl[a] = h.ang_flag[ga0 + a];
     }
+    const double *wd = h.wd + N * HP_WD;
+    for (int t = tid; t < HP_NM + NSP; t += HP_THREADS) sh.wd[t] = A(wd[t]);
+    if (tid < NSP) {
+        const int i = tid / N, j = tid - i * N;
+        const double w2 = wd[i] * wd[j];
+        sh.nf[2 * tid] = A(w2 * m.kappa[sp0 + tid]);
+        sh.nf[2 * tid + 1] = A(dx * dy * m.sigma[sp0 + tid] * w2);
+    }
+    __syncthreads();
+    // DOF t of the column belongs to the cell of angle t / NSP (a cell's DOFs
+    // start at NSP times its first angle)
     for (int t0 = tid; t0 < ncd; t0 += XU * HP_THREADS) {
         if (t0 != tid) {
 #pragma unroll
@@ -334,14 +415,12 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, uint32_t ops, int ac
             const int t = t0 + u * HP_THREADS;
             if (t >= ncd) break;
             A v = vv[u];
-            const int kk = acell[t / NSP] & 255;
-            const int nt = sh.c_nth[kk], ao = sh.c_ao[kk];
+            const int ta = t / NSP, w = pk[ta];
+            const int nt = (w >> 20) & 31, ao = ta - (w >> 25);
             const int lt = t - NSP * ao;
             const int s = hp_div(lt, 1.0f / float(nt)), a = lt - s * nt;
-            if (sh.c_bd[kk]) {
-                const int p = s / N, q = s - p * N;
-                if (hp_on_bdry(sh.c_bd[kk], p, q, N, N)) v = A(0);
-            }
+            const int bd = restrict_ ? (fl[ta] & 15) : 0;
+            if (bd && hp_on_bdry(bd, s / N, s % N, N, N)) v = A(0);
             xs[(ao + a) * S + s] = v;
             if constexpr (PREC == RTX_PREC_MIXED) xb[s * XSB + ao + a] = hp_bf16(float(v));
         }
@@ -356,271 +435,158 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, uint32_t ops, int ac
     }
     __syncthreads();
 
-    // ---- phase 2
-    constexpr int NTG = (MT + HP_TG - 1) / HP_TG;
+    // ---- 16 output angles per wavefront, every node
+    typedef typename HpMma<A>::v4 acc4;
+    typedef const A __attribute__((address_space(4))) *CPtr;
+    // the derivative matrix in scalar registers
+    const CPtr wdc = (CPtr)(uintptr_t)((sizeof(A) == 8 ? (const void *)(h.wd + N * HP_WD)
+                                                       : (const void *)(h.wd_f + N * HP_WD)));
     const int NRT = (na + 15) / 16;
-    typedef typename std::conditional<PREC == RTX_PREC_F64, hp_d4, hp_f4>::type acc4;
-    for (int item = wave; item < NRT * NTG; item += HP_WAVES) {
-        const int rt = item / NTG, tg = (item - rt * NTG) * HP_TG;
+    auto item = [&](int it) {
+        const int rt = it / NI, lb = it - rt * NI;
         const int R = rt * 16 + l16;
-        const bool rok = R < na;
-        // lanes past the last angle read valid addresses; their output
-        // column is never stored
-        const int Rc = rok ? R : na - 1;
-        acc4 acc[HP_TG];
+        const int Rc = R < na ? R : na - 1;
+        acc4 acc[MT];
 #pragma unroll
-        for (int t = 0; t < HP_TG; ++t) acc[t] = acc4{0, 0, 0, 0};
-        if (ops & RTX_OP_SCAT) {
-            // operand rows: node (tg + t) * 16 + l16 of this lane (rows past
-            // the last node read the last node; their outputs are not stored)
-            int arow[HP_TG];
+        for (int t = 0; t < MT; ++t) acc[t] = acc4{0, 0, 0, 0};
+        if (scat) {
+            int arow[MT], li = l16;
+            asm volatile("" : "+v"(li));
 #pragma unroll
-            for (int t = 0; t < HP_TG; ++t) {
-                const int s = (tg + t) * 16 + l16;
-                arow[t] = (s < NSP ? s : NSP - 1);
-            }
-            if constexpr (PREC != RTX_PREC_MIXED) {
-                typedef typename std::conditional<PREC == RTX_PREC_F64, double, float>::type E;
-                const E *G = (PREC == RTX_PREC_F64) ? (const E *)(m.G + m.col_G_off[c])
-                                                    : (const E *)(m.G_f + m.col_G_off[c]);
-                const E *gcol = G + Rc;
-                // G rows past na are clamped to the last row: the angle rows of
-                // the copy are zero there, so they add nothing
-                auto gload = [&](int Ak) -> E { return gcol[size_t(Ak < na ? Ak : na - 1) * na]; };
-                const A *xcol = xs + lg * S;
-                // four K steps of G per load group; the next two groups are
-                // in flight while the current one multiplies (three: 20 bytes
-                // per lane of register spills in FP64)
-                E bc[4], bn[4], bf[4];
+            for (int t = 0; t < MT; ++t) arow[t] = hp_node<A, N>(t, li, lb);
+            for (int kb = 0; kb < na; kb += 16) {
+                const Group cur = gq[0];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    bc[u] = gload(4 * u + lg);
-                    bn[u] = gload(16 + 4 * u + lg);
-                }
-                for (int kb = 0; kb < na; kb += 16) {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) bf[u] = gload(kb + 32 + 4 * u + lg);
+                for (int d = 0; d + 1 < PD; ++d) gq[d] = gq[d + 1];
+                gq[PD - 1] = gload(Rc, kb + 16 * PD);
+                if constexpr (PREC != RTX_PREC_MIXED) {
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         if (kb + 4 * u < na) {            // uniform across the wave
-                            const A *xk = xcol + (kb + 4 * u) * S;
+                            const A *xk = xs + (kb + 4 * u + lg) * S;
 #pragma unroll
-                            for (int t = 0; t < HP_TG; ++t) {
-                                if ((tg + t) < MT) {
-                                    const E a = E(xk[arow[t]]);
-                                    if constexpr (PREC == RTX_PREC_F64)
-                                        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bc[u], acc[t], 0, 0, 0);
-                                    else
-                                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bc[u], acc[t], 0, 0, 0);
-                                }
-                            }
+                            for (int t = 0; t < MT; ++t)
+                                acc[t] = HpMma<A>::step(xk[arow[t]], cur.g[u], acc[t]);
                         }
                     }
+                } else {
+                    const hp_s4 bv = {short(cur.g[0]), short(cur.g[1]), short(cur.g[2]), short(cur.g[3])};
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        bc[u] = bn[u];
-                        bn[u] = bf[u];
-                    }
-                }
-            } else {
-                const uint16_t *gcol = m.G_bf16 + m.col_G_off[c] + Rc;
-                const uint16_t *xrow[HP_TG];
-#pragma unroll
-                for (int t = 0; t < HP_TG; ++t) xrow[t] = xb + arow[t] * XSB + 4 * lg;
-                for (int kb = 0; kb < na; kb += 16) {
-                    hp_s4 bv;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const int Ak = kb + 4 * lg + u;
-                        bv[u] = short(gcol[size_t(Ak < na ? Ak : na - 1) * na]);
-                    }
-#pragma unroll
-                    for (int t = 0; t < HP_TG; ++t) {
-                        if ((tg + t) < MT) {
-                            const hp_s4 av = *reinterpret_cast<const hp_s4 *>(xrow[t] + kb);
-                            acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[t], 0, 0, 0);
-                        }
+                    for (int t = 0; t < MT; ++t) {
+                        const hp_s4 av = *reinterpret_cast<const hp_s4 *>(xb + arow[t] * XSB + 4 * lg + kb);
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[t], 0, 0, 0);
                     }
                 }
             }
         }
-        if (!rok) continue;
+        if (R >= na) return;
         // the output angle's cell and constants
-        const int ac = acell[R];
-        const int kk = ac & 255, r = ac >> 8;
-        const int nt = sh.c_nth[kk], bd = sh.c_bd[kk], quad = sh.c_quad[kk];
-        const int lf = bconv ? sh.c_lf[kk] : 0;
-        const A dth = sh.c_dth[kk], ct = cth[R], sn = sth[R], w_r = wr[R];
-        const A vol = A(dx * dy * 0.125) * dth * w_r;
-        const A cx = A(dy * 0.25) * dth * w_r * ct, cy = A(dx * 0.25) * dth * w_r * sn;
-        const A fx = A(dy * 0.25) * dth, fy = A(dx * 0.25) * dth;   // face factors, x / y faces
-        T *yc = y + cdof + NSP * sh.c_ao[kk] + r;                  // y[cell + s nt + r]
+        const int w = pk[R], nt = (w >> 20) & 31, f = fl[R];
+        const int bd = restrict_ ? (f & 15) : 0, quad = ((f >> 4) & 7) - 1;
+        const int lf = bconv ? (f >> 8) & 15 : 0;
+        const A dth = dt[R], cR = ct[R], sR = sn[R], w_r = wr[R];
+        const A vol = (ops & RTX_OP_MASS) ? A(dx * dy * 0.125) * dth * w_r : A(0);
+        const A ic = (ops & RTX_OP_ICONV) ? A(1) : A(0);
+        const A cx = ic * A(dy * 0.25) * dth * w_r * cR, cy = ic * A(dx * 0.25) * dth * w_r * sR;
+        // outflow factors of the faces +x, +y, -x, -y (quadrant Q flows out of
+        // faces Q and Q + 1)
+        const A fx = A(dy * 0.25) * dth, fy = A(dx * 0.25) * dth;
+        const bool ob = bconv && quad >= 0;
+        const A ox1 = ob && (quad == 0 || quad == 3) ? fx * w_r * cR : A(0);
+        const A ox0 = ob && (quad == 1 || quad == 2) ? -fx * w_r * cR : A(0);
+        const A oy1 = ob && quad < 2 ? fy * w_r * sR : A(0);
+        const A oy0 = ob && quad >= 2 ? -fy * w_r * sR : A(0);
+        T *yb = y + cdof;
+        const int yo = (w & 0xfffff) + (w >> 25);                  // + s nt: node s
         const A *xr = xs + R * S;                                  // angle row R of the copy
 #pragma unroll
-        for (int t = 0; t < HP_TG; ++t) {
-            if (tg + t >= MT) break;
-            // one output at a time (the line reads of an output are in
-            // flight together; rolling this loop keeps them in registers)
-#pragma unroll 1
-            for (int v = 0; v < 4; ++v) {
-                // f64 D row = l/16 + 4 v; f32 D row = 4 (l/16) + v
-                const int s = (tg + t) * 16 + ((PREC == RTX_PREC_F64) ? (lg + 4 * v) : (4 * lg + v));
-                if (s >= NSP) continue;
-                const int p = s / N, q = s - p * N;
-                const A xv = xr[s];
-                A val = A(0);
-                if (ops & RTX_OP_MASS) val += vol * sh.w2k[s] * xv;
-                if (ops & RTX_OP_ICONV) {
-                    const A *lx = xr + q, *ly = xr + p * N;
-                    const A *wdx = sh.WDx + p * HP_NM, *wdy = sh.WDy + q * HP_NM;
-                    A sx = A(0), sy = A(0);
+        for (int l = 0; l < LI; ++l) {
+            int q = lg + 4 * (lb + l);
+            // opaque: addresses and factors of the line are computed here, not
+            // hoisted out of the items and lines to be held (and spilled)
+            asm volatile("" : "+v"(q));
+            if (q >= N) continue;
+            // faces of the line's nodes (bit F: face F); the end nodes also
+            // lie on face 2 (p = 0) or 0 (p = N - 1)
+            const int qf = (q == N - 1 ? 2 : 0) | (q == 0 ? 8 : 0);
+            auto faces = [&](int p) { return qf | (p == 0 ? 4 : 0) | (p == N - 1 ? 1 : 0); };
+            // the inflow-face sums that k_hp_flux left in y, one node ahead
+            auto face_sum = [&](int p) {
+                A v = A(0);
+                if (faces(p) & lf) v = A(yb[yo + (p * N + q) * nt]);
+                return v;
+            };
+            A fs = face_sum(0);
+            A lx[N];
 #pragma unroll
-                    for (int i = 0; i < N; ++i) {
-                        sx += wdx[i] * lx[i * N];
-                        sy += wdy[i] * ly[i];
-                    }
-                    val -= cx * sh.wys[q] * sx + cy * sh.wxs[p] * sy;
-                }
-                // faces this node lies on (bit F: face F)
-                const int onf = ((p == N - 1) ? 1 : 0) | ((q == N - 1) ? 2 : 0) |
-                                ((p == 0) ? 4 : 0) | ((q == 0) ? 8 : 0);
-                if (bconv && quad >= 0 && onf) {
+            for (int i = 0; i < N; ++i) lx[i] = xr[i * N + q];
+            const A *wy = sh.wd + HP_NM + q * N;
+            const A wq = sh.wd[q];
+            // y-faces' outflow factor of this line, times w_p below
+            const A oy = q == N - 1 ? oy1 : (q == 0 ? oy0 : A(0));
+            // one output's reads at a time, and none kept for the next line:
+            // hoisted, they spill
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int hh = 0; hh < 2; ++hh) {
-                        const int F = (quad + hh) & 3;
-                        if (onf & (1 << F)) {
-                            const A tf = F == 0 ? ct : (F == 1 ? sn : (F == 2 ? -ct : -sn));
-                            val += ((F & 1) ? fy * sh.wxs[p] : fx * sh.wys[q]) * w_r * tf * xv;
-                        }
-                    }
+            for (int p = 0; p < N; ++p) {
+                const int s = p * N + q;
+                const A *ly = xr + p * N;
+                const A fn = p + 1 < N ? face_sum(p + 1) : A(0);
+                A sx = A(0), sy = A(0);
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    sx += wdc[HP_NM + p * N + i] * lx[i];
+                    sy += wy[i] * ly[i];
                 }
-                if (onf & lf) {
-                    // the cell's inflow-face sums on the node's faces, by face
-                    const int fo = sh.c_fo[kk];
-                    int slot = 0;
-                    // kept rolled: unrolled, the compiler's schedule of this
-                    // loop spills phase 2's registers
-#pragma unroll 1
-                    for (int F = 0; F < 4; ++F) {
-                        if ((lf >> F) & 1) {
-                            if ((onf >> F) & 1) {
-                                const int m0 = (F & 1) ? p : q;
-                                val += inn[fo + (slot * N + m0) * nt + r];
-                            }
-                            ++slot;
-                        }
-                    }
-                }
-                if (ops & RTX_OP_SCAT) val -= sh.sgw[s] * A(acc[t][v]);
-                const bool masked = bd && (onf & bd);
-                T *yp = yc + s * nt;
+                const A wp = wdc[p], xv = lx[p];
+                A val = vol * sh.nf[2 * s] * xv - (cx * wq * sx + cy * wp * sy);
+                if (p == N - 1) val += ox1 * wq * xv;
+                if (p == 0) val += ox0 * wq * xv;
+                val += oy * wp * xv;
+                val += fs;
+                fs = fn;
+                if (scat) val -= sh.nf[2 * s + 1] * A(acc[(l * N + p) / 4][(l * N + p) % 4]);
+                const int on = faces(p), o = yo + s * nt;
                 if (accumulate) {
-                    if (!masked) *yp = T(A(*yp) + val);
+                    // (face sums were added to y by k_hp_flux)
+                    if (!(on & bd)) yb[o] = T((on & lf) ? val : A(yb[o]) + val);
                 } else {
-                    *yp = T(masked ? A(0) : val);
+                    yb[o] = T((on & bd) ? A(0) : val);
                 }
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+    };
+    // the first item apart from the others: in one loop, the G rows loaded
+    // ahead for it would hold registers through every item's lines
+    if (wave < NRT * NI) item(wave);
+    for (int it = wave + HP_WAVES; it < NRT * NI; it += HP_WAVES) {
+        if (scat) {
+            const int R = it / NI * 16 + l16;
+#pragma unroll
+            for (int d = 0; d < PD; ++d) gq[d] = gload(R < na ? R : na - 1, 16 * d);
+        }
+        item(it);
     }
 }
 
 template <typename T, typename A, int PREC>
 __global__ __launch_bounds__(HP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
-             const int32_t *__restrict__ cols, int ncols, const T *__restrict__ x,
+             const int32_t *__restrict__ hdr, int ncols, const T *__restrict__ x,
              T *__restrict__ y) {
     extern __shared__ __align__(16) unsigned char hp_lds[];
     __shared__ HpShared<A> sh;
-
-    // XCD-aware block -> column: block b runs on XCD b % 8, and XCD j takes
-    // the j-th contiguous run of the (key-ordered) list, so the neighbour
-    // columns whose traces a column reads are mostly cached on the same XCD
-    const int per = (ncols + HP_XCD - 1) / HP_XCD;
-    const int bi = blockIdx.x % HP_XCD, bj = blockIdx.x / HP_XCD;
-    if (bj >= per) return;
-    const int ci = bi * per + bj;
-    if (ci >= ncols) return;
-    const int c = cols[ci];
-    const int tid = threadIdx.x;
-    // the column's scalars from its header (square columns: ny = nx)
-    const int32_t *hd = h.col_hdr + size_t(c) * HP_HDR;
-    const int k0 = hd[0], ncells = hd[1], nx = hd[2], ny = nx, nsp = nx * ny;
-    const int na = hd[3], cdof = hd[4], L0 = hd[5], nl = hd[6], ga0 = hd[7];
-    const int ninn = hd[8], nffc = hd[9], ntr = hd[10], es0 = hd[11], nes = hd[12];
-    const int sp0 = hd[13];
-    const bool restrict_ = (ops & RTX_OP_RESTRICT) != 0;
-    const double x0 = m.col_geom[4 * c + 0], y0 = m.col_geom[4 * c + 1];
-    const double dx = m.col_geom[4 * c + 2] - x0, dy = m.col_geom[4 * c + 3] - y0;
-    const HpLayout Lo = hp_layout<A, PREC>(nsp, na, ninn > nffc ? ninn : nffc, ntr, nes);
-    A *cth = reinterpret_cast<A *>(hp_lds + Lo.cth);
-    A *sth = reinterpret_cast<A *>(hp_lds + Lo.sth);
-    A *wr = reinterpret_cast<A *>(hp_lds + Lo.wr);
-    int *acell = reinterpret_cast<int *>(hp_lds + Lo.acell);
-
-    // ---- phase 0: tables
-    if (tid < ncells) {
-        const int k = k0 + tid;
-        const int nt = m.cell_nth[k], ao = m.cell_ang_off[k];
-        sh.c_nth[tid] = nt;
-        sh.c_bd[tid] = restrict_ ? m.cell_bdry[k] : 0;
-        sh.c_quad[tid] = m.cell_quad[k];
-        sh.c_ao[tid] = ao;
-        sh.c_l0[tid] = m.link_start[k] - L0;
-        sh.c_fo[tid] = h.cell_fo[k];
-        sh.c_dth[tid] = A(m.cell_geom[2 * k + 1] - m.cell_geom[2 * k]);
-        sh.c_lf[tid] = h.cell_lf[k];
-        for (int a = 0; a < nt; ++a) acell[ao + a] = tid | (a << 8);
-    }
-    if (tid == 0) {
-        sh.c_ao[ncells] = na;
-        sh.c_l0[ncells] = nl;
-        sh.l_inn[nl] = ninn;
-        sh.c_fo[ncells] = nffc;
-        sh.l_tr[nl] = ntr;
-    }
-    for (int a = tid; a < na; a += HP_THREADS) {
-        cth[a] = A(m.ang_trig[3 * (ga0 + a)]);
-        sth[a] = A(m.ang_trig[3 * (ga0 + a) + 1]);
-        wr[a] = A(m.ang_trig[3 * (ga0 + a) + 2]);
-    }
-    for (int li = tid; li < nl; li += HP_THREADS) {
-        const int l = L0 + li;
-        sh.l_w[li] = h.link_w[l];
-        sh.l_inn[li] = h.link_inn[l];
-        sh.l_es[li] = h.link_esl[l];
-        sh.l_m1[li] = m.link_meta[4 * l + 1];
-        sh.l_src[li] = m.link_meta[4 * l];
-        sh.l_tr[li] = m.link_meta[4 * l + 2];
-        sh.l_et[li] = m.link_Eth_off[l];
-    }
-    if (tid < nsp) {
-        const int i = tid / ny, j = tid - (tid / ny) * ny;
-        const double w2 = m.lgl_w[nx * HP_NM + i] * m.lgl_w[ny * HP_NM + j];
-        sh.w2k[tid] = A(w2 * m.kappa[sp0 + tid]);
-        sh.sgw[tid] = A(dx * dy * m.sigma[sp0 + tid] * w2);
-    }
-    if (tid < HP_NM * HP_NM) {
-        const int pp = tid / HP_NM, ii = tid % HP_NM;
-        sh.WDx[tid] = (pp < nx && ii < nx)
-                          ? A(m.lgl_w[nx * HP_NM + ii] * m.lgl_D[(size_t(nx) * HP_NM + pp) * HP_NM + ii])
-                          : A(0);
-        sh.WDy[tid] = (pp < ny && ii < ny)
-                          ? A(m.lgl_w[ny * HP_NM + ii] * m.lgl_D[(size_t(ny) * HP_NM + pp) * HP_NM + ii])
-                          : A(0);
-    }
-    if (tid < HP_NM) {
-        sh.wxs[tid] = A(tid < nx ? m.lgl_w[nx * HP_NM + tid] : 0.0);
-        sh.wys[tid] = A(tid < ny ? m.lgl_w[ny * HP_NM + tid] : 0.0);
-    }
-    __syncthreads();
-
-    // phases 1 and 2, compiled per node count (square columns; the host
-    // admits only those)
-    switch (nx) {
-#define HP_CASE(NN)                                                                           \
-    case NN:                                                                                  \
-        hp_column<T, A, PREC, NN>(m, ops, accumulate, sh, hp_lds, c, k0, ncells, na, cdof, L0, \
-                                  nl, ninn, nffc, ntr, es0, nes, h.es_pool, dx, dy, x, y);   \
+    const int ci = hp_xcd(ncols);
+    if (ci < 0) return;
+    const int32_t *hd = hdr + size_t(ci) * HP_HDR;
+    // compiled per node count (square columns; the host admits only those)
+    switch (hd[2]) {
+#define HP_CASE(NN)                                                                    \
+    case NN:                                                                           \
+        hp_column<T, A, PREC, NN>(m, h, ops, accumulate, sh, hp_lds, hd, x, y);        \
         break;
         HP_CASE(3) HP_CASE(4) HP_CASE(5) HP_CASE(6) HP_CASE(7) HP_CASE(8) HP_CASE(9) HP_CASE(10)
 #undef HP_CASE
@@ -632,12 +598,10 @@ void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
 
 // Bytes of dynamic LDS a column needs (FP64 or FP32 storage, mixed adds the
 // BF16 copy).
-static size_t hp_bytes(int nsp, int na, int nin, int ntr, int nes, int prec) {
-    if (prec == RTX_PREC_F64)
-        return size_t(hp_layout<double, RTX_PREC_F64>(nsp, na, nin, ntr, nes).total);
-    if (prec == RTX_PREC_F32)
-        return size_t(hp_layout<float, RTX_PREC_F32>(nsp, na, nin, ntr, nes).total);
-    return size_t(hp_layout<float, RTX_PREC_MIXED>(nsp, na, nin, ntr, nes).total);
+static size_t hp_bytes(int nsp, int na, int prec) {
+    if (prec == RTX_PREC_F64) return size_t(hp_layout<double, RTX_PREC_F64>(nsp, na).total);
+    if (prec == RTX_PREC_F32) return size_t(hp_layout<float, RTX_PREC_F32>(nsp, na).total);
+    return size_t(hp_layout<float, RTX_PREC_MIXED>(nsp, na).total);
 }
 
 // Static LDS of k_hpcol (the tables above), for the capacity check.
@@ -646,158 +610,143 @@ constexpr size_t HP_STATIC_BYTES = sizeof(HpShared<double>) + 64;
 int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     const int nc = d->ncol;
     p->hp_ok = false;
-    std::vector<int32_t> link_inn(std::max(d->nlink, 1), 0), col_inn(nc, 0);
-    std::vector<int32_t> cell_fo(std::max(d->ncell, 1), 0), col_ffc(nc, 0);
-    std::vector<int32_t> link_esl(std::max(d->nlink, 1), 0), col_es0(nc, 0), col_nes(nc, 0);
-    std::vector<double> es_pool;
-    std::vector<int32_t> col_hdr(size_t(nc) * HP_HDR, 0), cell_lf(std::max(d->ncell, 1), 0);
-    std::vector<int32_t> link_w(std::max(d->nlink, 1), 0);
-    std::vector<std::pair<int64_t, int>> seen;   // (pool offset, staged offset) of one column
-    std::vector<char> fits(nc, 0);
-    std::vector<size_t> need[3];
-    for (int k = 0; k < 3; ++k) need[k].assign(nc, 0);
+    std::vector<int32_t> ang_flag(std::max<int64_t>(d->nang, 1), 0);
+    std::vector<double> ang_dth(std::max<int64_t>(d->nang, 1), 0.0);
     int max_lds = 0;
     RTX_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, p->device));
     const size_t cap = size_t(max_lds) > HP_STATIC_BYTES ? size_t(max_lds) - HP_STATIC_BYTES : 0;
-    int nfit = 0;
+    // a column whose workgroup (dynamic + static LDS) fits half of a CU's
+    // 160 KB runs two workgroups per CU (class 0), the others one (class 1)
+    const size_t half = 80 * 1024 > HP_STATIC_BYTES ? 80 * 1024 - HP_STATIC_BYTES : 0;
+    std::vector<int32_t> hdr[3][HP_NCLS], over, links;
+    std::vector<HpCell> cells;
+    p->hp_ncols = 0;
     for (int c = 0; c < nc; ++c) {
         const int k0 = d->col_cell_start[c], k1 = d->col_cell_start[c + 1];
         const int nsp = d->col_nx[c] * d->col_ny[c], na = d->col_nang[c];
-        int o = 0;
-        for (int l = d->link_start[k0]; l < d->link_start[k1]; ++l) {
-            const int s = d->link_src[l], F = d->link_face[l], c1 = d->cell_col[s];
-            const int n1 = (F & 1) ? d->col_nx[c1] : d->col_ny[c1];
-            link_inn[l] = o;
-            o += n1 * d->cell_nth[d->link_target[l]];
-        }
-        col_inn[c] = o;
-        // inflow-face sums: per cell, one block of nx x nth per face that
-        // carries links
-        int fo = 0;
+        // per angle: its cell's masked faces, quadrant + 1 and the faces that
+        // carry links, and the cell's width
+        int64_t a = d->col_ang_start[c];
         for (int k = k0; k < k1; ++k) {
             int lf = 0;
-            for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) {
-                const int F = d->link_face[l], c1 = d->cell_col[d->link_src[l]];
-                lf |= 1 << F;
-                link_w[l] = F | (((F & 1) ? d->col_nx[c1] : d->col_ny[c1]) << 2);
+            for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) lf |= 1 << d->link_face[l];
+            for (int r = 0; r < d->cell_nth[k]; ++r, ++a) {
+                ang_flag[a] = (d->cell_bdry[k] & 15) | (d->cell_quad[k] + 1) << 4 | lf << 8;
+                ang_dth[a] = d->cell_geom[2 * k + 1] - d->cell_geom[2 * k];
             }
-            cell_lf[k] = lf;
-            cell_fo[k] = fo;
-            fo += __builtin_popcount(lf) * d->col_nx[c] * d->cell_nth[k];
         }
-        col_ffc[c] = fo;
-        // the column's distinct E^s blocks (n0 x n1 each, keyed by pool
-        // offset), copied in link order
-        seen.clear();
-        col_es0[c] = int(es_pool.size());
-        int nes = 0;
-        for (int l = d->link_start[k0]; l < d->link_start[k1]; ++l) {
-            const int64_t off = d->link_Es_off[l];
-            int pos = -1;
-            for (const auto &sp : seen)
-                if (sp.first == off) { pos = sp.second; break; }
-            if (pos < 0) {
-                const int s = d->link_src[l], F = d->link_face[l], c1 = d->cell_col[s];
-                const int n0 = (F & 1) ? d->col_nx[c] : d->col_ny[c];
-                const int n1 = (F & 1) ? d->col_nx[c1] : d->col_ny[c1];
-                pos = nes;
-                seen.emplace_back(off, pos);
-                es_pool.insert(es_pool.end(), d->Es_pool + off, d->Es_pool + off + int64_t(n0) * n1);
-                nes += n0 * n1;
-            }
-            link_esl[l] = pos;
-        }
-        col_nes[c] = nes;
-        const int nlc = d->link_start[k1] - d->link_start[k0];
-        int32_t *hc = col_hdr.data() + size_t(c) * HP_HDR;
-        hc[0] = k0;
-        hc[1] = k1 - k0;
-        hc[2] = d->col_nx[c];
-        hc[3] = na;
-        hc[4] = d->cell_dof_off[k0];
-        hc[5] = d->link_start[k0];
-        hc[6] = nlc;
-        hc[7] = d->col_ang_start[c];
-        hc[8] = o;
-        hc[9] = fo;
-        hc[10] = d->col_ntrace[c];
-        hc[11] = col_es0[c];
-        hc[12] = nes;
-        hc[13] = d->col_sp_off[c];
+        const int32_t h[HP_HDR] = {k0, k1 - k0, d->col_nx[c], na, d->cell_dof_off[k0], 0, 0,
+                                   d->col_ang_start[c], 0, 0, 0, 0, 0, d->col_sp_off[c], c, 0};
         // square columns of HP_NMIN..RTX_NMAX nodes (the compiled node counts)
-        bool ok = (k1 - k0) <= HP_MAX_CELLS && nlc <= HP_MAX_LINKS &&
-                  d->col_nx[c] == d->col_ny[c] && d->col_nx[c] >= HP_NMIN && na <= 4096 &&
-                  fo <= HP_FV * HP_THREADS;
+        bool ok = (k1 - k0) <= HP_MAX_CELLS && d->col_nx[c] == d->col_ny[c] &&
+                  d->col_nx[c] >= HP_NMIN && na <= 4096 && k1 > k0;
+        for (int k = k0; k < k1; ++k) ok = ok && d->link_start[k + 1] - d->link_start[k] < 256;
+        size_t need[3];
         for (int pr = 0; pr < 3; ++pr) {
-            need[pr][c] = hp_bytes(nsp, na, std::max(o, fo), d->col_ntrace[c], nes, pr);
-            ok = ok && need[pr][c] <= cap;
+            need[pr] = hp_bytes(nsp, na, pr);
+            ok = ok && need[pr] <= cap;
         }
-        fits[c] = ok ? 1 : 0;
-        nfit += ok ? 1 : 0;
-    }
-    // LDS classes: columns whose workgroup (dynamic + static LDS) fits half
-    // of a CU's 160 KB run two workgroups per CU, the rest one (FP64 sizes;
-    // the FP32 and mixed launches of a class take the class's own maximum)
-    const size_t half = 80 * 1024 > HP_STATIC_BYTES ? 80 * 1024 - HP_STATIC_BYTES : 0;
-    const size_t lim[HP_NCLS] = {half, cap};
-    std::vector<int32_t> lists[HP_NCLS], over;
-    for (int c = 0; c < nc; ++c) {
-        if (!fits[c]) {
+        if (!ok) {
             over.push_back(c);
             continue;
         }
-        int cls = HP_NCLS - 1;
-        for (int k = 0; k < HP_NCLS; ++k)
-            if (need[0][c] <= lim[k]) { cls = k; break; }
-        lists[cls].push_back(c);
-        for (int pr = 0; pr < 3; ++pr)
-            p->hp_cls[cls].bytes[pr] = std::max(p->hp_cls[cls].bytes[pr], need[pr][c]);
+        ++p->hp_ncols;
+        const double dx = d->col_geom[4 * c + 2] - d->col_geom[4 * c];
+        const double dy = d->col_geom[4 * c + 3] - d->col_geom[4 * c + 1];
+        for (int k = k0; k < k1; ++k) {
+            const double dth = d->cell_geom[2 * k + 1] - d->cell_geom[2 * k];
+            HpCell cl;
+            cl.fx = dy * 0.25 * dth;
+            cl.fy = dx * 0.25 * dth;
+            cl.off = d->cell_dof_off[k];
+            cl.l0 = int32_t(links.size() / 4);
+            int lf = 0, nl = 0;
+            for (int F = 0; F < 4; ++F)
+                for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) {
+                    if (d->link_face[l] != F) continue;
+                    const int w1 = d->link_meta[4 * l + 1];
+                    const int nx1 = (w1 >> 2) & 15, ny1 = (w1 >> 6) & 15, nt1 = (w1 >> 10) & 15;
+                    const int bd1 = (w1 >> 14) & 15, n1 = (F & 1) ? nx1 : ny1;
+                    // the trace's first DOF, stride and masked nodes
+                    const int fixed = F < 2 ? 0 : (F == 2 ? nx1 : ny1) - 1;
+                    const int first = (F & 1) ? fixed * nt1 : fixed * ny1 * nt1;
+                    const int stride = (F & 1) ? ny1 * nt1 : nt1;
+                    int mk = 0;
+                    for (int m1 = 0; m1 < n1; ++m1) {
+                        const int i1 = (F & 1) ? m1 : fixed, j1 = (F & 1) ? fixed : m1;
+                        if (((bd1 & 1) && i1 == nx1 - 1) || ((bd1 & 2) && j1 == ny1 - 1) ||
+                            ((bd1 & 4) && i1 == 0) || ((bd1 & 8) && j1 == 0))
+                            mk |= 1 << m1;
+                    }
+                    const int32_t rec[4] = {d->link_meta[4 * l] + first,
+                                            F | n1 << 2 | nt1 << 6 | stride << 10 | mk << 18,
+                                            d->link_Es_off[l], d->link_Eth_off[l]};
+                    links.insert(links.end(), rec, rec + 4);
+                    lf |= 1 << F;
+                    ++nl;
+                }
+            cl.w = nl | d->col_nx[c] << 8 | d->cell_nth[k] << 12 | (d->cell_bdry[k] & 15) << 16 | lf << 20;
+            cells.push_back(cl);
+        }
+        for (int pr = 0; pr < 3; ++pr) {
+            const int cls = need[pr] <= half ? 0 : 1;
+            hdr[pr][cls].insert(hdr[pr][cls].end(), h, h + HP_HDR);
+            HpClass &hc = p->hp_cls[pr][cls];
+            hc.bytes = std::max(hc.bytes, need[pr]);
+        }
     }
     // the columns the kernel cannot take run on the generic kernels
     std::vector<int32_t> gcells;
     for (int c : over)
         for (int k = d->col_cell_start[c]; k < d->col_cell_start[c + 1]; ++k) gcells.push_back(k);
     const std::vector<int32_t> gitems = scatter_items(p, over);
-    size_t total = link_inn.size() + col_inn.size() + cell_fo.size() + col_ffc.size() +
-                   link_esl.size() + col_es0.size() + col_nes.size() + col_hdr.size() +
-                   cell_lf.size() + link_w.size() + gcells.size() + gitems.size();
-    for (int k = 0; k < HP_NCLS; ++k) total += lists[k].size();
+    // weights and w_i l'_p(xi_i) per node count
+    std::vector<double> wd(size_t(HP_NM + 1) * HP_WD, 0.0);
+    for (int n = 1; n <= HP_NM; ++n)
+        for (int i = 0; i < n; ++i) {
+            wd[size_t(n) * HP_WD + i] = d->lgl_w[n * HP_NM + i];
+            for (int pp = 0; pp < n; ++pp)
+                wd[size_t(n) * HP_WD + HP_NM + pp * n + i] =
+                    d->lgl_w[n * HP_NM + i] * d->lgl_D[(size_t(n) * HP_NM + pp) * HP_NM + i];
+        }
+    const std::vector<float> wd_f(wd.begin(), wd.end());
+    size_t total = ang_flag.size() + links.size() + gcells.size() + gitems.size() + wd_f.size() + 64;
+    for (auto &hp : hdr)
+        for (auto &l : hp) total += l.size();
     RTX_HIP(hipMalloc(&p->hp_alloc, total * sizeof(int32_t)));
-    int32_t *base = static_cast<int32_t *>(p->hp_alloc);
-    size_t o = 0;
-    auto put = [&](const std::vector<int32_t> &v) -> const int32_t * {
-        if (v.empty()) return nullptr;
-        const int32_t *ptr = base + o;
-        (void)hipMemcpy(base + o, v.data(), v.size() * sizeof(int32_t), hipMemcpyHostToDevice);
-        o += v.size();
+    RTX_HIP(hipMalloc(&p->hp_es, (wd.size() + ang_dth.size()) * sizeof(double) +
+                                    cells.size() * sizeof(HpCell) + 64));
+    char *base = static_cast<char *>(p->hp_alloc);
+    auto put = [&](const void *v, size_t bytes) -> const void * {
+        if (bytes == 0) return nullptr;
+        const void *ptr = base;
+        (void)hipMemcpy(base, v, bytes, hipMemcpyHostToDevice);
+        base += (bytes + 15) & ~size_t(15);
         return ptr;
     };
-    p->hp.link_inn = put(link_inn);
-    p->hp.col_inn = put(col_inn);
-    p->hp.cell_fo = put(cell_fo);
-    p->hp.col_ffc = put(col_ffc);
-    p->hp.link_esl = put(link_esl);
-    p->hp.col_es0 = put(col_es0);
-    p->hp.col_nes = put(col_nes);
-    p->hp.col_hdr = put(col_hdr);
-    p->hp.cell_lf = put(cell_lf);
-    p->hp.link_w = put(link_w);
-    if (es_pool.empty()) es_pool.push_back(0.0);
-    RTX_HIP(hipMalloc(&p->hp_es, es_pool.size() * sizeof(double)));
-    RTX_HIP(hipMemcpy(p->hp_es, es_pool.data(), es_pool.size() * sizeof(double),
-                      hipMemcpyHostToDevice));
-    p->hp.es_pool = static_cast<const double *>(p->hp_es);
-    for (int k = 0; k < HP_NCLS; ++k) {
-        p->hp_cls[k].cols = put(lists[k]);
-        p->hp_cls[k].n = int(lists[k].size());
-    }
-    p->hp_gen_cells = put(gcells);
+    auto put_i = [&](const std::vector<int32_t> &v) {
+        return static_cast<const int32_t *>(put(v.data(), v.size() * sizeof(int32_t)));
+    };
+    p->hp.ang_flag = put_i(ang_flag);
+    p->hp.links = reinterpret_cast<const int4 *>(put_i(links));
+    for (int pr = 0; pr < 3; ++pr)
+        for (int k = 0; k < HP_NCLS; ++k) {
+            p->hp_cls[pr][k].hdr = put_i(hdr[pr][k]);
+            p->hp_cls[pr][k].n = int(hdr[pr][k].size() / HP_HDR);
+        }
+    p->hp_gen_cells = put_i(gcells);
     p->hp_n_gen_cells = int(gcells.size());
-    p->hp_gen_items = put(gitems);
+    p->hp_gen_items = put_i(gitems);
     p->hp_n_gen_items = int(gitems.size() / 2);
+    p->hp.wd_f = static_cast<const float *>(put(wd_f.data(), wd_f.size() * sizeof(float)));
+    base = static_cast<char *>(p->hp_es);
+    p->hp.wd = static_cast<const double *>(put(wd.data(), wd.size() * sizeof(double)));
+    p->hp.ang_dth = static_cast<const double *>(put(ang_dth.data(), ang_dth.size() * sizeof(double)));
+    p->hp.cells = static_cast<const HpCell *>(put(cells.data(), cells.size() * sizeof(HpCell)));
+    p->hp_n_cells = int(cells.size());
     RTX_HIP(hipGetLastError());
     p->hp_over_cols = over;
-    p->hp_ok = nfit > 0;
+    p->hp_ok = p->hp_ncols > 0;
     // side stream (default priority) and fork / join events of the class launches
     if (p->hp_ok) {
         RTX_HIP(hipStreamCreateWithFlags(&p->hp_side, hipStreamNonBlocking));
@@ -811,57 +760,53 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
 }
 
 template <typename T, typename A, int PREC>
-static int launch_hp_class(const rtx_plan *p, const HpClass &hc, uint32_t ops, const void *dx,
-                           void *dy, hipStream_t st, int accumulate) {
-    const size_t lds = hc.bytes[PREC == RTX_PREC_F64 ? 0 : (PREC == RTX_PREC_F32 ? 1 : 2)];
-    const int per = (hc.n + HP_XCD - 1) / HP_XCD;
-    RTX_HIP(hipFuncSetAttribute((const void *)k_hpcol<T, A, PREC>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
-    k_hpcol<T, A, PREC><<<per * HP_XCD, HP_THREADS, lds, st>>>(p->m, p->hp, ops, accumulate,
-                                                               hc.cols, hc.n, (const T *)dx,
-                                                               (T *)dy);
-    RTX_HIP(hipGetLastError());
-    return RTX_OK;
-}
-
-// The column kernel on every column it takes.  The LDS classes write
-// disjoint outputs, so the large-column class runs on the caller's stream
-// and the others on the plan's side stream at the same time (the side
-// stream waits for the work queued before the call, and the caller's stream
-// waits for the side stream before returning): the few large-column
-// workgroups then share the GPU with the small ones instead of leaving
-// CUs idle through their tail.
-int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
-                 int accumulate) {
-    auto launch = [&](int k, hipStream_t s) -> int {
-        const HpClass &hc = p->hp_cls[k];
-        if (hc.n == 0) return RTX_OK;
-        if (prec == RTX_PREC_F64)
-            return launch_hp_class<double, double, RTX_PREC_F64>(p, hc, ops, dx, dy, s, accumulate);
-        if (prec == RTX_PREC_F32)
-            return launch_hp_class<float, float, RTX_PREC_F32>(p, hc, ops, dx, dy, s, accumulate);
-        return launch_hp_class<float, float, RTX_PREC_MIXED>(p, hc, ops, dx, dy, s, accumulate);
-    };
-    int busy = 0;
-    for (int k = 0; k < HP_NCLS; ++k) busy += p->hp_cls[k].n > 0 ? 1 : 0;
-    if (busy < 2 || !p->hp_side) {
-        for (int k = HP_NCLS - 1; k >= 0; --k) {
-            const int rc = launch(k, st);
-            if (rc) return rc;
-        }
-        return RTX_OK;
+static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, hipStream_t st,
+                     int accumulate) {
+    if (ops & RTX_OP_BCONV) {
+        const int nblk = (p->hp_n_cells + HF_WAVES - 1) / HF_WAVES;
+        k_hp_flux<T, A><<<(nblk + HP_XCD - 1) / HP_XCD * HP_XCD, 64 * HF_WAVES, 0, st>>>(
+            p->m, p->hp.cells, p->hp.links, p->hp_n_cells, (ops & RTX_OP_RESTRICT) ? 1 : 0,
+            accumulate, (const T *)dx, (T *)dy);
+        RTX_HIP(hipGetLastError());
     }
+    auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
+        const int per = (hc.n + HP_XCD - 1) / HP_XCD;
+        RTX_HIP(hipFuncSetAttribute((const void *)k_hpcol<T, A, PREC>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, int(hc.bytes)));
+        k_hpcol<T, A, PREC><<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(
+            p->m, p->hp, ops, accumulate, hc.hdr, hc.n, (const T *)dx, (T *)dy);
+        RTX_HIP(hipGetLastError());
+        return RTX_OK;
+    };
+    const HpClass *hc = p->hp_cls[PREC];
+    if (hc[0].n == 0 || hc[1].n == 0 || !p->hp_side) {
+        const HpClass &one = hc[0].n ? hc[0] : hc[1];
+        return one.n ? launch(one, st) : RTX_OK;
+    }
+    // The classes write disjoint outputs, so the large-column class runs on
+    // the caller's stream and the other on the plan's side stream at the same
+    // time (the side stream waits for the work queued before, and the
+    // caller's stream for the side stream): the few large columns then share
+    // the GPU with the small ones instead of leaving CUs idle in their tail.
     RTX_HIP(hipEventRecord(p->hp_fork, st));
     RTX_HIP(hipStreamWaitEvent(p->hp_side, p->hp_fork, 0));
-    int rc = launch(HP_NCLS - 1, st);
+    int rc = launch(hc[1], st);
     if (rc) return rc;
-    for (int k = HP_NCLS - 2; k >= 0; --k) {
-        rc = launch(k, p->hp_side);
-        if (rc) return rc;
-    }
+    rc = launch(hc[0], p->hp_side);
+    if (rc) return rc;
     RTX_HIP(hipEventRecord(p->hp_join, p->hp_side));
     RTX_HIP(hipStreamWaitEvent(st, p->hp_join, 0));
     return RTX_OK;
+}
+
+// The column kernels on every column they take.
+int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
+                 int accumulate) {
+    if (prec == RTX_PREC_F64)
+        return launch_hp<double, double, RTX_PREC_F64>(p, ops, dx, dy, st, accumulate);
+    if (prec == RTX_PREC_F32)
+        return launch_hp<float, float, RTX_PREC_F32>(p, ops, dx, dy, st, accumulate);
+    return launch_hp<float, float, RTX_PREC_MIXED>(p, ops, dx, dy, st, accumulate);
 }
 
 }  // namespace rtx

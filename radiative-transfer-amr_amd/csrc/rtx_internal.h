@@ -79,34 +79,40 @@ int fused_column_ok(int ncells, int nsp, int nang, int part_links, size_t bytes6
 size_t fused_bytes(int64_t col_dofs, int64_t nang, int64_t part_dofs, int64_t part_trace,
                    size_t a);
 
-// Column kernel of uneven-order hp meshes (one workgroup per column):
-// column-local offsets of each link's angle-contracted trace block and
-// the column totals.
+// Kernels of uneven-order hp meshes (one wavefront per cell for the face
+// coupling, one workgroup per column for the rest).
 constexpr int HP_MAX_CELLS = 64;    // cells per column on this path
-constexpr int HP_MAX_LINKS = 192;   // upwind links per column on this path
 constexpr int HP_NCLS = 2;          // LDS classes (one launch each)
-struct HpTables {
-    const int32_t *link_inn = nullptr, *col_inn = nullptr;
-    // per cell: column-local offset of its inflow-face sums; per column:
-    // their count
-    const int32_t *cell_fo = nullptr, *col_ffc = nullptr;
-    // E^s staging: per column, its distinct E^s blocks copied contiguously
-    // into es_pool from col_es0 (col_nes values); per link, the column-local
-    // offset of its block in that copy
-    const int32_t *link_esl = nullptr, *col_es0 = nullptr, *col_nes = nullptr;
-    const double *es_pool = nullptr;
-    // per column a header of HP_HDR ints (first cell, cells, nodes per
-    // direction, angles, first DOF, first link, links, first angle, the
-    // inn / face-sum / trace / E^s counts, E^s start, first spatial node), so
-    // the kernel reads a column's scalars in one step; per cell the mask of
-    // faces that carry links; per link face | (neighbour face nodes << 2)
-    const int32_t *col_hdr = nullptr, *cell_lf = nullptr, *link_w = nullptr;
+// A cell of the face-coupling kernel: its inflow faces' factors (dy or dx)
+// dth / 4, first DOF, first link record, and links | N << 8 | angles << 12 |
+// masked faces << 16 | faces that carry links << 20.
+struct HpCell {
+    double fx, fy;
+    int32_t off, l0, w, pad = 0;
 };
+struct HpTables {
+    const HpCell *cells = nullptr;
+    // per link, cell by cell with ascending faces: the trace's first DOF; face
+    // | its nodes << 2 | its angles << 6 | DOFs between nodes << 10 | masked
+    // nodes << 18; E^s and E^theta offsets
+    const int4 *links = nullptr;
+    // per angle (numbered cell by cell): masked faces of its cell | (quadrant
+    // + 1) << 4 | faces that carry links << 8; the cell's width in theta
+    const int32_t *ang_flag = nullptr;
+    const double *ang_dth = nullptr;
+    // per node count n: the n LGL weights, then (from RTX_NMAX on) the n x n
+    // products w_i l'_p(xi_i), row p
+    const double *wd = nullptr;
+    const float *wd_f = nullptr;
+};
+// per column of a class a header of HP_HDR ints (first cell, cells, nodes per
+// direction, angles, first DOF, -, -, first angle, .., [13] first spatial
+// node, [14] column), so the kernel reads a column's scalars in one step
 constexpr int HP_HDR = 16;
 struct HpClass {
     int n = 0;                      // columns
-    const int32_t *cols = nullptr;  // device list (key order)
-    size_t bytes[3] = {0, 0, 0};    // dynamic LDS per workgroup: FP64, FP32, mixed
+    const int32_t *hdr = nullptr;   // their headers (key order)
+    size_t bytes = 0;               // dynamic LDS per workgroup
 };
 int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d);
 int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
@@ -171,12 +177,14 @@ struct rtx_plan {
     const int32_t *sc_all = nullptr, *sc_gen = nullptr;
     int n_sc_all = 0, n_sc_gen = 0;
     void *gen_alloc = nullptr;   // device lists of the generic set
-    // column kernel of hp meshes: per-link tables, LDS classes, and the
-    // columns it cannot take (run on the generic kernels, lists in hp_alloc)
+    // kernels of hp meshes: tables, LDS classes, and the columns they cannot
+    // take (run on the generic kernels, lists in hp_alloc)
     bool hp_ok = false;
     bool hp_default = false;     // mode -1 uses the column kernel
     rtx::HpTables hp;
-    rtx::HpClass hp_cls[rtx::HP_NCLS];
+    rtx::HpClass hp_cls[3][rtx::HP_NCLS];   // per precision
+    int hp_ncols = 0;
+    int hp_n_cells = 0;                     // cells of those columns
     std::vector<int32_t> hp_over_cols;
     const int32_t *hp_gen_cells = nullptr, *hp_gen_items = nullptr;
     int hp_n_gen_cells = 0, hp_n_gen_items = 0;

@@ -454,3 +454,60 @@ def test_copy_f64_measurement_helper(cuda):
     _lib.check(lib.rtx_copy_f64(C.c_void_p(src.data_ptr()), C.c_void_p(dst.data_ptr()), 0, None),
                "rtx_copy_f64")
     assert lib.rtx_copy_f64(C.c_void_p(src.data_ptr()), C.c_void_p(dst.data_ptr()), -1, None) != 0
+
+
+def column_edge_mesh(n, nt, nref_ang):
+    """2 x 2 columns of n x n nodes with 2^nref_ang cells of nt angles (for
+    nref_ang < 2 a cell spans several quadrants and takes inflow through all
+    four faces), one column and one cell an order higher where the order
+    limit allows, so that faces of unlike orders meet."""
+    m = problems.uniform_mesh([1.0, 1.0], [n, n, nt], nref_ang, 1)
+    keys = sorted(m.cols)
+    if n < 10:
+        m.ref_col(keys[0], "spt", "p")
+    if nt < 10:
+        m.ref_cell(keys[-1], sorted(m.cols[keys[-1]].cells)[0], "p")
+    return m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nt,nref_ang", [(3, 3, 0), (4, 10, 1), (5, 7, 4), (6, 4, 2), (7, 9, 4),
+                                           (8, 5, 3), (9, 10, 4), (10, 3, 5)])
+def test_column_kernel_orders_and_angle_counts(cuda, n, nt, nref_ang):
+    """The column kernels at each node count, with 3 to 160 angles (below one
+    16-angle tile, remainders of a tile, more tiles than wavefronts, both LDS
+    classes): parts, boundary rows and accumulation against the oracle.
+
+    Bounds.  An output is a sum of at most about 220 products, each rounded
+    once: sqrt(220) eps = 15 eps of the terms' size, and the two chained face
+    interpolations at most double it; four times that leaves room for terms
+    that cancel: 120 eps = 1.4e-14 in FP64 (TOL64 is 1e-12) and 7e-6 in FP32.
+    Mixed rounds the scattering operands to BF16 (TOLMIX)."""
+    import torch
+    from rtx.operator import (TransportOperator, OP_MASS, OP_SCAT, OP_ICONV, OP_BCONV, OP_SYSTEM,
+                              OP_RESTRICT, OP_ACCUM, PREC_F64, PREC_F32, PREC_MIXED)
+    mesh = column_edge_mesh(n, nt, nref_ang)
+    wl = problems.two_scatterers()
+    print("column", n, nt, nref_ang, "ndof", mesh.get_ndof(), flush=True)
+    V = asm.assemble(mesh, wl.kappa, wl.sigma, wl.Phi)
+    A = (V["BC"] - V["IC"] + V["M"] + V["S"]).tocsr()
+    op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
+    op.set_path(3)
+    rng = np.random.default_rng(n)
+    x, y0 = rng.uniform(-1, 1, op.ndof), rng.uniform(-1, 1, op.ndof)
+    mask = asm.intr_mask(mesh)
+    for prec, dt, tol in [(PREC_F64, torch.float64, TOL64), (PREC_F32, torch.float32, 7e-6),
+                          (PREC_MIXED, torch.float32, TOLMIX)]:
+        xd = _dev(x).to(dt)
+        for name, ops, ref in [("M", OP_MASS, V["M"] @ x), ("IC", OP_ICONV, -(V["IC"] @ x)),
+                               ("BC", OP_BCONV, V["BC"] @ x), ("A", OP_SYSTEM, A @ x),
+                               ("R", OP_SYSTEM | OP_RESTRICT, mask * (A @ (mask * x)))]:
+            y = op.apply(xd, ops=ops, precision=prec).cpu().double().numpy()
+            assert _rel(y, ref) < tol, (name, prec, _rel(y, ref))
+        for name, ops, ref in [("A+", OP_SYSTEM, y0 + A @ x),
+                               ("R+", OP_SYSTEM | OP_RESTRICT, y0 + mask * (A @ (mask * x)))]:
+            yd = _dev(y0).to(dt)
+            op.apply(xd, yd, ops=ops | OP_ACCUM, precision=prec)
+            assert _rel(yd.cpu().double().numpy(), ref) < tol, (name, prec)
+    y = op.apply(_dev(x), ops=OP_SCAT).cpu().numpy()
+    assert _rel(y, V["S"] @ x) < TOL64
