@@ -109,17 +109,6 @@ __device__ inline int hp_xcd(int n) {
 
 constexpr int HF_WAVES = 4;       // cells per workgroup
 
-// v where keep, else 0.  Bits rather than a select: the compiler turns a
-// select of a loaded value into a branch around the load, and a link's loads
-// then wait for each other.
-__device__ inline float hp_keep(float v, bool keep) {
-    return __uint_as_float(__float_as_uint(v) & (keep ? ~0u : 0u));
-}
-__device__ inline double hp_keep(double v, bool keep) {
-    const int k = keep ? ~0 : 0;
-    return __hiloint2double(__double2hiint(v) & k, __double2loint(v) & k);
-}
-
 // One link's operands in matrix-core layout: the neighbour's trace, E^theta
 // and E^s.  Indices past the sizes read the last entry; the trace is zero
 // there (one mask serves both products: the rows past the face's nodes that
@@ -150,7 +139,7 @@ __device__ __forceinline__ HpLink<A> hp_load_link(const DevMesh &m, const int4 r
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
         const uint32_t a = 4 * s + lg, ac = min(a, nt1 - 1);
-        o.tv[s] = hp_keep(A(tr[row * stride + ac]), live && a < nt1);
+        o.tv[s] = keep_if(A(tr[row * stride + ac]), live && a < nt1);
         o.ev[s] = A(Et[ac * nt + r]);
     }
 #pragma unroll

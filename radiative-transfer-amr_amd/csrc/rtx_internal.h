@@ -52,6 +52,33 @@ struct DevMesh {
     const uint16_t *G_bf16;
 };
 
+// v where keep, else 0.  Bits rather than a select: the compiler turns a
+// select of a loaded value into a branch around the load, and the loads of a
+// group then wait for each other.
+__device__ inline float keep_if(float v, bool keep) {
+    return __uint_as_float(__float_as_uint(v) & (keep ? ~0u : 0u));
+}
+__device__ inline double keep_if(double v, bool keep) {
+    const int k = keep ? ~0 : 0;
+    return __hiloint2double(__double2hiint(v) & k, __double2loint(v) & k);
+}
+
+// v_mfma_f64_16x16x4f64.  A operand: row lane % 16, k = lane / 16; B operand:
+// k = lane / 16, column lane % 16; D: column lane % 16, register v of lane
+// group g (lane / 16) row g + 4 v - so register s of a D is the B operand of
+// step s of a next product as it stands.
+typedef double mm_d4 __attribute__((ext_vector_type(4)));
+__device__ inline mm_d4 mma_f64(double a, double b, mm_d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Sum over the wavefront in a fixed order; every lane gets it.
+__device__ inline double wave_sum(double v) {
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s);
+    return v;
+}
+
 }  // namespace rtx
 
 struct rtx_plan;

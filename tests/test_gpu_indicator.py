@@ -172,3 +172,58 @@ def test_error_high_resolution_method(cuda):
     # some cells flagged at 0.9 of the maximum
     assert 0 < ind.error < 0.5
     assert any(c.do_ref for col in ind.cols.values() for c in col.cells.values())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(2, 3, 1), (4, 4, 4), (5, 8, 9), (7, 3, 7), (8, 8, 2), (10, 9, 5),
+                               (10, 10, 10)], ids=str)
+def test_error_measures_at_tile_edges(cuda, n):
+    """Every error kernel at node counts on both sides of a matrix step (4, 8)
+    and of the unrolled sizes (4, 7, 10), non-square columns and unlike
+    neighbours included.
+
+    Bound: a value is a sum of at most 13^3 products of one sign, each of
+    them exact to about 60 eps (three chained interpolations of at most 13
+    terms): 1e-12 is 4,500 eps."""
+    from oracle import error as oerr
+    from rtx.error import ErrorEvaluator
+    from rtx.plan import MeshTables
+
+    def make(up):
+        m = problems.uniform_mesh([1.0, 1.0], list(n), 2, 1)
+        keys = sorted(m.cols)
+        if max(n) < 10:
+            m.ref_col(keys[0], "spt", "p")
+            m.ref_cell(keys[-1], sorted(m.cols[keys[-1]].cells)[0], "p")
+        if up and max(n) < 9:
+            m.ref_mesh(kind="ang", form="p")
+            m.ref_mesh(kind="spt", form="p")
+        return m
+    mesh, mesh_hr = make(False), make(True)
+    ev, t_hr = ErrorEvaluator(mesh), MeshTables(mesh_hr)
+    t = ev.t
+    print("error measures", n, "ndof", t.ndof, flush=True)
+    rng = np.random.default_rng(n[0] + 16 * n[2])
+    u, u_hr = rng.uniform(-1, 1, t.ndof), rng.uniform(-1, 1, t_hr.ndof)
+    ang, ref = ev.angular_jump(u), oind.angular_jump(mesh, u)
+    assert all(_close(ang[k], ref[key]) for k, key in enumerate(t.cell_keys))
+    spt, ref = ev.spatial_jump(u), oind.spatial_jump(mesh, u)
+    assert all(_close(spt[c], ref[ck]) for c, ck in enumerate(t.col_keys))
+    xy, th, n2 = ev.moments(u)
+    for c, ck in enumerate(t.col_keys):
+        s0, ref = int(t.col_sp_off[c]), oind.col_intg_th(mesh, u, ck)
+        assert np.allclose(th[s0:s0 + ref.size], ref.ravel(), rtol=0, atol=TOL)
+    for k, (ck, kk) in enumerate(t.cell_keys):
+        a0 = int(t.col_ang_start[t.cell_col[k]]) + int(t.cell_ang_off[k])
+        ref = oind.cell_intg_xy(mesh, u, ck, kk)
+        assert np.allclose(xy[a0:a0 + ref.size], ref, rtol=0, atol=TOL)
+    err, hr2 = ev.nodal_errors(u, u_hr, t_hr)
+    ref, intg = oind.high_resolution(mesh, u, mesh_hr, u_hr)
+    assert all(_close(err[k], ref[key]) for k, key in enumerate(t.cell_keys))
+    assert _close(float(np.sum(hr2)), intg)
+    own = oind.high_resolution(mesh, u, mesh, u)[1]
+    assert _close(float(np.sum(n2)), own)
+    wave = lambda x, y, a: np.cos(3.0 * x) * np.sin(2.0 * y + 1.0) * (1.5 + np.cos(a))
+    dev = ev.cell_errors(u, ev.hr_values(wave))
+    ref = np.array([e for _, _, e in oerr.cell_errors(mesh, u, wave)])
+    assert np.max(np.abs(dev - ref)) <= TOL * np.max(ref)
