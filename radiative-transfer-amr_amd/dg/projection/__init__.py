@@ -11,11 +11,9 @@ as headerless float64 (``to_file.py:10-19``), read back by ``from_file``.
 returns a matching shape; otherwise (e.g. it branches on scalar
 coordinates) it is called once per node like the reference does.
 """
-import copy
-
 import numpy as np
 
-from ..mesh import Mesh, from_file as mesh_from_file
+from ..mesh import Mesh, copy_mesh, from_file as mesh_from_file
 from ..quadrature import quad_xyth
 
 __all__ = ["Projection", "from_file", "push_forward", "pull_back",
@@ -46,8 +44,8 @@ def eval_nodal(func, *coords) -> np.ndarray:
     try:
         with np.errstate(all="ignore"):
             v = func(*grids)
-        v = np.broadcast_to(np.asarray(v, dtype=np.float64), shape)
-        return np.array(v, dtype=np.float64)
+        v = np.asarray(v, dtype=np.float64)
+        return np.array(v if v.shape == shape else np.broadcast_to(v, shape))
     except Exception:
         out = np.empty(shape)
         for idx in np.ndindex(*shape):
@@ -97,7 +95,7 @@ class Projection_Column:
 
 class Projection:
     def __init__(self, mesh: Mesh, func=None):
-        self.mesh = copy.deepcopy(mesh)
+        self.mesh = copy_mesh(mesh)
         if func is None:
             f = None
         elif not mesh.has_th:
@@ -111,22 +109,21 @@ class Projection:
             assert col.is_lf
             x0, y0, x1, y1 = col.pos
             nx, ny = col.ndofs
-            xb, _, yb, _, _, _ = quad_xyth(nnodes_x=nx, nnodes_y=ny)
-            xf, yf = push_forward(x0, x1, xb), push_forward(y0, y1, yb)
+            if f is not None:
+                xb, _, yb, _, _, _ = quad_xyth(nnodes_x=nx, nnodes_y=ny)
+                xf, yf = push_forward(x0, x1, xb), push_forward(y0, y1, yb)
             cells = {}
             for kkey in sorted(col.cells.keys()):
                 cell = col.cells[kkey]
                 assert cell.is_lf
-                if self.mesh.has_th:
-                    nth = cell.ndofs[0]
-                    thb = quad_xyth(nnodes_th=nth)[4]
-                    thf = push_forward(cell.pos[0], cell.pos[1], thb)
-                else:
-                    nth, thf = 1, np.zeros(1)
+                nth = cell.ndofs[0] if self.mesh.has_th else 1
                 if f is None:
                     vals = np.zeros((nx, ny, nth))
+                elif self.mesh.has_th:
+                    thb = quad_xyth(nnodes_th=nth)[4]
+                    vals = eval_nodal(f, xf, yf, push_forward(cell.pos[0], cell.pos[1], thb))
                 else:
-                    vals = eval_nodal(f, xf, yf, thf)
+                    vals = eval_nodal(f, xf, yf, np.zeros(1))
                 cells[kkey] = Projection_Cell(cell, vals)
             self.cols[ckey] = Projection_Column(col, cells)
 

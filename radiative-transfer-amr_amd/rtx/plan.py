@@ -359,18 +359,29 @@ class MeshTables:
         """func(x, y, th) at every DOF in the global order; one broadcast call
         per column over (x nodes, y nodes, all angular nodes of the column)."""
         out = np.zeros(self.ndof)
+        angles = {}             # angular nodes of each angular mesh, from its first column
         for ci in range(self.ncol):
             x0, y0, x1, y1 = self.col_geom[ci]
             nx, ny = int(self.col_nx[ci]), int(self.col_ny[ci])
             xf = push_forward(x0, x1, _lgl(nx)[0])
             yf = push_forward(y0, y1, _lgl(ny)[0])
             k0, k1 = self.col_cell_start[ci], self.col_cell_start[ci + 1]
-            ths = [push_forward(self.cell_geom[k, 0], self.cell_geom[k, 1],
-                                _lg(int(self.cell_nth[k]))[0]) for k in range(k0, k1)]
-            vals = eval_nodal(func, xf, yf, np.concatenate(ths))
+            sig = self.col_sig[ci]
+            if sig not in angles:
+                angles[sig] = np.concatenate(
+                    [push_forward(self.cell_geom[k, 0], self.cell_geom[k, 1],
+                                  _lg(int(self.cell_nth[k]))[0]) for k in range(k0, k1)])
+            vals = eval_nodal(func, xf, yf, angles[sig].copy())
+            nt = int(self.cell_nth[k0])
+            if vals.shape[2] == nt * (k1 - k0) and np.all(self.cell_nth[k0:k1] == nt):
+                # cells of equal order: one transposed store
+                o = self.cell_dof_off[k0]
+                out[o:o + vals.size].reshape(k1 - k0, nx, ny, nt)[:] = \
+                    vals.reshape(nx, ny, k1 - k0, nt).transpose(2, 0, 1, 3)
+                continue
             a = 0
-            for k, th in zip(range(k0, k1), ths):
-                nt = th.size
+            for k in range(k0, k1):
+                nt = int(self.cell_nth[k])
                 o = self.cell_dof_off[k]
                 out[o:o + nx * ny * nt] = vals[:, :, a:a + nt].ravel()
                 a += nt

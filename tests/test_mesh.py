@@ -298,3 +298,43 @@ def test_tables_reject_unsupported_orders():
         MeshTables(Mesh([1.0, 1.0], [False, False], [11, 3, 3], True))
     with pytest.raises(ValueError):
         MeshTables(Mesh([1.0, 1.0], [False, False], [3, 3, 3], False))
+
+
+@pytest.mark.parametrize("kind", ["mesh", "derived", "no_th"])
+def test_copy_mesh_equals_deepcopy(kind):
+    """A mesh copy has every attribute (added ones and shared lists too) and
+    shares no mutable part; the nodal vector of a mixed-order mesh equals the
+    projection's, cell by cell."""
+    import copy
+    from dg.mesh import Mesh, copy_mesh
+    from dg.projection import Projection
+
+    class Derived(Mesh):
+        def __deepcopy__(self, memo):
+            new = Mesh([1.0, 1.0], [False, False], [2, 2, 2], True)
+            new.tag = "derived"
+            return new
+    if kind == "no_th":
+        mesh = Mesh([1.0, 1.0], [True, False], [3, 4, 2])
+    else:
+        mesh = hp_mesh()
+    shared = [1, [2.0, np.arange(3)]]
+    mesh.extra, mesh.again, mesh.me = shared, shared, mesh
+    if kind == "derived":
+        mesh.__class__ = Derived
+        assert copy_mesh(mesh).tag == "derived"
+        return
+    new, ref = copy_mesh(mesh), copy.deepcopy(mesh)
+    assert new == mesh and new == ref and type(new) is Mesh and new.me is new
+    assert new.extra is new.again and new.extra is not shared
+    assert new.extra[1][1] is not shared[1][1] and new.extra[1][0] == 2.0
+    for ck, col in mesh.cols.items():
+        assert new.cols[ck] is not col and new.cols[ck].pos is not col.pos
+        assert all(a is not b or a is None for a, b in zip(new.cols[ck].nhbr_keys, col.nhbr_keys))
+        for kk, cell in col.cells.items():
+            assert new.cols[ck].cells[kk].__dict__ == cell.__dict__
+            assert new.cols[ck].cells[kk].ndofs is not cell.ndofs
+    if kind == "mesh":
+        from rtx.plan import MeshTables
+        f = lambda x, y, th: np.exp(x - 2.0 * y) * (2.0 + np.cos(th))
+        assert np.array_equal(MeshTables(mesh).eval_nodal_dofs(f), Projection(mesh, f).to_vector())
