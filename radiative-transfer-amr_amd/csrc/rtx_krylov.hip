@@ -7,6 +7,7 @@
 // normalisation) is a fixed sequence of fused FP64 kernels over the tall
 // basis V; reductions are two-phase and deterministic (per-block partial
 // sums, then one reduction per output).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -15,50 +16,97 @@
 namespace rtx {
 
 constexpr int KT = 256;          // threads per block
+constexpr int KW = KT / 64;      // wavefronts per block
 constexpr int KCH = 8;           // basis vectors per mdot block (gridDim.y chunks)
-constexpr int KNB = 1024;        // row blocks of the tall-skinny kernels
+constexpr int KNB = 1024;        // most row blocks of the tall-skinny kernels
 constexpr int KMAXV = 256;       // largest basis handled by one Arnoldi step
 constexpr double REORTH = 0.5;   // re-orthogonalise when |w'|^2 < 0.5 |w|^2
 // state block after the partials (doubles): [0] |w|^2, [1] |w'|^2, [4] flag (int)
 constexpr int WORK_TAIL = 16;
 
-template <int N>
-__device__ inline void block_sum(double (&v)[N], double *sh) {
-    // sh: KT * N doubles; result in sh[j * KT].  (Cross-lane shuffles of
-    // the doubles first, then one LDS stage, measured slower: 18.7 against
-    // 15.6 us for the FP16-basis dot products on 2,048,000 rows.)
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int j = 0; j < N; ++j) sh[j * KT + tid] = v[j];
-    __syncthreads();
-    for (int s = KT / 2; s > 0; s >>= 1) {
-        if (tid < s) {
-#pragma unroll
-            for (int j = 0; j < N; ++j) sh[j * KT + tid] += sh[j * KT + tid + s];
-        }
-        __syncthreads();
-    }
+// Values per thread and load: 16 bytes of the basis (8 bytes of an FP16 one
+// whose rows start on 8 bytes only), or one where rows are not aligned.
+template <typename T>
+constexpr int kvec() { return 16 / int(sizeof(T)); }
+
+// Row blocks: one pass of the block's threads each, up to KNB (fewer blocks
+// leave fewer partial sums to add; more would be nearly empty).
+static int row_blocks(int64_t n, int vw) {
+    const int64_t per = int64_t(KT) * vw;
+    return int(std::max<int64_t>(1, std::min<int64_t>(KNB, (n + per - 1) / per)));
 }
 
-// Four consecutive values as doubles (16-byte loads; the caller checks the
-// alignment).
-__device__ inline void ld4(const float *p, double (&o)[4]) {
-    const float4 f = *reinterpret_cast<const float4 *>(p);
-    o[0] = f.x; o[1] = f.y; o[2] = f.z; o[3] = f.w;
+// N sums over a wavefront at once (N = 8): each step halves the values a
+// lane carries, 10 exchanges instead of 6 N.  Lane l returns the sum of value
+// bit-reversed(l / 8): 4 (l >> 5 & 1) + 2 (l >> 4 & 1) + (l >> 3 & 1).
+__device__ inline double wave_sum8(double (&v)[8], int lane) {
+#pragma unroll
+    for (int h = 4, off = 32; h > 0; h >>= 1, off >>= 1) {
+        const bool up = lane & off;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < h) {
+                const double keep = up ? v[j + h] : v[j], send = up ? v[j] : v[j + h];
+                v[j] = keep + __shfl_xor(send, off);
+            }
+    }
+    double r = v[0];
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) r += __shfl_xor(r, off);
+    return r;
 }
-__device__ inline void ld4(const double *p, double (&o)[4]) {
-    const double2 a = *reinterpret_cast<const double2 *>(p);
-    const double2 b = *reinterpret_cast<const double2 *>(p + 2);
-    o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
+
+// Sum over the block in a fixed order, for every thread (sh: KW doubles).
+__device__ inline double block_sum1(double v, double *sh) {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = sh[0];
+#pragma unroll
+    for (int w = 1; w < KW; ++w) t += sh[w];
+    return t;
 }
-// FP16 basis vectors: four consecutive values in one 8-byte load / store
-typedef _Float16 kh4 __attribute__((ext_vector_type(4)));
-__device__ inline void ld4(const _Float16 *p, double (&o)[4]) {
-    const kh4 v = *reinterpret_cast<const kh4 *>(p);
-    o[0] = double(v[0]); o[1] = double(v[1]); o[2] = double(v[2]); o[3] = double(v[3]);
+
+// VW consecutive values, loaded and stored 16 bytes at a time (8 for four FP16
+// values); the caller checks the alignment.
+template <typename T, int VW> struct KVec {
+    T v[VW];
+};
+template <typename T, int VW>
+constexpr int kelem() { return VW * int(sizeof(T)) > 16 ? 16 / int(sizeof(T)) : VW; }
+
+template <typename T, int VW>
+__device__ inline KVec<T, VW> ldv(const T *p) {
+    KVec<T, VW> o;
+    if constexpr (VW == 1) {
+        o.v[0] = p[0];
+    } else {
+        constexpr int E = kelem<T, VW>();
+        typedef T V __attribute__((ext_vector_type(E)));
+#pragma unroll
+        for (int u = 0; u < VW / E; ++u) {
+            const V q = *reinterpret_cast<const V *>(p + u * E);
+#pragma unroll
+            for (int e = 0; e < E; ++e) o.v[u * E + e] = q[e];
+        }
+    }
+    return o;
 }
-__device__ inline void st4(_Float16 *p, const _Float16 (&v)[4]) {
-    *reinterpret_cast<kh4 *>(p) = kh4{v[0], v[1], v[2], v[3]};
+template <typename T, int VW>
+__device__ inline void stv(T *p, const T (&v)[VW]) {
+    if constexpr (VW == 1) {
+        p[0] = v[0];
+    } else {
+        constexpr int E = kelem<T, VW>();
+        typedef T V __attribute__((ext_vector_type(E)));
+#pragma unroll
+        for (int u = 0; u < VW / E; ++u) {
+            V q;
+#pragma unroll
+            for (int e = 0; e < E; ++e) q[e] = v[u * E + e];
+            *reinterpret_cast<V *>(p + u * E) = q;
+        }
+    }
 }
 // a double rounded to a basis storage type (FP16 through FP32)
 template <typename T>
@@ -66,85 +114,140 @@ __device__ inline T to_store(double x) {
     if constexpr (std::is_same<T, _Float16>::value) return _Float16(float(x));
     else return T(x);
 }
-__device__ inline void st4(float *p, const float (&v)[4]) {
-    *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
-__device__ inline void st4(double *p, const double (&v)[4]) {
-    *reinterpret_cast<double2 *>(p) = make_double2(v[0], v[1]);
-    *reinterpret_cast<double2 *>(p + 2) = make_double2(v[2], v[3]);
-}
 
-// Row range of block b; with VEC the range starts on a multiple of 4.
-template <bool VEC>
+// Row range of block b, starting on a multiple of VW.
+template <int VW>
 __device__ inline void row_range(int64_t n, int b, int nb, int64_t &i0, int64_t &i1) {
     int64_t per = (n + nb - 1) / nb;
-    if (VEC) per = (per + 3) & ~int64_t(3);
+    per = (per + VW - 1) / VW * VW;
     i0 = int64_t(b) * per;
     i1 = (i0 + per < n) ? i0 + per : n;
     if (i0 > n) i0 = n;
 }
 
-// partial[j * nb + b] = sum over block b's rows of V_j[i] w[i], j < nv;
-// if with_ww, partial[nv * nb + b] = sum w[i]^2 (computed by chunk 0).
-template <typename T, bool VEC, typename TW = T>
-__global__ __launch_bounds__(KT) void k_mdot(const T *__restrict__ V, int64_t ld, int nv,
-                                             const TW *__restrict__ w, int64_t n,
-                                             double *__restrict__ partial, int with_ww,
-                                             const int *__restrict__ skip) {
-    if (skip && *skip) return;
-    __shared__ double sh[KT * (KCH + 1)];
-    const int b = blockIdx.x, nb = gridDim.x;
-    const int j0 = blockIdx.y * KCH;
-    int64_t i0, i1;
-    row_range<VEC>(n, b, nb, i0, i1);
-    double acc[KCH + 1];
-#pragma unroll
-    for (int j = 0; j <= KCH; ++j) acc[j] = 0.0;
-    const int64_t nq = VEC ? (i1 - i0) / 4 : 0;
+// One block's dot products with NJ basis vectors: the loads of a pass are
+// independent (NJ is compiled in: a test per vector would make each load wait
+// for the one before).
+template <typename T, int VW, typename TW, int NJ>
+__device__ inline void mdot_rows(const T *V, int64_t ld, const TW *w, int64_t i0, int64_t i1,
+                                 double (&acc)[KCH], double &ww) {
+    const int64_t nq = (i1 - i0) / VW;
     for (int64_t q = threadIdx.x; q < nq; q += KT) {
-        const int64_t i = i0 + 4 * q;
-        double wv[4];
-        ld4(w + i, wv);
+        const int64_t i = i0 + VW * q;
+        const KVec<TW, VW> wv = ldv<TW, VW>(w + i);
+        KVec<T, VW> vv[NJ];
 #pragma unroll
-        for (int j = 0; j < KCH; ++j)
-            if (j0 + j < nv) {
-                double vv[4];
-                ld4(V + int64_t(j0 + j) * ld + i, vv);
-                acc[j] += vv[0] * wv[0] + vv[1] * wv[1] + vv[2] * wv[2] + vv[3] * wv[3];
-            }
-        acc[KCH] += wv[0] * wv[0] + wv[1] * wv[1] + wv[2] * wv[2] + wv[3] * wv[3];
+        for (int j = 0; j < NJ; ++j) vv[j] = ldv<T, VW>(V + j * ld + i);
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+            const double we = double(wv.v[e]);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[j] += double(vv[j].v[e]) * we;
+            ww += we * we;
+        }
     }
-    for (int64_t i = i0 + 4 * nq + threadIdx.x; i < i1; i += KT) {
+    const int64_t i = i0 + VW * nq + threadIdx.x;       // fewer than VW rows past the passes
+    if (VW > 1 && i < i1) {
         const double wi = double(w[i]);
 #pragma unroll
-        for (int j = 0; j < KCH; ++j)
-            if (j0 + j < nv) acc[j] += double(V[int64_t(j0 + j) * ld + i]) * wi;
-        acc[KCH] += wi * wi;
-    }
-    block_sum<KCH + 1>(acc, sh);
-    if (threadIdx.x == 0) {
-        for (int j = 0; j < KCH; ++j)
-            if (j0 + j < nv) partial[int64_t(j0 + j) * nb + b] = sh[j * KT];
-        if (with_ww && blockIdx.y == 0) partial[int64_t(nv) * nb + b] = sh[KCH * KT];
+        for (int j = 0; j < NJ; ++j) acc[j] += double(V[j * ld + i]) * wi;
+        ww += wi * wi;
     }
 }
 
-// out[j] (+)= sum_b partial[j * nb + b]; one block per j.
-__global__ __launch_bounds__(KT) void k_reduce(const double *__restrict__ partial, int nb,
+// partial[j * nb + b] = sum over block b's rows of V_j[i] w[i], j < nv;
+// if with_ww, partial[nv * nb + b] = sum w[i]^2 (computed by chunk 0).
+//
+// Bound by reading V where n is large; one pass of loads and the sums over
+// the block where it is not.  2,048,000 rows, FP16, 1 to 15 vectors: 12.0 ->
+// 10.9 us on average; 65,536 rows, FP64, 1 to 50 vectors: 15.8 -> 5.8 us
+// (1,024 blocks of 64 rows and a tree of eight barriers before).
+template <typename T, int VW, typename TW = T>
+__global__ __launch_bounds__(KT) void k_mdot(const T *__restrict__ V, int64_t ld, int nv,
+                                             const TW *__restrict__ w, int64_t n, int nb,
+                                             double *__restrict__ partial, int with_ww,
+                                             const int *__restrict__ skip) {
+    if (skip && *skip) return;
+    __shared__ double sh[KW][KCH + 1];
+    // workgroups go to the XCDs round-robin: the chunks of row block b one after
+    // another on XCD b % 8 (where k_update's block b runs too), so that w is
+    // read from memory once
+    const int nch = (nv + KCH - 1) / KCH, slot = blockIdx.x / 8;
+    const int b = slot / nch * 8 + blockIdx.x % 8;
+    const int chunk = slot % nch, j0 = chunk * KCH, nj = min(nv - j0, KCH);
+    if (b >= nb) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int64_t i0, i1;
+    row_range<VW>(n, b, nb, i0, i1);
+    double acc[KCH] = {0.0}, ww = 0.0;
+    const T *Vj = V + int64_t(j0) * ld;
+    switch (nj) {
+#define KCASE(NJ)                                                   \
+    case NJ:                                                        \
+        mdot_rows<T, VW, TW, NJ>(Vj, ld, w, i0, i1, acc, ww);       \
+        break;
+        KCASE(1) KCASE(2) KCASE(3) KCASE(4) KCASE(5) KCASE(6) KCASE(7) KCASE(8)
+#undef KCASE
+    }
+    const double s = wave_sum8(acc, lane);
+    if ((lane & 7) == 0)
+        sh[wave][((lane >> 5) & 1) * 4 + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1)] = s;
+    const bool sq = with_ww && chunk == 0;
+    if (sq) {
+        ww = wave_sum(ww);
+        if (lane == 0) sh[wave][KCH] = ww;
+    }
+    __syncthreads();
+    if (tid < nj || (sq && tid == KCH)) {
+        double t = sh[0][tid];
+#pragma unroll
+        for (int v = 1; v < KW; ++v) t += sh[v][tid];
+        partial[int64_t(tid == KCH ? nv : j0 + tid) * nb + b] = t;
+    }
+}
+
+// out[j] (+)= sum_b partial[j * nb + b], nb <= KNB; one wavefront per j.
+__global__ __launch_bounds__(KT) void k_reduce(const double *__restrict__ partial, int nb, int nj,
                                                double *__restrict__ out, int accumulate,
                                                const int *__restrict__ skip) {
     if (skip && *skip) return;
-    __shared__ double sh[KT];
-    const int j = blockIdx.x;
-    double v[1] = {0.0};
-    for (int b = threadIdx.x; b < nb; b += KT) v[0] += partial[int64_t(j) * nb + b];
-    block_sum<1>(v, sh);
-    if (threadIdx.x == 0) out[j] = accumulate ? out[j] + sh[0] : sh[0];
+    const int j = blockIdx.x * KW + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (j >= nj) return;
+    const double *p = partial + int64_t(j) * nb;
+    double v = 0.0;
+#pragma unroll
+    for (int u = 0; u < KNB / 64; ++u)
+        v += keep_if(p[min(lane + 64 * u, nb - 1)], lane + 64 * u < nb);
+    v = wave_sum(v);
+    if (lane == 0) out[j] = accumulate ? out[j] + v : v;
+}
+
+// acc -= V h at VW rows from i: eight (then four) basis vectors' loads at a
+// time; past the last one the last vector again with a zero factor.
+template <typename T, int VW>
+__device__ inline void subtract_rows(const T *V, int64_t ld, int nv, const double *hs, int64_t i,
+                                     double (&acc)[VW]) {
+    int j = 0;
+    const auto some = [&](auto cnt) {
+        constexpr int N = decltype(cnt)::value;
+        KVec<T, VW> vv[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) vv[u] = ldv<T, VW>(V + int64_t(min(j + u, nv - 1)) * ld + i);
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const double h = j + u < nv ? hs[j + u] : 0.0;
+#pragma unroll
+            for (int e = 0; e < VW; ++e) acc[e] -= double(vv[u].v[e]) * h;
+        }
+        j += N;
+    };
+    while (j + 8 <= nv) some(std::integral_constant<int, 8>());
+    while (j < nv) some(std::integral_constant<int, 4>());
 }
 
 // w -= V h (nv vectors); partial[b] = sum over block b of the new w^2
 // (accumulated in FP64 for either storage type).
-template <typename T, bool VEC>
+template <typename T, int VW>
 __global__ __launch_bounds__(KT) void k_update(const T *__restrict__ V, int64_t ld, int nv,
                                                const double *__restrict__ h,
                                                T *__restrict__ w, int64_t n,
@@ -152,59 +255,88 @@ __global__ __launch_bounds__(KT) void k_update(const T *__restrict__ V, int64_t 
                                                const int *__restrict__ skip) {
     if (skip && *skip) return;
     __shared__ double hs[KMAXV];
-    __shared__ double sh[KT];
+    __shared__ double sh[KW];
     for (int j = threadIdx.x; j < nv; j += KT) hs[j] = h[j];
     __syncthreads();
     const int b = blockIdx.x, nb = gridDim.x;
     int64_t i0, i1;
-    row_range<VEC>(n, b, nb, i0, i1);
-    double ss[1] = {0.0};
-    const int64_t nq = VEC ? (i1 - i0) / 4 : 0;
+    row_range<VW>(n, b, nb, i0, i1);
+    double ss = 0.0;
+    const int64_t nq = (i1 - i0) / VW;
     for (int64_t q = threadIdx.x; q < nq; q += KT) {
-        const int64_t i = i0 + 4 * q;
-        double acc[4];
-        ld4(w + i, acc);
-        for (int j = 0; j < nv; ++j) {
-            double vv[4];
-            ld4(V + int64_t(j) * ld + i, vv);
-            const double hj = hs[j];
-            acc[0] -= vv[0] * hj; acc[1] -= vv[1] * hj;
-            acc[2] -= vv[2] * hj; acc[3] -= vv[3] * hj;
-        }
-        T out[4];
+        const int64_t i = i0 + VW * q;
+        const KVec<T, VW> wv = ldv<T, VW>(w + i);
+        double acc[VW];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            out[u] = T(acc[u]);
-            ss[0] += double(out[u]) * double(out[u]);
+        for (int e = 0; e < VW; ++e) acc[e] = double(wv.v[e]);
+        subtract_rows<T, VW>(V, ld, nv, hs, i, acc);
+        T out[VW];
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+            out[e] = T(acc[e]);
+            ss += double(out[e]) * double(out[e]);
         }
-        st4(w + i, out);
+        stv<T, VW>(w + i, out);
     }
-    for (int64_t i = i0 + 4 * nq + threadIdx.x; i < i1; i += KT) {
-        double acc = double(w[i]);
-        int j = 0;
-        for (; j + 4 <= nv; j += 4) {
-            acc -= double(V[int64_t(j) * ld + i]) * hs[j] +
-                   double(V[int64_t(j + 1) * ld + i]) * hs[j + 1] +
-                   double(V[int64_t(j + 2) * ld + i]) * hs[j + 2] +
-                   double(V[int64_t(j + 3) * ld + i]) * hs[j + 3];
-        }
-        for (; j < nv; ++j) acc -= double(V[int64_t(j) * ld + i]) * hs[j];
-        const T wn = T(acc);
+    const int64_t i = i0 + VW * nq + threadIdx.x;
+    if (VW > 1 && i < i1) {
+        double acc[1] = {double(w[i])};
+        subtract_rows<T, 1>(V, ld, nv, hs, i, acc);
+        const T wn = T(acc[0]);
         w[i] = wn;
-        ss[0] += double(wn) * double(wn);
+        ss += double(wn) * double(wn);
     }
-    block_sum<1>(ss, sh);
-    if (threadIdx.x == 0) partial[b] = sh[0];
+    ss = block_sum1(ss, sh);
+    if (threadIdx.x == 0) partial[b] = ss;
+}
+
+// Fold Hessenberg column j (hc[0..j] in LDS, then beta) into the QR
+// factorisation of the cycle's least-squares problem (k_gmres_givens's
+// recurrence), by one block with the rotations staged in LDS; hc is
+// overwritten.
+__device__ inline void givens_column(double *hc, double beta, int j, int m, double *state) {
+    __shared__ double cs_[KMAXV], sn_[KMAXV];
+    double *cs = state, *sn = state + m, *g = state + 2 * m;
+    double *Rj = state + 3 * m + 1 + int64_t(j) * m;
+    double *Hj = state + 3 * m + 1 + int64_t(m) * m + int64_t(j) * (m + 1);
+    double *est = state + 3 * m + 1 + int64_t(m) * m + int64_t(m + 1) * m;
+    const int tid = threadIdx.x;
+    for (int t = tid; t < j; t += KT) {
+        cs_[t] = cs[t];
+        sn_[t] = sn[t];
+    }
+    for (int t = tid; t <= j + 1; t += KT) Hj[t] = t <= j ? hc[t] : beta;
+    const double gj = g[j];
+    __syncthreads();                 // hc is rotated in place below
+    if (tid == 0) {
+        double carry = hc[0];
+        for (int t = 0; t < j; ++t) {
+            const double b = hc[t + 1];
+            hc[t] = cs_[t] * carry + sn_[t] * b;
+            carry = -sn_[t] * carry + cs_[t] * b;
+        }
+        const double den = hypot(carry, beta);
+        const double c = den != 0.0 ? carry / den : 1.0;
+        const double sv = den != 0.0 ? beta / den : 0.0;
+        cs[j] = c;
+        sn[j] = sv;
+        hc[j] = den;
+        g[j + 1] = -sv * gj;
+        g[j] = c * gj;
+        est[j] = fabs(sv * gj);
+    }
+    __syncthreads();
+    for (int t = tid; t <= j; t += KT) Rj[t] = hc[t];
 }
 
 // One Arnoldi update for an FP32 basis with the norm taken from the dot
 // products: hd[0..nv-1] = V^T w, hd[nv] = |w|^2 (FP64 sums of FP32 data),
-// |w'|^2 = |w|^2 - sum h_j^2 (every block computes it, in the same order),
-// v_out = (w - V h) / |w'| written directly (w itself is left as it was);
-// a relative norm below 1e-6 counts as a breakdown (v_out = 0, h = 0).
-// Block 0 writes hcol[0..nv] and, when state is given, folds the column
-// into the Givens factorisation (k_normalize_givens's recurrence).
-template <typename T, bool VEC, typename TW = T>
+// |w'|^2 = |w|^2 - sum h_j^2 (every wavefront computes it, in the same
+// order), v_out = (w - V h) / |w'| written directly (w itself is left as it
+// was); a relative norm below 1e-6 counts as a breakdown (v_out = 0, h = 0).
+// The last block has no rows: it writes hcol[0..nv] and, when state is given,
+// folds the column into the Givens factorisation while the others work.
+template <typename T, int VW, typename TW = T>
 __global__ __launch_bounds__(KT) void k_update_pyth(const T *__restrict__ V, int64_t ld, int nv,
                                                     const double *__restrict__ hd,
                                                     const TW *__restrict__ w,
@@ -212,69 +344,41 @@ __global__ __launch_bounds__(KT) void k_update_pyth(const T *__restrict__ V, int
                                                     double *__restrict__ hcol, int j, int m,
                                                     double *state) {
     __shared__ double hs[KMAXV + 1];
-    __shared__ double beta_sh;
     for (int q = threadIdx.x; q <= nv; q += KT) hs[q] = hd[q];
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double hh = 0.0;
-        for (int q = 0; q < nv; ++q) hh += hs[q] * hs[q];
-        const double r2 = hs[nv] - hh;
-        beta_sh = (r2 > 1e-12 * hs[nv]) ? sqrt(r2) : 0.0;
-    }
-    __syncthreads();
-    const double beta = beta_sh;
+    double hh = 0.0;
+    for (int q = threadIdx.x & 63; q < nv; q += 64) hh += hs[q] * hs[q];
+    hh = wave_sum(hh);
+    const double r2 = hs[nv] - hh;
+    const double beta = (r2 > 1e-12 * hs[nv]) ? sqrt(r2) : 0.0;
     const double sc = beta > 0.0 ? 1.0 / beta : 0.0;
-    const int b = blockIdx.x, nb = gridDim.x;
+    const int b = blockIdx.x, nb = gridDim.x - 1;
+    if (b == nb) {
+        for (int q = threadIdx.x; q <= nv; q += KT) hcol[q] = q < nv ? hs[q] : beta;
+        if (state) givens_column(hs, beta, j, m, state);
+        return;
+    }
     int64_t i0, i1;
-    row_range<VEC>(n, b, nb, i0, i1);
-    const int64_t nq = VEC ? (i1 - i0) / 4 : 0;
+    row_range<VW>(n, b, nb, i0, i1);
+    const int64_t nq = (i1 - i0) / VW;
     for (int64_t q = threadIdx.x; q < nq; q += KT) {
-        const int64_t i = i0 + 4 * q;
-        double acc[4];
-        ld4(w + i, acc);
-        for (int jj = 0; jj < nv; ++jj) {
-            double vv[4];
-            ld4(V + int64_t(jj) * ld + i, vv);
-            const double hj = hs[jj];
-            acc[0] -= vv[0] * hj; acc[1] -= vv[1] * hj;
-            acc[2] -= vv[2] * hj; acc[3] -= vv[3] * hj;
-        }
-        T out[4];
+        const int64_t i = i0 + VW * q;
+        const KVec<TW, VW> wv = ldv<TW, VW>(w + i);
+        double acc[VW];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) out[u] = to_store<T>(acc[u] * sc);
-        st4(v_out + i, out);
+        for (int e = 0; e < VW; ++e) acc[e] = double(wv.v[e]);
+        subtract_rows<T, VW>(V, ld, nv, hs, i, acc);
+        T out[VW];
+#pragma unroll
+        for (int e = 0; e < VW; ++e) out[e] = to_store<T>(acc[e] * sc);
+        stv<T, VW>(v_out + i, out);
     }
-    for (int64_t i = i0 + 4 * nq + threadIdx.x; i < i1; i += KT) {
-        double acc = double(w[i]);
-        for (int jj = 0; jj < nv; ++jj) acc -= double(V[int64_t(jj) * ld + i]) * hs[jj];
-        v_out[i] = to_store<T>(acc * sc);
+    const int64_t i = i0 + VW * nq + threadIdx.x;
+    if (VW > 1 && i < i1) {
+        double acc[1] = {double(w[i])};
+        subtract_rows<T, 1>(V, ld, nv, hs, i, acc);
+        v_out[i] = to_store<T>(acc[0] * sc);
     }
-    if (b != 0 || threadIdx.x != 0) return;
-    for (int q = 0; q < nv; ++q) hcol[q] = hs[q];
-    hcol[nv] = beta;
-    if (!state) return;
-    double *cs = state, *sn = state + m, *g = state + 2 * m;
-    double *Rj = state + 3 * m + 1 + int64_t(j) * m;
-    double *Hj = state + 3 * m + 1 + int64_t(m) * m + int64_t(j) * (m + 1);
-    double *est = state + 3 * m + 1 + int64_t(m) * m + int64_t(m + 1) * m;
-    for (int t = 0; t <= j; ++t) Hj[t] = hs[t];
-    Hj[j + 1] = beta;
-    double carry = hs[0];
-    for (int t = 0; t < j; ++t) {
-        const double bb = hs[t + 1];
-        Rj[t] = cs[t] * carry + sn[t] * bb;
-        carry = -sn[t] * carry + cs[t] * bb;
-    }
-    const double den = hypot(carry, beta);
-    const double c = den != 0.0 ? carry / den : 1.0;
-    const double sv = den != 0.0 ? beta / den : 0.0;
-    cs[j] = c;
-    sn[j] = sv;
-    Rj[j] = den;
-    const double gj = g[j];
-    g[j + 1] = -sv * gj;
-    g[j] = c * gj;
-    est[j] = fabs(g[j + 1]);
 }
 
 // state layout (doubles): [0] |w|^2 before projection, [1] |w'|^2 after;
@@ -287,15 +391,35 @@ __global__ void k_set_flag(int *flag, int v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *flag = v;
 }
 
-// v_out = w / sqrt(nrm2); hcol[nv] = sqrt(nrm2).  nrm2 comes from state.
+// v_out = w / |w|, |w|^2 the sum of the nrm2 partials (every block adds them,
+// in the same order).  The last block has no rows: it sets hcol[nv] = |w| and,
+// when state is given, folds Hessenberg column j into the Givens factorisation.
 template <typename T>
-__global__ void k_normalize(const T *__restrict__ w, T *__restrict__ v_out, int64_t n,
-                            const double *__restrict__ nrm2, double *__restrict__ hcol, int nv) {
-    const double beta = sqrt(*nrm2);
+__global__ __launch_bounds__(KT) void k_normalize(const T *__restrict__ w, T *__restrict__ v_out,
+                                                  int64_t n, const double *__restrict__ nrm2,
+                                                  int nparts, double *__restrict__ hcol, int nv,
+                                                  int j, int m, double *state) {
+    __shared__ double sh[KW];
+    double v = 0.0;
+#pragma unroll
+    for (int u = 0; u < KNB / KT; ++u) {
+        const int q = threadIdx.x + KT * u;
+        v += keep_if(nrm2[min(q, nparts - 1)], q < nparts);
+    }
+    const double beta = sqrt(block_sum1(v, sh));
     const double s = beta > 0.0 ? 1.0 / beta : 0.0;
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    for (; i < n; i += int64_t(gridDim.x) * blockDim.x) v_out[i] = T(double(w[i]) * s);
-    if (blockIdx.x == 0 && threadIdx.x == 0) hcol[nv] = beta;
+    const int nb = gridDim.x - 1;
+    if (int(blockIdx.x) == nb) {
+        if (threadIdx.x == 0) hcol[nv] = beta;
+        if (!state) return;
+        __shared__ double hc[KMAXV + 1];
+        for (int t = threadIdx.x; t <= j; t += KT) hc[t] = hcol[t];
+        __syncthreads();
+        givens_column(hc, beta, j, m, state);
+        return;
+    }
+    int64_t i = int64_t(blockIdx.x) * KT + threadIdx.x;
+    for (; i < n; i += int64_t(nb) * KT) v_out[i] = T(double(w[i]) * s);
 }
 
 // x += sum_j y_j V_j  (y on the device)
@@ -375,68 +499,48 @@ __global__ void k_gmres_givens(int j, int m, const double *__restrict__ hcol, do
     s.est[j] = fabs(s.g[j + 1]);
 }
 
-// v_out = w / |w| (as k_normalize) and, in block 0, the Givens update of
-// column j (as k_gmres_givens) with the rotations staged in LDS, so the
-// serial recurrence runs on LDS values while the other blocks normalise.
-template <typename T>
-__global__ __launch_bounds__(KT) void k_normalize_givens(const T *__restrict__ w,
-                                                         T *__restrict__ v_out, int64_t n,
-                                                         const double *__restrict__ nrm2,
-                                                         double *__restrict__ hcol, int nv,
-                                                         int j, int m, double *state) {
-    const double beta = sqrt(*nrm2);
-    const double s = beta > 0.0 ? 1.0 / beta : 0.0;
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    for (; i < n; i += int64_t(gridDim.x) * blockDim.x) v_out[i] = T(double(w[i]) * s);
-    if (blockIdx.x != 0) return;
-    __shared__ double hc[KMAXV + 1], cs[KMAXV], sn[KMAXV];
-    GState g(state, m);
-    const int tid = threadIdx.x;
-    for (int t = tid; t <= j; t += KT) hc[t] = hcol[t];
-    if (tid == 0) hc[j + 1] = beta;
-    for (int t = tid; t < j; t += KT) {
-        cs[t] = g.cs[t];
-        sn[t] = g.sn[t];
-    }
-    __syncthreads();
-    double *Hj = g.H + int64_t(j) * (m + 1);
-    for (int t = tid; t <= j + 1; t += KT) Hj[t] = hc[t];
-    __syncthreads();                 // hc is rotated in place below
-    if (tid == 0) {
-        hcol[nv] = beta;
-        double carry = hc[0];
-        for (int t = 0; t < j; ++t) {
-            const double b = hc[t + 1];
-            hc[t] = cs[t] * carry + sn[t] * b;
-            carry = -sn[t] * carry + cs[t] * b;
+// y = R_k^{-1} g_k (back substitution over the first k columns), one
+// wavefront: lane l holds rows l, l + 64, .. and takes the columns from the
+// last to the first, the next one (contiguous in R) loading meanwhile.  Row by
+// row on one thread it was 110 us at k = 50, each term waiting for a load:
+// 14 us now.
+template <int ROWS>
+__device__ inline void back_substitute(int k, int m, const GState &s, double *y, int lane) {
+    double acc[ROWS], col[ROWS], nxt[ROWS];
+    const auto load = [&](int l, double (&c)[ROWS]) {
+        const double *R = s.R + int64_t(max(l, 0)) * m;
+#pragma unroll
+        for (int q = 0; q < ROWS; ++q) c[q] = R[min(lane + 64 * q, max(l, 0))];
+    };
+#pragma unroll
+    for (int q = 0; q < ROWS; ++q) acc[q] = s.g[min(lane + 64 * q, k - 1)];
+    load(k - 1, col);
+    for (int l = k - 1; l >= 0; --l) {
+        load(l - 1, nxt);
+        double num = acc[0], d = col[0];
+#pragma unroll
+        for (int q = 1; q < ROWS; ++q)
+            if (l >> 6 == q) {
+                num = acc[q];
+                d = col[q];
+            }
+        num = __shfl(num, l & 63);
+        d = __shfl(d, l & 63);
+        const double yl = d != 0.0 ? num / d : 0.0;
+        if (lane == 0) y[l] = yl;
+#pragma unroll
+        for (int q = 0; q < ROWS; ++q) {
+            if (lane + 64 * q < l) acc[q] -= col[q] * yl;
+            col[q] = nxt[q];
         }
-        const double hj1 = beta;
-        const double den = hypot(carry, hj1);
-        const double c = den != 0.0 ? carry / den : 1.0;
-        const double sv = den != 0.0 ? hj1 / den : 0.0;
-        g.cs[j] = c;
-        g.sn[j] = sv;
-        hc[j] = den;
-        const double gj = g.g[j];
-        g.g[j + 1] = -sv * gj;
-        g.g[j] = c * gj;
-        g.est[j] = fabs(g.g[j + 1]);
     }
-    __syncthreads();
-    double *Rj = g.R + int64_t(j) * m;
-    for (int t = tid; t <= j; t += KT) Rj[t] = hc[t];
 }
 
-// y = R_k^{-1} g_k (back substitution over the first k columns).
-__global__ void k_gmres_solve(int k, int m, const double *state, double *__restrict__ y) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ __launch_bounds__(64) void k_gmres_solve(int k, int m, const double *state,
+                                                    double *__restrict__ y) {
     GState s(const_cast<double *>(state), m);
-    for (int i = k - 1; i >= 0; --i) {
-        double acc = s.g[i];
-        for (int l = i + 1; l < k; ++l) acc -= s.R[int64_t(l) * m + i] * y[l];
-        const double d = s.R[int64_t(i) * m + i];
-        y[i] = d != 0.0 ? acc / d : 0.0;
-    }
+    if (k <= 64) back_substitute<1>(k, m, s, y, threadIdx.x);
+    else back_substitute<KMAXV / 64>(k, m, s, y, threadIdx.x);
 }
 
 template <typename S, typename D>
@@ -469,22 +573,65 @@ static bool aligned16(const T *p) {
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-template <typename T>
-static void launch_mdot(bool vec, dim3 grid, hipStream_t st, const T *V, int64_t ld, int nv,
-                        const T *w, int64_t n, double *part, int with_ww, const int *flag) {
-    if (vec)
-        k_mdot<T, true><<<grid, KT, 0, st>>>(V, ld, nv, w, n, part, with_ww, flag);
-    else
-        k_mdot<T, false><<<grid, KT, 0, st>>>(V, ld, nv, w, n, part, with_ww, flag);
+// Values per load that the basis and w allow (rows of nv > 1 vectors start
+// ld apart).
+template <typename T, typename TW>
+static int vec_width(const T *V, int64_t ld, int nv, const TW *w) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(V) | (nv > 1 ? uintptr_t(ld) * sizeof(T) : 0);
+    if (!aligned16(w)) return 1;
+    if (at % 16 == 0) return kvec<T>();
+    return sizeof(T) == 2 && at % 8 == 0 ? 4 : 1;
+}
+
+// f(std::integral_constant<int, VW>) for the width vec_width gave.
+template <typename T, typename F>
+static void with_width(int vw, F f) {
+    if (vw == kvec<T>()) return f(std::integral_constant<int, kvec<T>()>());
+    if constexpr (sizeof(T) == 2)
+        if (vw == 4) return f(std::integral_constant<int, 4>());
+    f(std::integral_constant<int, 1>());
+}
+
+template <typename T, typename TW>
+static void launch_mdot(int vw, int nb, hipStream_t st, const T *V, int64_t ld, int nv,
+                        const TW *w, int64_t n, double *part, int with_ww, const int *flag) {
+    const int grid = (nb + 7) / 8 * 8 * ((nv + KCH - 1) / KCH);
+    with_width<T>(vw, [&](auto v) {
+        k_mdot<T, decltype(v)::value, TW><<<grid, KT, 0, st>>>(V, ld, nv, w, n, nb, part, with_ww,
+                                                               flag);
+    });
+}
+
+static void launch_reduce(const double *part, int nb, int nj, double *out, int accumulate,
+                          const int *flag, hipStream_t st) {
+    k_reduce<<<(nj + KW - 1) / KW, KT, 0, st>>>(part, nb, nj, out, accumulate, flag);
 }
 
 template <typename T>
-static void launch_update(bool vec, hipStream_t st, const T *V, int64_t ld, int nv,
+static void launch_update(int vw, int nb, hipStream_t st, const T *V, int64_t ld, int nv,
                           const double *h, T *w, int64_t n, double *part, const int *flag) {
-    if (vec)
-        k_update<T, true><<<KNB, KT, 0, st>>>(V, ld, nv, h, w, n, part, flag);
-    else
-        k_update<T, false><<<KNB, KT, 0, st>>>(V, ld, nv, h, w, n, part, flag);
+    with_width<T>(vw, [&](auto v) {
+        k_update<T, decltype(v)::value><<<nb, KT, 0, st>>>(V, ld, nv, h, w, n, part, flag);
+    });
+}
+
+// Classical Gram-Schmidt, one pass, with the norm from the dot products, in
+// three launches: dots, their reduction, the update writing the normalised
+// vector (and the Givens update).  Widths count V_out's row too.
+template <typename T, typename TW>
+static int arnoldi_pyth(const T *d_V, int64_t ld, int nv, int64_t n, const TW *d_w, double *d_hcol,
+                        double *part, double *hd, hipStream_t st, int gj, int gm,
+                        double *d_state) {
+    T *V_out = const_cast<T *>(d_V) + int64_t(nv) * ld;
+    const int vw = vec_width(d_V, ld, nv + 1, d_w), nb = row_blocks(n, vw);
+    launch_mdot(vw, nb, st, d_V, ld, nv, d_w, n, part, 1, nullptr);
+    launch_reduce(part, nb, nv + 1, hd, 0, nullptr, st);
+    with_width<T>(vw, [&](auto v) {
+        k_update_pyth<T, decltype(v)::value, TW><<<nb + 1, KT, 0, st>>>(
+            d_V, ld, nv, hd, d_w, V_out, n, d_hcol, gj, gm, d_state);
+    });
+    RTX_HIP(hipGetLastError());
+    return RTX_OK;
 }
 
 // One Arnoldi step; with d_state, the final normalisation also folds the
@@ -503,59 +650,43 @@ static int arnoldi_step(const T *d_V, int64_t ld, int nv, int64_t n, T *d_w, dou
     double *part2 = d_work + int64_t(KMAXV + 1) * KNB;      // KNB
     double *state = part2 + KNB;                            // [ww0, ww1, h2...]
     int *flag = reinterpret_cast<int *>(state + 4);
-    const int nchunk = (nv + KCH - 1) / KCH;
     T *V_out = const_cast<T *>(d_V) + int64_t(nv) * ld;
-    const bool vec = (ld % 4 == 0) && aligned16(d_V) && aligned16(d_w);
-    if (refine == 0 && std::is_same<T, float>::value) {
-        // FP32 basis (the inner solves of mixed refinement): classical
-        // Gram-Schmidt, one pass, with the norm from the dot products, in
-        // three launches: dots, their reduction, the update writing the
-        // normalised vector (and the Givens update)
-        double *hd = part2;                     // nv + 1 reduced values
-        launch_mdot<T>(vec, dim3(KNB, nchunk), st, d_V, ld, nv, d_w, n, part, 1, nullptr);
-        k_reduce<<<nv + 1, KT, 0, st>>>(part, KNB, hd, 0, nullptr);
-        if (vec)
-            k_update_pyth<T, true><<<KNB, KT, 0, st>>>(d_V, ld, nv, hd, d_w, V_out, n, d_hcol,
-                                                     gj, gm, d_state);
-        else
-            k_update_pyth<T, false><<<KNB, KT, 0, st>>>(d_V, ld, nv, hd, d_w, V_out, n, d_hcol,
-                                                      gj, gm, d_state);
-        RTX_HIP(hipGetLastError());
-        return RTX_OK;
-    }
-    auto normalize = [&]() {
-        if (d_state)
-            k_normalize_givens<T><<<2048, KT, 0, st>>>(d_w, V_out, n, state + 1, d_hcol, nv, gj,
-                                                       gm, d_state);
-        else
-            k_normalize<T><<<2048, KT, 0, st>>>(d_w, V_out, n, state + 1, d_hcol, nv);
+    // FP32 basis (the inner solves of mixed refinement)
+    if constexpr (std::is_same<T, float>::value)
+        if (refine == 0)
+            return arnoldi_pyth(d_V, ld, nv, n, d_w, d_hcol, part, part2, st, gj, gm,
+                                d_state);
+    const int vw = vec_width(d_V, ld, nv, d_w), nb = row_blocks(n, vw);
+    auto normalize = [&](const double *nrm2, int nparts) {
+        const int blocks = int(std::min<int64_t>(2048, (n + KT - 1) / KT));
+        k_normalize<T><<<blocks + 1, KT, 0, st>>>(d_w, V_out, n, nrm2, nparts, d_hcol, nv, gj, gm,
+                                                  d_state);
     };
     // pass 1: h = V^T w, |w|^2
-    launch_mdot<T>(vec, dim3(KNB, nchunk), st, d_V, ld, nv, d_w, n, part, refine == 1 ? 1 : 0,
-                   nullptr);
-    k_reduce<<<nv, KT, 0, st>>>(part, KNB, d_hcol, 0, nullptr);
-    if (refine == 1) k_reduce<<<1, KT, 0, st>>>(part + int64_t(nv) * KNB, KNB, state + 0, 0, nullptr);
+    launch_mdot(vw, nb, st, d_V, ld, nv, d_w, n, part, refine == 1 ? 1 : 0, nullptr);
+    launch_reduce(part, nb, nv, d_hcol, 0, nullptr, st);
+    if (refine == 1) launch_reduce(part + int64_t(nv) * nb, nb, 1, state + 0, 0, nullptr, st);
     // w -= V h, |w'|^2
-    launch_update<T>(vec, st, d_V, ld, nv, d_hcol, d_w, n, part2, nullptr);
-    k_reduce<<<1, KT, 0, st>>>(part2, KNB, state + 1, 0, nullptr);
+    launch_update<T>(vw, nb, st, d_V, ld, nv, d_hcol, d_w, n, part2, nullptr);
     if (refine == 0) {     // classical Gram-Schmidt, one pass (PETSc's default)
-        normalize();
+        normalize(part2, nb);
         RTX_HIP(hipGetLastError());
         return RTX_OK;
     }
+    launch_reduce(part2, nb, 1, state + 1, 0, nullptr, st);
     if (refine == 1)
         k_reorth_test<<<1, 1, 0, st>>>(state, flag);
     else
         k_set_flag<<<1, 1, 0, st>>>(flag, 0);
     // optional pass 2 (skipped on the device when flag == 1)
-    launch_mdot<T>(vec, dim3(KNB, nchunk), st, d_V, ld, nv, d_w, n, part, 0, flag);
+    launch_mdot(vw, nb, st, d_V, ld, nv, d_w, n, part, 0, flag);
     // accumulate the correction into hcol, keep it separately for the update
     double *hcorr = part + int64_t(KMAXV) * KNB;            // nv doubles, after the partials
-    k_reduce<<<nv, KT, 0, st>>>(part, KNB, hcorr, 0, flag);
-    launch_update<T>(vec, st, d_V, ld, nv, hcorr, d_w, n, part2, flag);
-    k_reduce<<<1, KT, 0, st>>>(part2, KNB, state + 1, 0, flag);
-    k_reduce<<<nv, KT, 0, st>>>(hcorr, 1, d_hcol, 1, flag);  // hcol += hcorr
-    normalize();
+    launch_reduce(part, nb, nv, hcorr, 0, flag, st);
+    launch_update<T>(vw, nb, st, d_V, ld, nv, hcorr, d_w, n, part2, flag);
+    launch_reduce(part2, nb, 1, state + 1, 0, flag, st);
+    launch_reduce(hcorr, 1, nv, d_hcol, 1, flag, st);       // hcol += hcorr
+    normalize(state + 1, 1);
     RTX_HIP(hipGetLastError());
     return RTX_OK;
 }
@@ -575,25 +706,7 @@ static int arnoldi_step_h(const _Float16 *d_V, int64_t ld, int nv, int64_t n, co
     hipStream_t st = static_cast<hipStream_t>(stream);
     double *part = d_work;
     double *hd = d_work + int64_t(KMAXV + 1) * KNB;
-    const int nchunk = (nv + KCH - 1) / KCH;
-    _Float16 *V_out = const_cast<_Float16 *>(d_V) + int64_t(nv) * ld;
-    const bool vec = (ld % 4 == 0) && aligned16(d_V) && aligned16(d_w) &&
-                     (reinterpret_cast<uintptr_t>(V_out) & 7) == 0;
-    if (vec) {
-        k_mdot<_Float16, true, float><<<dim3(KNB, nchunk), KT, 0, st>>>(d_V, ld, nv, d_w, n, part,
-                                                                        1, nullptr);
-        k_reduce<<<nv + 1, KT, 0, st>>>(part, KNB, hd, 0, nullptr);
-        k_update_pyth<_Float16, true, float><<<KNB, KT, 0, st>>>(d_V, ld, nv, hd, d_w, V_out, n,
-                                                                d_hcol, gj, gm, d_state);
-    } else {
-        k_mdot<_Float16, false, float><<<dim3(KNB, nchunk), KT, 0, st>>>(d_V, ld, nv, d_w, n,
-                                                                         part, 1, nullptr);
-        k_reduce<<<nv + 1, KT, 0, st>>>(part, KNB, hd, 0, nullptr);
-        k_update_pyth<_Float16, false, float><<<KNB, KT, 0, st>>>(d_V, ld, nv, hd, d_w, V_out, n,
-                                                                 d_hcol, gj, gm, d_state);
-    }
-    RTX_HIP(hipGetLastError());
-    return RTX_OK;
+    return arnoldi_pyth(d_V, ld, nv, n, d_w, d_hcol, part, hd, st, gj, gm, d_state);
 }
 
 /* One Arnoldi step: orthogonalise w against V_0..V_{nv-1} (columns of length n,
@@ -726,11 +839,9 @@ extern "C" int rtx_mdot(const double *d_V, int64_t ld, int nv, int64_t n, const 
                         double *d_out, double *d_work, void *stream) {
     RTX_CHECK(d_V && d_w && d_out && d_work && nv >= 1 && nv < KMAXV, "rtx_mdot: bad argument");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int nchunk = (nv + KCH - 1) / KCH;
-    // vector loads need every V_j on 16 bytes: any ld for a single vector
-    const bool vec = (nv == 1 || ld % 4 == 0) && aligned16(d_V) && aligned16(d_w);
-    launch_mdot<double>(vec, dim3(KNB, nchunk), st, d_V, ld, nv, d_w, n, d_work, 0, nullptr);
-    k_reduce<<<nv, KT, 0, st>>>(d_work, KNB, d_out, 0, nullptr);
+    const int vw = vec_width(d_V, ld, nv, d_w), nb = row_blocks(n, vw);
+    launch_mdot(vw, nb, st, d_V, ld, nv, d_w, n, d_work, 0, nullptr);
+    launch_reduce(d_work, nb, nv, d_out, 0, nullptr, st);
     RTX_HIP(hipGetLastError());
     return RTX_OK;
 }

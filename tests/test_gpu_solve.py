@@ -827,3 +827,90 @@ def test_block_jacobi_fp4_apply(cuda):
         rhs = op.mask(fd - op.apply(bd, ops=OP_SYSTEM), keep_interior=True)
         x, info = learned.Session(op, bj=pc, precision="mixed").solve(rhs, rtol=1e-8)
         assert info["converged_reason"] > 0 and info["rel_residual"] <= 1e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("basis", [0, 1, 2], ids=["f64", "f32", "f16"])
+@pytest.mark.parametrize("n,pad", [(1, 0), (5, 3), (513, 0), (1024, 0), (4100, 0), (4100, 4),
+                                   (300_001, 7)])
+def test_arnoldi_step_widths(cuda, basis, n, pad):
+    """One Arnoldi step against numpy at lengths around a pass of a block and
+    its load widths (rows on 16 bytes, on 8, unaligned), 1 to 17 vectors (one,
+    two and three chunks, remainders of the update's groups).
+
+    Bounds.  Dot products: sums in FP64 of at most 300,001 products of
+    stored values, each error below 300,001 eps / 2 = 3.3e-11 of |v||w| at
+    the very worst, and 600 eps for rounding errors of random sign: 1e-12.
+    The new vector: the same, plus its rounding to FP32 (2^-24) or FP16
+    (2^-11, and 2^-25 below its normal range)."""
+    import ctypes as C
+    import torch
+    from rtx import _lib
+    from rtx.krylov import _vp
+    lib = _lib.load()
+    dt = (torch.float64, torch.float32, torch.float16)[basis]
+    wt = torch.float32 if basis else torch.float64
+    m, ld = 20, n + pad
+    ws, ss = C.c_int64(), C.c_int64()
+    _lib.check(lib.rtx_arnoldi_workspace(m + 1, C.byref(ws)), "ws")
+    _lib.check(lib.rtx_gmres_state_size(m, C.byref(ss)), "ss")
+    rng = np.random.default_rng(n + pad)
+    for nv in (1, 7, 8, 9, 17):
+        print("arnoldi", basis, n, ld, nv, flush=True)
+        V = torch.zeros((nv + 1, ld), dtype=dt, device="cuda")
+        rows = rng.normal(size=(nv, n)) / (8.0 * np.sqrt(n))
+        V[:nv, :n] = torch.from_numpy(rows).cuda().to(dt)
+        w = torch.from_numpy(rng.normal(size=n)).cuda().to(wt)
+        Vh, wh = V[:nv, :n].double().cpu().numpy(), w.double().cpu().numpy()
+        work = torch.full((int(ws.value),), float("nan"), dtype=torch.float64, device="cuda")
+        state = torch.zeros(int(ss.value), dtype=torch.float64, device="cuda")
+        hcol = torch.zeros(m + 2, dtype=torch.float64, device="cuda")
+        _lib.check(lib.rtx_gmres_begin(m, 2.0, _vp(state), None), "begin")
+        _lib.check(lib.rtx_gmres_arnoldi(basis, _vp(V), ld, n, _vp(w), _vp(hcol), _vp(work), 0,
+                                         nv - 1, m, _vp(state), None), "step")
+        h = Vh @ wh
+        new = wh - h @ Vh
+        beta = np.sqrt(wh @ wh - h @ h) if basis else np.linalg.norm(new)
+        got = hcol[:nv + 1].cpu().numpy()
+        scale = np.linalg.norm(wh)
+        assert np.abs(got[:nv] - h).max() <= 1e-12 * scale
+        assert abs(got[nv] - beta) <= 1e-12 * scale
+        out = V[nv, :n].double().cpu().numpy()
+        tol = (0.0, 2.0 ** -24, 2.0 ** -11)[basis]
+        assert (np.abs(out - new / beta) <= tol * np.abs(new / beta) + 1e-12
+                + (2.0 ** -25 if basis == 2 else 0.0)).all()
+        assert not V[nv, n:].any()
+        # column nv - 1 of the raw Hessenberg matrix
+        H0 = 3 * m + 1 + m * m + (nv - 1) * (m + 1)
+        assert np.array_equal(state[H0:H0 + nv + 1].cpu().numpy(), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [1, 2, 63, 64, 65, 130, 200])
+def test_gmres_back_substitution(cuda, k):
+    """y = R^-1 g against numpy up to and past one wavefront's rows, with a
+    zero pivot (its entry of y is zero).  R = I + N, |N| <= 1 / (2 k): its
+    inverse is bounded by 2, so 1e-13 holds with room for k eps."""
+    import ctypes as C
+    import torch
+    from rtx import _lib
+    from rtx.krylov import _vp
+    lib, m = _lib.load(), 200
+    ss = C.c_int64()
+    _lib.check(lib.rtx_gmres_state_size(m, C.byref(ss)), "ss")
+    rng = np.random.default_rng(k)
+    R = np.triu(rng.uniform(-0.5, 0.5, (k, k)) / k, 1) + np.eye(k)
+    if k > 2:
+        R[k // 2, k // 2] = 0.0
+    g = rng.uniform(-1, 1, k)
+    st = np.full(int(ss.value), np.nan)
+    st[2 * m:2 * m + k] = g
+    for j in range(k):
+        st[3 * m + 1 + j * m:3 * m + 1 + j * m + j + 1] = R[:j + 1, j]
+    y = np.zeros(k)
+    for i in range(k - 1, -1, -1):
+        y[i] = (g[i] - R[i, i + 1:] @ y[i + 1:]) / R[i, i] if R[i, i] != 0.0 else 0.0
+    state, yd = _dev(st), _dev(np.zeros(m))
+    _lib.check(lib.rtx_gmres_solve(k, m, _vp(state), _vp(yd), None), "solve")
+    assert np.abs(yd[:k].cpu().numpy() - y).max() <= 1e-13
+    assert not yd[k:].any()
