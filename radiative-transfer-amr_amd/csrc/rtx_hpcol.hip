@@ -10,8 +10,8 @@
 //              the matrix cores with operands read from memory; the links of
 //              a face add up in the accumulators.  The sums of the cell's
 //              inflow faces are stored at their DOFs of y.
-//   k_hpcol    everything else, one workgroup of 512 threads per column of
-//              N x N nodes: x of the column -> LDS (angle-major); each
+//   k_hpcol    everything else, one workgroup of 512 threads per column:
+//              x of the column -> LDS (angle-major); each
 //              wavefront owns 16 output angles R and every node: it
 //              accumulates the scattering sum_A x[s, A] G^T[A, R] on the
 //              matrix cores (scattering_matrix.py:142-237), then adds mass
@@ -169,7 +169,7 @@ void k_hp_flux(DevMesh m, const HpCell *__restrict__ cells, const int4 *__restri
     if (blk < 0 || ci >= ncells) return;
     // the cell's scalars are uniform over the wavefront
     const HpCell cl = cells[ci];
-    const int nl = cl.w & 255, N = (cl.w >> 8) & 15, nt = (cl.w >> 12) & 15;
+    const int nl = cl.w & 255, nt = (cl.w >> 12) & 15, nx = (cl.w >> 8) & 15, ny = (cl.w >> 24) & 15;
     const int bd = restrict_ ? (cl.w >> 16) & 15 : 0, lf = (cl.w >> 20) & 15;
     if (nl == 0) return;
     const v4 zero = v4{0, 0, 0, 0};
@@ -180,7 +180,9 @@ void k_hp_flux(DevMesh m, const HpCell *__restrict__ cells, const int4 *__restri
     // last node, [F] (faces 1, 2, 3)
     A c0[4] = {A(0), A(0), A(0), A(0)}, c1[4] = {A(0), A(0), A(0), A(0)};
     for (int i = 0; i < nl; ++i) {           // ascending faces
-        const HpLink<A> lk = hp_load_link<T, A>(m, links[cl.l0 + i], N, nt, restrict_, l16, lg, x);
+        const int4 rec = links[cl.l0 + i];
+        const int N = (rec.y & 1) ? nx : ny;             // nodes of this face
+        const HpLink<A> lk = hp_load_link<T, A>(m, rec, N, nt, restrict_, l16, lg, x);
         // inn[m1, r] = sum_a tr[m1, a] E^theta[a, r], then
         // sum_m1 E^s[m1, m0] inn[m1, r] onto the face's sums
         v4 inn = zero;
@@ -209,9 +211,9 @@ void k_hp_flux(DevMesh m, const HpCell *__restrict__ cells, const int4 *__restri
             const A add1 = F == 1 ? c1[1] : F == 2 ? c1[2] : F == 3 ? c1[3] : A(0);
             const bool skip0 = ((bd >> f0) & 1) || (((lf >> f0) & 1) && f0 > F);
             const bool skip1 = ((bd >> f1) & 1) || (((lf >> f1) & 1) && f1 > F);
-            const int fixed = F < 2 ? N - 1 : 0;
-            const int ms = (F & 1) ? N * nt : nt;
-            T *yf = y + cl.off + ((F & 1) ? fixed * nt : fixed * N * nt) + l16;
+            const int first_s = F == 0 ? (nx - 1) * ny : F == 1 ? ny - 1 : 0;    // its first node
+            const int ms = (F & 1) ? ny * nt : nt;
+            T *yf = y + cl.off + first_s * nt + l16;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if (Mma::row(0, v) >= N) continue;           // uniform
@@ -289,9 +291,9 @@ struct HpShared {
 // of lane group g holds node p = e % N of line q = g + 4 (l0 + e / N).  Rows
 // past the lines read a valid node; their outputs are not stored.
 template <typename A, int N>
-__device__ inline int hp_node(int t, int i, int l0) {
+__device__ inline int hp_node(int t, int i, int l0, int ny) {
     const int e = 4 * t + HpMma<A>::reg(i), q = HpMma<A>::group(i) + 4 * (l0 + e / N);
-    return (e % N) * N + (q < N ? q : N - 1);
+    return (e % N) * ny + (q < ny ? q : ny - 1);
 }
 
 // What bounds a column: latency in its phases and the LDS pipe in the lines.
@@ -301,19 +303,30 @@ __device__ inline int hp_node(int t, int i, int l0) {
 // together, against one kernel with the contraction's operands in LDS and 30
 // LDS reads per output: hp mesh of 34,279 cells FP64 283 -> 226 us, 9,150
 // cells mixed 87 -> 45 us, 1,024 columns of 7 x 7 nodes FP32 52 -> 35 us.
-template <typename T, typename A, int PREC, int N>
+//
+// RECT: N nodes along x and another number along y, read at run time.  The
+// lines have their compiled length; only the sums along y and the divisions
+// by the node count are left to run time, and every precision takes one line
+// per lane group and item.  A kernel apart: in one with the square columns its
+// scalar registers slow those down by 2 to 5 %.  Against the generic kernels:
+// 8 x 6 nodes, 7 angles per cell, 1,024 columns FP64 100 -> 49 us, mixed 91 ->
+// 35 us; 4 x 5 nodes, 8 angles, 4,096 columns FP64 366 -> 251 us, mixed 329 ->
+// 168 us; 3 x 5 nodes, 4 angles, 256 columns FP64 20 -> 12 us.
+template <typename T, typename A, int PREC, int N, bool RECT>
 __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, uint32_t ops,
                                           int accumulate, HpShared<A> &sh, unsigned char *lds,
                                           const int32_t *hd, const T *__restrict__ x,
                                           T *__restrict__ y) {
-    constexpr int NSP = N * N;
+    const int NY = RECT ? hd[5] : N;
+    const int NSP = N * NY;
     // x-lines: NL per lane group, LI of them in one item (16 output angles x
     // 4 LI lines).  FP64 takes one: with all of them its accumulators leave
     // too few of the 128 registers of 4 wavefronts per SIMD for the lines
     // (252 spilled, against 24), and two or three times the items spread
     // better over the wavefronts; G is then read from L2 once per item.
     constexpr int NL = (N + 3) / 4;
-    constexpr int LI = sizeof(A) == 8 ? 1 : NL, NI = NL / LI;
+    constexpr int LI = sizeof(A) == 8 || RECT ? 1 : NL;
+    const int NI = RECT ? (NY + 3) / 4 : NL / LI;
     constexpr int MT = (N * LI + 3) / 4;         // node tiles
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -365,7 +378,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     // ---- x of the column and its tables.  The first batch of x is loaded
     // while the angles' tables go to LDS.
     // x values per thread and pass: a column of 96 angles in one
-    constexpr int XU = (NSP * 96 + HP_THREADS - 1) / HP_THREADS < 16 ? (NSP * 96 + HP_THREADS - 1) / HP_THREADS : 16;
+    constexpr int XM = (N * N * 96 + HP_THREADS - 1) / HP_THREADS, XU = RECT || XM > 16 ? 16 : XM;
     A vv[XU];
 #pragma unroll
     for (int u = 0; u < XU; ++u) {
@@ -380,11 +393,11 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
         pk[a] = m.ang_pack[ga0 + a];
         fl[a] = h.ang_flag[ga0 + a];
     }
-    const double *wd = h.wd + N * HP_WD;
-    for (int t = tid; t < HP_NM + NSP; t += HP_THREADS) sh.wd[t] = A(wd[t]);
+    const double *wd = h.wd + NY * HP_WD;
+    for (int t = tid; t < HP_NM + NY * NY; t += HP_THREADS) sh.wd[t] = A(wd[t]);
     if (tid < NSP) {
-        const int i = tid / N, j = tid - i * N;
-        const double w2 = wd[i] * wd[j];
+        const int i = tid / NY, j = tid - i * NY;
+        const double w2 = h.wd[N * HP_WD + i] * wd[j];
         sh.nf[2 * tid] = A(w2 * m.kappa[sp0 + tid]);
         sh.nf[2 * tid + 1] = A(dx * dy * m.sigma[sp0 + tid] * w2);
     }
@@ -404,12 +417,15 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
             const int t = t0 + u * HP_THREADS;
             if (t >= ncd) break;
             A v = vv[u];
-            const int ta = t / NSP, w = pk[ta];
+            const int ta = RECT ? hp_div(t, 1.0f / float(NSP)) : t / (N * N), w = pk[ta];
             const int nt = (w >> 20) & 31, ao = ta - (w >> 25);
             const int lt = t - NSP * ao;
             const int s = hp_div(lt, 1.0f / float(nt)), a = lt - s * nt;
             const int bd = restrict_ ? (fl[ta] & 15) : 0;
-            if (bd && hp_on_bdry(bd, s / N, s % N, N, N)) v = A(0);
+            if (bd) {
+                const int i = RECT ? hp_div(s, 1.0f / float(NY)) : s / N;
+                if (hp_on_bdry(bd, i, s - i * NY, N, NY)) v = A(0);
+            }
             xs[(ao + a) * S + s] = v;
             if constexpr (PREC == RTX_PREC_MIXED) xb[s * XSB + ao + a] = hp_bf16(float(v));
         }
@@ -427,7 +443,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     // ---- 16 output angles per wavefront, every node
     typedef typename HpMma<A>::v4 acc4;
     typedef const A __attribute__((address_space(4))) *CPtr;
-    // the derivative matrix in scalar registers
+    // the derivative matrix along x in scalar registers
     const CPtr wdc = (CPtr)(uintptr_t)((sizeof(A) == 8 ? (const void *)(h.wd + N * HP_WD)
                                                        : (const void *)(h.wd_f + N * HP_WD)));
     const int NRT = (na + 15) / 16;
@@ -442,7 +458,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
             int arow[MT], li = l16;
             asm volatile("" : "+v"(li));
 #pragma unroll
-            for (int t = 0; t < MT; ++t) arow[t] = hp_node<A, N>(t, li, lb);
+            for (int t = 0; t < MT; ++t) arow[t] = hp_node<A, N>(t, li, lb, NY);
             for (int kb = 0; kb < na; kb += 16) {
                 const Group cur = gq[0];
 #pragma unroll
@@ -494,39 +510,52 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
             // opaque: addresses and factors of the line are computed here, not
             // hoisted out of the items and lines to be held (and spilled)
             asm volatile("" : "+v"(q));
-            if (q >= N) continue;
+            if (q >= NY) continue;
             // faces of the line's nodes (bit F: face F); the end nodes also
             // lie on face 2 (p = 0) or 0 (p = N - 1)
-            const int qf = (q == N - 1 ? 2 : 0) | (q == 0 ? 8 : 0);
+            const int qf = (q == NY - 1 ? 2 : 0) | (q == 0 ? 8 : 0);
             auto faces = [&](int p) { return qf | (p == 0 ? 4 : 0) | (p == N - 1 ? 1 : 0); };
             // the inflow-face sums that k_hp_flux left in y, one node ahead
             auto face_sum = [&](int p) {
                 A v = A(0);
-                if (faces(p) & lf) v = A(yb[yo + (p * N + q) * nt]);
+                if (faces(p) & lf) v = A(yb[yo + (p * NY + q) * nt]);
                 return v;
             };
             A fs = face_sum(0);
             A lx[N];
 #pragma unroll
-            for (int i = 0; i < N; ++i) lx[i] = xr[i * N + q];
-            const A *wy = sh.wd + HP_NM + q * N;
+            for (int i = 0; i < N; ++i) lx[i] = xr[i * NY + q];
+            const A *wy = sh.wd + HP_NM + q * NY;
             const A wq = sh.wd[q];
             // y-faces' outflow factor of this line, times w_p below
-            const A oy = q == N - 1 ? oy1 : (q == 0 ? oy0 : A(0));
+            const A oy = q == NY - 1 ? oy1 : (q == 0 ? oy0 : A(0));
             // one output's reads at a time, and none kept for the next line:
             // hoisted, they spill
             asm volatile("" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int p = 0; p < N; ++p) {
-                const int s = p * N + q;
-                const A *ly = xr + p * N;
+                const int s = p * NY + q;
+                const A *ly = xr + p * NY;
                 const A fn = p + 1 < N ? face_sum(p + 1) : A(0);
                 A sx = A(0), sy = A(0);
 #pragma unroll
                 for (int i = 0; i < N; ++i) {
                     sx += wdc[HP_NM + p * N + i] * lx[i];
-                    sy += wy[i] * ly[i];
+                    if constexpr (!RECT) sy += wy[i] * ly[i];
+                }
+                if constexpr (RECT) {
+                    // four at a time; past the last node that node again
+                    // with a zero factor
+#pragma unroll
+                    for (int jb = 0; jb < HP_NM; jb += 4)
+                        if (jb < NY) {                    // uniform
+#pragma unroll
+                            for (int j = jb; j < jb + 4; ++j) {
+                                const int jc = j < NY ? j : NY - 1;
+                                sy += keep_if(wy[jc], j < NY) * ly[jc];
+                            }
+                        }
                 }
                 const A wp = wdc[p], xv = lx[p];
                 A val = vol * sh.nf[2 * s] * xv - (cx * wq * sx + cy * wp * sy);
@@ -561,7 +590,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     }
 }
 
-template <typename T, typename A, int PREC>
+template <typename T, typename A, int PREC, bool RECT>
 __global__ __launch_bounds__(HP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
              const int32_t *__restrict__ hdr, int ncols, const T *__restrict__ x,
@@ -571,11 +600,11 @@ void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
     const int ci = hp_xcd(ncols);
     if (ci < 0) return;
     const int32_t *hd = hdr + size_t(ci) * HP_HDR;
-    // compiled per node count (square columns; the host admits only those)
+    // compiled per node count along x
     switch (hd[2]) {
-#define HP_CASE(NN)                                                                    \
-    case NN:                                                                           \
-        hp_column<T, A, PREC, NN>(m, h, ops, accumulate, sh, hp_lds, hd, x, y);        \
+#define HP_CASE(NN)                                                                   \
+    case NN:                                                                          \
+        hp_column<T, A, PREC, NN, RECT>(m, h, ops, accumulate, sh, hp_lds, hd, x, y); \
         break;
         HP_CASE(3) HP_CASE(4) HP_CASE(5) HP_CASE(6) HP_CASE(7) HP_CASE(8) HP_CASE(9) HP_CASE(10)
 #undef HP_CASE
@@ -607,7 +636,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     // a column whose workgroup (dynamic + static LDS) fits half of a CU's
     // 160 KB runs two workgroups per CU (class 0), the others one (class 1)
     const size_t half = 80 * 1024 > HP_STATIC_BYTES ? 80 * 1024 - HP_STATIC_BYTES : 0;
-    std::vector<int32_t> hdr[3][HP_NCLS], over, links;
+    std::vector<int32_t> hdr[3][HP_NCLS], rect[3][HP_NCLS], over, links;
     std::vector<HpCell> cells;
     p->hp_ncols = 0;
     for (int c = 0; c < nc; ++c) {
@@ -624,11 +653,12 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
                 ang_dth[a] = d->cell_geom[2 * k + 1] - d->cell_geom[2 * k];
             }
         }
-        const int32_t h[HP_HDR] = {k0, k1 - k0, d->col_nx[c], na, d->cell_dof_off[k0], 0, 0,
+        const int32_t h[HP_HDR] = {k0, k1 - k0, d->col_nx[c], na, d->cell_dof_off[k0],
+                                   d->col_ny[c], 0,
                                    d->col_ang_start[c], 0, 0, 0, 0, 0, d->col_sp_off[c], c, 0};
-        // square columns of HP_NMIN..RTX_NMAX nodes (the compiled node counts)
-        bool ok = (k1 - k0) <= HP_MAX_CELLS && d->col_nx[c] == d->col_ny[c] &&
-                  d->col_nx[c] >= HP_NMIN && na <= 4096 && k1 > k0;
+        // HP_NMIN..RTX_NMAX nodes per direction (the compiled node counts)
+        bool ok = (k1 - k0) <= HP_MAX_CELLS && std::min(d->col_nx[c], d->col_ny[c]) >= HP_NMIN &&
+                  na <= 4096 && k1 > k0;
         for (int k = k0; k < k1; ++k) ok = ok && d->link_start[k + 1] - d->link_start[k] < 256;
         size_t need[3];
         for (int pr = 0; pr < 3; ++pr) {
@@ -674,12 +704,14 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
                     lf |= 1 << F;
                     ++nl;
                 }
-            cl.w = nl | d->col_nx[c] << 8 | d->cell_nth[k] << 12 | (d->cell_bdry[k] & 15) << 16 | lf << 20;
+            cl.w = nl | d->col_nx[c] << 8 | d->cell_nth[k] << 12 | (d->cell_bdry[k] & 15) << 16 |
+                   lf << 20 | d->col_ny[c] << 24;
             cells.push_back(cl);
         }
         for (int pr = 0; pr < 3; ++pr) {
             const int cls = need[pr] <= half ? 0 : 1;
-            hdr[pr][cls].insert(hdr[pr][cls].end(), h, h + HP_HDR);
+            auto &list = d->col_nx[c] == d->col_ny[c] ? hdr[pr][cls] : rect[pr][cls];
+            list.insert(list.end(), h, h + HP_HDR);
             HpClass &hc = p->hp_cls[pr][cls];
             hc.bytes = std::max(hc.bytes, need[pr]);
         }
@@ -700,8 +732,13 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         }
     const std::vector<float> wd_f(wd.begin(), wd.end());
     size_t total = ang_flag.size() + links.size() + gcells.size() + gitems.size() + wd_f.size() + 64;
-    for (auto &hp : hdr)
-        for (auto &l : hp) total += l.size();
+    for (int pr = 0; pr < 3; ++pr)
+        for (int k = 0; k < HP_NCLS; ++k) {
+            auto &l = hdr[pr][k];
+            p->hp_cls[pr][k].n_square = int(l.size() / HP_HDR);
+            l.insert(l.end(), rect[pr][k].begin(), rect[pr][k].end());
+            total += l.size();
+        }
     RTX_HIP(hipMalloc(&p->hp_alloc, total * sizeof(int32_t)));
     RTX_HIP(hipMalloc(&p->hp_es, (wd.size() + ang_dth.size()) * sizeof(double) +
                                     cells.size() * sizeof(HpCell) + 64));
@@ -758,14 +795,21 @@ static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, 
             accumulate, (const T *)dx, (T *)dy);
         RTX_HIP(hipGetLastError());
     }
-    auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
-        const int per = (hc.n + HP_XCD - 1) / HP_XCD;
-        RTX_HIP(hipFuncSetAttribute((const void *)k_hpcol<T, A, PREC>,
+    // a class's square columns, then the others
+    auto launch_kind = [&](auto kern, const HpClass &hc, int c0, int n, hipStream_t s) -> int {
+        if (n == 0) return RTX_OK;
+        const int per = (n + HP_XCD - 1) / HP_XCD;
+        RTX_HIP(hipFuncSetAttribute((const void *)kern,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(hc.bytes)));
-        k_hpcol<T, A, PREC><<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(
-            p->m, p->hp, ops, accumulate, hc.hdr, hc.n, (const T *)dx, (T *)dy);
+        kern<<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(
+            p->m, p->hp, ops, accumulate, hc.hdr + size_t(c0) * HP_HDR, n, (const T *)dx, (T *)dy);
         RTX_HIP(hipGetLastError());
         return RTX_OK;
+    };
+    auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
+        const int rc = launch_kind(k_hpcol<T, A, PREC, false>, hc, 0, hc.n_square, s);
+        return rc ? rc : launch_kind(k_hpcol<T, A, PREC, true>, hc, hc.n_square,
+                                     hc.n - hc.n_square, s);
     };
     const HpClass *hc = p->hp_cls[PREC];
     if (hc[0].n == 0 || hc[1].n == 0 || !p->hp_side) {

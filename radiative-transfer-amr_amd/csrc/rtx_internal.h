@@ -111,8 +111,9 @@ size_t fused_bytes(int64_t col_dofs, int64_t nang, int64_t part_dofs, int64_t pa
 constexpr int HP_MAX_CELLS = 64;    // cells per column on this path
 constexpr int HP_NCLS = 2;          // LDS classes (one launch each)
 // A cell of the face-coupling kernel: its inflow faces' factors (dy or dx)
-// dth / 4, first DOF, first link record, and links | N << 8 | angles << 12 |
-// masked faces << 16 | faces that carry links << 20.
+// dth / 4, first DOF, first link record, and links | nodes along x << 8 |
+// angles << 12 | masked faces << 16 | faces that carry links << 20 | nodes
+// along y << 24.
 struct HpCell {
     double fx, fy;
     int32_t off, l0, w, pad = 0;
@@ -132,13 +133,13 @@ struct HpTables {
     const double *wd = nullptr;
     const float *wd_f = nullptr;
 };
-// per column of a class a header of HP_HDR ints (first cell, cells, nodes per
-// direction, angles, first DOF, -, -, first angle, .., [13] first spatial
-// node, [14] column), so the kernel reads a column's scalars in one step
+// per column of a class a header of HP_HDR ints (first cell, cells, nodes
+// along x, angles, first DOF, nodes along y, -, first angle, .., [13] first
+// spatial node, [14] column), so the kernel reads a column's scalars in one step
 constexpr int HP_HDR = 16;
 struct HpClass {
-    int n = 0;                      // columns
-    const int32_t *hdr = nullptr;   // their headers (key order)
+    int n = 0, n_square = 0;        // columns, those with as many nodes along x as along y
+    const int32_t *hdr = nullptr;   // their headers (the square ones first, each kind in key order)
     size_t bytes = 0;               // dynamic LDS per workgroup
 };
 int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d);

@@ -456,14 +456,14 @@ def test_copy_f64_measurement_helper(cuda):
     assert lib.rtx_copy_f64(C.c_void_p(src.data_ptr()), C.c_void_p(dst.data_ptr()), -1, None) != 0
 
 
-def column_edge_mesh(n, nt, nref_ang):
-    """2 x 2 columns of n x n nodes with 2^nref_ang cells of nt angles (for
+def column_edge_mesh(n, nt, nref_ang, ny=None):
+    """2 x 2 columns of n x n (or n x ny) nodes with 2^nref_ang cells of nt angles (for
     nref_ang < 2 a cell spans several quadrants and takes inflow through all
     four faces), one column and one cell an order higher where the order
     limit allows, so that faces of unlike orders meet."""
-    m = problems.uniform_mesh([1.0, 1.0], [n, n, nt], nref_ang, 1)
+    m = problems.uniform_mesh([1.0, 1.0], [n, ny or n, nt], nref_ang, 1)
     keys = sorted(m.cols)
-    if n < 10:
+    if max(n, ny or n) < 10:
         m.ref_col(keys[0], "spt", "p")
     if nt < 10:
         m.ref_cell(keys[-1], sorted(m.cols[keys[-1]].cells)[0], "p")
@@ -483,17 +483,32 @@ def test_column_kernel_orders_and_angle_counts(cuda, n, nt, nref_ang):
     interpolations at most double it; four times that leaves room for terms
     that cancel: 120 eps = 1.4e-14 in FP64 (TOL64 is 1e-12) and 7e-6 in FP32.
     Mixed rounds the scattering operands to BF16 (TOLMIX)."""
+    check_column_kernels(column_edge_mesh(n, nt, nref_ang), n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny,nt,nref_ang", [(3, 4, 3, 2), (4, 3, 5, 1), (5, 9, 7, 4),
+                                               (9, 5, 10, 3), (10, 3, 4, 2), (3, 10, 10, 4),
+                                               (6, 7, 2, 3), (7, 8, 5, 0), (8, 5, 9, 4)])
+def test_column_kernel_unlike_orders(cuda, nx, ny, nt, nref_ang):
+    """Columns with other orders along y than along x, on both sides of every
+    line count (4, 8): as above, with the same bounds, and no column left to
+    the generic kernels."""
+    op = check_column_kernels(column_edge_mesh(nx, nt, nref_ang, ny), nx + ny)
+    assert op.plan_info()["column_kernel_cols"] == 4
+
+
+def check_column_kernels(mesh, seed):
     import torch
     from rtx.operator import (TransportOperator, OP_MASS, OP_SCAT, OP_ICONV, OP_BCONV, OP_SYSTEM,
                               OP_RESTRICT, OP_ACCUM, PREC_F64, PREC_F32, PREC_MIXED)
-    mesh = column_edge_mesh(n, nt, nref_ang)
     wl = problems.two_scatterers()
-    print("column", n, nt, nref_ang, "ndof", mesh.get_ndof(), flush=True)
+    print("column kernels, ndof", mesh.get_ndof(), flush=True)
     V = asm.assemble(mesh, wl.kappa, wl.sigma, wl.Phi)
     A = (V["BC"] - V["IC"] + V["M"] + V["S"]).tocsr()
     op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
     op.set_path(3)
-    rng = np.random.default_rng(n)
+    rng = np.random.default_rng(seed)
     x, y0 = rng.uniform(-1, 1, op.ndof), rng.uniform(-1, 1, op.ndof)
     mask = asm.intr_mask(mesh)
     for prec, dt, tol in [(PREC_F64, torch.float64, TOL64), (PREC_F32, torch.float32, 7e-6),
@@ -511,3 +526,4 @@ def test_column_kernel_orders_and_angle_counts(cuda, n, nt, nref_ang):
             assert _rel(yd.cpu().double().numpy(), ref) < tol, (name, prec)
     y = op.apply(_dev(x), ops=OP_SCAT).cpu().numpy()
     assert _rel(y, V["S"] @ x) < TOL64
+    return op
