@@ -9,7 +9,8 @@
 //              neighbour's angles, then with E^s over its face nodes, both on
 //              the matrix cores with operands read from memory; the links of
 //              a face add up in the accumulators.  The sums of the cell's
-//              inflow faces are stored at their DOFs of y.
+//              inflow faces are stored at their DOFs of y.  Cells whose
+//              neighbours have the same nodes and angles are left out.
 //   k_hpcol    everything else, one workgroup of 512 threads per column:
 //              x of the column -> LDS (angle-major); each
 //              wavefront owns 16 output angles R and every node: it
@@ -18,7 +19,8 @@
 //              (mass_matrix.py:140-173), interior convection
 //              (interior_convection_matrix.py:161-243), the outflow faces
 //              (boundary_convection_matrix.py:284-346) and the sums that
-//              k_hp_flux left in y, and stores y.
+//              k_hp_flux left in y, or, where the neighbours are alike, their
+//              values of x times the (then diagonal) coupling; stores y.
 //
 // The two share no workspace: y itself carries the face sums from one to the
 // other, so concurrent applies on several streams stay independent.
@@ -39,6 +41,7 @@
 // (v_mfma_f32_16x16x4f32) or mixed (FP32 transport terms, BF16 scattering
 // operands on v_mfma_f32_16x16x16bf16_1k with FP32 accumulation).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "rtx_internal.h"
@@ -242,16 +245,17 @@ __host__ __device__ inline int hp_stride(int na, int kstep, int c, int M) {
 }
 
 struct HpLayout {           // dynamic LDS of one column, in bytes from the base
-    int xs, xb, ct, sn, wr, dth, pk, fl, total;
+    int xs, xb, ct, sn, wr, dth, pk, fl, src, total;
     int S, NA, XSB;         // angle-major row (node) stride, padded angle rows, BF16 stride
 };
 
 // Angle-major copy: NA rows (the column's angles, padded to the K step with
 // zero rows) of S = nsp rounded up to odd entries, so that lanes on
 // consecutive angles or nodes read distinct banks; mixed adds the node-major
-// BF16 copy.  Then four values and two words per angle.  A: LDS element type.
+// BF16 copy.  Then four values and two words per angle, and two more where
+// alike neighbours are read directly.  A: LDS element type.
 template <typename A, int PREC>
-__host__ __device__ inline HpLayout hp_layout(int nsp, int na) {
+__host__ __device__ inline HpLayout hp_layout(int nsp, int na, bool alike) {
     HpLayout L;
     const int ea = int(sizeof(A));
     const int kstep = (PREC == RTX_PREC_MIXED) ? 16 : 4;
@@ -277,6 +281,8 @@ __host__ __device__ inline HpLayout hp_layout(int nsp, int na) {
     o += na * 4;
     L.fl = o;
     o += na * 4;
+    L.src = (o + 7) & ~7;
+    o = L.src + (alike ? na * 8 : 0);
     L.total = (o + 15) & ~15;
     return L;
 }
@@ -302,7 +308,8 @@ __device__ inline int hp_node(int t, int i, int l0, int ny) {
 // (lines), those of the second round 15,100.  Times of the two kernels
 // together, against one kernel with the contraction's operands in LDS and 30
 // LDS reads per output: hp mesh of 34,279 cells FP64 283 -> 226 us, 9,150
-// cells mixed 87 -> 45 us, 1,024 columns of 7 x 7 nodes FP32 52 -> 35 us.
+// cells mixed 87 -> 45 us, 1,024 columns of 7 x 7 nodes FP32 52 -> 35 us (29
+// with alike neighbours read directly).
 //
 // RECT: N nodes along x and another number along y, read at run time.  The
 // lines have their compiled length; only the sums along y and the divisions
@@ -311,8 +318,9 @@ __device__ inline int hp_node(int t, int i, int l0, int ny) {
 // scalar registers slow those down by 2 to 5 %.  Against the generic kernels:
 // 8 x 6 nodes, 7 angles per cell, 1,024 columns FP64 100 -> 49 us, mixed 91 ->
 // 35 us; 4 x 5 nodes, 8 angles, 4,096 columns FP64 366 -> 251 us, mixed 329 ->
-// 168 us; 3 x 5 nodes, 4 angles, 256 columns FP64 20 -> 12 us.
-template <typename T, typename A, int PREC, int N, bool RECT>
+// 168 us; 3 x 5 nodes, 4 angles, 256 columns FP64 20 -> 12 us (and with alike
+// neighbours read directly 42, 30, 229, 140 and 9 us).
+template <typename T, typename A, int PREC, int N, bool RECT, bool ALIKE>
 __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, uint32_t ops,
                                           int accumulate, HpShared<A> &sh, unsigned char *lds,
                                           const int32_t *hd, const T *__restrict__ x,
@@ -337,7 +345,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     const int ncd = NSP * na;
     const double dx = m.col_geom[4 * c + 2] - m.col_geom[4 * c + 0];
     const double dy = m.col_geom[4 * c + 3] - m.col_geom[4 * c + 1];
-    const HpLayout Lo = hp_layout<A, PREC>(NSP, na);
+    const HpLayout Lo = hp_layout<A, PREC>(NSP, na, ALIKE);
     const int S = Lo.S, XSB = Lo.XSB;
     A *xs = reinterpret_cast<A *>(lds + Lo.xs);
     uint16_t *xb = reinterpret_cast<uint16_t *>(lds + Lo.xb);
@@ -347,6 +355,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     A *dt = reinterpret_cast<A *>(lds + Lo.dth);
     int *pk = reinterpret_cast<int *>(lds + Lo.pk);
     int *fl = reinterpret_cast<int *>(lds + Lo.fl);
+    int2 *sr = reinterpret_cast<int2 *>(lds + Lo.src);
 
     // ---- the first G rows of this wavefront's first 16 output angles, in
     // flight through the staging phases.  PD load groups of four K steps (one
@@ -392,6 +401,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
         dt[a] = A(h.ang_dth[ga0 + a]);
         pk[a] = m.ang_pack[ga0 + a];
         fl[a] = h.ang_flag[ga0 + a];
+        if constexpr (ALIKE) sr[a] = h.ang_src[ga0 + a];
     }
     const double *wd = h.wd + NY * HP_WD;
     for (int t = tid; t < HP_NM + NY * NY; t += HP_THREADS) sh.wd[t] = A(wd[t]);
@@ -501,6 +511,15 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
         const A ox0 = ob && (quad == 1 || quad == 2) ? -fx * w_r * cR : A(0);
         const A oy1 = ob && quad < 2 ? fy * w_r * sR : A(0);
         const A oy0 = ob && quad >= 2 ? -fy * w_r * sR : A(0);
+        // ALIKE: inflow from alike neighbours: the outflow factors of the
+        // opposite faces, and the neighbours' first face nodes (-1: none)
+        int2 src = make_int2(-1, -1);
+        if constexpr (ALIKE)
+            if (bconv) src = sr[R];
+        const bool xlow = quad == 0 || quad == 3;   // inflow at p = 0
+        const A ix = -(ox1 + ox0), iy = -(oy1 + oy0);
+        // their masked end nodes: x first, x last, y first, y last
+        const int mk = restrict_ ? f >> 12 : 0;
         T *yb = y + cdof;
         const int yo = (w & 0xfffff) + (w >> 25);                  // + s nt: node s
         const A *xr = xs + R * S;                                  // angle row R of the copy
@@ -515,10 +534,14 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
             // lie on face 2 (p = 0) or 0 (p = N - 1)
             const int qf = (q == NY - 1 ? 2 : 0) | (q == 0 ? 8 : 0);
             auto faces = [&](int p) { return qf | (p == 0 ? 4 : 0) | (p == N - 1 ? 1 : 0); };
-            // the inflow-face sums that k_hp_flux left in y, one node ahead
+            // the inflow-face sums that k_hp_flux left in y, or the value of
+            // the alike y-neighbour; one node ahead
+            const bool yin = src.y >= 0 && q == (quad < 2 ? 0 : NY - 1);
             auto face_sum = [&](int p) {
                 A v = A(0);
+                const bool dead = (p == 0 && (mk & 4)) || (p == N - 1 && (mk & 8));
                 if (faces(p) & lf) v = A(yb[yo + (p * NY + q) * nt]);
+                if (yin && !dead) v = iy * A(x[uint32_t(src.y + p * NY * nt)]);
                 return v;
             };
             A fs = face_sum(0);
@@ -527,6 +550,10 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
             for (int i = 0; i < N; ++i) lx[i] = xr[i * NY + q];
             const A *wy = sh.wd + HP_NM + q * NY;
             const A wq = sh.wd[q];
+            // and of the alike x-neighbour
+            A xin = A(0);
+            if (src.x >= 0 && !(q == 0 && (mk & 1)) && !(q == NY - 1 && (mk & 2)))
+                xin = wq * ix * A(x[uint32_t(src.x + q * nt)]);
             // y-faces' outflow factor of this line, times w_p below
             const A oy = q == NY - 1 ? oy1 : (q == 0 ? oy0 : A(0));
             // one output's reads at a time, and none kept for the next line:
@@ -561,8 +588,10 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
                 A val = vol * sh.nf[2 * s] * xv - (cx * wq * sx + cy * wp * sy);
                 if (p == N - 1) val += ox1 * wq * xv;
                 if (p == 0) val += ox0 * wq * xv;
+                if (p == 0) val += xlow ? xin : A(0);
+                if (p == N - 1) val += xlow ? A(0) : xin;
                 val += oy * wp * xv;
-                val += fs;
+                val += yin ? wp * fs : fs;
                 fs = fn;
                 if (scat) val -= sh.nf[2 * s + 1] * A(acc[(l * N + p) / 4][(l * N + p) % 4]);
                 const int on = faces(p), o = yo + s * nt;
@@ -590,7 +619,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     }
 }
 
-template <typename T, typename A, int PREC, bool RECT>
+template <typename T, typename A, int PREC, bool RECT, bool ALIKE>
 __global__ __launch_bounds__(HP_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
              const int32_t *__restrict__ hdr, int ncols, const T *__restrict__ x,
@@ -604,7 +633,8 @@ void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
     switch (hd[2]) {
 #define HP_CASE(NN)                                                                   \
     case NN:                                                                          \
-        hp_column<T, A, PREC, NN, RECT>(m, h, ops, accumulate, sh, hp_lds, hd, x, y); \
+        hp_column<T, A, PREC, NN, RECT, ALIKE>(m, h, ops, accumulate, sh, hp_lds, hd, \
+                                               x, y);                                 \
         break;
         HP_CASE(3) HP_CASE(4) HP_CASE(5) HP_CASE(6) HP_CASE(7) HP_CASE(8) HP_CASE(9) HP_CASE(10)
 #undef HP_CASE
@@ -616,20 +646,61 @@ void k_hpcol(DevMesh m, HpTables h, uint32_t ops, int accumulate,
 
 // Bytes of dynamic LDS a column needs (FP64 or FP32 storage, mixed adds the
 // BF16 copy).
-static size_t hp_bytes(int nsp, int na, int prec) {
-    if (prec == RTX_PREC_F64) return size_t(hp_layout<double, RTX_PREC_F64>(nsp, na).total);
-    if (prec == RTX_PREC_F32) return size_t(hp_layout<float, RTX_PREC_F32>(nsp, na).total);
-    return size_t(hp_layout<float, RTX_PREC_MIXED>(nsp, na).total);
+static size_t hp_bytes(int nsp, int na, int prec, bool alike) {
+    if (prec == RTX_PREC_F64) return size_t(hp_layout<double, RTX_PREC_F64>(nsp, na, alike).total);
+    if (prec == RTX_PREC_F32) return size_t(hp_layout<float, RTX_PREC_F32>(nsp, na, alike).total);
+    return size_t(hp_layout<float, RTX_PREC_MIXED>(nsp, na, alike).total);
 }
 
 // Static LDS of k_hpcol (the tables above), for the capacity check.
 constexpr size_t HP_STATIC_BYTES = sizeof(HpShared<double>) + 64;
+
+// Whether cell k's links all join it to cells with the same nodes and angles,
+// through an inflow face each.  E^s and E^theta are then diagonal (weights;
+// weights x direction) up to the rounding of the node positions, and the
+// column kernel reads the neighbours' values directly.  src: the x- and the
+// y-neighbour's first face node (-1: none); masked: its masked end nodes
+// (bits: x first, x last, y first, y last).
+static bool alike_cell(const rtx_mesh_desc *d, int k, int32_t *src, int32_t *masked) {
+    const int c = d->cell_col[k], nx = d->col_nx[c], ny = d->col_ny[c], nt = d->cell_nth[k];
+    const int quad = d->cell_quad[k];
+    src[0] = src[1] = -1;
+    *masked = 0;
+    if (quad < 0) return false;
+    const auto diagonal = [](const double *E, int n, auto diag) {
+        for (int a = 0; a < n; ++a)
+            for (int b = 0; b < n; ++b)
+                if (!(std::fabs(E[a * n + b] - (a == b ? diag(a) : 0.0)) <= 1e-13)) return false;
+        return true;
+    };
+    for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) {
+        const int s = d->link_src[l], F = d->link_face[l], c1 = d->cell_col[s], odd = F & 1;
+        if ((F != ((quad + 2) & 3) && F != ((quad + 3) & 3)) || src[odd] >= 0) return false;
+        if (d->col_nx[c1] != nx || d->col_ny[c1] != ny || d->cell_nth[s] != nt) return false;
+        const int n = odd ? nx : ny;
+        const double *trig = d->ang_trig + 3 * (d->col_ang_start[c] + d->cell_ang_off[k]);
+        if (!diagonal(d->Es_pool + d->link_Es_off[l], n,
+                      [&](int a) { return d->lgl_w[n * HP_NM + a]; }) ||
+            !diagonal(d->Eth_pool + d->link_Eth_off[l], nt, [&](int a) {
+                return trig[3 * a + 2] * trig[3 * a + odd] * (F < 2 ? 1.0 : -1.0);
+            }))
+            return false;
+        // the neighbour's opposite face: its first node and masked ends (the
+        // masked faces next to it; never the face itself, which has links)
+        const int bd = d->cell_bdry[s] & 15, node = F == 2 ? (nx - 1) * ny : F == 3 ? ny - 1 : 0;
+        if (bd >> ((F + 2) & 3) & 1) return false;
+        src[odd] = d->cell_dof_off[s] + node * nt;
+        *masked |= ((bd >> (odd ? 2 : 3) & 1) | (bd >> (odd ? 0 : 1) & 1) << 1) << 2 * odd;
+    }
+    return true;
+}
 
 int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     const int nc = d->ncol;
     p->hp_ok = false;
     std::vector<int32_t> ang_flag(std::max<int64_t>(d->nang, 1), 0);
     std::vector<double> ang_dth(std::max<int64_t>(d->nang, 1), 0.0);
+    std::vector<int32_t> ang_src(2 * std::max<int64_t>(d->nang, 1), -1);
     int max_lds = 0;
     RTX_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, p->device));
     const size_t cap = size_t(max_lds) > HP_STATIC_BYTES ? size_t(max_lds) - HP_STATIC_BYTES : 0;
@@ -639,6 +710,20 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     std::vector<int32_t> hdr[3][HP_NCLS], rect[3][HP_NCLS], over, links;
     std::vector<HpCell> cells;
     p->hp_ncols = 0;
+    // Neighbours are read directly where at least a quarter of the cells have
+    // alike ones.  The kernel that does so holds more registers: with no such
+    // cell it takes 5 % longer (an hp mesh in FP64, 227 -> 239 us), with
+    // nothing else it saves the face kernel (1,024 columns of 7 x 7 nodes in
+    // FP32 35 -> 29 us, 256 columns of 3 x 5 nodes in FP64 12.4 -> 8.7 us).
+    std::vector<int32_t> cell_src(size_t(2) * d->ncell), cell_mask(d->ncell);
+    std::vector<char> direct(d->ncell);
+    int64_t ndirect = 0;
+    for (int k = 0; k < d->ncell; ++k) {
+        direct[k] = alike_cell(d, k, &cell_src[size_t(2) * k], &cell_mask[k]);
+        ndirect += direct[k];
+    }
+    p->hp_alike = 4 * ndirect >= d->ncell;
+    if (!p->hp_alike) std::fill(direct.begin(), direct.end(), char(0));
     for (int c = 0; c < nc; ++c) {
         const int k0 = d->col_cell_start[c], k1 = d->col_cell_start[c + 1];
         const int nsp = d->col_nx[c] * d->col_ny[c], na = d->col_nang[c];
@@ -647,10 +732,18 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         int64_t a = d->col_ang_start[c];
         for (int k = k0; k < k1; ++k) {
             int lf = 0;
-            for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) lf |= 1 << d->link_face[l];
+            if (!direct[k])
+                for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l)
+                    lf |= 1 << d->link_face[l];
             for (int r = 0; r < d->cell_nth[k]; ++r, ++a) {
                 ang_flag[a] = (d->cell_bdry[k] & 15) | (d->cell_quad[k] + 1) << 4 | lf << 8;
                 ang_dth[a] = d->cell_geom[2 * k + 1] - d->cell_geom[2 * k];
+                if (!direct[k]) continue;
+                ang_flag[a] |= cell_mask[k] << 12;
+                for (int e = 0; e < 2; ++e) {
+                    const int32_t src = cell_src[size_t(2) * k + e];
+                    ang_src[2 * a + e] = src < 0 ? -1 : src + r;
+                }
             }
         }
         const int32_t h[HP_HDR] = {k0, k1 - k0, d->col_nx[c], na, d->cell_dof_off[k0],
@@ -662,7 +755,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         for (int k = k0; k < k1; ++k) ok = ok && d->link_start[k + 1] - d->link_start[k] < 256;
         size_t need[3];
         for (int pr = 0; pr < 3; ++pr) {
-            need[pr] = hp_bytes(nsp, na, pr);
+            need[pr] = hp_bytes(nsp, na, pr, p->hp_alike);
             ok = ok && need[pr] <= cap;
         }
         if (!ok) {
@@ -673,6 +766,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         const double dx = d->col_geom[4 * c + 2] - d->col_geom[4 * c];
         const double dy = d->col_geom[4 * c + 3] - d->col_geom[4 * c + 1];
         for (int k = k0; k < k1; ++k) {
+            if (direct[k]) continue;
             const double dth = d->cell_geom[2 * k + 1] - d->cell_geom[2 * k];
             HpCell cl;
             cl.fx = dy * 0.25 * dth;
@@ -731,7 +825,8 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
                     d->lgl_w[n * HP_NM + i] * d->lgl_D[(size_t(n) * HP_NM + pp) * HP_NM + i];
         }
     const std::vector<float> wd_f(wd.begin(), wd.end());
-    size_t total = ang_flag.size() + links.size() + gcells.size() + gitems.size() + wd_f.size() + 64;
+    size_t total = ang_flag.size() + ang_src.size() + links.size() + gcells.size() + gitems.size() +
+                   wd_f.size() + 64;
     for (int pr = 0; pr < 3; ++pr)
         for (int k = 0; k < HP_NCLS; ++k) {
             auto &l = hdr[pr][k];
@@ -754,6 +849,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         return static_cast<const int32_t *>(put(v.data(), v.size() * sizeof(int32_t)));
     };
     p->hp.ang_flag = put_i(ang_flag);
+    p->hp.ang_src = reinterpret_cast<const int2 *>(put_i(ang_src));
     p->hp.links = reinterpret_cast<const int4 *>(put_i(links));
     for (int pr = 0; pr < 3; ++pr)
         for (int k = 0; k < HP_NCLS; ++k) {
@@ -788,7 +884,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
 template <typename T, typename A, int PREC>
 static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, hipStream_t st,
                      int accumulate) {
-    if (ops & RTX_OP_BCONV) {
+    if ((ops & RTX_OP_BCONV) && p->hp_n_cells > 0) {
         const int nblk = (p->hp_n_cells + HF_WAVES - 1) / HF_WAVES;
         k_hp_flux<T, A><<<(nblk + HP_XCD - 1) / HP_XCD * HP_XCD, 64 * HF_WAVES, 0, st>>>(
             p->m, p->hp.cells, p->hp.links, p->hp_n_cells, (ops & RTX_OP_RESTRICT) ? 1 : 0,
@@ -807,9 +903,13 @@ static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, 
         return RTX_OK;
     };
     auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
-        const int rc = launch_kind(k_hpcol<T, A, PREC, false>, hc, 0, hc.n_square, s);
-        return rc ? rc : launch_kind(k_hpcol<T, A, PREC, true>, hc, hc.n_square,
-                                     hc.n - hc.n_square, s);
+        const int rc = p->hp_alike
+                           ? launch_kind(k_hpcol<T, A, PREC, false, true>, hc, 0, hc.n_square, s)
+                           : launch_kind(k_hpcol<T, A, PREC, false, false>, hc, 0, hc.n_square, s);
+        if (rc) return rc;
+        const int n = hc.n - hc.n_square;
+        return p->hp_alike ? launch_kind(k_hpcol<T, A, PREC, true, true>, hc, hc.n_square, n, s)
+                           : launch_kind(k_hpcol<T, A, PREC, true, false>, hc, hc.n_square, n, s);
     };
     const HpClass *hc = p->hp_cls[PREC];
     if (hc[0].n == 0 || hc[1].n == 0 || !p->hp_side) {

@@ -125,8 +125,11 @@ struct HpTables {
     // nodes << 18; E^s and E^theta offsets
     const int4 *links = nullptr;
     // per angle (numbered cell by cell): masked faces of its cell | (quadrant
-    // + 1) << 4 | faces that carry links << 8; the cell's width in theta
+    // + 1) << 4 | faces whose sums k_hp_flux leaves in y << 8 | masked end nodes
+    // of alike neighbours << 12; the first face node of the alike x- and
+    // y-neighbour (-1: none); the cell's width in theta
     const int32_t *ang_flag = nullptr;
+    const int2 *ang_src = nullptr;
     const double *ang_dth = nullptr;
     // per node count n: the n LGL weights, then (from RTX_NMAX on) the n x n
     // products w_i l'_p(xi_i), row p
@@ -212,7 +215,8 @@ struct rtx_plan {
     rtx::HpTables hp;
     rtx::HpClass hp_cls[3][rtx::HP_NCLS];   // per precision
     int hp_ncols = 0;
-    int hp_n_cells = 0;                     // cells of those columns
+    int hp_n_cells = 0;                     // cells of those columns for k_hp_flux
+    bool hp_alike = false;                  // alike neighbours are read directly
     std::vector<int32_t> hp_over_cols;
     const int32_t *hp_gen_cells = nullptr, *hp_gen_items = nullptr;
     int hp_n_gen_cells = 0, hp_n_gen_items = 0;
