@@ -661,7 +661,7 @@ constexpr size_t HP_STATIC_BYTES = sizeof(HpShared<double>) + 64;
 // column kernel reads the neighbours' values directly.  src: the x- and the
 // y-neighbour's first face node (-1: none); masked: its masked end nodes
 // (bits: x first, x last, y first, y last).
-static bool alike_cell(const rtx_mesh_desc *d, int k, int32_t *src, int32_t *masked) {
+bool alike_cell(const rtx_mesh_desc *d, int k, int32_t *src, int32_t *masked) {
     const int c = d->cell_col[k], nx = d->col_nx[c], ny = d->col_ny[c], nt = d->cell_nth[k];
     const int quad = d->cell_quad[k];
     src[0] = src[1] = -1;

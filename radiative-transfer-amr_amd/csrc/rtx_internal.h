@@ -145,6 +145,7 @@ struct HpClass {
     const int32_t *hdr = nullptr;   // their headers (the square ones first, each kind in key order)
     size_t bytes = 0;               // dynamic LDS per workgroup
 };
+bool alike_cell(const rtx_mesh_desc *d, int k, int32_t *src, int32_t *masked);
 int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d);
 int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
                  int accumulate);
@@ -191,6 +192,10 @@ struct rtx_plan {
     bool uni_ok = false;
     int32_t uni_n = 0, uni_nth = 0, uni_ncells = 0;
     int uni_H = 0;                // parts per column of the uniform kernel (0: default)
+    // per cell, from alike_cell: the x- and y-neighbour's first face node (-1:
+    // none) and the masked end nodes
+    const int4 *uni_src = nullptr;
+    void *uni_alloc = nullptr;
     // largest own-DOF count and own-trace count of a column part when the
     // fused kernel splits every column into H = 1, 2, 4 cell ranges
     int32_t max_part_dofs[5] = {0, 0, 0, 0, 0}, max_part_trace[5] = {0, 0, 0, 0, 0};

@@ -292,26 +292,22 @@ extern "C" int rtx_plan_create(const rtx_mesh_desc *d, rtx_plan **out) {
             ok = d->col_cell_start[c] == c * NC &&
                  int64_t(d->cell_dof_off[c * NC]) == int64_t(c) * N * N * NTH * NC &&
                  d->col_sp_off[c] == c * N * N && d->col_ang_start[c] == c * NTH * NC;
-        // every link must couple equal shapes (trace of N x NTH values), and a
-        // cell may have at most one link on an x-face (F even) and one on a
-        // y-face (F odd): the kernel adds a corner node's two face fluxes in
-        // one thread, without atomics
-        for (int l = 0; l < nl && ok; ++l) {
-            const int s = d->link_src[l];
-            ok = d->cell_nth[s] == NTH && d->col_nx[d->cell_col[s]] == N;
-        }
-        for (int k = 0; k < nk && ok; ++k) {
-            int par = 0;
-            for (int l = d->link_start[k]; l < d->link_start[k + 1] && ok; ++l) {
-                const int bit = 1 << (d->link_face[l] & 1);
-                ok = (par & bit) == 0;
-                par |= bit;
-            }
-        }
-        p->uni_ok = ok && uniform_shape_compiled(N, NTH, NC);
+        // every cell has alike neighbours, at most one through an x-face and
+        // one through a y-face
+        ok = ok && uniform_shape_compiled(N, NTH, NC);
+        std::vector<int32_t> src(ok ? size_t(4) * nk : 0, 0);
+        for (int k = 0; k < nk && ok; ++k)
+            ok = alike_cell(d, k, &src[size_t(4) * k], &src[size_t(4) * k + 2]);
+        p->uni_ok = ok;
         p->uni_n = N;
         p->uni_nth = NTH;
         p->uni_ncells = NC;
+        if (p->uni_ok) {
+            RTX_HIP(hipMalloc(&p->uni_alloc, src.size() * sizeof(int32_t)));
+            RTX_HIP(hipMemcpy(p->uni_alloc, src.data(), src.size() * sizeof(int32_t),
+                              hipMemcpyHostToDevice));
+            p->uni_src = static_cast<const int4 *>(p->uni_alloc);
+        }
     }
     for (int c = 0; c < nc; ++c) {
         const int k0 = d->col_cell_start[c], k1 = d->col_cell_start[c + 1], ncl = k1 - k0;
@@ -537,6 +533,7 @@ extern "C" void rtx_plan_destroy(rtx_plan *p) {
     if (p->coarse) (void)hipFree(p->coarse);
     if (p->bins) (void)hipFree(p->bins);
     if (p->gen_alloc) (void)hipFree(p->gen_alloc);
+    if (p->uni_alloc) (void)hipFree(p->uni_alloc);
     if (p->hp_alloc) (void)hipFree(p->hp_alloc);
     if (p->hp_es) (void)hipFree(p->hp_es);
     if (p->hp_fork) (void)hipEventDestroy(p->hp_fork);

@@ -3,16 +3,18 @@
 // When every column has nx = ny = N, every cell nth = NTH angular nodes and
 // every column NC cells with one shared angular mesh (one G^T block), the
 // per-column work has compile-time shape: NSP = N^2 spatial nodes,
-// NA = NC NTH angles, NCD = NSP NA DOFs.  The kernel is the same five-phase
-// computation as rtx_fused.hip (same reference formulas), specialised:
-// no searches, constant divisions, batched register prefetch of the column,
-// the part's neighbour traces and the MFMA B operands, and XCD-aware
-// (column, part) blocks: each XCD owns a contiguous run of columns.
+// NA = NC NTH angles, NCD = NSP NA DOFs.  The same terms as rtx_fused.hip
+// (same reference formulas), specialised: no searches, constant divisions,
+// batched register prefetch of the column and the MFMA B operands, and
+// XCD-aware (column, part) blocks: each XCD owns a contiguous run of columns.
 //
 // Two kernels: k_uniform adds the cell-local terms by lines of nodes into an
-// output tile in LDS (1, 2 or 4 parts per column); k_uniform_e computes
-// every term of an output in the scattering MFMA's accumulator layout, with
-// no output tile, so more columns are resident per CU (the FP64 default).
+// output tile in LDS (1, 2 or 4 parts per column) and takes the inflow from
+// the neighbours' values directly; k_uniform_e computes every term of an
+// output in the scattering MFMA's accumulator layout, with no output tile, so
+// more columns are resident per CU (the FP64 default), and stages the
+// neighbours' traces in LDS (read by the output lanes instead, they are
+// scattered loads: 27 -> 30 us for 1,024 columns of 5 x 5 x 80).
 #include <type_traits>
 
 #include "rtx_internal.h"
@@ -56,6 +58,28 @@ constexpr int u_pad(int na, int nth) {
     return v;
 }
 
+// Inflow through a face from the neighbour's node at the same place.  Both
+// columns have the same nodes and angles there, so the coupling matrices
+// E^s and E^theta are diagonal (weights, weights x direction) and the flux at
+// a node is the outflow term's product with the neighbour's value and the
+// opposite direction: no traces to stage, no contraction.  tf: the direction
+// factor of the outflow face opposite.
+template <typename A>
+__device__ inline A u_inflow(A len4, A dth, A w, A wr, A tf, A xn) {
+    return -(len4 * dth * w * wr * tf) * xn;
+}
+
+// Outflow faces quad and quad + 1 of a cell: the x-face (F even), the y-face,
+// and the node rows they lie on.
+struct UFaces {
+    int Fx, Fy;
+    bool yfirst;
+    __device__ explicit UFaces(int quad) : yfirst((quad & 1) != 0) {
+        Fx = yfirst ? ((quad + 1) & 3) : quad;
+        Fy = yfirst ? quad : ((quad + 1) & 3);
+    }
+};
+
 // BF16 copy of the column for the MIXED scattering MFMA: rows padded to
 // whole 16-node tiles, columns to whole 16-angle k-steps, both with zeros;
 // row stride na16 + 4 (a multiple of 4 elements, so one 8-byte read per
@@ -75,11 +99,18 @@ constexpr int u_threads() {
     return ((NC / H) * NTH + 15) / 16 > 4 ? 512 : 256;
 }
 
+// Bound by LDS traffic and latency; what counts is how many columns a CU
+// holds.  The bounds below hold three (FP64) or four workgroups of eight
+// wavefronts, at most 80 or 64 registers, so the neighbours' values are loaded
+// where the scattering's operands are not live.  With the traces and the face
+// contraction in LDS and no bound (columns of 5 x 5 x 80): 4,096 columns mixed
+// 51.7 -> 43.2 us, FP32 64 -> 60 us, FP64 97 -> 89 us; 1,024 columns mixed
+// 16.2 -> 14.7 us.
 template <typename T, typename A, int PREC, int N, int NTH, int NC, int H,
           int UTHREADS = u_threads<NTH, NC, H>()>
-__global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops, int accumulate,
-                                                      const T *__restrict__ x,
-                                                      T *__restrict__ y, int nlink_lds) {
+__global__ __launch_bounds__(UTHREADS, PREC == RTX_PREC_F64 ? 6 : 8)
+void k_uniform(DevMesh m, uint32_t ops, int accumulate, const int4 *__restrict__ src,
+               const T *__restrict__ x, T *__restrict__ y) {
     constexpr int NSP = N * N, NA = NC * NTH, NCD = NSP * NA, CD = NSP * NTH;
     constexpr int OC = NC / H;                 // cells per part
     constexpr int NOWN = OC * CD, NOA = OC * NTH;
@@ -87,19 +118,15 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
     constexpr int NTILE = (NOA + 15) / 16;     // output-angle tiles of the part
     constexpr int NKS = (NA + 3) / 4;          // f64/f32 k-steps
     constexpr int NKB = (NA + 15) / 16;        // bf16 k-steps
-    constexpr int MAXL = 4 * OC;               // links of the part (<= 2 per cell per
-                                               // face pair; 4 leaves room for hp-free meshes)
-    constexpr int TRL = N * NTH;               // trace values per link
     // DOF passes t = t0 + u XS over a column (cell-major, CD DOFs per cell):
-    // when a cell fits the workgroup, a pass covers CPP whole cells and a
-    // thread keeps one in-cell position in every pass, so its (node, angle)
-    // indices are computed once; threads past CPP CD idle (t0 = NCD)
-    constexpr int CPP = CD <= UTHREADS ? UTHREADS / CD : 0;
-    constexpr int XS = CPP ? CPP * CD : UTHREADS;
+    // a pass covers CPP whole cells and a thread keeps one in-cell position
+    // in every pass, so its (node, angle) indices are computed once; threads
+    // past CPP CD idle (t0 = NCD)
+    static_assert(CD <= UTHREADS, "a cell fits the workgroup");
+    constexpr int CPP = UTHREADS / CD;
+    constexpr int XS = CPP * CD;
     constexpr int XU = (NCD + XS - 1) / XS;
-    // the same for trace and flux slots (TRL values per link, TRL <= 81)
-    constexpr int LPP = UTHREADS / TRL;
-    constexpr int TS = LPP * TRL;
+    constexpr int YU = (OC + CPP - 1) / CPP;   // passes over the part's outputs
     // LDS rows per spatial node, angle-contiguous, strides from u_pad
     constexpr int NAP = u_pad(NA, NTH), NOAP = u_pad(NOA, NTH);
     static_assert(NTILE <= UTHREADS / 64, "one output-angle tile per wavefront");
@@ -112,20 +139,14 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
     constexpr int NAPB = u_bf_stride(NA);
     constexpr size_t XB_OFF = u_bf_off(size_t(NSP * NAP + NSP * NOAP) * sizeof(A));
     uint16_t *xb = reinterpret_cast<uint16_t *>(u_lds + XB_OFF);
-    A *tr = XB ? reinterpret_cast<A *>(u_lds + XB_OFF + u_bf_bytes(NSP, NA))
-               : ys + NSP * NOAP;              // links * TRL: neighbour traces
-    A *fl = tr + nlink_lds * TRL;              // links * TRL: face fluxes (phase 3)
     __shared__ A cth[NA], sth[NA], cw[NA];
     __shared__ A kap[NSP], sgw[NSP];
     __shared__ A wx_[N], WD[N * N];
     __shared__ A dth_[NC];
     __shared__ int cbd[NC], cqd[NC];
     __shared__ int nfc[NSP];                   // u_node_faces of each spatial node
-    __shared__ int l_src[MAXL], l_meta[MAXL], l_es[MAXL], l_et[MAXL];
-    // per part cell, its inflow x- / y-face link's flux slots: (first slot
-    // << 4) | (1 + the node row i / column j on that face), 0 without one
-    __shared__ int cfx[OC], cfy[OC];
-                                               // link, -1 without one
+    // per part cell, the neighbours' first face nodes (-1: none) and masked ends
+    __shared__ int4 nbr[OC];
 
     // workgroups go to the XCDs round-robin (b mod 8); XCD j takes the
     // contiguous columns [j cpx, (j + 1) cpx) in order, all parts of a column
@@ -144,8 +165,6 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
     const int cdof = c * NCD;
     const int kk_lo = h * OC;
     const int own0 = kk_lo * CD;
-    const int L0 = m.link_start[k0 + kk_lo];
-    const int nl = m.link_start[k0 + kk_lo + OC] - L0;
     const bool restrict_ = (ops & RTX_OP_RESTRICT) != 0;
     const bool bconv = (ops & RTX_OP_BCONV) != 0;
     const double dx = m.col_geom[4 * c + 2] - m.col_geom[4 * c + 0];
@@ -196,7 +215,8 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
         xv[u] = (t < NCD) ? A(x[cdof + t]) : A(0);
     }
     double r_c = 0, r_s = 0, r_w = 0, r_kap = 0, r_sig = 0, r_wd = 0, r_g = 0;
-    int r_bd = 0, r_q = -1, r_src = 0, r_meta = 0, r_es = 0, r_et = 0;
+    int r_bd = 0, r_q = -1;
+    int4 r_nbr = make_int4(-1, -1, 0, 0);
     if (tid < NA) {
         r_c = m.ang_trig[3 * (ga0 + tid)];
         r_s = m.ang_trig[3 * (ga0 + tid) + 1];
@@ -216,13 +236,7 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
         r_q = m.cell_quad[k];
         r_g = m.cell_geom[2 * k + 1] - m.cell_geom[2 * k];
     }
-    if (bconv && tid < nl) {
-        const int l = L0 + tid;
-        r_src = m.link_meta[4 * l + 0];
-        r_meta = m.link_meta[4 * l + 1];
-        r_es = m.link_Es_off[l];
-        r_et = m.link_Eth_off[l];
-    }
+    if (bconv && tid < OC) r_nbr = src[k0 + kk_lo + tid];
     if (tid < NA) {
         cth[tid] = A(r_c);
         sth[tid] = A(r_s);
@@ -240,25 +254,42 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
         cqd[tid] = r_q;
         dth_[tid] = A(r_g);
     }
-    if (bconv && tid < nl) {
-        l_src[tid] = r_src;
-        l_meta[tid] = r_meta;
-        l_es[tid] = r_es;
-        l_et[tid] = r_et;
-    }
-    if (tid < OC) {
-        cfx[tid] = 0;
-        cfy[tid] = 0;
-    }
+    if (tid < OC) nbr[tid] = r_nbr;
     __syncthreads();
-    if (bconv && tid < nl) {
-        const int kl = (r_meta >> 18) - kk_lo, F = r_meta & 3;
-        const int slots = (tid * TRL) << 4;
-        if (F & 1) cfy[kl] = slots | (1 + (F == 1 ? N - 1 : 0));
-        else cfx[kl] = slots | (1 + (F == 0 ? N - 1 : 0));
-    }
 
-    // ---- phase 1: column input (masked) and the part's neighbour traces
+    // ---- the neighbours' values of this thread's outputs, in flight until the
+    // write-back: after the scattering in FP64 and before it in FP32, where its
+    // operands hold registers (loaded with the column they spill), with the
+    // column in mixed precision
+    const int le = tid % CD, sne = le / NTH, ae = le % NTH, ie = sne / N, je = sne % N;
+    A xi[YU], yi[YU];
+    auto load_inflow = [&]() {
+        int ax[YU], ay[YU];
+#pragma unroll
+        for (int u = 0; u < YU; ++u) {
+            const int kl = tid / CD + u * CPP;
+            ax[u] = ay[u] = -1;
+            if (tid < XS && kl < OC) {
+                const int4 nb = nbr[kl];
+                const UFaces f(cqd[kk_lo + kl]);
+                const int mk = restrict_ ? nb.z : 0;
+                if (ie == (f.Fx == 0 ? 0 : N - 1) && nb.x >= 0 &&
+                    !(je == 0 && (mk & 1)) && !(je == N - 1 && (mk & 2)))
+                    ax[u] = nb.x + je * NTH + ae;
+                if (je == (f.Fy == 1 ? 0 : N - 1) && nb.y >= 0 &&
+                    !(ie == 0 && (mk & 4)) && !(ie == N - 1 && (mk & 8)))
+                    ay[u] = nb.y + ie * N * NTH + ae;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < YU; ++u) {
+            xi[u] = ax[u] >= 0 ? A(x[ax[u]]) : A(0);
+            yi[u] = ay[u] >= 0 ? A(x[ay[u]]) : A(0);
+        }
+    };
+    if constexpr (XB) load_inflow();
+
+    // ---- phase 1: column input (masked)
     {
         const int lt0 = t0 % CD, sn0 = lt0 / NTH, a0 = lt0 % NTH, nf0 = nfc[sn0 < NSP ? sn0 : 0];
 #pragma unroll
@@ -266,22 +297,10 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
             const int t = t0 + u * XS;
             if (t < NCD) {
                 A v = xv[u];
-                int kk, sn, a, nf;
-                if constexpr (CPP > 0) {
-                    kk = t0 / CD + u * CPP;
-                    sn = sn0;
-                    a = a0;
-                    nf = nf0;
-                } else {
-                    const int lt = t % CD;
-                    kk = t / CD;
-                    sn = lt / NTH;
-                    a = lt % NTH;
-                    nf = nfc[sn];
-                }
-                if (cbd[kk] & nf) v = A(0);   // cbd is 0 without RESTRICT
-                xs[sn * NAP + kk * NTH + a] = v;
-                if constexpr (XB) xb[sn * NAPB + kk * NTH + a] = u_bf16(float(v));
+                const int kk = t0 / CD + u * CPP;
+                if (cbd[kk] & nf0) v = A(0);   // cbd is 0 without RESTRICT
+                xs[sn0 * NAP + kk * NTH + a0] = v;
+                if constexpr (XB) xb[sn0 * NAPB + kk * NTH + a0] = u_bf16(float(v));
             }
         }
     }
@@ -294,47 +313,15 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
         for (int e = tid; e < PR; e += UTHREADS)
             xb[(NSP + e / (NKB * 16)) * NAPB + e % (NKB * 16)] = 0;
     }
-    if (bconv) {
-        constexpr int TU = (MAXL * TRL + TS - 1) / TS;
-        const int e0 = tid < TS ? tid : MAXL * TRL;
-        const int le = e0 % TRL, m1 = le / NTH, a = le % NTH;
-        int addr[TU];
-        bool zero[TU];
-        A v[TU];
-#pragma unroll
-        for (int u = 0; u < TU; ++u) {
-            const int li = e0 / TRL + u * LPP;
-            addr[u] = -1;
-            zero[u] = false;
-            if (li < nl) {
-                const int w1 = l_meta[li];
-                const int F = w1 & 3, bd1 = restrict_ ? ((w1 >> 14) & 15) : 0;
-                int i1, j1;
-                if (F == 0) { i1 = 0; j1 = m1; }
-                else if (F == 2) { i1 = N - 1; j1 = m1; }
-                else if (F == 1) { i1 = m1; j1 = 0; }
-                else { i1 = m1; j1 = N - 1; }
-                addr[u] = l_src[li] + (i1 * N + j1) * NTH + a;
-                zero[u] = (bd1 & nfc[i1 * N + j1]) != 0;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < TU; ++u) v[u] = (addr[u] >= 0) ? A(x[addr[u]]) : A(0);
-#pragma unroll
-        for (int u = 0; u < TU; ++u) {
-            const int li = e0 / TRL + u * LPP;
-            if (li < nl) tr[li * TRL + le] = zero[u] ? A(0) : v[u];
-        }
-    }
     if constexpr (MFMA_FIRST) load_b();
     __syncthreads();
 
     // ---- scattering for the part's output angles on MFMA, into registers,
-    // subtracted from the outputs in phase 4.  In FP64 it is issued here,
-    // before phases 2 and 3, so the matrix pipe runs while the cell-local and
-    // face terms go through the vector units (measured faster); in FP32 and
-    // BF16, whose MFMA work is short and whose operand conversion competes
-    // with phase 2, it runs after phase 3 (measured faster).
+    // subtracted from the outputs in phase 3.  In FP64 it is issued here,
+    // before phase 2, so the matrix pipe runs while the cell-local terms go
+    // through the vector units (measured faster); in FP32 and BF16, whose MFMA
+    // work is short and whose operand conversion competes with phase 2, it
+    // runs after it (measured faster).
     typedef typename std::conditional<PREC == RTX_PREC_F64, u_dbl4, u_flt4>::type acc4;
     constexpr bool EARLY = MFMA_FIRST;
     acc4 sacc[MT];
@@ -390,6 +377,7 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
         }
     };
     if (EARLY && scat_w) scatter();
+    if constexpr (EARLY) load_inflow();
 
     // ---- phase 2: cell-local terms on the part's DOFs, by lines of nodes:
     // pass x: one (cell, q, angle) line per thread reads x[0..N-1][q] once
@@ -465,40 +453,8 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
     }
     __syncthreads();
 
-    // ---- phase 3: upwind inflow couplings, one (link, face node, angle) per
-    // thread, into a flux slot of its own; phase 5 adds a DOF's slots (its
-    // cell has at most one x-face and one y-face link, the plan admits no
-    // other mesh here) in a fixed order: bit-reproducible without atomics.
-    // Phase 4 does not read the slots, so no barrier separates them.
-    if (bconv) {
-        const int f0 = tid < TS ? tid : MAXL * TRL;
-        const int le = f0 % TRL, m0 = le / NTH, r = le % NTH;
-        for (int li = f0 / TRL; li < nl; li += LPP) {
-            const int w1 = l_meta[li];
-            const int F = w1 & 3, kk = w1 >> 18;
-            const double *Es = m.Es_pool + l_es[li];
-            const double *Et = m.Eth_pool + l_et[li];
-            A et[NTH], es[N];
-#pragma unroll
-            for (int a = 0; a < NTH; ++a) et[a] = A(Et[a * NTH + r]);
-#pragma unroll
-            for (int a = 0; a < N; ++a) es[a] = A(Es[a * N + m0]);
-            const A *trl = tr + li * TRL;
-            A acc = A(0);
-            // one trace row at a time: keeps the registers of this phase
-            // below those of the MFMA phase
-#pragma unroll 1
-            for (int m1 = 0; m1 < N; ++m1) {
-                A inner = A(0);
-#pragma unroll
-                for (int a = 0; a < NTH; ++a) inner += et[a] * trl[m1 * NTH + a];
-                acc += es[m1] * inner;
-            }
-            fl[li * TRL + le] = A(((F & 1) ? dx : dy) * 0.25) * dth_[kk] * acc;
-        }
-    }
-
-    // ---- phase 4: the scattering, subtracted from the outputs
+    // ---- phase 3: the scattering, subtracted from the outputs
+    if constexpr (!EARLY && !XB) load_inflow();
     if (!EARLY && scat_w) scatter();
     if (scat_w && rok) {
 #pragma unroll
@@ -512,20 +468,23 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
     }
     __syncthreads();
 
-    // ---- phase 5: write back the part's DOFs (own DOF e = kl CD + lt of
-    // part cell kl), by whole-cell passes as in phase 1 when a cell fits the
-    // workgroup
-    auto emit = [&](int kl, int lt, int sn) {
-        const int kk = kk_lo + kl, a = lt % NTH;
-        const int t = own0 + kl * CD + lt;
-        const bool masked = (cbd[kk] & nfc[sn]) != 0;
-        A v = ys[sn * NOAP + kl * NTH + a];
+    // ---- phase 4: the inflow through the x-face, then the y-face, and the
+    // write-back of the part's DOFs by whole-cell passes as in phase 1
+    if (tid >= XS) return;
+#pragma unroll
+    for (int u = 0; u < YU; ++u) {
+        const int kl = tid / CD + u * CPP;
+        if (kl >= OC) break;
+        const int kk = kk_lo + kl, ca = kk * NTH + ae, t = own0 + kl * CD + le;
+        const bool masked = (cbd[kk] & nfc[sne]) != 0;
+        A v = ys[sne * NOAP + kl * NTH + ae];
         if (bconv) {
-            // inflow face fluxes: x-face, then y-face
-            const int i = sn / N, j = sn % N;
-            const int fx = cfx[kl], fy = cfy[kl];
-            if (i + 1 == (fx & 15)) v += fl[(fx >> 4) + j * NTH + a];
-            if (j + 1 == (fy & 15)) v += fl[(fy >> 4) + i * NTH + a];
+            const UFaces f(cqd[kk]);
+            const A xtf = f.Fx == 0 ? cth[ca] : -cth[ca], ytf = f.Fy == 1 ? sth[ca] : -sth[ca];
+            if (ie == (f.Fx == 0 ? 0 : N - 1))
+                v += u_inflow(A(dy * 0.25), dth_[kk], wx_[je], cw[ca], xtf, xi[u]);
+            if (je == (f.Fy == 1 ? 0 : N - 1))
+                v += u_inflow(A(dx * 0.25), dth_[kk], wx_[ie], cw[ca], ytf, yi[u]);
         }
         if (masked) v = A(0);
         if (accumulate) {
@@ -533,14 +492,6 @@ __global__ __launch_bounds__(UTHREADS, 4) void k_uniform(DevMesh m, uint32_t ops
         } else {
             y[cdof + t] = T(v);
         }
-    };
-    if constexpr (CPP > 0) {
-        if (tid < XS) {
-            const int lt = tid % CD, sn = lt / NTH;
-            for (int kl = tid / CD; kl < OC; kl += CPP) emit(kl, lt, sn);
-        }
-    } else {
-        for (int e = tid; e < NOWN; e += UTHREADS) emit(e / CD, e % CD, (e % CD) / NTH);
     }
 }
 
@@ -988,21 +939,16 @@ template <typename T, typename A, int PREC, int N, int NTH, int NC, int H>
 int launch_one(rtx_plan *p, uint32_t ops, const void *dx, void *dy, hipStream_t st, int acc) {
     constexpr int NSP = N * N, NA = NC * NTH;
     constexpr int NAP = u_pad(NA, NTH), NOAP = u_pad((NC / H) * NTH, NTH);
-    constexpr int MAXL = 4 * (NC / H), TRL = N * NTH;
-    RTX_CHECK(p->max_part_links[H] <= MAXL, "uniform apply: %d links in a column part (max %d)",
-              p->max_part_links[H], MAXL);
-    // column and output rows, then trace and flux slots for the largest link
-    // count of any part
     constexpr bool XB = PREC == RTX_PREC_MIXED;
     const size_t tiles = XB ? u_bf_off(size_t(NSP * NAP + NSP * NOAP) * sizeof(A)) + u_bf_bytes(NSP, NA)
                             : size_t(NSP * NAP + NSP * NOAP) * sizeof(A);
-    const size_t lds = tiles + size_t(2 * p->max_part_links[H] * TRL) * sizeof(A);
+    const size_t lds = tiles;
     auto kern = k_uniform<T, A, PREC, N, NTH, NC, H>;
     RTX_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(lds)));
     const int nblocks = ((p->m.ncol + UXCD - 1) / UXCD) * UXCD * H;   // 8 cpx H
-    kern<<<nblocks, u_threads<NTH, NC, H>(), lds, st>>>(p->m, ops, acc, (const T *)dx, (T *)dy,
-                                                        p->max_part_links[H]);
+    kern<<<nblocks, u_threads<NTH, NC, H>(), lds, st>>>(p->m, ops, acc, p->uni_src, (const T *)dx,
+                                                        (T *)dy);
     RTX_HIP(hipGetLastError());
     return RTX_OK;
 }
@@ -1038,11 +984,11 @@ template <int N, int NTH, int NC>
 int launch_shape(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
                  int acc) {
     // default: FP64 runs the output-layout kernel when every column is
-    // resident at once (four workgroups per CU; C2, 1024 columns: 29.5 us
-    // against 30.4 us), else the line-pass kernel, whose eight-wave
-    // workgroups pipeline better over several rounds (64 x 64 x 16 cells:
-    // 94 us against 109 us); FP32 and mixed run the line-pass kernel (mixed
-    // C2 15.3 us against 15.7 us).  A part count set by
+    // resident at once (four workgroups per CU; 1,024 columns of 5 x 5 x 80:
+    // 26.4 us against 27.3 us), else the line-pass kernel, whose eight-wave
+    // workgroups pipeline better over several rounds (4,096 columns: 89 us
+    // against 109 us); FP32 and mixed run the line-pass kernel (1,024 columns
+    // mixed: 14.7 us against 15.7 us).  A part count set by
     // rtx_set_uniform_parts or rtx_autotune selects the line-pass kernel
     // with that many parts.
     int H = p->uni_H;
