@@ -316,10 +316,10 @@ __device__ inline int hp_node(int t, int i, int l0, int ny) {
 // by the node count are left to run time, and every precision takes one line
 // per lane group and item.  A kernel apart: in one with the square columns its
 // scalar registers slow those down by 2 to 5 %.  Against the generic kernels:
-// 8 x 6 nodes, 7 angles per cell, 1,024 columns FP64 100 -> 49 us, mixed 91 ->
-// 35 us; 4 x 5 nodes, 8 angles, 4,096 columns FP64 366 -> 251 us, mixed 329 ->
-// 168 us; 3 x 5 nodes, 4 angles, 256 columns FP64 20 -> 12 us (and with alike
-// neighbours read directly 42, 30, 229, 140 and 9 us).
+// 8 x 6 nodes, 7 angles per cell, 1,024 columns FP64 100 -> 49 us, FP32 91 ->
+// 40 us; 4 x 5 nodes, 8 angles, 4,096 columns FP64 366 -> 251 us, FP32 331 ->
+// 223 us; 3 x 5 nodes, 4 angles, 256 columns FP64 20 -> 12 us (and with alike
+// neighbours read directly 42, 32, 229, 182 and 9 us).  Mixed runs FP32.
 template <typename T, typename A, int PREC, int N, bool RECT, bool ALIKE>
 __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, uint32_t ops,
                                           int accumulate, HpShared<A> &sh, unsigned char *lds,
@@ -763,6 +763,22 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
             continue;
         }
         ++p->hp_ncols;
+        // In mixed precision, columns of unlike orders and those with very many
+        // couplings are applied in FP32, the accuracy they have always had
+        // there: they go with the columns of the RECT kernel.
+        int sums = 0, inner = 0;
+        for (int k = k0; k < k1; ++k) {
+            int lf = 0;
+            for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) {
+                const int c1 = d->cell_col[d->link_src[l]], odd = d->link_face[l] & 1;
+                lf |= 1 << d->link_face[l];
+                inner += (odd ? d->col_nx[c1] : d->col_ny[c1]) * d->cell_nth[k];
+            }
+            sums += __builtin_popcount(lf) * d->col_nx[c] * d->cell_nth[k];
+        }
+        const bool square = d->col_nx[c] == d->col_ny[c] &&
+                            d->link_start[k1] - d->link_start[k0] <= 192 && sums <= 4096 &&
+                            need[RTX_PREC_MIXED] + 4 * size_t(std::max(sums, inner)) + 8192 <= cap;
         const double dx = d->col_geom[4 * c + 2] - d->col_geom[4 * c];
         const double dy = d->col_geom[4 * c + 3] - d->col_geom[4 * c + 1];
         for (int k = k0; k < k1; ++k) {
@@ -804,7 +820,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         }
         for (int pr = 0; pr < 3; ++pr) {
             const int cls = need[pr] <= half ? 0 : 1;
-            auto &list = d->col_nx[c] == d->col_ny[c] ? hdr[pr][cls] : rect[pr][cls];
+            auto &list = square ? hdr[pr][cls] : rect[pr][cls];
             list.insert(list.end(), h, h + HP_HDR);
             HpClass &hc = p->hp_cls[pr][cls];
             hc.bytes = std::max(hc.bytes, need[pr]);
@@ -903,18 +919,23 @@ static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, 
         return RTX_OK;
     };
     auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
-        const int rc = p->hp_alike
-                           ? launch_kind(k_hpcol<T, A, PREC, false, true>, hc, 0, hc.n_square, s)
-                           : launch_kind(k_hpcol<T, A, PREC, false, false>, hc, 0, hc.n_square, s);
-        if (rc) return rc;
-        const int n = hc.n - hc.n_square;
-        return p->hp_alike ? launch_kind(k_hpcol<T, A, PREC, true, true>, hc, hc.n_square, n, s)
-                           : launch_kind(k_hpcol<T, A, PREC, true, false>, hc, hc.n_square, n, s);
+        return p->hp_alike
+                   ? launch_kind(k_hpcol<T, A, PREC, false, true>, hc, 0, hc.n_square, s)
+                   : launch_kind(k_hpcol<T, A, PREC, false, false>, hc, 0, hc.n_square, s);
     };
+    // the other columns (mixed precision: in FP32)
+    constexpr int RP = PREC == RTX_PREC_MIXED ? RTX_PREC_F32 : PREC;
+    for (const HpClass &hc : p->hp_cls[RP]) {
+        const int n = hc.n - hc.n_square;
+        const int rc = p->hp_alike
+                           ? launch_kind(k_hpcol<T, A, RP, true, true>, hc, hc.n_square, n, st)
+                           : launch_kind(k_hpcol<T, A, RP, true, false>, hc, hc.n_square, n, st);
+        if (rc) return rc;
+    }
     const HpClass *hc = p->hp_cls[PREC];
-    if (hc[0].n == 0 || hc[1].n == 0 || !p->hp_side) {
-        const HpClass &one = hc[0].n ? hc[0] : hc[1];
-        return one.n ? launch(one, st) : RTX_OK;
+    if (hc[0].n_square == 0 || hc[1].n_square == 0 || !p->hp_side) {
+        const HpClass &one = hc[0].n_square ? hc[0] : hc[1];
+        return launch(one, st);
     }
     // The classes write disjoint outputs, so the large-column class runs on
     // the caller's stream and the other on the plan's side stream at the same
