@@ -39,7 +39,8 @@
 // by LDS need into two classes (one launch each) sized so that the first runs
 // two workgroups per CU.  Arithmetic: FP64 (v_mfma_f64_16x16x4f64), FP32
 // (v_mfma_f32_16x16x4f32) or mixed (FP32 transport terms, BF16 scattering
-// operands on v_mfma_f32_16x16x16bf16_1k with FP32 accumulation).
+// operands on v_mfma_f32_16x16x16bf16_1k with FP32 accumulation); columns that
+// hp_wide names keep FP64 arithmetic in the last two.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -311,15 +312,16 @@ __device__ inline int hp_node(int t, int i, int l0, int ny) {
 // cells mixed 87 -> 45 us, 1,024 columns of 7 x 7 nodes FP32 52 -> 35 us (29
 // with alike neighbours read directly).
 //
-// RECT: N nodes along x and another number along y, read at run time.  The
-// lines have their compiled length; only the sums along y and the divisions
-// by the node count are left to run time, and every precision takes one line
-// per lane group and item.  A kernel apart: in one with the square columns its
-// scalar registers slow those down by 2 to 5 %.  Against the generic kernels:
-// 8 x 6 nodes, 7 angles per cell, 1,024 columns FP64 100 -> 49 us, FP32 91 ->
-// 40 us; 4 x 5 nodes, 8 angles, 4,096 columns FP64 366 -> 251 us, FP32 331 ->
-// 223 us; 3 x 5 nodes, 4 angles, 256 columns FP64 20 -> 12 us (and with alike
-// neighbours read directly 42, 32, 229, 182 and 9 us).  Mixed runs FP32.
+// RECT: N nodes along x, the number along y read at run time.  The lines have
+// their compiled length; only the sums along y and the divisions by the node
+// count are left to run time, and one item takes one line per lane group.  A
+// kernel apart: in one with the other columns its scalar registers slow those
+// down by 2 to 5 %.  Always in FP64 arithmetic (see hp_wide), on FP64 or FP32
+// vectors.  Against the generic kernels, alike neighbours read directly: 1,024
+// columns of 8 x 6 nodes and 56 angles FP64 96 -> 38 us, FP32 87 -> 36 us; 4,096
+// of 4 x 5 nodes and 64 angles 185 -> 94 and 168 -> 97 us; 256 of 3 x 5 nodes and
+// 16 angles 16 -> 8 us.  With hanging nodes, 856 columns of 8 x 6 nodes and 56
+// angles: 84 -> 47 and 76 -> 45 us.
 template <typename T, typename A, int PREC, int N, bool RECT, bool ALIKE>
 __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, uint32_t ops,
                                           int accumulate, HpShared<A> &sh, unsigned char *lds,
@@ -655,6 +657,43 @@ static size_t hp_bytes(int nsp, int na, int prec, bool alike) {
 // Static LDS of k_hpcol (the tables above), for the capacity check.
 constexpr size_t HP_STATIC_BYTES = sizeof(HpShared<double>) + 64;
 
+// Whether FP32 and mixed precision apply column c in FP64 arithmetic (T float,
+// A double, on the RECT kernel): columns of unlike orders, and square ones that
+// with their couplings hold more FP64 values than a CU's LDS less 11 KB of
+// tables, or more than 192 links or 4,096 inflow-face values.  Those have
+// always run like that in reduced precision (on the generic kernels, with FP64
+// transport terms), and what a caller gets there is not to depend on the kernel:
+// relative error 2.5e-8 (generic 3.6e-8), against 1e-7 in FP32 arithmetic and
+// 2e-5 with BF16 scattering.  (FP32 arithmetic took 30 us where this takes 36,
+// 1,024 columns of 8 x 6 nodes and 56 angles.)
+static bool hp_wide(const rtx_mesh_desc *d, int c) {
+    constexpr size_t LDS_VALUES = 152712;
+    const int k0 = d->col_cell_start[c], k1 = d->col_cell_start[c + 1];
+    const int nx = d->col_nx[c], ny = d->col_ny[c], na = d->col_nang[c];
+    if (nx != ny || d->link_start[k1] - d->link_start[k0] > 192) return true;
+    // values of the inflow faces, of the traces contracted over their angles,
+    // and of the distinct E^s blocks
+    int sums = 0, inner = 0, nes = 0;
+    std::vector<int32_t> seen;
+    for (int k = k0; k < k1; ++k) {
+        int lf = 0;
+        for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) {
+            const int c1 = d->cell_col[d->link_src[l]], odd = d->link_face[l] & 1;
+            const int n1 = odd ? d->col_nx[c1] : d->col_ny[c1];
+            lf |= 1 << d->link_face[l];
+            inner += n1 * d->cell_nth[k];
+            if (std::find(seen.begin(), seen.end(), d->link_Es_off[l]) == seen.end()) {
+                seen.push_back(d->link_Es_off[l]);
+                nes += nx * n1;
+            }
+        }
+        sums += __builtin_popcount(lf) * nx * d->cell_nth[k];
+    }
+    const size_t own = std::max((na + 3) / 4 * 4 * (nx * ny | 1), d->col_ntrace[c]);
+    const size_t bytes = (8 * own + 15) / 16 * 16 + 8 * size_t(std::max(sums, inner) + nes) + 28 * na;
+    return sums > 4096 || (bytes + 15) / 16 * 16 > LDS_VALUES;
+}
+
 // Whether cell k's links all join it to cells with the same nodes and angles,
 // through an inflow face each.  E^s and E^theta are then diagonal (weights;
 // weights x direction) up to the rounding of the node positions, and the
@@ -707,8 +746,8 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     // a column whose workgroup (dynamic + static LDS) fits half of a CU's
     // 160 KB runs two workgroups per CU (class 0), the others one (class 1)
     const size_t half = 80 * 1024 > HP_STATIC_BYTES ? 80 * 1024 - HP_STATIC_BYTES : 0;
-    std::vector<int32_t> hdr[3][HP_NCLS], rect[3][HP_NCLS], over, links;
-    std::vector<HpCell> cells;
+    std::vector<int32_t> hdr[3][HP_NCLS], wide[2][HP_NCLS], over, links;
+    std::vector<HpCell> cells, wide_cells;
     p->hp_ncols = 0;
     // Neighbours are read directly where at least a quarter of the cells have
     // alike ones.  The kernel that does so holds more registers: with no such
@@ -763,22 +802,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
             continue;
         }
         ++p->hp_ncols;
-        // In mixed precision, columns of unlike orders and those with very many
-        // couplings are applied in FP32, the accuracy they have always had
-        // there: they go with the columns of the RECT kernel.
-        int sums = 0, inner = 0;
-        for (int k = k0; k < k1; ++k) {
-            int lf = 0;
-            for (int l = d->link_start[k]; l < d->link_start[k + 1]; ++l) {
-                const int c1 = d->cell_col[d->link_src[l]], odd = d->link_face[l] & 1;
-                lf |= 1 << d->link_face[l];
-                inner += (odd ? d->col_nx[c1] : d->col_ny[c1]) * d->cell_nth[k];
-            }
-            sums += __builtin_popcount(lf) * d->col_nx[c] * d->cell_nth[k];
-        }
-        const bool square = d->col_nx[c] == d->col_ny[c] &&
-                            d->link_start[k1] - d->link_start[k0] <= 192 && sums <= 4096 &&
-                            need[RTX_PREC_MIXED] + 4 * size_t(std::max(sums, inner)) + 8192 <= cap;
+        const bool rect = d->col_nx[c] != d->col_ny[c], in_f64 = hp_wide(d, c);
         const double dx = d->col_geom[4 * c + 2] - d->col_geom[4 * c];
         const double dy = d->col_geom[4 * c + 3] - d->col_geom[4 * c + 1];
         for (int k = k0; k < k1; ++k) {
@@ -816,16 +840,24 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
                 }
             cl.w = nl | d->col_nx[c] << 8 | d->cell_nth[k] << 12 | (d->cell_bdry[k] & 15) << 16 |
                    lf << 20 | d->col_ny[c] << 24;
-            cells.push_back(cl);
+            (in_f64 ? wide_cells : cells).push_back(cl);
         }
-        for (int pr = 0; pr < 3; ++pr) {
-            const int cls = need[pr] <= half ? 0 : 1;
-            auto &list = square ? hdr[pr][cls] : rect[pr][cls];
-            list.insert(list.end(), h, h + HP_HDR);
-            HpClass &hc = p->hp_cls[pr][cls];
-            hc.bytes = std::max(hc.bytes, need[pr]);
+        const auto take = [&](std::vector<int32_t> *lists, HpClass *classes, size_t bytes) {
+            const int cls = bytes <= half ? 0 : 1;
+            lists[cls].insert(lists[cls].end(), h, h + HP_HDR);
+            classes[cls].bytes = std::max(classes[cls].bytes, bytes);
+        };
+        if (!rect) take(hdr[RTX_PREC_F64], p->hp_cls[RTX_PREC_F64], need[RTX_PREC_F64]);
+        else take(wide[0], p->hp_wide[0], need[RTX_PREC_F64]);
+        if (in_f64) {
+            take(wide[1], p->hp_wide[1], need[RTX_PREC_F64]);
+        } else {
+            take(hdr[RTX_PREC_F32], p->hp_cls[RTX_PREC_F32], need[RTX_PREC_F32]);
+            take(hdr[RTX_PREC_MIXED], p->hp_cls[RTX_PREC_MIXED], need[RTX_PREC_MIXED]);
         }
     }
+    p->hp_n_narrow = int(cells.size());
+    cells.insert(cells.end(), wide_cells.begin(), wide_cells.end());
     // the columns the kernel cannot take run on the generic kernels
     std::vector<int32_t> gcells;
     for (int c : over)
@@ -843,13 +875,10 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     const std::vector<float> wd_f(wd.begin(), wd.end());
     size_t total = ang_flag.size() + ang_src.size() + links.size() + gcells.size() + gitems.size() +
                    wd_f.size() + 64;
-    for (int pr = 0; pr < 3; ++pr)
-        for (int k = 0; k < HP_NCLS; ++k) {
-            auto &l = hdr[pr][k];
-            p->hp_cls[pr][k].n_square = int(l.size() / HP_HDR);
-            l.insert(l.end(), rect[pr][k].begin(), rect[pr][k].end());
-            total += l.size();
-        }
+    for (int k = 0; k < HP_NCLS; ++k) {
+        for (const auto &lists : hdr) total += lists[k].size();
+        for (const auto &lists : wide) total += lists[k].size();
+    }
     RTX_HIP(hipMalloc(&p->hp_alloc, total * sizeof(int32_t)));
     RTX_HIP(hipMalloc(&p->hp_es, (wd.size() + ang_dth.size()) * sizeof(double) +
                                     cells.size() * sizeof(HpCell) + 64));
@@ -867,11 +896,14 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     p->hp.ang_flag = put_i(ang_flag);
     p->hp.ang_src = reinterpret_cast<const int2 *>(put_i(ang_src));
     p->hp.links = reinterpret_cast<const int4 *>(put_i(links));
-    for (int pr = 0; pr < 3; ++pr)
-        for (int k = 0; k < HP_NCLS; ++k) {
-            p->hp_cls[pr][k].hdr = put_i(hdr[pr][k]);
-            p->hp_cls[pr][k].n = int(hdr[pr][k].size() / HP_HDR);
-        }
+    const auto put_class = [&](HpClass &hc, const std::vector<int32_t> &list) {
+        hc.hdr = put_i(list);
+        hc.n = int(list.size() / HP_HDR);
+    };
+    for (int k = 0; k < HP_NCLS; ++k) {
+        for (int pr = 0; pr < 3; ++pr) put_class(p->hp_cls[pr][k], hdr[pr][k]);
+        for (int w = 0; w < 2; ++w) put_class(p->hp_wide[w][k], wide[w][k]);
+    }
     p->hp_gen_cells = put_i(gcells);
     p->hp_n_gen_cells = int(gcells.size());
     p->hp_gen_items = put_i(gitems);
@@ -897,46 +929,52 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     return RTX_OK;
 }
 
+template <typename T, typename A>
+static int launch_hp_flux(const rtx_plan *p, uint32_t ops, int c0, int n, const T *x, T *y,
+                          hipStream_t st, int accumulate) {
+    if (n == 0) return RTX_OK;
+    const int nblk = (n + HF_WAVES - 1) / HF_WAVES;
+    k_hp_flux<T, A><<<(nblk + HP_XCD - 1) / HP_XCD * HP_XCD, 64 * HF_WAVES, 0, st>>>(
+        p->m, p->hp.cells + c0, p->hp.links, n, (ops & RTX_OP_RESTRICT) ? 1 : 0, accumulate, x, y);
+    RTX_HIP(hipGetLastError());
+    return RTX_OK;
+}
+
 template <typename T, typename A, int PREC>
 static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, hipStream_t st,
                      int accumulate) {
-    if ((ops & RTX_OP_BCONV) && p->hp_n_cells > 0) {
-        const int nblk = (p->hp_n_cells + HF_WAVES - 1) / HF_WAVES;
-        k_hp_flux<T, A><<<(nblk + HP_XCD - 1) / HP_XCD * HP_XCD, 64 * HF_WAVES, 0, st>>>(
-            p->m, p->hp.cells, p->hp.links, p->hp_n_cells, (ops & RTX_OP_RESTRICT) ? 1 : 0,
-            accumulate, (const T *)dx, (T *)dy);
-        RTX_HIP(hipGetLastError());
+    const T *x = static_cast<const T *>(dx);
+    T *y = static_cast<T *>(dy);
+    if (ops & RTX_OP_BCONV) {
+        const int nn = PREC == RTX_PREC_F64 ? 0 : p->hp_n_narrow;
+        int rc = launch_hp_flux<T, A>(p, ops, 0, nn, x, y, st, accumulate);
+        if (rc) return rc;
+        rc = launch_hp_flux<T, double>(p, ops, nn, p->hp_n_cells - nn, x, y, st, accumulate);
+        if (rc) return rc;
     }
-    // a class's square columns, then the others
-    auto launch_kind = [&](auto kern, const HpClass &hc, int c0, int n, hipStream_t s) -> int {
-        if (n == 0) return RTX_OK;
-        const int per = (n + HP_XCD - 1) / HP_XCD;
+    auto launch_class = [&](auto kern, const HpClass &hc, hipStream_t s) -> int {
+        if (hc.n == 0) return RTX_OK;
+        const int per = (hc.n + HP_XCD - 1) / HP_XCD;
         RTX_HIP(hipFuncSetAttribute((const void *)kern,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(hc.bytes)));
-        kern<<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(
-            p->m, p->hp, ops, accumulate, hc.hdr + size_t(c0) * HP_HDR, n, (const T *)dx, (T *)dy);
+        kern<<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(p->m, p->hp, ops, accumulate, hc.hdr, hc.n,
+                                                        x, y);
         RTX_HIP(hipGetLastError());
         return RTX_OK;
     };
-    auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
-        return p->hp_alike
-                   ? launch_kind(k_hpcol<T, A, PREC, false, true>, hc, 0, hc.n_square, s)
-                   : launch_kind(k_hpcol<T, A, PREC, false, false>, hc, 0, hc.n_square, s);
-    };
-    // the other columns (mixed precision: in FP32)
-    constexpr int RP = PREC == RTX_PREC_MIXED ? RTX_PREC_F32 : PREC;
-    for (const HpClass &hc : p->hp_cls[RP]) {
-        const int n = hc.n - hc.n_square;
+    // the columns of the RECT kernel, in FP64 arithmetic whatever the precision
+    for (const HpClass &hc : p->hp_wide[PREC == RTX_PREC_F64 ? 0 : 1]) {
         const int rc = p->hp_alike
-                           ? launch_kind(k_hpcol<T, A, RP, true, true>, hc, hc.n_square, n, st)
-                           : launch_kind(k_hpcol<T, A, RP, true, false>, hc, hc.n_square, n, st);
+                           ? launch_class(k_hpcol<T, double, RTX_PREC_F64, true, true>, hc, st)
+                           : launch_class(k_hpcol<T, double, RTX_PREC_F64, true, false>, hc, st);
         if (rc) return rc;
     }
+    auto launch = [&](const HpClass &hc, hipStream_t s) -> int {
+        return p->hp_alike ? launch_class(k_hpcol<T, A, PREC, false, true>, hc, s)
+                           : launch_class(k_hpcol<T, A, PREC, false, false>, hc, s);
+    };
     const HpClass *hc = p->hp_cls[PREC];
-    if (hc[0].n_square == 0 || hc[1].n_square == 0 || !p->hp_side) {
-        const HpClass &one = hc[0].n_square ? hc[0] : hc[1];
-        return launch(one, st);
-    }
+    if (hc[0].n == 0 || hc[1].n == 0 || !p->hp_side) return launch(hc[0].n ? hc[0] : hc[1], st);
     // The classes write disjoint outputs, so the large-column class runs on
     // the caller's stream and the other on the plan's side stream at the same
     // time (the side stream waits for the work queued before, and the

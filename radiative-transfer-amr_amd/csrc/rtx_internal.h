@@ -136,13 +136,13 @@ struct HpTables {
     const double *wd = nullptr;
     const float *wd_f = nullptr;
 };
-// per column of a class a header of HP_HDR ints (first cell, cells, nodes
+// Per column of a class a header of HP_HDR ints (first cell, cells, nodes
 // along x, angles, first DOF, nodes along y, -, first angle, .., [13] first
 // spatial node, [14] column), so the kernel reads a column's scalars in one step
 constexpr int HP_HDR = 16;
 struct HpClass {
-    int n = 0, n_square = 0;        // columns, those with as many nodes along x as along y
-    const int32_t *hdr = nullptr;   // their headers (the square ones first, each kind in key order)
+    int n = 0;                      // columns
+    const int32_t *hdr = nullptr;   // their headers, in key order
     size_t bytes = 0;               // dynamic LDS per workgroup
 };
 bool alike_cell(const rtx_mesh_desc *d, int k, int32_t *src, int32_t *masked);
@@ -218,9 +218,13 @@ struct rtx_plan {
     bool hp_ok = false;
     bool hp_default = false;     // mode -1 uses the column kernel
     rtx::HpTables hp;
-    rtx::HpClass hp_cls[3][rtx::HP_NCLS];   // per precision
+    // columns in a precision's own arithmetic, and those that the RECT kernel
+    // applies in FP64 arithmetic ([0] FP64 applies, [1] FP32 and mixed)
+    rtx::HpClass hp_cls[3][rtx::HP_NCLS], hp_wide[2][rtx::HP_NCLS];
     int hp_ncols = 0;
-    int hp_n_cells = 0;                     // cells of those columns for k_hp_flux
+    // cells of those columns for k_hp_flux; the first hp_n_narrow are those of
+    // hp_cls in FP32 and mixed precision, the others those of hp_wide[1]
+    int hp_n_cells = 0, hp_n_narrow = 0;
     bool hp_alike = false;                  // alike neighbours are read directly
     std::vector<int32_t> hp_over_cols;
     const int32_t *hp_gen_cells = nullptr, *hp_gen_items = nullptr;

@@ -527,3 +527,62 @@ def check_column_kernels(mesh, seed):
     y = op.apply(_dev(x), ops=OP_SCAT).cpu().numpy()
     assert _rel(y, V["S"] @ x) < TOL64
     return op
+
+
+def _links_of(t, c):
+    return int(t.link_start[t.col_cell_start[c + 1]] - t.link_start[t.col_cell_start[c]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["unlike", "unlike_hp", "large", "many_links"])
+@pytest.mark.parametrize("path", [-1, 3], ids=["auto", "column"])
+def test_reduced_precision_of_wide_columns(cuda, case, path):
+    """Columns of unlike orders, and square ones too large for LDS in FP64 or
+    with many links, are applied in FP64 arithmetic when FP32 or mixed
+    precision is asked for, as by the generic kernels.
+
+    Bound: the generic kernels round every output to FP32 twice (transport
+    part, then with the scattering), the column kernel once, and at inflow
+    nodes twice.  So its error is at most the generic kernels' one; over the
+    15,000 values and more of a case the root mean square of the roundings
+    varies by about 1 %, and 5 % are allowed.  (FP32 arithmetic is off by
+    three times as much, BF16 scattering by 500 times.)"""
+    import torch
+    from rtx.operator import TransportOperator, OP_SYSTEM, OP_RESTRICT, PREC_F32, PREC_MIXED
+    if case == "unlike":
+        mesh = problems.uniform_mesh([1.0, 1.0], [8, 6, 7], 3, 2)
+    elif case == "unlike_hp":
+        mesh = problems.uniform_mesh([1.0, 1.0], [5, 7, 6], 3, 2)
+        keys = sorted(mesh.cols)
+        mesh.ref_col(keys[0], "spt", "p")
+        mesh.ref_col(keys[5], "spt", "h")
+        mesh.ref_cell(keys[-1], sorted(mesh.cols[keys[-1]].cells)[0], "h")
+    elif case == "large":      # periodic: every cell has two inflow faces
+        mesh = problems.uniform_mesh([1.0, 1.0], [10, 10, 10], 4, 1, pbcs=(True, True))
+    else:
+        # two columns with four refined neighbours: 256 links each
+        mesh = problems.uniform_mesh([1.0, 1.0], [7, 7, 3], 6, 2, pbcs=(True, True))
+        mids = [k for k in sorted(mesh.cols) if mesh.cols[k].pos[:2] in ([0.0, 0.0], [0.5, 0.5])]
+        for key in {n for k in mids for face in mesh.cols[k].nhbr_keys for n in face if n is not None}:
+            mesh.ref_col(key, "spt", "h")
+    wl = problems.two_scatterers()
+    op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
+    t = op.t
+    print("wide columns", case, "path", path, "ndof", t.ndof, flush=True)
+    keep = np.zeros(t.ndof, bool)
+    for c in range(t.ncol):
+        if case != "many_links" or _links_of(t, c) > 192:
+            k0, k1 = t.col_cell_start[c], t.col_cell_start[c + 1]
+            end = t.cell_dof_off[k1 - 1] + t.col_nx[c] * t.col_ny[c] * t.cell_nth[k1 - 1]
+            keep[t.cell_dof_off[k0]:end] = True
+    assert keep.sum() > 15_000
+    x = _dev(np.random.default_rng(3).uniform(-1.0, 1.0, t.ndof)).float()
+    for ops in (OP_SYSTEM, OP_SYSTEM | OP_RESTRICT):
+        op.set_path(0)
+        ref = op.apply(x.double(), ops=ops).cpu().numpy()[keep]
+        generic = _rel(op.apply(x, ops=ops, precision=PREC_F32).cpu().double().numpy()[keep], ref)
+        op.set_path(path)
+        for prec in (PREC_F32, PREC_MIXED):
+            err = _rel(op.apply(x, ops=ops, precision=prec).cpu().double().numpy()[keep], ref)
+            print("  precision", prec, "error", err, "generic", generic, flush=True)
+            assert err <= 1.05 * generic, (prec, err, generic)
