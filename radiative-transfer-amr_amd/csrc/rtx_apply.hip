@@ -441,14 +441,16 @@ extern "C" int rtx_apply(rtx_plan *p, uint32_t op_mask, int precision, const voi
         RTX_CHECK(!(op_mask & RTX_OP_QUADW) || p->fused_mode != 3,
                   "rtx_apply: the hp column path does not apply quadrature weights");
         if (!(op_mask & RTX_OP_QUADW)) {
-            int rc = launch_hpcol(p, op_mask, precision, d_x, d_y, st, acc);
-            if (rc || p->hp_over_cols.empty()) return rc;
+            const int all = p->fused_mode == 3 ? 1 : 0;
+            int rc = launch_hpcol(p, op_mask, precision, d_x, d_y, st, acc, all);
+            if (rc || p->hp_n_gen_cells[all] == 0) return rc;
             if (precision == RTX_PREC_F64)
-                return launch_apply<double>(p, op_mask, d_x, d_y, st, p->hp_gen_cells,
-                                            p->hp_n_gen_cells, p->hp_gen_items,
-                                            p->hp_n_gen_items);
-            return launch_apply<float>(p, op_mask, d_x, d_y, st, p->hp_gen_cells,
-                                       p->hp_n_gen_cells, p->hp_gen_items, p->hp_n_gen_items);
+                return launch_apply<double>(p, op_mask, d_x, d_y, st, p->hp_gen_cells[all],
+                                            p->hp_n_gen_cells[all], p->hp_gen_items[all],
+                                            p->hp_n_gen_items[all]);
+            return launch_apply<float>(p, op_mask, d_x, d_y, st, p->hp_gen_cells[all],
+                                       p->hp_n_gen_cells[all], p->hp_gen_items[all],
+                                       p->hp_n_gen_items[all]);
         }
     }
     const bool forced = p->fused_mode == 1;
@@ -644,7 +646,7 @@ extern "C" int rtx_set_uniform_parts(rtx_plan *p, int H) {
 /* Launch-shape summary: out[0] uniform bin usable, [1] its parts per column,
    [2 + 3 b .. 4 + 3 b] parts, columns and generic flag of fused bin b
    (b < 6), [20], [21] columns and cells on the generic kernels, [22] the hp
-   column kernel is the default path, [23] columns it takes, [24] the uniform
+   column kernel is the default path, [23] columns it can take, [24] the uniform
    bin's FP64 apply runs the output-layout kernel (1: the default when every
    column is resident at once, four per CU) or the line-pass kernel (0).
    Returns the count (25). */

@@ -694,6 +694,16 @@ static bool hp_wide(const rtx_mesh_desc *d, int c) {
     return sums > 4096 || (bytes + 15) / 16 * 16 > LDS_VALUES;
 }
 
+// Whether the RECT kernel needs long for column c: its wavefronts' rounds of
+// items (16 angles, a line per lane group) times an item's work, the matrix steps
+// (angles x node tiles / 4) and the lines' products at half the weight.
+static bool hp_long(const rtx_mesh_desc *d, int c) {
+    const int nx = d->col_nx[c], ny = d->col_ny[c], na = d->col_nang[c];
+    const int items = (na + 15) / 16 * ((ny + 3) / 4);
+    const int work = na * ((nx + 3) / 4) / 2 + nx * (nx + ny);
+    return (items + HP_WAVES - 1) / HP_WAVES * work > 500;
+}
+
 // Whether cell k's links all join it to cells with the same nodes and angles,
 // through an inflow face each.  E^s and E^theta are then diagonal (weights;
 // weights x direction) up to the rounding of the node positions, and the
@@ -763,7 +773,29 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     }
     p->hp_alike = 4 * ndirect >= d->ncell;
     if (!p->hp_alike) std::fill(direct.begin(), direct.end(), char(0));
+    // A workgroup works a column off alone, so few columns that need long leave
+    // the chip idle, and the generic kernels spread them better.  Where they
+    // are at most three for every four CUs, the default path leaves the long
+    // ones of the columns that hp_wide names to the generic kernels.  Generic
+    // against column kernel: 16 columns of 10 x 9 nodes and 80 angles (work 620)
+    // FP32 32 / 36 us, of 8 x 7 nodes and 112 angles (464) 33 / 30 us; 16 of 8 x 7
+    // nodes and 256 angles FP64 50 / 79 us, 64 of them 61 / 79, 160 115 / 90; of
+    // 6 x 5 nodes and 192 angles in FP32 160 columns 51 / 54 us, 193 53 / 52.
+    std::vector<char> in_f64(nc), late(nc);
+    int nlate = 0;
     for (int c = 0; c < nc; ++c) {
+        in_f64[c] = hp_wide(d, c);
+        late[c] = in_f64[c] && hp_long(d, c);
+        nlate += late[c];
+    }
+    if (4 * nlate > 3 * p->n_cu) std::fill(late.begin(), late.end(), char(0));
+    // late columns last, so that each list begins with the default path's part
+    std::vector<int32_t> order;
+    for (int l = 0; l < 2; ++l)
+        for (int c = 0; c < nc; ++c)
+            if (late[c] == l) order.push_back(c);
+    std::vector<int32_t> deferred;
+    for (const int c : order) {
         const int k0 = d->col_cell_start[c], k1 = d->col_cell_start[c + 1];
         const int nsp = d->col_nx[c] * d->col_ny[c], na = d->col_nang[c];
         // per angle: its cell's masked faces, quadrant + 1 and the faces that
@@ -802,7 +834,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
             continue;
         }
         ++p->hp_ncols;
-        const bool rect = d->col_nx[c] != d->col_ny[c], in_f64 = hp_wide(d, c);
+        if (late[c]) deferred.push_back(c);
         const double dx = d->col_geom[4 * c + 2] - d->col_geom[4 * c];
         const double dy = d->col_geom[4 * c + 3] - d->col_geom[4 * c + 1];
         for (int k = k0; k < k1; ++k) {
@@ -840,16 +872,18 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
                 }
             cl.w = nl | d->col_nx[c] << 8 | d->cell_nth[k] << 12 | (d->cell_bdry[k] & 15) << 16 |
                    lf << 20 | d->col_ny[c] << 24;
-            (in_f64 ? wide_cells : cells).push_back(cl);
+            (in_f64[c] ? wide_cells : cells).push_back(cl);
+            if (!late[c]) ++p->hp_n_cells[0];
         }
         const auto take = [&](std::vector<int32_t> *lists, HpClass *classes, size_t bytes) {
             const int cls = bytes <= half ? 0 : 1;
             lists[cls].insert(lists[cls].end(), h, h + HP_HDR);
             classes[cls].bytes = std::max(classes[cls].bytes, bytes);
+            if (!late[c]) ++classes[cls].n[0];
         };
-        if (!rect) take(hdr[RTX_PREC_F64], p->hp_cls[RTX_PREC_F64], need[RTX_PREC_F64]);
+        if (d->col_nx[c] == d->col_ny[c]) take(hdr[RTX_PREC_F64], p->hp_cls[RTX_PREC_F64], need[RTX_PREC_F64]);
         else take(wide[0], p->hp_wide[0], need[RTX_PREC_F64]);
-        if (in_f64) {
+        if (in_f64[c]) {
             take(wide[1], p->hp_wide[1], need[RTX_PREC_F64]);
         } else {
             take(hdr[RTX_PREC_F32], p->hp_cls[RTX_PREC_F32], need[RTX_PREC_F32]);
@@ -858,11 +892,18 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     }
     p->hp_n_narrow = int(cells.size());
     cells.insert(cells.end(), wide_cells.begin(), wide_cells.end());
-    // the columns the kernel cannot take run on the generic kernels
-    std::vector<int32_t> gcells;
-    for (int c : over)
-        for (int k = d->col_cell_start[c]; k < d->col_cell_start[c + 1]; ++k) gcells.push_back(k);
-    const std::vector<int32_t> gitems = scatter_items(p, over);
+    // generic kernels: the columns the kernel cannot take, and in the default
+    // path those left to them
+    std::vector<int32_t> gcells[2], gitems[2];
+    for (int f = 0; f < 2; ++f) {
+        std::vector<int32_t> cols(over);
+        if (f == 0) cols.insert(cols.end(), deferred.begin(), deferred.end());
+        std::sort(cols.begin(), cols.end());
+        for (int c : cols)
+            for (int k = d->col_cell_start[c]; k < d->col_cell_start[c + 1]; ++k)
+                gcells[f].push_back(k);
+        gitems[f] = scatter_items(p, cols);
+    }
     // weights and w_i l'_p(xi_i) per node count
     std::vector<double> wd(size_t(HP_NM + 1) * HP_WD, 0.0);
     for (int n = 1; n <= HP_NM; ++n)
@@ -873,8 +914,8 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
                     d->lgl_w[n * HP_NM + i] * d->lgl_D[(size_t(n) * HP_NM + pp) * HP_NM + i];
         }
     const std::vector<float> wd_f(wd.begin(), wd.end());
-    size_t total = ang_flag.size() + ang_src.size() + links.size() + gcells.size() + gitems.size() +
-                   wd_f.size() + 64;
+    size_t total = ang_flag.size() + ang_src.size() + links.size() + wd_f.size() + 96;
+    for (int f = 0; f < 2; ++f) total += gcells[f].size() + gitems[f].size();
     for (int k = 0; k < HP_NCLS; ++k) {
         for (const auto &lists : hdr) total += lists[k].size();
         for (const auto &lists : wide) total += lists[k].size();
@@ -898,24 +939,25 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     p->hp.links = reinterpret_cast<const int4 *>(put_i(links));
     const auto put_class = [&](HpClass &hc, const std::vector<int32_t> &list) {
         hc.hdr = put_i(list);
-        hc.n = int(list.size() / HP_HDR);
+        hc.n[1] = int(list.size() / HP_HDR);
     };
     for (int k = 0; k < HP_NCLS; ++k) {
         for (int pr = 0; pr < 3; ++pr) put_class(p->hp_cls[pr][k], hdr[pr][k]);
         for (int w = 0; w < 2; ++w) put_class(p->hp_wide[w][k], wide[w][k]);
     }
-    p->hp_gen_cells = put_i(gcells);
-    p->hp_n_gen_cells = int(gcells.size());
-    p->hp_gen_items = put_i(gitems);
-    p->hp_n_gen_items = int(gitems.size() / 2);
+    for (int f = 0; f < 2; ++f) {
+        p->hp_gen_cells[f] = put_i(gcells[f]);
+        p->hp_n_gen_cells[f] = int(gcells[f].size());
+        p->hp_gen_items[f] = put_i(gitems[f]);
+        p->hp_n_gen_items[f] = int(gitems[f].size() / 2);
+    }
     p->hp.wd_f = static_cast<const float *>(put(wd_f.data(), wd_f.size() * sizeof(float)));
     base = static_cast<char *>(p->hp_es);
     p->hp.wd = static_cast<const double *>(put(wd.data(), wd.size() * sizeof(double)));
     p->hp.ang_dth = static_cast<const double *>(put(ang_dth.data(), ang_dth.size() * sizeof(double)));
     p->hp.cells = static_cast<const HpCell *>(put(cells.data(), cells.size() * sizeof(HpCell)));
-    p->hp_n_cells = int(cells.size());
+    p->hp_n_cells[1] = int(cells.size());
     RTX_HIP(hipGetLastError());
-    p->hp_over_cols = over;
     p->hp_ok = p->hp_ncols > 0;
     // side stream (default priority) and fork / join events of the class launches
     if (p->hp_ok) {
@@ -942,23 +984,24 @@ static int launch_hp_flux(const rtx_plan *p, uint32_t ops, int c0, int n, const 
 
 template <typename T, typename A, int PREC>
 static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, hipStream_t st,
-                     int accumulate) {
+                     int accumulate, int all) {
     const T *x = static_cast<const T *>(dx);
     T *y = static_cast<T *>(dy);
     if (ops & RTX_OP_BCONV) {
         const int nn = PREC == RTX_PREC_F64 ? 0 : p->hp_n_narrow;
         int rc = launch_hp_flux<T, A>(p, ops, 0, nn, x, y, st, accumulate);
         if (rc) return rc;
-        rc = launch_hp_flux<T, double>(p, ops, nn, p->hp_n_cells - nn, x, y, st, accumulate);
+        rc = launch_hp_flux<T, double>(p, ops, nn, p->hp_n_cells[all] - nn, x, y, st, accumulate);
         if (rc) return rc;
     }
     auto launch_class = [&](auto kern, const HpClass &hc, hipStream_t s) -> int {
-        if (hc.n == 0) return RTX_OK;
-        const int per = (hc.n + HP_XCD - 1) / HP_XCD;
+        const int n = hc.n[all];
+        if (n == 0) return RTX_OK;
+        const int per = (n + HP_XCD - 1) / HP_XCD;
         RTX_HIP(hipFuncSetAttribute((const void *)kern,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(hc.bytes)));
-        kern<<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(p->m, p->hp, ops, accumulate, hc.hdr, hc.n,
-                                                        x, y);
+        kern<<<per * HP_XCD, HP_THREADS, hc.bytes, s>>>(p->m, p->hp, ops, accumulate, hc.hdr, n, x,
+                                                        y);
         RTX_HIP(hipGetLastError());
         return RTX_OK;
     };
@@ -974,7 +1017,8 @@ static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, 
                            : launch_class(k_hpcol<T, A, PREC, false, false>, hc, s);
     };
     const HpClass *hc = p->hp_cls[PREC];
-    if (hc[0].n == 0 || hc[1].n == 0 || !p->hp_side) return launch(hc[0].n ? hc[0] : hc[1], st);
+    if (hc[0].n[all] == 0 || hc[1].n[all] == 0 || !p->hp_side)
+        return launch(hc[0].n[all] ? hc[0] : hc[1], st);
     // The classes write disjoint outputs, so the large-column class runs on
     // the caller's stream and the other on the plan's side stream at the same
     // time (the side stream waits for the work queued before, and the
@@ -991,14 +1035,15 @@ static int launch_hp(const rtx_plan *p, uint32_t ops, const void *dx, void *dy, 
     return RTX_OK;
 }
 
-// The column kernels on every column they take.
+// The column kernels on their columns: all they can take (all = 1) or the
+// default path's (0).
 int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
-                 int accumulate) {
+                 int accumulate, int all) {
     if (prec == RTX_PREC_F64)
-        return launch_hp<double, double, RTX_PREC_F64>(p, ops, dx, dy, st, accumulate);
+        return launch_hp<double, double, RTX_PREC_F64>(p, ops, dx, dy, st, accumulate, all);
     if (prec == RTX_PREC_F32)
-        return launch_hp<float, float, RTX_PREC_F32>(p, ops, dx, dy, st, accumulate);
-    return launch_hp<float, float, RTX_PREC_MIXED>(p, ops, dx, dy, st, accumulate);
+        return launch_hp<float, float, RTX_PREC_F32>(p, ops, dx, dy, st, accumulate, all);
+    return launch_hp<float, float, RTX_PREC_MIXED>(p, ops, dx, dy, st, accumulate, all);
 }
 
 }  // namespace rtx

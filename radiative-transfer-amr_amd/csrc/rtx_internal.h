@@ -141,14 +141,14 @@ struct HpTables {
 // spatial node, [14] column), so the kernel reads a column's scalars in one step
 constexpr int HP_HDR = 16;
 struct HpClass {
-    int n = 0;                      // columns
-    const int32_t *hdr = nullptr;   // their headers, in key order
+    int n[2] = {0, 0};              // columns: the default path's (the first ones), all
+    const int32_t *hdr = nullptr;   // their headers
     size_t bytes = 0;               // dynamic LDS per workgroup
 };
 bool alike_cell(const rtx_mesh_desc *d, int k, int32_t *src, int32_t *masked);
 int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d);
 int launch_hpcol(rtx_plan *p, uint32_t ops, int prec, const void *dx, void *dy, hipStream_t st,
-                 int accumulate);
+                 int accumulate, int all);
 
 constexpr int BJ_NCLS = 8;          // size classes of the block-Jacobi build
 constexpr int RTX_NBINS = 6;
@@ -213,8 +213,7 @@ struct rtx_plan {
     const int32_t *sc_all = nullptr, *sc_gen = nullptr;
     int n_sc_all = 0, n_sc_gen = 0;
     void *gen_alloc = nullptr;   // device lists of the generic set
-    // kernels of hp meshes: tables, LDS classes, and the columns they cannot
-    // take (run on the generic kernels, lists in hp_alloc)
+    // kernels of hp meshes: tables and LDS classes (lists in hp_alloc)
     bool hp_ok = false;
     bool hp_default = false;     // mode -1 uses the column kernel
     rtx::HpTables hp;
@@ -222,13 +221,15 @@ struct rtx_plan {
     // applies in FP64 arithmetic ([0] FP64 applies, [1] FP32 and mixed)
     rtx::HpClass hp_cls[3][rtx::HP_NCLS], hp_wide[2][rtx::HP_NCLS];
     int hp_ncols = 0;
-    // cells of those columns for k_hp_flux; the first hp_n_narrow are those of
-    // hp_cls in FP32 and mixed precision, the others those of hp_wide[1]
-    int hp_n_cells = 0, hp_n_narrow = 0;
+    // cells of those columns for k_hp_flux (the default path's, all); the first
+    // hp_n_narrow are those of hp_cls in FP32 and mixed precision, the others
+    // those of hp_wide[1]
+    int hp_n_cells[2] = {0, 0}, hp_n_narrow = 0;
     bool hp_alike = false;                  // alike neighbours are read directly
-    std::vector<int32_t> hp_over_cols;
-    const int32_t *hp_gen_cells = nullptr, *hp_gen_items = nullptr;
-    int hp_n_gen_cells = 0, hp_n_gen_items = 0;
+    // the columns beside them on the generic kernels: [0] the default path's
+    // (those it leaves out, too), [1] those the kernel cannot take
+    const int32_t *hp_gen_cells[2] = {}, *hp_gen_items[2] = {};
+    int hp_n_gen_cells[2] = {0, 0}, hp_n_gen_items[2] = {0, 0};
     void *hp_alloc = nullptr, *hp_es = nullptr;
     hipStream_t hp_side = nullptr;
     hipEvent_t hp_fork = nullptr, hp_join = nullptr;

@@ -586,3 +586,39 @@ def test_reduced_precision_of_wide_columns(cuda, case, path):
             err = _rel(op.apply(x, ops=ops, precision=prec).cpu().double().numpy()[keep], ref)
             print("  precision", prec, "error", err, "generic", generic, flush=True)
             assert err <= 1.05 * generic, (prec, err, generic)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nref_spt,expect", [((10, 9, 9), 1, "generic"), ((10, 9, 9), 4, "column"),
+                                               ((8, 7, 7), 1, "column"), ((8, 8, 8), 1, "generic"),
+                                               ((10, 10, 10), 2, "both")], ids=str)
+def test_default_path_of_long_columns(cuda, n, nref_spt, expect):
+    """Few columns that keep a workgroup long run the generic kernels by
+    default: bit for bit their results.  More than three for every four
+    CUs, and short ones at any number, run the column kernel.  A mesh of both
+    kinds (4 corner columns on the column kernel, 12 not) agrees with the
+    generic kernels to rounding (as check_column_kernels: TOL64, 7e-6), with
+    boundary rows and accumulation."""
+    import torch
+    from rtx.operator import (TransportOperator, OP_SYSTEM, OP_RESTRICT, OP_ACCUM, PREC_F64,
+                              PREC_F32)
+    mesh = problems.uniform_mesh([1.0, 1.0], list(n), 5 if n == (8, 8, 8) else 4, nref_spt,
+                                 pbcs=(n == (8, 8, 8),) * 2)
+    wl = problems.two_scatterers()
+    op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
+    print("long columns", n, "cols", op.t.ncol, "ndof", op.ndof, flush=True)
+    assert op.plan_info()["column_kernel_cols"] == op.t.ncol
+    x = _dev(np.random.default_rng(4).uniform(-1.0, 1.0, op.ndof))
+    y0 = torch.rand_like(x)
+    for prec, dt, tol in ((PREC_F64, torch.float64, TOL64), (PREC_F32, torch.float32, 7e-6)):
+        for ops in (OP_SYSTEM | OP_RESTRICT, OP_SYSTEM | OP_ACCUM):
+            out = {}
+            for path in (-1, 0, 3):
+                op.set_path(path)
+                out[path] = op.apply(x.to(dt), y0.to(dt).clone(), ops=ops, precision=prec)
+            if expect != "both":
+                assert torch.equal(out[-1], out[0 if expect == "generic" else 3])
+                assert not torch.equal(out[0], out[3])
+            else:
+                assert not torch.equal(out[-1], out[0]) and not torch.equal(out[-1], out[3])
+            assert float((out[-1] - out[0]).norm() / out[0].norm()) < tol
