@@ -6,10 +6,10 @@
 // neighbouring columns, projected onto a common node set) and the
 // projection integrals of src/dg/projection/cell_intg_xy.py:13-36 and
 // col_intg_th.py:13-37 that cell_hp_steer.py / col_hp_steer.py read.  The
-// reference walks every cell in Python; here one workgroup owns a column and
-// each of its wavefronts takes cells (or face pairs) of it; sums stay inside
-// a wavefront until a last step over the workgroup's wavefronts, always in
-// the same order.
+// reference walks every cell in Python; here a wavefront owns a cell (angular
+// jumps), or a workgroup a column and each of its wavefronts cells or face
+// pairs of it; sums stay inside a wavefront until a last step over the
+// workgroup's wavefronts, always in the same order.
 #include <type_traits>
 
 #include "rtx_internal.h"
@@ -19,6 +19,7 @@ namespace rtx {
 constexpr int INM = RTX_NMAX;
 constexpr int IWAVES = 8;
 constexpr int ITHREADS = 64 * IWAVES;
+constexpr int AWAVES = 4;           // cells per workgroup of the angular jumps
 
 // w2[s] = wx_i wy_j of the column's nodes s = i ny + j, to LDS.
 __device__ inline void node_weights(const DevMesh &m, int nx, int ny, double *w2) {
@@ -99,40 +100,65 @@ __global__ __launch_bounds__(ITHREADS) void k_moments(DevMesh m, const double *_
 // the cell and of its lower / upper neighbours in the column, and
 // err[k] = (1/4) sum_ij wx_i wy_j (1/2)((bot_k - top_lo)^2 + (top_k - bot_up)^2)
 // (error_angular_jump.py:36-81).  lend[(n 2 + s) INM + a] = l_a(2 s - 1) of
-// the n-point Gauss-Legendre basis.  A wavefront per cell, a lane per node:
-// 16,384 cells of 5 x 5 x 5 30 -> 14 us against a workgroup per cell.
-__global__ __launch_bounds__(ITHREADS) void k_angular_jump(DevMesh m, const double *__restrict__ u,
-                                                          const int32_t *__restrict__ nbr,
-                                                          const double *__restrict__ lend,
-                                                          double *__restrict__ err) {
-    __shared__ double w2[INM * INM];
-    const int c = blockIdx.x, lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// the n-point Gauss-Legendre basis.
+//
+// Bound by reading u three times (a cell and its two neighbours, mostly from
+// the cache).  A wavefront per cell of the mesh, a lane per node, so that
+// columns of many cells fill the chip as well as many columns do:
+// 16,384 cells of 5 x 5 x 5 in 1,024 columns 12 us, 1,024 cells of 10 x 10 x 10
+// in 16 columns 7.8 us (a workgroup per column of cells took 12 and 57 us, a
+// workgroup per cell 28 and 8.3 us).
+__global__ __launch_bounds__(64 * AWAVES) void k_angular_jump(DevMesh m, const double *__restrict__ u,
+                                                             const int32_t *__restrict__ nbr,
+                                                             const double *__restrict__ lend,
+                                                             double *__restrict__ err) {
+    const int lane = threadIdx.x & 63;
+    // workgroups go to the 8 XCDs round-robin; XCD j takes the j-th eighth of
+    // the cells, so a cell's neighbours are read through the same L2
+    const int blk = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+    const int k = blk * AWAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (k >= m.ncell) return;
+    const int c = m.cell_col[k];
     const int nx = m.col_nx[c], ny = m.col_ny[c], nsp = nx * ny;
-    node_weights(m, nx, ny, w2);
-    const int k1 = m.col_cell_start[c + 1];
-    for (int k = m.col_cell_start[c] + wave; k < k1; k += IWAVES) {
-        const int lo = nbr[2 * k], up = nbr[2 * k + 1];
-        const int nt = m.cell_nth[k], ntl = m.cell_nth[lo], ntu = m.cell_nth[up];
-        const double *uk = u + m.cell_dof_off[k], *ul = u + m.cell_dof_off[lo],
-                     *uu = u + m.cell_dof_off[up];
-        const double *bot_k = lend + (nt * 2 + 0) * INM, *top_k = lend + (nt * 2 + 1) * INM;
-        const double *top_l = lend + (ntl * 2 + 1) * INM, *bot_u = lend + (ntu * 2 + 0) * INM;
-        double acc = 0.0;
-        for (int s = lane; s < nsp; s += 64) {
-            double b0 = 0.0, t0 = 0.0, tl = 0.0, bu = 0.0;
-            for (int a = 0; a < nt; ++a) {
-                b0 += uk[s * nt + a] * bot_k[a];
-                t0 += uk[s * nt + a] * top_k[a];
+    const int lo = nbr[2 * k], up = nbr[2 * k + 1];
+    const int nt = m.cell_nth[k], ntl = m.cell_nth[lo], ntu = m.cell_nth[up];
+    const double *uk = u + m.cell_dof_off[k], *ul = u + m.cell_dof_off[lo],
+                 *uu = u + m.cell_dof_off[up];
+    const double *bot_k = lend + (nt * 2 + 0) * INM, *top_k = lend + (nt * 2 + 1) * INM;
+    const double *top_l = lend + (ntl * 2 + 1) * INM, *bot_u = lend + (ntu * 2 + 0) * INM;
+    const double *wx = m.lgl_w + nx * INM, *wy = m.lgl_w + ny * INM;
+    double acc = 0.0;
+    // Q nodes per lane, side by side; past the last node that node again
+    const auto nodes = [&](auto per_lane) {
+        constexpr int Q = decltype(per_lane)::value;
+        int at[Q];
+        double b0[Q] = {}, t0[Q] = {}, tl[Q] = {}, bu[Q] = {};
+#pragma unroll
+        for (int q = 0; q < Q; ++q) at[q] = min(lane + 64 * q, nsp - 1);
+        for (int a = 0; a < nt; ++a)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const double v = uk[at[q] * nt + a];
+                b0[q] += v * bot_k[a];
+                t0[q] += v * top_k[a];
             }
-            for (int a = 0; a < ntl; ++a) tl += ul[s * ntl + a] * top_l[a];
-            for (int a = 0; a < ntu; ++a) bu += uu[s * ntu + a] * bot_u[a];
-            const double jl = (b0 - tl) * (b0 - tl), ju = (t0 - bu) * (t0 - bu);
-            acc += w2[s] * 0.5 * (jl + ju);
+        for (int a = 0; a < ntl; ++a)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) tl[q] += ul[at[q] * ntl + a] * top_l[a];
+        for (int a = 0; a < ntu; ++a)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) bu[q] += uu[at[q] * ntu + a] * bot_u[a];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const double jl = (b0[q] - tl[q]) * (b0[q] - tl[q]), ju = (t0[q] - bu[q]) * (t0[q] - bu[q]);
+            if (lane + 64 * q < nsp) acc += wx[at[q] / ny] * wy[at[q] % ny] * 0.5 * (jl + ju);
         }
-        acc = wave_sum(acc);
-        if (lane == 0) err[k] = 0.25 * acc;
-    }
+    };
+    static_assert(INM * INM <= 128, "two nodes per lane cover a column");
+    if (nsp <= 64) nodes(std::integral_constant<int, 1>());
+    else nodes(std::integral_constant<int, 2>());
+    acc = wave_sum(acc);
+    if (lane == 0) err[k] = 0.25 * acc;
 }
 
 // One side of a face pair, U[b][r] = sum_t psi[t][b] sum_a h[t][a] xsi[a][r],
@@ -282,7 +308,8 @@ extern "C" int rtx_error_angular_jump(rtx_plan *p, const double *d_u, const int3
     RTX_CHECK(p && d_u && d_nbr && d_lend && d_cell_err, "rtx_error_angular_jump: null argument");
     if (int rc = check_cells(p, "rtx_error_angular_jump")) return rc;
     if (p->m.ncell == 0) return RTX_OK;
-    k_angular_jump<<<p->m.ncol, ITHREADS, 0, static_cast<hipStream_t>(stream)>>>(
+    const int nblk = (p->m.ncell + AWAVES - 1) / AWAVES;
+    k_angular_jump<<<(nblk + 7) / 8 * 8, 64 * AWAVES, 0, static_cast<hipStream_t>(stream)>>>(
         p->m, d_u, d_nbr, d_lend, d_cell_err);
     RTX_HIP(hipGetLastError());
     return RTX_OK;

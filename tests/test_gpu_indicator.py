@@ -227,3 +227,24 @@ def test_error_measures_at_tile_edges(cuda, n):
     dev = ev.cell_errors(u, ev.hr_values(wave))
     ref = np.array([e for _, _, e in oerr.cell_errors(mesh, u, wave)])
     assert np.max(np.abs(dev - ref)) <= TOL * np.max(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nref_ang,nref_spt", [((3, 3, 2), 5, 1), ((2, 4, 3), 2, 0),
+                                                 ((10, 9, 3), 3, 1), ((8, 8, 4), 2, 1)], ids=str)
+def test_angular_jump_across_columns(cuda, n, nref_ang, nref_spt):
+    """Cell counts that end inside a workgroup and columns that begin inside
+    one, on both sides of one node per lane (64), with cells of unlike angles
+    side by side (bound: see test_error_measures_at_tile_edges)."""
+    from rtx.error import ErrorEvaluator
+    mesh = problems.uniform_mesh([1.0, 1.0], list(n), nref_ang, nref_spt)
+    keys = sorted(mesh.cols)
+    for i, key in enumerate(keys):
+        cells = sorted(mesh.cols[key].cells)
+        mesh.ref_cell(key, cells[i % len(cells)], "h")
+    mesh.ref_cell(keys[0], sorted(mesh.cols[keys[0]].cells)[-1], "p")
+    ev = ErrorEvaluator(mesh)
+    print("angular jumps", n, "cells", ev.t.ncell, flush=True)
+    u = np.random.default_rng(8).uniform(-1, 1, ev.t.ndof)
+    ang, ref = ev.angular_jump(u), oind.angular_jump(mesh, u)
+    assert all(_close(ang[k], ref[key]) for k, key in enumerate(ev.t.cell_keys))
