@@ -24,11 +24,13 @@ struct ErrCell {
     const double *Px, *Py, *Pt, *wx, *wy, *wt;  // n x m matrices, m weights
 };
 
-// Sums over this lane's target nodes of w (u_hr - I u)^2 (and w u_hr^2).
+// Sums over this lane's target nodes of w (u_hr - I u)^2 (and w u_hr^2), of the
+// target x-planes p0, p0 + step, ..
 // IM >= max(nx, ny, nt): loads without branches (indices past a size read its
 // last entry, and u is zero there, so the rows and terms past the sizes are).
 template <bool NODAL, int IM>
-__device__ inline void error_cell(const ErrCell &c, int l16, int lg, double &acc, double &acc2) {
+__device__ inline void error_cell(const ErrCell &c, int l16, int lg, int p0, int step, double &acc,
+                                  double &acc2) {
     constexpr int KS = (IM + 3) / 4;            // K steps of four
     double pt[KS], py[KS], uv[IM][KS];
     const int r = min(l16, c.mt - 1), qr = min(l16, c.my - 1), jr = min(l16, c.ny - 1);
@@ -70,9 +72,9 @@ __device__ inline void error_cell(const ErrCell &c, int l16, int lg, double &acc
         for (int v = 0; v < 4; ++v)
             if (4 * v < c.my) o[v] = c.hr[min(p, c.mx - 1) * c.my * c.mt + off[v]];
     };
-    hr_load(0, hv);
-    for (int p = 0; p < c.mx; ++p) {
-        hr_load(p + 1, hn);
+    hr_load(p0, hv);
+    for (int p = p0; p < c.mx; p += step) {
+        hr_load(p + step, hn);
         double px[IM];
 #pragma unroll
         for (int i = 0; i < IM; ++i) px[i] = c.Px[min(i, c.nx - 1) * c.mx + p];   // uniform
@@ -103,16 +105,21 @@ __device__ inline void error_cell(const ErrCell &c, int l16, int lg, double &acc
 // Bound by reading u_hr (512 values of a cell of 5 x 5 x 5).  One wavefront
 // per cell and no LDS: the workgroup of 256 threads with the three products
 // in LDS spent the time on barriers and on index divisions.  16,384 such
-// cells (84 MB): 128 -> 59 us.  (Px one plane
-// ahead as well spills scalar registers: 62 us.)
-template <bool NODAL>
+// cells (84 MB): 122 -> 57 us.  (Px one plane ahead as well spills scalar
+// registers: 3 us more.)
+//
+// WPC wavefronts per cell, 1 or EWAVES: each contracts the cell and takes every
+// WPC-th of its target x-planes.
+template <bool NODAL, int WPC>
 __global__ __launch_bounds__(64 * EWAVES) __attribute__((amdgpu_waves_per_eu(4)))
 void k_error_l2(DevMesh m, const double *__restrict__ uh, const double *__restrict__ u_hr,
                 const int64_t *__restrict__ hr_off, const int32_t *__restrict__ hr_dims,
                 const double *__restrict__ tab, double *__restrict__ cell_err,
                 double *__restrict__ hr_norm2) {
     const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
-    const int k = blockIdx.x * EWAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int k = WPC == 1 ? blockIdx.x * EWAVES + wave : blockIdx.x;
+    const int p0 = WPC == 1 ? 0 : wave;
     if (k >= m.ncell) return;
     const int c = m.cell_col[k];
     ErrCell e;
@@ -136,18 +143,54 @@ void k_error_l2(DevMesh m, const double *__restrict__ uh, const double *__restri
     double acc = 0.0, acc2 = 0.0;
     // the smallest of three unrolled sizes (one, two or three K steps)
     const int n = max(max(e.nx, e.ny), e.nt);
-    if (n <= 4) error_cell<NODAL, 4>(e, l16, lg, acc, acc2);
-    else if (n <= 7) error_cell<NODAL, 7>(e, l16, lg, acc, acc2);
-    else error_cell<NODAL, ENM>(e, l16, lg, acc, acc2);
+    if (n <= 4) error_cell<NODAL, 4>(e, l16, lg, p0, WPC, acc, acc2);
+    else if (n <= 7) error_cell<NODAL, 7>(e, l16, lg, p0, WPC, acc, acc2);
+    else error_cell<NODAL, ENM>(e, l16, lg, p0, WPC, acc, acc2);
     const double dx = m.col_geom[4 * c + 2] - m.col_geom[4 * c + 0];
     const double dy = m.col_geom[4 * c + 3] - m.col_geom[4 * c + 1];
     const double dth = m.cell_geom[2 * k + 1] - m.cell_geom[2 * k + 0];
     acc = wave_sum(acc);
-    if (lane == 0) cell_err[k] = dx * dy * dth / 8.0 * acc;
-    if (NODAL) {
-        acc2 = wave_sum(acc2);
-        if (lane == 0) hr_norm2[k] = dx * dy * dth / 8.0 * acc2;
+    if (NODAL) acc2 = wave_sum(acc2);
+    if constexpr (WPC > 1) {
+        __shared__ double part[2][WPC];
+        if (lane == 0) {
+            part[0][wave] = acc;
+            part[1][wave] = acc2;
+        }
+        __syncthreads();
+        acc = acc2 = 0.0;
+#pragma unroll
+        for (int w = 0; w < WPC; ++w) {
+            acc += part[0][w];
+            acc2 += part[1][w];
+        }
+        if (wave != 0) return;
     }
+    if (lane == 0) {
+        cell_err[k] = dx * dy * dth / 8.0 * acc;
+        if (NODAL) hr_norm2[k] = dx * dy * dth / 8.0 * acc2;
+    }
+}
+
+// A cell's wavefronts wait for its values, so few cells are a chain of one
+// wavefront's target planes: up to two cells per CU they are shared by EWAVES
+// wavefronts.  256 cells of 5 x 5 x 5 8.4 -> 6.5 us, of 8 x 8 x 8 12.1 -> 8.8,
+// 512 of 10 x 10 x 10 14.8 -> 13.0, of 5 x 5 x 5 8.4 either way; from 1,024 cells
+// on (8.7, 13.1 and 16.1 us) one wavefront per cell fills the chip.
+template <bool NODAL>
+static int launch_error(const rtx_plan *p, const double *uh, const double *u_hr,
+                        const int64_t *hr_off, const int32_t *hr_dims, const double *tab,
+                        double *cell_err, double *hr_norm2, void *stream) {
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    const int ncell = p->m.ncell;
+    if (ncell <= 2 * p->n_cu)
+        k_error_l2<NODAL, EWAVES><<<ncell, 64 * EWAVES, 0, st>>>(p->m, uh, u_hr, hr_off, hr_dims,
+                                                                 tab, cell_err, hr_norm2);
+    else
+        k_error_l2<NODAL, 1><<<(ncell + EWAVES - 1) / EWAVES, 64 * EWAVES, 0, st>>>(
+            p->m, uh, u_hr, hr_off, hr_dims, tab, cell_err, hr_norm2);
+    RTX_HIP(hipGetLastError());
+    return RTX_OK;
 }
 
 }  // namespace rtx
@@ -161,11 +204,8 @@ extern "C" int rtx_error_l2(rtx_plan *p, const double *d_uh, const double *d_u_h
               "rtx_error_l2: null argument");
     RTX_CHECK(p->max_cell_ndof <= ENM * ENM * ENM, "rtx_error_l2: cell too large");
     if (p->m.ncell == 0) return RTX_OK;
-    const int nblk = (p->m.ncell + EWAVES - 1) / EWAVES;
-    k_error_l2<false><<<nblk, 64 * EWAVES, 0, static_cast<hipStream_t>(stream)>>>(
-        p->m, d_uh, d_u_hr, d_hr_off, nullptr, d_tab, d_cell_err, nullptr);
-    RTX_HIP(hipGetLastError());
-    return RTX_OK;
+    return launch_error<false>(p, d_uh, d_u_hr, d_hr_off, nullptr, d_tab, d_cell_err, nullptr,
+                               stream);
 }
 
 extern "C" int rtx_error_l2_nodal(rtx_plan *p, const double *d_uh, const double *d_u_hr,
@@ -176,9 +216,6 @@ extern "C" int rtx_error_l2_nodal(rtx_plan *p, const double *d_uh, const double 
               "rtx_error_l2_nodal: null argument");
     RTX_CHECK(p->max_cell_ndof <= ENM * ENM * ENM, "rtx_error_l2_nodal: cell too large");
     if (p->m.ncell == 0) return RTX_OK;
-    const int nblk = (p->m.ncell + EWAVES - 1) / EWAVES;
-    k_error_l2<true><<<nblk, 64 * EWAVES, 0, static_cast<hipStream_t>(stream)>>>(
-        p->m, d_uh, d_u_hr, d_hr_off, d_hr_dims, d_tab, d_cell_err, d_hr_norm2);
-    RTX_HIP(hipGetLastError());
-    return RTX_OK;
+    return launch_error<true>(p, d_uh, d_u_hr, d_hr_off, d_hr_dims, d_tab, d_cell_err, d_hr_norm2,
+                              stream);
 }

@@ -248,3 +248,39 @@ def test_angular_jump_across_columns(cuda, n, nref_ang, nref_spt):
     u = np.random.default_rng(8).uniform(-1, 1, ev.t.ndof)
     ang, ref = ev.angular_jump(u), oind.angular_jump(mesh, u)
     assert all(_close(ang[k], ref[key]) for k, key in enumerate(ev.t.cell_keys))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nref_spt", [((2, 3, 2), 1), ((4, 3, 4), 1), ((2, 2, 2), 3),
+                                        ((4, 4, 3), 3)], ids=str)
+def test_error_l2_few_and_many_cells(cuda, n, nref_spt):
+    """The L2 errors with a cell shared by the wavefronts of a workgroup (few
+    cells: 35) and with one wavefront per cell (more than two cells per CU:
+    515), target planes that do not divide among the wavefronts included
+    (bound: see test_error_measures_at_tile_edges)."""
+    from oracle import error as oerr
+    from rtx.error import ErrorEvaluator
+    from rtx.plan import MeshTables
+
+    def make(p):
+        mesh = problems.uniform_mesh([1.0, 1.0], list(n), 3, nref_spt)
+        key = sorted(mesh.cols)[0]
+        for cell in sorted(mesh.cols[key].cells)[:3]:
+            mesh.ref_cell(key, cell, "h")
+        if p:
+            mesh.ref_mesh(kind="ang", form="p")
+            mesh.ref_mesh(kind="spt", form="p")
+        return mesh
+    mesh, mesh_hr = make(False), make(True)
+    ev, t_hr = ErrorEvaluator(mesh), MeshTables(mesh_hr)
+    print("L2 errors", n, "cells", ev.t.ncell, flush=True)
+    rng = np.random.default_rng(9)
+    u, u_hr = rng.uniform(-1, 1, ev.t.ndof), rng.uniform(-1, 1, t_hr.ndof)
+    err, hr2 = ev.nodal_errors(u, u_hr, t_hr)
+    ref, intg = oind.high_resolution(mesh, u, mesh_hr, u_hr)
+    assert all(_close(err[k], ref[key]) for k, key in enumerate(ev.t.cell_keys))
+    assert _close(float(np.sum(hr2)), intg)
+    wave = lambda x, y, a: np.cos(3.0 * x) * np.sin(2.0 * y + 1.0) * (1.5 + np.cos(a))
+    dev = ev.cell_errors(u, ev.hr_values(wave))
+    ref = np.array([e for _, _, e in oerr.cell_errors(mesh, u, wave)])
+    assert np.max(np.abs(dev - ref)) <= TOL * np.max(ref)
