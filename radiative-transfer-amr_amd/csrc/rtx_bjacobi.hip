@@ -368,9 +368,9 @@ __device__ inline uint32_t bj_key(double v) {
     return static_cast<uint32_t>(__double2hiint(v)) & 0x7fffff80u;
 }
 __device__ inline uint32_t bj_key(float v) { return __float_as_uint(v) & 0x7fffff80u; }
-// keys of infinities and NaN start here
+// keys of NaN start here
 template <typename T>
-__device__ constexpr uint32_t bj_key_inf() { return sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u; }
+__device__ constexpr uint32_t bj_key_nan() { return sizeof(T) == 8 ? 0x7ff00080u : 0x7f800080u; }
 
 __device__ inline double bj_lane(double v, int lane) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
@@ -420,20 +420,23 @@ __device__ inline void bj_wave_sync() {
 }
 
 // 1 / p to an ulp (hardware reciprocal and Newton steps): a pivot's relative
-// perturbation of that size is one rounding of the elimination.
+// perturbation of that size is one rounding of the elimination.  0 for an
+// infinite p (where a Newton step gives NaN).
 __device__ inline double bj_recip(double p) {
-    double r = __builtin_amdgcn_rcp(p);
-    r = fma(fma(-p, r, 1.0), r, r);
-    return fma(fma(-p, r, 1.0), r, r);
+    const double r = __builtin_amdgcn_rcp(p);
+    double q = fma(fma(-p, r, 1.0), r, r);
+    q = fma(fma(-p, q, 1.0), q, q);
+    return r == 0.0 ? 0.0 : q;
 }
 __device__ inline float bj_recip(float p) {
     const float r = __builtin_amdgcn_rcpf(p);
-    return fmaf(fmaf(-p, r, 1.f), r, r);
+    const float q = fmaf(fmaf(-p, r, 1.f), r, r);
+    return r == 0.f ? 0.f : q;
 }
 
 // Sweep the 16 columns of a panel held one row (H rows, 64 apart) per lane.
 // q: byte table of the step that each row was pivot of (BJMma::slot order);
-// perm: pivot row of each step.  False on a zero or non-finite pivot (the
+// perm: pivot row of each step.  False on a zero or NaN pivot (the
 // same for every lane; what the panel holds then is void).
 template <int H, typename T>
 __device__ __forceinline__ bool bj_panel(T (&P0)[16], T (&P1)[16], int k0, int lane, bool used0,
@@ -458,7 +461,7 @@ __device__ __forceinline__ bool bj_panel(T (&P0)[16], T (&P1)[16], int k0, int l
             key = v > key ? v : key;
         }
         key = bj_wave_max(key);
-        bad |= key < 0x80u || key >= bj_key_inf<T>();
+        bad |= key < 0x80u || key >= bj_key_nan<T>();
         const int pr = 127 - int(key & 127u), pl = pr & 63;
         const bool low = H == 1 || pr < 64;
         T row[16];

@@ -104,6 +104,37 @@ def test_nonfinite_coefficient_is_a_singular_block(cuda):
 
 
 @pytest.mark.gpu
+def test_infinite_absorption_has_a_zero_inverse(cuda):
+    """An infinite absorption in one column is no singular block: an infinite
+    pivot's inverse is zero, so the inverses of that column's cells are zero but
+    for the identity on masked DOFs, and the other cells' are those without it."""
+    import ctypes as C
+    import torch
+    from rtx._lib import check, ptr
+    from rtx.krylov import BlockJacobi
+    from rtx.operator import TransportOperator
+    mesh, wl = _c1_small()
+    op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
+    t = op.t
+    k1 = int(t.col_cell_start[1])
+    n = int(t.col_nx[0] * t.col_ny[0] * t.cell_nth[0])
+    assert list(t.col_geom[0]) == [0.0, 0.0, 0.25, 0.25] and n == 64
+    free = op.mask(torch.ones(op.ndof, dtype=torch.float64, device="cuda"))[:k1 * n].cpu().numpy()
+    want = [BlockJacobi(op).inv, BlockJacobi(op, keep_f64=False, keep_f32=True).inv32]
+    kap = t.eval_spatial(wl.kappa)
+    kap[:int(t.col_nx[0] * t.col_ny[0])] = np.inf
+    check(op.lib.rtx_plan_set_coeffs(op.plan, t.nsp, ptr(kap, C.c_double),
+                                     ptr(op.sigma_nodes, C.c_double), op.G_pool.size,
+                                     ptr(op.G_pool, C.c_double)), "set_coeffs")
+    got = [BlockJacobi(op).inv, BlockJacobi(op, keep_f64=False, keep_f32=True).inv32]
+    for g, w in zip(got, want):
+        assert torch.equal(g[k1 * n * n:], w[k1 * n * n:])
+        g = g[:k1 * n * n].cpu().numpy().reshape(k1, n, n)
+        for k in range(k1):
+            assert np.array_equal(g[k], np.diag(1.0 - free[k * n:(k + 1) * n]))
+
+
+@pytest.mark.gpu
 def test_kaczmarz_is_reported_not_silent(cuda):
     from rt.problem import KaczmarzSubstituted
     mesh, wl = _c1_small()
