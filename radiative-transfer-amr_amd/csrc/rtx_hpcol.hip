@@ -759,11 +759,13 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
     std::vector<int32_t> hdr[3][HP_NCLS], wide[2][HP_NCLS], over, links;
     std::vector<HpCell> cells, wide_cells;
     p->hp_ncols = 0;
-    // Neighbours are read directly where at least a quarter of the cells have
-    // alike ones.  The kernel that does so holds more registers: with no such
-    // cell it takes 5 % longer (an hp mesh in FP64, 227 -> 239 us), with
-    // nothing else it saves the face kernel (1,024 columns of 7 x 7 nodes in
-    // FP32 35 -> 29 us, 256 columns of 3 x 5 nodes in FP64 12.4 -> 8.7 us).
+    // Neighbours are read directly where at least half of the cells have alike
+    // ones.  The kernel that does so holds more registers: with no such cell it
+    // takes 3 to 6 % longer (an hp mesh in FP64, 208 -> 221 us), with nothing else
+    // it saves the face kernel (1,024 columns of 5 x 5 nodes and 40 angles FP64 29
+    // -> 21 us, FP32 25 -> 20).  That mesh with columns p-refined: 69 % alike 29.4
+    // -> 26.7 and 25.7 -> 24.6 us, 50 % 29.8 -> 28.2 and 25.9 -> 26.0, 36 % 29.9 ->
+    // 29.2 and 26.1 -> 27.7, 28 % 30.1 -> 30.4 and 26.3 -> 28.5.
     std::vector<int32_t> cell_src(size_t(2) * d->ncell), cell_mask(d->ncell);
     std::vector<char> direct(d->ncell);
     int64_t ndirect = 0;
@@ -771,7 +773,7 @@ int hpcol_build(rtx_plan *p, const rtx_mesh_desc *d) {
         direct[k] = alike_cell(d, k, &cell_src[size_t(2) * k], &cell_mask[k]);
         ndirect += direct[k];
     }
-    p->hp_alike = 4 * ndirect >= d->ncell;
+    p->hp_alike = 2 * ndirect >= d->ncell;
     if (!p->hp_alike) std::fill(direct.begin(), direct.end(), char(0));
     // A workgroup works a column off alone, so few columns that need long leave
     // the chip idle, and the generic kernels spread them better.  Where they
