@@ -351,9 +351,10 @@ __device__ inline double bj_entry(const DevMesh &m, const BJCell &x, const BJSel
 // FP32 (this: 6.9).  One barrier per panel is left; the next panel's wave
 // starts as soon as its own tile is updated (W is double-buffered), at raised
 // priority because the panels are the serial chain.  Registers: two blocks of
-// eight waves per CU in FP64 (128 VGPRs); in FP32 four (64 VGPRs with a few
-// spills: 16,384 blocks of 125 in 1.83 ms, against 2.0 at 80 VGPRs and 2.5
-// without a limit, before the assembly's index tables took it to 1.68).
+// eight waves per CU in FP64 (128 VGPRs); in FP32 four (64 VGPRs with 2 to 15
+// spilled, 43 where NT is 6 and the inverse is stored: 16,384 blocks of 125 in
+// 1.83 ms, against 2.0 at 80 VGPRs and 2.5 without a limit, before the
+// assembly's index tables took it to 1.68).  Measured at NT = 8 alone.
 template <int NT, typename T>
 struct BJReg {
     static constexpr int NR = 16 * NT;

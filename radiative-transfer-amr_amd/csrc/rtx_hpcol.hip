@@ -23,7 +23,8 @@
 //              values of x times the (then diagonal) coupling; stores y.
 //
 // The two share no workspace: y itself carries the face sums from one to the
-// other, so concurrent applies on several streams stay independent.
+// other.  The plan's side stream and its two events are shared by all applies, so
+// a plan serves one stream at a time.
 //
 // The nodes are the rows of the scattering product in an order of our own: a
 // lane's accumulators are whole lines of nodes (x-lines q = lane group,
@@ -65,8 +66,9 @@ __device__ inline bool hp_on_bdry(int bd, int i, int j, int nx, int ny) {
            ((bd & 8) && j == 0);
 }
 
-// floor(v / n) for 0 <= v < 2^16 and 1 <= n <= 16, by a float product: the
-// quotient's fractional part stays >= 0.5 / n away from an integer.
+// floor(v / n) for 0 <= v < 2^16 and 1 <= n <= 100, by a float product: (v + 0.5)
+// / n stays 0.5 / n away from an integer, and the product is off by at most
+// 2^-22 of itself, 2^-6 / n.
 __device__ inline int hp_div(int v, float rcp) { return int((float(v) + 0.5f) * rcp); }
 
 __device__ inline uint16_t hp_bf16(float f) {

@@ -196,10 +196,6 @@ struct rtx_plan {
     // none) and the masked end nodes
     const int4 *uni_src = nullptr;
     void *uni_alloc = nullptr;
-    // largest own-DOF count and own-trace count of a column part when the
-    // fused kernel splits every column into H = 1, 2, 4 cell ranges
-    int32_t max_part_dofs[5] = {0, 0, 0, 0, 0}, max_part_trace[5] = {0, 0, 0, 0, 0};
-    int32_t max_part_links[5] = {0, 0, 0, 0, 0};
     int fused_mode = -1;   // -1 auto, 0 generic kernels, 1 fused per-column kernel
     // order bins of the apply (non-uniform meshes): fused-kernel bins by part
     // count, and the columns (and their cells) left to the generic kernels

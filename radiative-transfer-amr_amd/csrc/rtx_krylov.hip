@@ -562,12 +562,6 @@ extern "C" int rtx_arnoldi_workspace(int max_vecs, int64_t *n_doubles) {
     return RTX_OK;
 }
 
-/* One Arnoldi step: orthogonalise w against V_0..V_{nv-1} (columns of length n,
-   stride ld) by classical Gram-Schmidt; refine 0: one pass, 1: a second pass
-   when the norm dropped by more than the "twice is enough" factor, 2: always
-   two passes; normalise into V_nv and write the Hessenberg column
-   h_0..h_{nv-1}, h_nv = |w| to d_hcol (device, nv + 1 doubles).  w is
-   overwritten.  Everything is enqueued on `stream`; no host sync. */
 template <typename T>
 static bool aligned16(const T *p) {
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0;

@@ -312,22 +312,6 @@ extern "C" int rtx_plan_create(const rtx_mesh_desc *d, rtx_plan **out) {
     for (int c = 0; c < nc; ++c) {
         const int k0 = d->col_cell_start[c], k1 = d->col_cell_start[c + 1], ncl = k1 - k0;
         if (ncl < p->min_col_cells) p->min_col_cells = ncl;
-        const int nsp = d->col_nx[c] * d->col_ny[c];
-        for (int H : {1, 2, 4}) {
-            for (int h = 0; h < H; ++h) {
-                const int lo = k0 + (h * ncl) / H, hi = k0 + ((h + 1) * ncl) / H;
-                int dofs = 0, tr = 0;
-                for (int k = lo; k < hi; ++k) dofs += nsp * d->cell_nth[k];
-                const int l0 = d->link_start[lo], l1 = d->link_start[hi];
-                for (int l = l0; l < l1; ++l) {
-                    const int s = d->link_src[l], F = d->link_face[l], c1 = d->cell_col[s];
-                    tr += ((F & 1) ? d->col_nx[c1] : d->col_ny[c1]) * d->cell_nth[s];
-                }
-                if (dofs > p->max_part_dofs[H]) p->max_part_dofs[H] = dofs;
-                if (tr > p->max_part_trace[H]) p->max_part_trace[H] = tr;
-                if (l1 - l0 > p->max_part_links[H]) p->max_part_links[H] = l1 - l0;
-            }
-        }
     }
     // Order bins: every column goes to the fused kernel with the smallest
     // part count H whose part fits 32 KB of LDS (else the smallest within the

@@ -113,7 +113,7 @@ void k_uniform(DevMesh m, uint32_t ops, int accumulate, const int4 *__restrict__
                const T *__restrict__ x, T *__restrict__ y) {
     constexpr int NSP = N * N, NA = NC * NTH, NCD = NSP * NA, CD = NSP * NTH;
     constexpr int OC = NC / H;                 // cells per part
-    constexpr int NOWN = OC * CD, NOA = OC * NTH;
+    constexpr int NOA = OC * NTH;
     constexpr int MT = (NSP + 15) / 16;
     constexpr int NTILE = (NOA + 15) / 16;     // output-angle tiles of the part
     constexpr int NKS = (NA + 3) / 4;          // f64/f32 k-steps
@@ -506,16 +506,17 @@ constexpr int ue_waves() {
 // output computed where the scattering MFMA leaves it: lane (l16, lg) of wave
 // w owns output angle R = 16 w + l16 and the nodes of its accumulator rows,
 // and adds to the MFMA result the mass, convection, outflow and inflow-face
-// terms of those (node, angle) outputs in the order k_uniform adds them (so
-// the two kernels agree bit for bit).  No output tile in LDS: the column
-// tile, the traces and the flux slots are all the LDS it needs, so more
-// columns are resident per CU (C2: 34 KB, four per CU, every column of the
-// mesh in one round).  The outputs go through the dead column tile for a
-// coalesced store.
+// terms of those (node, angle) outputs in the order k_uniform adds them.  The
+// two agree to rounding: here the inflow is the neighbours' traces contracted
+// with E^s and E^theta, there its diagonal alone.  No output tile in LDS: the
+// column tile, the traces and the flux slots are all the LDS it needs, so more
+// columns are resident per CU (5 x 5 x 80: 34 KB, four per CU, 1,024 columns in
+// one round).  The outputs go through the dead column tile for a coalesced
+// store.
 template <typename T, typename A, int PREC, int N, int NTH, int NC,
           int ETHREADS = 64 * ue_waves<NTH, NC>()>
 // at least as many waves per SIMD as the workgroup has waves: four columns
-// per CU (C2: 5 waves per SIMD, at most 102 VGPRs)
+// per CU (5 x 5 x 80: 5 waves per SIMD, at most 102 VGPRs)
 __global__ __launch_bounds__(ETHREADS, ETHREADS / 64) void k_uniform_e(DevMesh m, uint32_t ops, int accumulate,
                                                         const T *__restrict__ x,
                                                         T *__restrict__ y, int nlink_lds) {
@@ -785,7 +786,8 @@ __global__ __launch_bounds__(ETHREADS, ETHREADS / 64) void k_uniform_e(DevMesh m
     if (MFMA_FIRST && scat_w) scatter();
 
     // ---- upwind inflow couplings, one (link, face node, angle) per thread,
-    // into a flux slot of its own (as k_uniform's phase 3)
+    // into a flux slot of its own; a DOF's slots are added below in a fixed
+    // order (its cell has at most one x-face and one y-face link)
     if (bconv) {
         const int f0 = tid < TS ? tid : MAXL * TRL;
         const int le = f0 % TRL, m0 = le / NTH, r = le % NTH;
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(ETHREADS, ETHREADS / 64) void k_uniform_e(DevMesh m
 
     // ---- every term of this lane's outputs, in k_uniform's order: mass,
     // x-derivative, outflow faces (phase 2 x-lines), y-derivative (y-lines),
-    // scattering (phase 4), inflow faces x then y (phase 5)
+    // scattering (phase 3), inflow faces x then y (phase 4)
     A outv[MT][4];
     if (wave < NTILE) {
         const int Rc = rok ? R : NA - 1;
@@ -919,18 +921,18 @@ int launch_e(rtx_plan *p, uint32_t ops, const void *dx, void *dy, hipStream_t st
     constexpr int NSP = N * N, NA = NC * NTH;
     constexpr int NAP = u_pad(NA, NTH);
     constexpr int MAXL = 4 * NC, TRL = N * NTH;
-    RTX_CHECK(p->max_part_links[1] <= MAXL, "uniform apply: %d links in a column (max %d)",
-              p->max_part_links[1], MAXL);
+    RTX_CHECK(p->max_col_links <= MAXL, "uniform apply: %d links in a column (max %d)",
+              p->max_col_links, MAXL);
     constexpr bool XB = PREC == RTX_PREC_MIXED;
     const size_t tiles = XB ? u_bf_off(size_t(NSP * NAP) * sizeof(A)) + u_bf_bytes(NSP, NA)
                             : size_t(NSP * NAP) * sizeof(A);
-    const size_t lds = tiles + size_t(2 * p->max_part_links[1] * TRL) * sizeof(A);
+    const size_t lds = tiles + size_t(2 * p->max_col_links * TRL) * sizeof(A);
     auto kern = k_uniform_e<T, A, PREC, N, NTH, NC>;
     RTX_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 int(lds)));
     const int nblocks = ((p->m.ncol + UXCD - 1) / UXCD) * UXCD;
     kern<<<nblocks, 64 * ue_waves<NTH, NC>(), lds, st>>>(p->m, ops, acc, (const T *)dx, (T *)dy,
-                                                         p->max_part_links[1]);
+                                                         p->max_col_links);
     RTX_HIP(hipGetLastError());
     return RTX_OK;
 }
