@@ -1,16 +1,20 @@
 """CPU model of the uniform-bin apply kernel's index arithmetic (test-only).
 
 Restates the compile-time shapes of ``csrc/rtx_uniform.hip`` (threads per
-workgroup, LDS row strides, whole-cell DOF passes, trace and flux-slot
-passes, phase-2 line mapping) for every compiled order bin and part count,
-and checks the properties the kernel relies on: every DOF, trace slot and
-line is visited exactly once, every LDS index stays inside its tile, and
-lanes walking a cell's DOFs in order hit distinct LDS banks (32 banks of
-4 bytes; 8-byte elements).
+workgroup, LDS row strides, whole-cell DOF passes, phase-2 line mapping, and
+the trace and flux-slot passes of the output-layout kernel) for every compiled
+order bin and part count, and checks the properties the kernels rely on: every
+DOF, trace slot and line is visited exactly once, every LDS index stays inside
+its tile, and lanes walking a cell's DOFs in order hit distinct LDS banks (32
+banks of 4 bytes; 8-byte elements).
 """
 import pytest
 
 BINS = [(5, 5, 16), (4, 4, 16), (4, 4, 4), (3, 3, 8), (5, 5, 8), (4, 4, 8), (3, 3, 4)]
+
+
+# static LDS of k_uniform, 5 x 5 x 80 (hipcc resource report), by element size
+STATIC = {8: 3216, 4: 1888}
 
 
 def u_threads(nth, nc, h):
@@ -43,8 +47,9 @@ def test_passes_cover_each_index_once(n, nth, nc, h):
     noa = oc * nth
     nap, noap = u_pad(na, nth), u_pad(noa, nth)
     assert nap >= na and noap >= noa and nap % 2 == 1 and noap % 2 == 1
-    cpp = ut // cd if cd <= ut else 0
-    xs_ = cpp * cd if cpp else ut
+    assert cd <= ut                   # a cell fits the workgroup
+    cpp = ut // cd
+    xs_ = cpp * cd
     xu = (ncd + xs_ - 1) // xs_
     # phase 1: column DOFs t = t0 + u XS, t0 = tid (tid < XS) else NCD
     seen, lds = [], set()
@@ -54,8 +59,7 @@ def test_passes_cover_each_index_once(n, nth, nc, h):
             t = t0 + u * xs_
             if t >= ncd:
                 continue
-            kk = t0 // cd + u * cpp if cpp else t // cd
-            lt = t0 % cd if cpp else t % cd
+            kk, lt = t0 // cd + u * cpp, t0 % cd
             assert kk * cd + lt == t
             sn, a = lt // nth, lt % nth
             li = sn * nap + kk * nth + a
@@ -63,34 +67,18 @@ def test_passes_cover_each_index_once(n, nth, nc, h):
             seen.append(t)
             lds.add(li)
     assert sorted(seen) == list(range(ncd)) and len(lds) == ncd
-    # phase 5: own DOFs (kl, lt) of the part, kl = tid / CD + k CPP
+    # phase 4: own DOFs (kl, lt) of the part, kl = tid / CD + u CPP, and the
+    # neighbours' values loaded for them before
+    yu = (oc + cpp - 1) // cpp
     own = []
-    for tid in range(ut):
-        if cpp:
-            if tid >= xs_:
-                continue
-            lt = tid % cd
-            kl = tid // cd
-            while kl < oc:
+    for tid in range(xs_):
+        lt = tid % cd
+        for u in range(yu):
+            kl = tid // cd + u * cpp
+            if kl < oc:
                 own.append(kl * cd + lt)
                 assert (lt // nth) * noap + kl * nth + lt % nth < nsp * noap
-                kl += cpp
-        else:
-            own.extend(range(tid, oc * cd, ut))
     assert sorted(own) == list(range(oc * cd))
-    # traces and flux slots: (link li, slot le), li = tid / TRL + u LPP
-    trl, maxl = n * nth, 4 * oc
-    lpp = ut // trl
-    ts = lpp * trl
-    tu = (maxl * trl + ts - 1) // ts
-    slots = []
-    for tid in range(ut):
-        e0 = tid if tid < ts else maxl * trl
-        for u in range(tu):
-            li = e0 // trl + u * lpp
-            if li < maxl:
-                slots.append(li * trl + e0 % trl)
-    assert sorted(slots) == list(range(maxl * trl))
     # phase-2 lines (q or p, part angle)
     nline = oc * n * nth
     lines = sorted((e // noa, e % noa) for e in range(nline))
@@ -117,16 +105,36 @@ def test_cell_walk_hits_distinct_banks(n, nth, nc):
 
 
 @pytest.mark.parametrize("n,nth,nc,h", CASES)
-def test_lds_fits_three_workgroups_for_the_c2_bin(n, nth, nc, h):
-    """Dynamic LDS of an FP64 launch at the largest link count a part may
-    have (4 per cell), plus about 4.2 KB of static arrays."""
+def test_inflow_reads_the_neighbours_face(n, nth, nc, h):
+    """The direct inflow: a neighbour of the same shape has its first face node
+    at (N - 1) N (through face 2), N - 1 (face 3) or 0 (faces 0, 1); node je of
+    an x-face lies je rows of NTH values further, node ie of a y-face ie rows
+    of N NTH, and all stay inside the neighbour's cell on its opposite face."""
+    cd = n * n * nth
+    for F, first in ((0, 0), (1, 0), (2, (n - 1) * n), (3, n - 1)):
+        for node in range(n):
+            for a in range(nth):
+                at = first * nth + node * (n * nth if F & 1 else nth) + a
+                assert 0 <= at < cd
+                i, j = at // nth // n, at // nth % n
+                assert at % nth == a
+                assert (i, j) == {0: (0, node), 1: (node, 0), 2: (n - 1, node), 3: (node, n - 1)}[F]
+
+
+@pytest.mark.parametrize("n,nth,nc,h", CASES)
+def test_lds_of_the_line_pass_kernel(n, nth, nc, h):
+    """Dynamic LDS of a launch (column and output rows, and the BF16 column in
+    mixed precision) plus its static arrays; three workgroups per CU in FP64
+    and four in FP32 and mixed for columns of 5 x 5 x 80."""
     nsp, na, oc = n * n, nc * nth, nc // h
-    lds = (nsp * u_pad(na, nth) + nsp * u_pad(oc * nth, nth) + 2 * 4 * oc * n * nth) * 8 + 4400
-    assert lds <= 160 * 1024
-    if (n, nth, nc, h) == (5, 5, 16, 1):
-        # the C2 bin has at most 2 links per cell: 3 workgroups per CU
-        lds2 = (nsp * u_pad(na, nth) * 2 + 2 * 2 * oc * n * nth) * 8 + 4400
-        assert 3 * lds2 <= 160 * 1024
+    rows = nsp * u_pad(na, nth) + nsp * u_pad(oc * nth, nth)
+    bf16 = (nsp + 15) // 16 * 16 * ((na + 15) // 16 * 16 + 4) * 2 + 16
+    for size, extra, static, wgs in ((8, 0, STATIC[8], 3), (4, 0, STATIC[4], 4),
+                                     (4, bf16, STATIC[4], 4)):
+        lds = rows * size + extra + static
+        assert lds <= 160 * 1024
+        if (n, nth, nc, h) == (5, 5, 16, 1):
+            assert wgs * lds <= 160 * 1024
 
 
 @pytest.mark.parametrize("n,nth,nc", BINS)
@@ -199,8 +207,19 @@ def test_output_layout_kernel_indices(n, nth, nc):
                             assert 0 <= (p * n + i) * nap + R < nsp * nap
                         staged.append(kk * cd + s * nth + r)
         assert sorted(staged) == list(range(ncd))
+    # traces and flux slots: (link li, slot le), li = e0 / TRL + u LPP
+    trl, maxl, ut = n * nth, 4 * nc, 64 * waves
+    lpp = ut // trl
+    ts = lpp * trl
+    tu = (maxl * trl + ts - 1) // ts
+    slots = []
+    for tid in range(ut):
+        e0 = tid if tid < ts else maxl * trl
+        slots += [(e0 // trl + u * lpp) * trl + e0 % trl for u in range(tu)
+                  if e0 // trl + u * lpp < maxl]
+    assert sorted(slots) == list(range(maxl * trl))
     if (n, nth, nc) == (5, 5, 16):
-        trl, links = n * nth, 2 * nc
+        links = 2 * nc
         dyn = nsp * nap * 8 + 2 * links * trl * 8
         static = 4112                    # the FP64 instance's static LDS (hipcc resource report)
         assert 4 * (dyn + static) <= 160 * 1024
