@@ -30,9 +30,10 @@
 // lane's accumulators are whole lines of nodes (x-lines q = lane group,
 // lane group + 4, ..), so the derivative along x reads a line once for all of
 // its outputs, with the derivative matrix in scalar registers, and the
-// derivative along y reads each row of nodes once per line.  That is about 6
-// LDS reads per output; evaluated output by output it was about 30, and the
-// LDS pipe was what bounded the column.
+// derivative along y reads each row of nodes once per line.  On an hp mesh of
+// 8.3 M DOF that is 28 LDS instructions per 64 outputs in FP64 and 21 in mixed
+// precision; evaluated output by output, with the face coupling in LDS, it was
+// 71 and 70, and the LDS pipe was what bounded the column.
 //
 // Every output has one owner and a fixed order of additions, so results are
 // bit-reproducible; x is read from HBM once (plus the neighbours' face
@@ -309,8 +310,8 @@ __device__ inline int hp_node(int t, int i, int l0, int ny) {
 // FP64, N = 6, 88 angles, two workgroups per CU, cycles: tables and first G
 // rows 7,900, x to LDS 4,200, a wavefront's 16 angles 9,700 (matrix) + 6,600
 // (lines), those of the second round 15,100.  Times of the two kernels
-// together, against one kernel with the contraction's operands in LDS and 30
-// LDS reads per output: hp mesh of 34,279 cells FP64 283 -> 226 us, 9,150
+// together, against one kernel with the contraction's operands in LDS that
+// evaluated output by output: hp mesh of 34,279 cells FP64 283 -> 226 us, 9,150
 // cells mixed 87 -> 45 us, 1,024 columns of 7 x 7 nodes FP32 52 -> 35 us (29
 // with alike neighbours read directly).
 //
