@@ -23,7 +23,8 @@
 //              values of x times the (then diagonal) coupling; stores y.
 //
 // The two share no workspace: y itself carries the face sums from one to the
-// other.  The plan's side stream and its two events are shared by all applies, so
+// other (with accumulation a node that has some is therefore rounded twice, in
+// FP32 up to 1.5 times the error of one rounding).  The plan's side stream and its two events are shared by all applies, so
 // a plan serves one stream at a time.
 //
 // The nodes are the rows of the scattering product in an order of our own: a
@@ -249,14 +250,14 @@ __host__ __device__ inline int hp_stride(int na, int kstep, int c, int M) {
 }
 
 struct HpLayout {           // dynamic LDS of one column, in bytes from the base
-    int xs, xb, ct, sn, wr, dth, pk, fl, src, total;
+    int xs, xb, vo, cx, cy, pk, fl, src, total;
     int S, NA, XSB;         // angle-major row (node) stride, padded angle rows, BF16 stride
 };
 
 // Angle-major copy: NA rows (the column's angles, padded to the K step with
 // zero rows) of S = nsp rounded up to odd entries, so that lanes on
 // consecutive angles or nodes read distinct banks; mixed adds the node-major
-// BF16 copy.  Then four values and two words per angle, and two more where
+// BF16 copy.  Then three values and two words per angle, and two more where
 // alike neighbours are read directly.  A: LDS element type.
 template <typename A, int PREC>
 __host__ __device__ inline HpLayout hp_layout(int nsp, int na, bool alike) {
@@ -273,13 +274,11 @@ __host__ __device__ inline HpLayout hp_layout(int nsp, int na, bool alike) {
     L.xb = o;
     o += nsp * L.XSB * 2;
     o = (o + 15) & ~15;
-    L.ct = o;
+    L.vo = o;
     o += na * ea;
-    L.sn = o;
+    L.cx = o;
     o += na * ea;
-    L.wr = o;
-    o += na * ea;
-    L.dth = o;
+    L.cy = o;
     o += na * ea;
     L.pk = o;
     o += na * 4;
@@ -354,10 +353,9 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     const int S = Lo.S, XSB = Lo.XSB;
     A *xs = reinterpret_cast<A *>(lds + Lo.xs);
     uint16_t *xb = reinterpret_cast<uint16_t *>(lds + Lo.xb);
-    A *ct = reinterpret_cast<A *>(lds + Lo.ct);
-    A *sn = reinterpret_cast<A *>(lds + Lo.sn);
-    A *wr = reinterpret_cast<A *>(lds + Lo.wr);
-    A *dt = reinterpret_cast<A *>(lds + Lo.dth);
+    A *vo = reinterpret_cast<A *>(lds + Lo.vo);
+    A *fcx = reinterpret_cast<A *>(lds + Lo.cx);
+    A *fcy = reinterpret_cast<A *>(lds + Lo.cy);
     int *pk = reinterpret_cast<int *>(lds + Lo.pk);
     int *fl = reinterpret_cast<int *>(lds + Lo.fl);
     int2 *sr = reinterpret_cast<int2 *>(lds + Lo.src);
@@ -399,11 +397,12 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
         const int t = tid + u * HP_THREADS;
         vv[u] = (t < ncd) ? A(x[cdof + t]) : A(0);
     }
+    // per angle the mass factor and the fluxes along x and y, rounded once
     for (int a = tid; a < na; a += HP_THREADS) {
-        ct[a] = A(m.ang_trig[3 * (ga0 + a)]);
-        sn[a] = A(m.ang_trig[3 * (ga0 + a) + 1]);
-        wr[a] = A(m.ang_trig[3 * (ga0 + a) + 2]);
-        dt[a] = A(h.ang_dth[ga0 + a]);
+        const double w = h.ang_dth[ga0 + a] * m.ang_trig[3 * (ga0 + a) + 2];
+        vo[a] = A(dx * dy * 0.125 * w);
+        fcx[a] = A(dy * 0.25 * w * m.ang_trig[3 * (ga0 + a)]);
+        fcy[a] = A(dx * 0.25 * w * m.ang_trig[3 * (ga0 + a) + 1]);
         pk[a] = m.ang_pack[ga0 + a];
         fl[a] = h.ang_flag[ga0 + a];
         if constexpr (ALIKE) sr[a] = h.ang_src[ga0 + a];
@@ -504,18 +503,15 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
         const int w = pk[R], nt = (w >> 20) & 31, f = fl[R];
         const int bd = restrict_ ? (f & 15) : 0, quad = ((f >> 4) & 7) - 1;
         const int lf = bconv ? (f >> 8) & 15 : 0;
-        const A dth = dt[R], cR = ct[R], sR = sn[R], w_r = wr[R];
-        const A vol = (ops & RTX_OP_MASS) ? A(dx * dy * 0.125) * dth * w_r : A(0);
-        const A ic = (ops & RTX_OP_ICONV) ? A(1) : A(0);
-        const A cx = ic * A(dy * 0.25) * dth * w_r * cR, cy = ic * A(dx * 0.25) * dth * w_r * sR;
+        const A vol = (ops & RTX_OP_MASS) ? vo[R] : A(0), gx = fcx[R], gy = fcy[R];
+        const A cx = (ops & RTX_OP_ICONV) ? gx : A(0), cy = (ops & RTX_OP_ICONV) ? gy : A(0);
         // outflow factors of the faces +x, +y, -x, -y (quadrant Q flows out of
         // faces Q and Q + 1)
-        const A fx = A(dy * 0.25) * dth, fy = A(dx * 0.25) * dth;
         const bool ob = bconv && quad >= 0;
-        const A ox1 = ob && (quad == 0 || quad == 3) ? fx * w_r * cR : A(0);
-        const A ox0 = ob && (quad == 1 || quad == 2) ? -fx * w_r * cR : A(0);
-        const A oy1 = ob && quad < 2 ? fy * w_r * sR : A(0);
-        const A oy0 = ob && quad >= 2 ? -fy * w_r * sR : A(0);
+        const A ox1 = ob && (quad == 0 || quad == 3) ? gx : A(0);
+        const A ox0 = ob && (quad == 1 || quad == 2) ? -gx : A(0);
+        const A oy1 = ob && quad < 2 ? gy : A(0);
+        const A oy0 = ob && quad >= 2 ? -gy : A(0);
         // ALIKE: inflow from alike neighbours: the outflow factors of the
         // opposite faces, and the neighbours' first face nodes (-1: none)
         int2 src = make_int2(-1, -1);

@@ -62,11 +62,13 @@ constexpr int u_pad(int na, int nth) {
 // columns have the same nodes and angles there, so the coupling matrices
 // E^s and E^theta are diagonal (weights, weights x direction) and the flux at
 // a node is the outflow term's product with the neighbour's value and the
-// opposite direction: no traces to stage, no contraction.  tf: the direction
-// factor of the outflow face opposite.
+// opposite direction: no traces to stage, no contraction.  flux: side / 4 x
+// width x angle weight x direction of the axis (rounded once, from FP64: in
+// FP32 the error of the coupling is then below that of the contraction); high:
+// the outflow face opposite lies at the axis' upper end; w: node weight.
 template <typename A>
-__device__ inline A u_inflow(A len4, A dth, A w, A wr, A tf, A xn) {
-    return -(len4 * dth * w * wr * tf) * xn;
+__device__ inline A u_inflow(A flux, bool high, A w, A xn) {
+    return (high ? -flux : flux) * w * xn;
 }
 
 // Outflow faces quad and quad + 1 of a cell: the x-face (F even), the y-face,
@@ -140,6 +142,7 @@ void k_uniform(DevMesh m, uint32_t ops, int accumulate, const int4 *__restrict__
     constexpr size_t XB_OFF = u_bf_off(size_t(NSP * NAP + NSP * NOAP) * sizeof(A));
     uint16_t *xb = reinterpret_cast<uint16_t *>(u_lds + XB_OFF);
     __shared__ A cth[NA], sth[NA], cw[NA];
+    __shared__ A flx[NA], fly[NA];             // x- and y-flux of each angle (u_inflow)
     __shared__ A kap[NSP], sgw[NSP];
     __shared__ A wx_[N], WD[N * N];
     __shared__ A dth_[NC];
@@ -214,13 +217,15 @@ void k_uniform(DevMesh m, uint32_t ops, int accumulate, const int4 *__restrict__
         const int t = t0 + u * XS;
         xv[u] = (t < NCD) ? A(x[cdof + t]) : A(0);
     }
-    double r_c = 0, r_s = 0, r_w = 0, r_kap = 0, r_sig = 0, r_wd = 0, r_g = 0;
+    double r_c = 0, r_s = 0, r_w = 0, r_ag = 0, r_kap = 0, r_sig = 0, r_wd = 0, r_g = 0;
     int r_bd = 0, r_q = -1;
     int4 r_nbr = make_int4(-1, -1, 0, 0);
     if (tid < NA) {
         r_c = m.ang_trig[3 * (ga0 + tid)];
         r_s = m.ang_trig[3 * (ga0 + tid) + 1];
         r_w = m.ang_trig[3 * (ga0 + tid) + 2];
+        const int k = k0 + tid / NTH;
+        r_ag = m.cell_geom[2 * k + 1] - m.cell_geom[2 * k];
     }
     if (tid < NSP) {
         r_kap = m.kappa[c * NSP + tid];
@@ -241,6 +246,8 @@ void k_uniform(DevMesh m, uint32_t ops, int accumulate, const int4 *__restrict__
         cth[tid] = A(r_c);
         sth[tid] = A(r_s);
         cw[tid] = A(r_w);
+        flx[tid] = A(dy * 0.25 * r_ag * r_w * r_c);
+        fly[tid] = A(dx * 0.25 * r_ag * r_w * r_s);
     }
     if (tid < NSP) {
         kap[tid] = A(r_kap);
@@ -480,11 +487,8 @@ void k_uniform(DevMesh m, uint32_t ops, int accumulate, const int4 *__restrict__
         A v = ys[sne * NOAP + kl * NTH + ae];
         if (bconv) {
             const UFaces f(cqd[kk]);
-            const A xtf = f.Fx == 0 ? cth[ca] : -cth[ca], ytf = f.Fy == 1 ? sth[ca] : -sth[ca];
-            if (ie == (f.Fx == 0 ? 0 : N - 1))
-                v += u_inflow(A(dy * 0.25), dth_[kk], wx_[je], cw[ca], xtf, xi[u]);
-            if (je == (f.Fy == 1 ? 0 : N - 1))
-                v += u_inflow(A(dx * 0.25), dth_[kk], wx_[ie], cw[ca], ytf, yi[u]);
+            if (ie == (f.Fx == 0 ? 0 : N - 1)) v += u_inflow(flx[ca], f.Fx == 0, wx_[je], xi[u]);
+            if (je == (f.Fy == 1 ? 0 : N - 1)) v += u_inflow(fly[ca], f.Fy == 1, wx_[ie], yi[u]);
         }
         if (masked) v = A(0);
         if (accumulate) {

@@ -622,3 +622,64 @@ def test_default_path_of_long_columns(cuda, n, nref_spt, expect):
             else:
                 assert not torch.equal(out[-1], out[0]) and not torch.equal(out[-1], out[3])
             assert float((out[-1] - out[0]).norm() / out[0].norm()) < tol
+
+
+def contraction_fp32(t, x):
+    """The face coupling and outflow terms in FP32 by contraction with E^theta
+    and E^s, factors rounded one by one (numpy)."""
+    f = np.float32
+    y = np.zeros(t.ndof, f)
+    x = x.astype(f)
+
+    def face(k, F, own):
+        c = int(t.cell_col[k])
+        nx, ny, nt = int(t.col_nx[c]), int(t.col_ny[c]), int(t.cell_nth[k])
+        at = np.arange(nx * ny * nt).reshape(nx, ny, nt) + int(t.cell_dof_off[k])
+        end = -1 if (F in (0, 1)) == own else 0
+        return at[end] if F % 2 == 0 else at[:, end]
+    for k in range(t.ncell):
+        c, quad, nt = int(t.cell_col[k]), int(t.cell_quad[k]), int(t.cell_nth[k])
+        side = (t.col_geom[c, 3] - t.col_geom[c, 1], t.col_geom[c, 2] - t.col_geom[c, 0])
+        dth = f(t.cell_geom[k, 1] - t.cell_geom[k, 0])
+        a0 = int(t.col_ang_start[c]) + int(t.cell_ang_off[k])
+        trig = t.ang_trig[3 * a0:3 * (a0 + nt)].reshape(nt, 3).astype(f)
+        for F in (quad, (quad + 1) % 4):
+            at = face(k, F, True)
+            n = at.shape[0]
+            w = t.lgl_w[10 * n:10 * n + n].astype(f)
+            tf = trig[:, F % 2] * f(1 if F < 2 else -1)
+            y[at] += f(side[F % 2] * 0.25) * dth * w[:, None] * trig[:, 2] * tf * x[at]
+        for l in range(int(t.link_start[k]), int(t.link_start[k + 1])):
+            s, F = int(t.link_src[l]), int(t.link_face[l])
+            own, other = face(k, F, True), face(s, F, False)
+            es, et = int(t.link_Es_off[l]), int(t.link_Eth_off[l])
+            Es = t.Es_pool[es:es + len(other) * len(own)].reshape(len(other), -1).astype(f)
+            Et = t.Eth_pool[et:et + int(t.cell_nth[s]) * nt].reshape(-1, nt).astype(f)
+            y[own] += f(side[F % 2] * 0.25) * dth * (Es.T @ (x[other] @ Et))
+    return y
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nref_ang", [((3, 3, 4), 4), ((6, 6, 6), 3), ((10, 10, 5), 3),
+                                        ((5, 5, 5), 4), ((4, 4, 4), 2), ((3, 3, 3), 3)], ids=str)
+def test_fp32_face_coupling_error(cuda, n, nref_ang):
+    """Neighbours read directly (column kernel and uniform line-pass kernel):
+    the FP32 error of the face terms against FP64 is no larger than that of
+    the contraction with E^theta and E^s in FP32 that it replaces.  The factors of
+    a term are constants of the mesh, so their roundings do not average out, and
+    the fewer there are the better: from FP64 one, the weight's and the
+    products', against two matrix entries, the side, the width and theirs.  10 %
+    are allowed for the luck of single constants."""
+    from rtx.operator import TransportOperator, OP_BCONV, PREC_F32
+    mesh = problems.uniform_mesh([1.0, 1.0], list(n), nref_ang, 3)
+    wl = problems.two_scatterers()
+    op = TransportOperator(mesh, wl.kappa, wl.sigma, wl.Phi)
+    x = np.random.default_rng(2).uniform(-1, 1, op.ndof).astype(np.float32)
+    op.set_path(0)
+    ref = op.apply(_dev(x.astype(np.float64)), ops=OP_BCONV).cpu().numpy()
+    op.set_path(-1)
+    err = _rel(op.apply(_dev(x), ops=OP_BCONV, precision=PREC_F32).cpu().double().numpy(), ref)
+    old = _rel(contraction_fp32(op.t, x).astype(np.float64), ref)
+    print("FP32 face terms", n, "uniform", op.plan_info()["uniform"], "error", err,
+          "contraction", old, flush=True)
+    assert err <= 1.1 * old

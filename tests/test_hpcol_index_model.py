@@ -48,7 +48,7 @@ def hp_layout(nsp, na, prec, alike):
     XSB = hp_stride(na, 16, 8, 16) if prec == "mixed" else 0
     o = (NA * S * ea + 15) & ~15
     o = (o + nsp * XSB * 2 + 15) & ~15
-    o += 4 * na * ea + 2 * na * 4
+    o += 3 * na * ea + 2 * na * 4
     o = ((o + 7) & ~7) + (8 * na if alike else 0)
     return S, NA, XSB, (o + 15) & ~15
 

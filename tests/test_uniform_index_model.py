@@ -14,7 +14,7 @@ BINS = [(5, 5, 16), (4, 4, 16), (4, 4, 4), (3, 3, 8), (5, 5, 8), (4, 4, 8), (3, 
 
 
 # static LDS of k_uniform, 5 x 5 x 80 (hipcc resource report), by element size
-STATIC = {8: 3216, 4: 1888}
+STATIC = {8: 4496, 4: 2528}
 
 
 def u_threads(nth, nc, h):
