@@ -334,7 +334,7 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     // x-lines: NL per lane group, LI of them in one item (16 output angles x
     // 4 LI lines).  FP64 takes one: with all of them its accumulators leave
     // too few of the 128 registers of 4 wavefronts per SIMD for the lines
-    // (252 spilled, against 24), and two or three times the items spread
+    // (252 spilled, against 2), and two or three times the items spread
     // better over the wavefronts; G is then read from L2 once per item.
     constexpr int NL = (N + 3) / 4;
     constexpr int LI = sizeof(A) == 8 || RECT ? 1 : NL;
