@@ -362,10 +362,10 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
 
     // ---- the first G rows of this wavefront's first 16 output angles, in
     // flight through the staging phases.  PD load groups of four K steps (one
-    // of 16 in mixed precision); lanes past the last angle, and rows past it,
-    // read valid addresses: those angle rows of the copy are zero, and those
-    // lanes' outputs are not stored.
-    constexpr int PD = PREC == RTX_PREC_F32 && N <= 7 ? 4 : 2;
+    // of 16 in mixed precision; four groups in FP32 are 1 to 2 % slower); lanes
+    // past the last angle, and rows past it, read valid addresses: those angle
+    // rows of the copy are zero, and those lanes' outputs are not stored.
+    constexpr int PD = 2;
     typedef typename std::conditional<PREC == RTX_PREC_MIXED, uint16_t, A>::type GT;
     const GT *Gc = PREC == RTX_PREC_MIXED ? (const GT *)(m.G_bf16 + m.col_G_off[c])
                    : PREC == RTX_PREC_F64 ? (const GT *)(m.G + m.col_G_off[c])
@@ -389,7 +389,9 @@ __device__ __forceinline__ void hp_column(const DevMesh &m, const HpTables &h, u
     }
     // ---- x of the column and its tables.  The first batch of x is loaded
     // while the angles' tables go to LDS.
-    // x values per thread and pass: a column of 96 angles in one
+    // x values per thread and pass: a column of 96 angles in one (for 48 angles
+    // the FP64 hp mesh of 2.0 M DOF takes 93.5 us against 90, for 160 its and
+    // the 7 x 7 columns 2 to 5 % more)
     constexpr int XM = (N * N * 96 + HP_THREADS - 1) / HP_THREADS, XU = RECT || XM > 16 ? 16 : XM;
     A vv[XU];
 #pragma unroll
