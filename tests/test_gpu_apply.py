@@ -213,8 +213,8 @@ def test_apply_c3_rows_and_linearity(cuda, path):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,nref_ang,nref_spt", [(5, 4, 3), (4, 2, 2)], ids=["p4", "p3"])
 def test_uniform_apply_bit_reproducible(cuda, n, nref_ang, nref_spt):
-    """The uniform kernel adds every output in a fixed order (face fluxes
-    staged, no atomics): repeated FP64 and mixed applies are bit-identical, and
+    """The uniform kernel adds every output in a fixed order (one thread per
+    output, no atomics): repeated FP64 and mixed applies are bit-identical, and
     so are the FP64 applies of every valid part count (the per-DOF arithmetic
     does not depend on how a column is split)."""
     import torch
@@ -253,8 +253,9 @@ def test_uniform_apply_bit_reproducible(cuda, n, nref_ang, nref_spt):
 def test_uniform_output_layout_kernel(cuda, n, nref_ang, nref_spt):
     """The default FP64 uniform kernel (every term of an output added where
     the scattering MFMA leaves it) against the line-pass kernel (one part per
-    column) on compiled shapes: the same operations in the same order, so the
-    results agree to the last bits (1e-15 relative; equality is reported);
+    column) on compiled shapes: the same terms in the same order, but the inflow
+    contracted from the neighbours' traces in one and read directly in the other,
+    so the results agree to rounding (1e-15 relative; equality is reported);
     both match the oracle at 1e-12; repeated applies are bit-identical, also
     into a y that is only 8-byte aligned (element-wise write-back instead of
     16-byte copies); accumulate mode adds exactly.  FP32 and mixed default to
